@@ -1,43 +1,56 @@
-// NT-GEMM workgroup tile for gfx950 (CDNA4): C^[BM x BN] = A[BM x K] * B[BN x K]^T,
+// NT-GEMM workgroup tile for gfx950 (CDNA4): C^[256 x 256] = A[256 x K] * B[256 x K]^T,
 // both operands K-contiguous in memory, fp32 accumulation on the matrix cores.
 //
-// One workgroup of WAVES_M x WAVES_N wavefronts (64 lanes each) owns a BM x BN
-// tile.  K is walked in slabs of 128 bytes per row (64 bf16 or 32 fp32
-// elements).  A slab of A (BM rows) and of B (BN rows) travels HBM/L2 -> LDS
-// directly (buffer loads with an LDS destination; no registers, no LDS store
-// instructions).  Such a load fills LDS in lane order, so rows are 128 bytes
-// apart with no padding; bank conflicts are avoided by an XOR swizzle of the
-// 16-byte K-chunks within a row, applied on the global side of the load and
-// undone by the fragment reads.  Two LDS stages: while the matrix cores work on
-// stage s, the next slab lands in stage s^1; one workgroup barrier per slab,
-// placed before the last K-step so that step's matrix instructions cover the
-// first fragment reads of the next slab; that barrier is preceded by an
-// explicit wait for the wave's outstanding loads, because a barrier alone does
-// not wait for loads whose destination is LDS.
+// One workgroup of 2 x 2 wavefronts (64 lanes each, one per SIMD of a CU) owns a 256 x 256 tile; a wave
+// owns 128 x 128 of it as 8 x 8 blocks of 16 x 16.  K is walked in slabs of 128 bytes per row (64 bf16 or 32
+// fp32 elements), each slab in two halves of 64 bytes.
 //
-// Operands are either row-major (the caller's hidden states and weight) or
-// K-blocked (the library's own intermediates: per tile and slab one contiguous
-// 32 KB piece, see Operand).  Consecutive K loops of a workgroup that keep the
-// same B rows can stream into each other: the last two slab periods of one loop
-// already request the first two slabs of the next (see Stream).
+// What bounds it: on random operands the chip runs at its power limit (the shader clock settles at 1.5 -
+// 1.6 GHz), so the rate is what is left after data movement and idle issue slots have taken their energy.
+//  - 128 x 128 per wave reads 16 fragments per 64 matrix instructions; the 128 x 64 of eight waves read 12 per 32.
+//  - v_mfma 16x16x32 against 32x32x16 on the same operands: 2 % more rate out of registers (1870 against 1827
+//    TFLOP/s), 6 % in this loop.
+//  - every instruction's place is fixed in the source: a fragment read of the next half after every second
+//    matrix instruction, an operand load after every eighth (more often and the loads back up behind the
+//    vector memory path, which takes a wave's kilobyte per 16 cycles, and the wave with them), scalar address
+//    work one piece at a time in between.  With one wave per SIMD nothing else would fill a gap.
+// Measured on operands of M = 4096, N = 12288, K = 32768 (bf16): 1493 TFLOP/s row-major, 1505 K-blocked; the
+// eight-wave 32x32x16 form of this tile with two 64 KB stages ran 1310.
 //
-// Accumulator layout (v_mfma_f32_32x32x*): for the 32x32 block (mi, ni) of a
-// wave, lane l, register r hold
-//     row (A index) = mi*32 + 8*(r/4) + 4*(l/32) + (r%4)
-//     col (B index) = ni*32 + (l%32)
-// so a lane owns ONE B row per ni and 16 A rows per (mi, ni).  The callers put
-// the dimension they reduce over (vocabulary, for the softmax statistics) on A,
-// which makes that reduction mostly lane-local.
+// Operand slabs travel HBM/L2 -> LDS directly (buffer loads with an LDS destination; no registers, no LDS
+// store instructions) into two rings of 32 KB slots, three for A and two for B: all 160 KB.  While the matrix
+// cores work on slab s, B(s+1) and A(s+1), A(s+2) land; a slot is requested again right after the barrier
+// behind its last fragment read.  The third A slot is what makes the loads of a slab early enough: with two
+// 64 KB stages (same loop) the row-major rate is 1398.  One barrier per slab, preceded by an explicit
+// wait for this wave's own loads, because a barrier alone does not wait for loads whose destination is LDS; the
+// youngest eight (the A slab after next) stay outstanding.
+//
+// A load fills LDS in lane order, so rows are 128 bytes apart with no padding; bank conflicts are
+// avoided by an XOR swizzle of the 16-byte K-chunks within a row, applied on the global side of the load and
+// undone by the fragment reads (0 conflict cycles).
+//
+// Operands are either row-major (the caller's hidden states and weight) or K-blocked (the library's own
+// intermediates: per tile and slab one contiguous 32 KB piece, see Operand).  Consecutive tiles of a
+// workgroup stream into each other: requests that run past a tile's last slab continue with the next
+// tile's first ones, whose first fragments are in registers when the tile ends.
+//
+// Accumulators (v_mfma_f32_16x16x*): lane l = 16 g + c holds, in register r of block (i, j), the product of
+//     A row a_row(i, 4 g + r)   and   B row b_row(j, c).
+// Which rows of the wave's 128 make up a block is free, because it only decides where a fragment is read
+// from.  a_row gives a lane VEC = 16 / sizeof(T) consecutive A rows (bf16: over a pair of blocks), b_row BV
+// consecutive B rows over BV blocks, so that 16-byte pieces of either orientation of the result are in one
+// lane and leave without a shuffle.  The callers put the dimension they reduce over (vocabulary, for the
+// softmax statistics) on A, which makes that reduction mostly lane-local.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <utility>
 
 namespace clgrpo {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kRowBytes = 128;    // K-slab bytes per tile row
 constexpr int kChunksPerRow = 8;  // 16-byte chunks per slab row
@@ -55,90 +68,97 @@ __host__ __device__ __forceinline__ int64_t blocked_index(int64_t row, int64_t k
   return (((row / kBlockRows) * n_kslab + k / E) * kBlockRows + (row % kBlockRows)) * E + (k % E);
 }
 
-// Kept logits ("z-native" layout).  The forward leaves a chunk's raw logits for the backward in the
-// order its accumulators hold them, so that storing them costs no shuffle: the buffer is cut into the
-// same 32 KB units as a K-blocked operand (256 rows x one 128-byte K slab of vocabulary, unit (rb, ks) at
-// byte (rb * n_kslab + ks) * 32768), and inside a unit into sub-blocks of 32 rows x 32 vocabulary entries,
-// sub-block (rs, vs) at (rs * VSUB + vs) * PIECES KB.  A sub-block is one 32x32 accumulator block: lane
-// (h, t32) = (lane / 32, lane % 32) owns row t32 and the 16 entries 8 * (r / 4) + 4 * h + r % 4, r = 0..15,
-// which it stores as PIECES 16-byte pieces; piece j of all 64 lanes is one contiguous KB.  The kernel that
-// turns logits into d(logits) reads a unit whole and writes the K-blocked result over it.
-// 16-bit inputs keep their logits as IEEE half (10 mantissa bits against bf16's 7: the softmax the
-// backward rebuilds from them is 8x closer to the fp32 one), fp32 inputs as fp32.
+// Kept logits: the forward leaves a chunk's raw logits for the backward in the K-blocked layout (rows =
+// tokens, K = vocabulary) that the d(logits) operand will have, so that the kernel that turns one into the
+// other works in place.  16-bit inputs keep their logits as IEEE half (10 mantissa bits against bf16's 7: the
+// softmax the backward rebuilds from them is 8x closer to the fp32 one), fp32 inputs as fp32.
 template <typename T> struct KeptLogit;
 template <> struct KeptLogit<__bf16> { typedef _Float16 type; };
 template <> struct KeptLogit<float> { typedef float type; };
 
-template <typename T> struct ZNative {
-  static constexpr int ES = (int)sizeof(T);
-  static constexpr int kSlabElems = kRowBytes / ES;     // vocabulary entries per unit
-  static constexpr int VSUB = kSlabElems / 32;          // sub-blocks along the vocabulary per unit
-  static constexpr int PIECES = ES;                     // 16-byte pieces per lane and sub-block (16 values)
-  static constexpr int kPerPiece = 16 / PIECES;         // values per piece
-  static constexpr int kUnitBytes = kBlockRows * kRowBytes;
-  // byte offset of piece j of lane half h for `row` and the 32-aligned vocabulary block `v32` (= vocab / 32)
-  __host__ __device__ static __forceinline__ int64_t piece_offset(int64_t row, int64_t v32, int64_t n_kslab, int h, int j) {
-    const int64_t rb = row / kBlockRows;
-    const int R = (int)(row % kBlockRows);
-    const int64_t unit = (rb * n_kslab + v32 / VSUB) * kUnitBytes;
-    const int sb = (R >> 5) * VSUB + (int)(v32 % VSUB);
-    return unit + (int64_t)sb * (PIECES * 1024) + j * 1024 + (h * 32 + (R & 31)) * 16;
+// Matrix instructions of slot m (0 .. 63) of a slab half: 64 bytes of K of block (i, j) = (m / 8, m % 8), odd
+// rows walked backwards so that neighbours share an operand.  Written as assembly because that is what ties the
+// accumulators to the accumulation registers: left to itself the compiler moves all 256 of them between the
+// register files around every loop, and spills what is in their way.  The compiler does not see the
+// instruction's latency either: see settle().  Everything else that touches an accumulator goes through
+// acc_get / acc_set for the same reason.
+template <typename T> struct Mma;
+template <> struct Mma<__bf16> {
+  __device__ static __forceinline__ void slot(f32x4 (&acc)[8][8], const u32x4 (&a)[8], const u32x4 (&b)[8], int m) {
+    const int i = m / 8, j = (i & 1) ? 7 - m % 8 : m % 8;
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(a[i]), "v"(b[j]));
   }
-  // vocabulary offset inside its 32-block of value e of piece j for lane half h
-  __host__ __device__ static __forceinline__ int col_of(int h, int j, int e) {
-    const int r = j * kPerPiece + e;
-    return 8 * (r >> 2) + 4 * h + (r & 3);
+};
+template <> struct Mma<float> {
+  // 16 bytes hold four K=4 steps: lane group g, element e stands for k = 4g + e in both operands.  A slot takes
+  // step m % 8 / 2 of four blocks of row i, so that an accumulator comes up again eight instructions later.
+  __device__ static __forceinline__ void slot(f32x4 (&acc)[8][8], const u32x4 (&a)[8], const u32x4 (&b)[8], int m) {
+    const int i = m / 8, e = m % 8 / 2;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int j = (m % 2) * 4 + k;
+      asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(a[i][e]), "v"(b[j][e]));
+    }
   }
 };
 
-// One 32-byte-of-K step for a 32x32 block: a and b each hold 16 bytes per lane.
-template <typename T>
-__device__ __forceinline__ void mma_block(f32x16& acc, const u32x4& a, const u32x4& b);
-
-template <>
-__device__ __forceinline__ void mma_block<__bf16>(f32x16& acc, const u32x4& a, const u32x4& b) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+__device__ __forceinline__ float acc_get(const f32x4& acc, int r) {
+  float v;
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(acc[r]));
+  return v;
+}
+__device__ __forceinline__ void acc_set(f32x4& acc, float v0, float v1, float v2, float v3) {
+  float a0, a1, a2, a3;
+  asm volatile("v_accvgpr_write_b32 %0, %1" : "=a"(a0) : "v"(v0));
+  asm volatile("v_accvgpr_write_b32 %0, %1" : "=a"(a1) : "v"(v1));
+  asm volatile("v_accvgpr_write_b32 %0, %1" : "=a"(a2) : "v"(v2));
+  asm volatile("v_accvgpr_write_b32 %0, %1" : "=a"(a3) : "v"(v3));
+  acc = f32x4{a0, a1, a2, a3};
 }
 
-template <>
-__device__ __forceinline__ void mma_block<float>(f32x16& acc, const u32x4& a, const u32x4& b) {
-  // Four K=2 steps; lane half h, element j stands for k = 4h + j in both operands.
-  f32x4 af = __builtin_bit_cast(f32x4, a);
-  f32x4 bf = __builtin_bit_cast(f32x4, b);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[0], bf[0], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[1], bf[1], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[2], bf[2], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[3], bf[3], acc, 0, 0, 0);
-}
+// fn(constant 0), ..., fn(constant N - 1), spelled out: an unrolled loop of this many instructions is over the
+// compiler's limit, and what is left rolled up would index registers in memory.
+template <int N> struct Const { static constexpr int value = N; };
+template <typename Fn, int... M>
+__device__ __forceinline__ void each(Fn fn, std::integer_sequence<int, M...>) { (fn(Const<M>{}), ...); }
+template <int N, typename Fn>
+__device__ __forceinline__ void each(Fn fn) { each(fn, std::make_integer_sequence<int, N>{}); }
 
-// Row of the accumulator register r within a 32x32 block for this lane.
-__device__ __forceinline__ int acc_row(int r, int lane) {
-  return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-}
-
-template <typename T, int BM_, int BN_, int WAVES_M_, int WAVES_N_>
+// BV: consecutive B rows a lane holds (see above), 8 or 4.
+template <typename T, int BV>
 struct GemmTile {
-  static constexpr int BM = BM_, BN = BN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;
-  static constexpr int kWaves = WAVES_M * WAVES_N;
-  static constexpr int kThreads = 64 * kWaves;
-  static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
-  static constexpr int MI = WM / 32, NI = WN / 32;
-  static constexpr int kRowsPerPass = kThreads / kChunksPerRow;
-  static constexpr int kPassA = BM / kRowsPerPass, kPassB = BN / kRowsPerPass;
-  static constexpr int kStageBytes = (BM + BN) * kRowBytes;
-  static constexpr int kLdsBytes = 2 * kStageBytes;
+  static constexpr int BM = 256, BN = 256, WM = 128, WN = 128;
+  static constexpr int MI = 8, NI = 8;                 // 16 x 16 blocks per wave along A / B
+  static constexpr int kThreads = 256;
+  static constexpr int kSlotBytes = 256 * kRowBytes;   // one operand's slab
+  static constexpr int kASlots = 3, kBSlots = 2;
+  static constexpr int kLdsBytes = (kASlots + kBSlots) * kSlotBytes;
   static constexpr int kSlabK = Elem<T>::kSlabK;
-  static_assert(BM % kRowsPerPass == 0 && BN % kRowsPerPass == 0, "tile rows vs threads");
-  static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile must be whole 32x32 blocks");
+  static constexpr int VEC = 16 / (int)sizeof(T);      // elements per 16-byte piece
+  static constexpr int kBB = kASlots * kSlotBytes;     // LDS offset of the B ring
+  static_assert(BV == 8 || BV == 4, "B rows per lane");
 
-  // State a caller carries between consecutive K loops of one workgroup that share B (same
-  // token rows, next block of A rows): which LDS stage holds slab 0, and whether the first two
-  // slabs of the coming loop have already been requested.
-  struct Stream {
-    int phase = 0;
-    bool loaded = false;
-  };
+  typedef f32x4 Acc[MI][NI];
+  typedef __attribute__((address_space(3))) char lds_char;
+  typedef __attribute__((address_space(3))) const u32x4 lds_vec;
+
+  // This lane's rows within the wave's 128: a_row(i, r) of register r of blocks i, b_row(j) of blocks j.
+  __device__ static __forceinline__ constexpr int a_block(int i) {
+    return VEC == 8 ? (i >> 1) * 32 + (i & 1) * 4 : i * 16;
+  }
+  __device__ static __forceinline__ int a_lane(int rho) { return VEC == 8 ? (rho >> 2) * 8 + (rho & 3) : rho; }
+  __device__ static __forceinline__ constexpr int b_block(int j) { return (j / BV) * 16 * BV + j % BV; }
+  __device__ static __forceinline__ int lane_a0() {     // first A row of this lane (block 0, register 0)
+    const int g = (threadIdx.x & 63) >> 4;
+    return VEC == 8 ? g * 8 : g * 4;
+  }
+  __device__ static __forceinline__ int lane_b0() { return (threadIdx.x & 15) * BV; }
+  __device__ static __forceinline__ int wave_m() { return ((threadIdx.x >> 6) & 1) * WM; }
+  __device__ static __forceinline__ int wave_n() { return (threadIdx.x >> 7) * WN; }
+
+  // Swizzle of LDS row R's chunks: eight rows that one fragment read takes together get eight values.
+  __device__ static __forceinline__ int a_swz(int row) { return VEC == 8 ? (row & 3) | ((row >> 3) & 1) << 2 : row & 7; }
+  __device__ static __forceinline__ int b_swz(int row) { return (BV == 8 ? row >> 3 : row >> 2) & 7; }
 
   // Where an operand's tile lives in memory: `rows` valid rows starting at `base`, consecutive
   // rows `row_bytes` apart, consecutive 128-byte K slabs of a row `slab_bytes` apart.
@@ -158,204 +178,196 @@ struct GemmTile {
     }
   };
 
-  // Per-thread constants of the global -> LDS loads of one operand pair.
-  struct Loader {
-    const char* a_ptr;
-    const char* b_ptr;
-    int a_bytes, b_bytes;     // bytes the valid rows span from the tile base at slab 0
-    int a_shrink, b_shrink;   // by how much that span shrinks per slab step (row-major: one slab; blocked: 0)
-    int a_slab, b_slab;
-    int a_voff, b_voff, a_pass, b_pass, dma_off;
+  // The next slab to request of one operand.  Loads go through range-checked buffer descriptors that cover
+  // exactly the valid rows, so rows past them read as zero and nothing outside the operands is touched: the
+  // row offset is in the per-lane part, which is what the hardware checks, the K-slab offset in the base
+  // address, and the size is what is left of the valid rows from there.
+  struct Cursor {
+    const char* p;
+    int bytes;
+    int left;       // slabs of this tile from here on
   };
 
-  typedef __attribute__((address_space(3))) char lds_char;
+  int slab_a, slab_b, shrink_a, shrink_b;     // address step and size step per slab
+  int pass_a, pass_b;                         // bytes between the rows of two loads of a slab
+  Cursor a, b, next_a, next_b;
+  lds_char* lds;
+  __amdgpu_buffer_rsrc_t rsrc_a, rsrc_b;
+  int voff_a, voff_b[2];
+  u32x4 af[2][MI], bf[2][NI];
+  uint32_t a0, b0;                            // this lane's fragment address in slot 0 of either ring
+  uint32_t ra, rb, na, nb;                    // the same in the slab being read and in the one after it
+  uint32_t da, db;                            // where the next requested slab goes
+  uint32_t w0;
 
-  // Loads go through range-checked buffer descriptors that cover exactly the valid rows, so rows
-  // past them read as zero and nothing outside the operands is touched.  The hardware checks the
-  // sum of the per-lane and the scalar offset against the descriptor's size, so the K-slab offset
-  // travels in the descriptor's base address instead (a few scalar instructions per slab) and the
-  // size is what is left of the valid rows from there.
-  __device__ static __forceinline__ Loader make_loader(const Operand& a, const Operand& b) {
-    const int tid = threadIdx.x;
-    const int ld_row = tid >> 3;
-    const int ld_chunk = tid & 7;
-    Loader L;
-    L.a_ptr = reinterpret_cast<const char*>(a.base);
-    L.b_ptr = reinterpret_cast<const char*>(b.base);
-    L.a_bytes = a.rows * a.row_bytes;
-    L.b_bytes = b.rows * b.row_bytes;
-    L.a_shrink = a.slab_bytes == kRowBytes ? kRowBytes : 0;
-    L.b_shrink = b.slab_bytes == kRowBytes ? kRowBytes : 0;
-    L.a_slab = a.slab_bytes;
-    L.b_slab = b.slab_bytes;
-    // A wave's load instruction fills 1 KB of LDS in lane order: 8 rows x 8 chunks of 16 bytes.
-    // The lane that lands on (row, slot) fetches K-chunk slot ^ swz(row), so a fragment read of
-    // K-chunk q goes to slot q ^ swz(row).
-    const int ld_swz = (ld_row & 7) ^ ((ld_row >> 3) & 1);
-    L.a_voff = ld_row * a.row_bytes + ((ld_chunk ^ ld_swz) * 16);
-    L.b_voff = ld_row * b.row_bytes + ((ld_chunk ^ ld_swz) * 16);
-    L.a_pass = kRowsPerPass * a.row_bytes;
-    L.b_pass = kRowsPerPass * b.row_bytes;
-    L.dma_off = __builtin_amdgcn_readfirstlane(tid >> 6) * 8 * kRowBytes;   // this wave's 8 rows within a pass
-    return L;
+  __device__ static __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
+  __device__ __forceinline__ void make_a() {
+    rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.p), 0, a.bytes, 0x00020000);
+  }
+  __device__ __forceinline__ void make_b() {
+    rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(b.p), 0, b.bytes, 0x00020000);
+  }
+  // Load p (0 .. 7) of the slab at the cursor: 8 rows per wave, 32 per workgroup.
+  __device__ __forceinline__ void load_a(int p) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, lds + da + p * 4096, 16, voff_a + p * pass_a, 0, 0, 0);
+  }
+  __device__ __forceinline__ void load_b(int p) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, lds + db + p * 4096, 16, voff_b[BV == 8 ? (p & 1) : 0] + p * pass_b, 0, 0, 0);
+  }
+  __device__ __forceinline__ void step_a() { step_a1(); step_a2(); step_a3(); }
+  // in pieces, to be placed between matrix instructions; masks, because a select would become a branch
+  __device__ __forceinline__ void step_a1() { a.left -= 1; }
+  __device__ __forceinline__ void step_a2() {
+    const int64_t sw = -(int64_t)(a.left == 0);
+    a.p += ((next_a.p - a.p) & sw) | (slab_a & ~sw);
+  }
+  __device__ __forceinline__ void step_a3() {
+    const int sw = -(int)(a.left == 0);
+    a.bytes += ((next_a.bytes - a.bytes) & sw) | (-shrink_a & ~sw);
+    a.left |= next_a.left & sw;
+  }
+  __device__ __forceinline__ void step_b() { step_b1(); step_b2(); step_b3(); }
+  // in pieces, to be placed between matrix instructions; masks, because a select would become a branch
+  __device__ __forceinline__ void step_b1() { b.left -= 1; }
+  __device__ __forceinline__ void step_b2() {
+    const int64_t sw = -(int64_t)(b.left == 0);
+    b.p += ((next_b.p - b.p) & sw) | (slab_b & ~sw);
+  }
+  __device__ __forceinline__ void step_b3() {
+    const int sw = -(int)(b.left == 0);
+    b.bytes += ((next_b.bytes - b.bytes) & sw) | (-shrink_b & ~sw);
+    b.left |= next_b.left & sw;
+  }
+  __device__ __forceinline__ void slot_a() { const uint32_t t = da + kSlotBytes; da = t >= (uint32_t)kBB ? t - kBB : t; }
+  __device__ __forceinline__ void slot_b() { db = 2 * (kBB + w0) + kSlotBytes - db; }
+  // Fragment read n (0 .. 15) of a half: the first A fragment, all of B, the rest of A.
+  __device__ __forceinline__ void read(int set, uint32_t pa, uint32_t pb, int n) {
+    if (n == 0) af[set][0] = *(lds_vec*)(lds + pa);
+    else if (n <= NI) bf[set][n - 1] = *(lds_vec*)(lds + pb + b_block(n - 1) * kRowBytes);
+    else af[set][n - NI] = *(lds_vec*)(lds + pa + a_block(n - NI) * kRowBytes);
   }
 
-  // global -> LDS without passing registers; completion must be awaited (wait_loads) before the
-  // workgroup barrier that publishes the stage.
-  __device__ static __forceinline__ void dma_slab(const Loader& L, char* stage, int slab) {
-    lds_char* dst = (lds_char*)(stage) + L.dma_off;
-    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(L.a_ptr + (int64_t)slab * L.a_slab), 0, L.a_bytes - slab * L.a_shrink, 0x00020000);
-    const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(L.b_ptr + (int64_t)slab * L.b_slab), 0, L.b_bytes - slab * L.b_shrink, 0x00020000);
-#pragma unroll
-    for (int p = 0; p < kPassA; ++p)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, dst + p * kRowsPerPass * kRowBytes, 16,
-                                               L.a_voff + p * L.a_pass, 0, 0, 0);
-#pragma unroll
-    for (int p = 0; p < kPassB; ++p)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, dst + (BM + p * kRowsPerPass) * kRowBytes, 16,
-                                               L.b_voff + p * L.b_pass, 0, 0, 0);
+  __device__ static __forceinline__ Cursor cursor(const Operand& o, int nslab) {
+    return Cursor{reinterpret_cast<const char*>(o.base), o.rows * o.row_bytes, nslab};
+  }
+  // What the cursor does behind the last slab of the last tile: request that slab again.
+  __device__ static __forceinline__ Cursor hold(const Operand& o, int nslab) {
+    const int shrink = o.slab_bytes == kRowBytes ? kRowBytes : 0;
+    return Cursor{reinterpret_cast<const char*>(o.base) + (int64_t)(nslab - 1) * o.slab_bytes,
+                  o.rows * o.row_bytes - (nslab - 1) * shrink, 1};
   }
 
-  // A workgroup barrier does not wait for loads whose destination is LDS: wait for this wave's
-  // outstanding ones explicitly (s_waitcnt vmcnt(0), the other counters left alone).
-  __device__ static __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
-  // acc[mi][ni] must be initialised by the caller.  `a` / `b` describe the tile's rows from K offset 0;
-  // K must be a multiple of kSlabK and every row 16-byte aligned.  With next != nullptr the last
-  // two slab periods request the first two slabs of the next K loop, which keeps one operand and
-  // takes the other's rows from `next` (next_rows valid rows, same layout as the operand it replaces:
-  // A unless next_is_b), and LDS stays in use on return; otherwise, with release_lds, all loads have
-  // landed and every wave is past its last fragment read on return.
-  __device__ static __forceinline__ void run(f32x16 (&acc)[MI][NI], const Operand& a, const Operand& b, int K,
-                                             char* lds, Stream& st, const T* next, int next_rows,
-                                             bool release_lds, bool next_is_b = false) {
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int wm = wave % WAVES_M;
-    const int wn = wave / WAVES_M;
-    const Loader L = make_loader(a, b);
-    const int nslab = K / kSlabK;
-    const bool stream_on = next != nullptr && nslab >= 2;
-    Loader LN = L;
-    if (stream_on) {
-      if (next_is_b) {
-        LN.b_ptr = reinterpret_cast<const char*>(next);
-        LN.b_bytes = next_rows * b.row_bytes;
-      } else {
-        LN.a_ptr = reinterpret_cast<const char*>(next);
-        LN.a_bytes = next_rows * a.row_bytes;
-      }
-    }
-
-    const int fr_swz = (lane & 7) ^ ((lane >> 3) & 1);
-    int xk[4];
+  // First tile of a workgroup (or of a run that does not stream): nothing is in flight, LDS is free.
+  __device__ __forceinline__ void start(const Operand& A, const Operand& B, int nslab, char* shared) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    lds = (lds_char*)shared;
+    slab_a = A.slab_bytes; slab_b = B.slab_bytes;
+    shrink_a = A.slab_bytes == kRowBytes ? kRowBytes : 0;
+    shrink_b = B.slab_bytes == kRowBytes ? kRowBytes : 0;
+    pass_a = 32 * A.row_bytes; pass_b = 32 * B.row_bytes;
+    w0 = __builtin_amdgcn_readfirstlane(wave) * 1024;
+    // A wave's load fills 1 KB of LDS in lane order: 8 rows x 8 chunks.  The lane that lands on (row, slot)
+    // fetches chunk slot ^ swz(row); load p of a slab starts 32 p rows further down, which leaves a_swz and
+    // b_swz<4> as they are and moves b_swz<8> by 4 p, so odd loads have an offset of their own.
+    const int row = wave * 8 + (lane >> 3), chunk = lane & 7;
+    voff_a = row * A.row_bytes + (chunk ^ a_swz(row)) * 16;
+    voff_b[0] = row * B.row_bytes + (chunk ^ b_swz(row)) * 16;
+    voff_b[1] = row * B.row_bytes + (chunk ^ b_swz(row + 32)) * 16;
+    const int g = lane >> 4, c = lane & 15;
+    const int fa = a_lane(c), fb = c * BV;
+    a0 = (wave_m() + fa) * kRowBytes + (g ^ a_swz(fa)) * 16;
+    b0 = kBB + (wave_n() + fb) * kRowBytes + (g ^ b_swz(fb)) * 16;
+    a = cursor(A, nslab); b = cursor(B, nslab);
+    next_a = hold(A, nslab); next_b = hold(B, nslab);
+    make_a(); make_b();
+    da = w0; db = kBB + w0;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) xk[kk] = ((kk * 2 + (lane >> 5)) ^ fr_swz) * 16;
-    const int a_frag_off = (wm * WM + (lane & 31)) * kRowBytes;
-    const int b_frag_off = BM * kRowBytes + (wn * WN + (lane & 31)) * kRowBytes;
-
-    u32x4 af[2][MI], bf[2][NI];
-    auto read_frags = [&](int set, const char* stage, int kk) {
+    for (int p = 0; p < 8; ++p) load_a(p);
 #pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
-        af[set][mi] = *reinterpret_cast<const u32x4*>(stage + a_frag_off + mi * 32 * kRowBytes + xk[kk]);
+    for (int p = 0; p < 8; ++p) load_b(p);
+    step_a(); step_b(); make_a(); make_b(); slot_a(); slot_b();
 #pragma unroll
-      for (int ni = 0; ni < NI; ++ni)
-        bf[set][ni] = *reinterpret_cast<const u32x4*>(stage + b_frag_off + ni * 32 * kRowBytes + xk[kk]);
-    };
-    auto mma = [&](int set) {
+    for (int p = 0; p < 8; ++p) load_a(p);
+    step_a(); make_a(); slot_a();
+    __builtin_amdgcn_s_waitcnt(0x0F78);    // all but the youngest eight loads
+    __syncthreads();
+    ra = a0; rb = b0; na = a0 + kSlotBytes; nb = b0 + kSlotBytes;
 #pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
+    for (int n = 0; n < 16; ++n) read(0, ra, rb, n);
 #pragma unroll
-        for (int ni = 0; ni < NI; ++ni) mma_block<T>(acc[mi][ni], af[set][mi], bf[set][ni]);
-    };
-    constexpr int kFragReads = MI + NI;
-    constexpr int kMma = MI * NI;
-    constexpr int kLoads = kPassA + kPassB;
-    // one K-step: `kFragReads` matrix ops each followed by one LDS read, then the rest
-    auto pace_reads = [&]() {
-#pragma unroll
-      for (int i = 0; i < kFragReads; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x008, kMma - kFragReads, 0);
-    };
-    // one slab: `cur` holds slab s, the loads of slab s+1 into `nxt` are in flight; `ld` and
-    // `ld_slab` name the slab requested into `cur` once everyone is done with it
-    auto slab_body = [&](char* cur, char* nxt, const Loader& ld, int ld_slab) {
-      read_frags(1, cur, 1);
-      mma(0);
-      pace_reads();
-      read_frags(0, cur, 2);
-      mma(1);
-      pace_reads();
-      read_frags(1, cur, 3);
-      mma(0);
-      pace_reads();
-      __builtin_amdgcn_sched_barrier(0);
-      // slab s+1 has landed in `nxt` for every wave; everyone holds the last fragments of `cur`
-      wait_loads();
-      __syncthreads();
-      read_frags(0, nxt, 0);
-      dma_slab(ld, cur, ld_slab);
-      mma(1);
-#pragma unroll
-      for (int i = 0; i < kFragReads; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x020, (kLoads + kFragReads - 1) / kFragReads, 0);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x008, kMma - kFragReads, 0);
-      __builtin_amdgcn_sched_barrier(0);
-    };
-
-    char* const buf0 = lds + st.phase * kStageBytes;
-    char* const buf1 = lds + (st.phase ^ 1) * kStageBytes;
-    if (!st.loaded) {
-      dma_slab(L, buf0, 0);
-      wait_loads();
-      __syncthreads();
-      if (nslab > 1) dma_slab(L, buf1, 1);
-    } else {
-      wait_loads();
-      __syncthreads();
-    }
-    read_frags(0, buf0, 0);
-    int s = 0;
-    for (; s + 2 < nslab; ++s)
-      slab_body((s & 1) ? buf1 : buf0, (s & 1) ? buf0 : buf1, L, s + 2);
-    // The last two slab periods have no slab of this loop left to request: they request the first
-    // two slabs of the next loop, or the last slab again.  (Measured: leaving the loads out here
-    // instead makes the whole loop slower, not faster.)
-    for (; s < nslab; ++s)
-      slab_body((s & 1) ? buf1 : buf0, (s & 1) ? buf0 : buf1, LN, stream_on ? s + 2 - nslab : nslab - 1);
-    st.phase = (st.phase + nslab) & 1;
-    st.loaded = stream_on;
-    if (release_lds && !stream_on) {
-      wait_loads();      // the repeated loads of the last slab still target LDS
-      __syncthreads();
-    }
+    for (int p = 0; p < 8; ++p) load_b(p);
   }
 
-  // Single K loop: nothing carried over, LDS free on return.
-  __device__ static __forceinline__ void run(f32x16 (&acc)[MI][NI], const Operand& a, const Operand& b, int K,
-                                             char* lds) {
-    Stream st;
-    run(acc, a, b, K, lds, st, nullptr, 0, true);
+  // One tile's K loop of `nslab` slabs; acc must be initialised by the caller.  Between tiles of a
+  // streaming workgroup LDS stays in use; after the last one call finish() before touching it.
+  __device__ __forceinline__ void run(Acc& acc, int nslab) {
+    settle();
+    for (int s = 0; s < nslab; ++s) {
+      each<MI * NI>([&](auto c) __attribute__((always_inline)) {            // first half of the slab
+        constexpr int m = decltype(c)::value;
+        Mma<T>::slot(acc, af[0], bf[0], m);
+        fence();
+        if constexpr (m % 2 == 0 && m < 32) { read(1, ra ^ 64, rb ^ 64, m / 2); fence(); }
+        if constexpr (m % 8 == 1) { load_a(m / 8); fence(); }
+        if constexpr (m == 35) { step_b1(); fence(); }
+        if constexpr (m == 37) { step_b2(); fence(); }
+        if constexpr (m == 43) { step_b3(); fence(); }
+        if constexpr (m == 45) { make_b(); fence(); }
+        if constexpr (m == 47) { slot_b(); fence(); }
+      });
+      fence();
+      // every wave has the last fragments of this slab, and the next one's loads have landed
+      __builtin_amdgcn_s_waitcnt(0x0078);
+      __builtin_amdgcn_s_barrier();
+      fence();
+      each<MI * NI>([&](auto c) __attribute__((always_inline)) {            // second half, while the next slab's first fragments come in
+        constexpr int m = decltype(c)::value;
+        Mma<T>::slot(acc, af[1], bf[1], m);
+        fence();
+        if constexpr (m % 2 == 0 && m < 32) { read(0, na, nb, m / 2); fence(); }
+        if constexpr (m % 8 == 1) { load_b(m / 8); fence(); }
+        if constexpr (m == 35) { step_a1(); fence(); }
+        if constexpr (m == 37) { step_a2(); fence(); }
+        if constexpr (m == 43) { step_a3(); fence(); }
+        if constexpr (m == 45) { make_a(); fence(); }
+        if constexpr (m == 47) { slot_a(); fence(); }
+        if constexpr (m == 51) { ra = na; rb = nb; fence(); }
+        if constexpr (m == 53) { const uint32_t t = na + kSlotBytes; na = t >= (uint32_t)kBB ? t - kBB : t; fence(); }
+        if constexpr (m == 55) { nb = 2 * b0 + kSlotBytes - nb; fence(); }
+      });
+    }
+    settle();
+  }
+
+  // Wait states between matrix instructions and other accesses to the accumulators, in either direction: at most
+  // 19 (result of a 16-pass instruction read by the vector unit).
+  __device__ static __forceinline__ void settle() {
+    fence();
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    fence();
+  }
+
+  // All loads have landed and every wave is past its last fragment read: LDS is free.
+  __device__ static __forceinline__ void finish() {
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    __syncthreads();
+  }
+
+  // Whether a workgroup's tiles of `nslab` slabs can stream: A is requested three slabs ahead, which must not
+  // reach beyond the next tile.
+  __device__ static __forceinline__ bool can_stream(int nslab) { return nslab >= kASlots; }
+
+  __device__ static __forceinline__ void zero(Acc& acc) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc_set(acc[i][j], 0.f, 0.f, 0.f, 0.f);
   }
 };
 
-// The tile every GEMM-shaped kernel of the head path uses: 256 x 256 outputs per workgroup,
-// 2 x kHeadWavesN wavefronts.
-#ifndef CLGRPO_WAVES_N
-#define CLGRPO_WAVES_N 4
-#endif
-constexpr int kHeadWavesN = CLGRPO_WAVES_N;
-constexpr int kHeadThreads = 64 * 2 * kHeadWavesN;
-template <typename T> using HeadTile = GemmTile<T, 256, 256, 2, kHeadWavesN>;
+constexpr int kHeadThreads = 256;
+// The tile of the kernels that hold logits (A = vocabulary, B = tokens): a lane's 16-byte pieces run along either.
+template <typename T> using LogitTile = GemmTile<T, 16 / (int)sizeof(T)>;
 
 // Workgroup id -> logical work item so that the workgroups resident on one XCD
 // (hardware deals consecutive ids round-robin over the 8 XCDs) own a contiguous

@@ -18,20 +18,17 @@ int validate_head_shape(const char* who, int64_t T, int64_t H, int64_t V, int32_
 
 constexpr float kLog2e = 1.4426950408889634f;
 
-template <typename T> struct Pack4;
-template <> struct Pack4<float> {
-  typedef float4 type;
-  __device__ static __forceinline__ type make(float a, float b, float c, float d) { return make_float4(a, b, c, d); }
-};
-template <> struct Pack4<__bf16> {
-  typedef uint2 type;
-  __device__ static __forceinline__ type make(float a, float b, float c, float d) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    bf16x2 lo = {(__bf16)a, (__bf16)b};
-    bf16x2 hi = {(__bf16)c, (__bf16)d};
-    return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
-  }
-};
+// VEC = 16 / sizeof(T) floats as one 16-byte piece of the operand dtype.
+__device__ __forceinline__ u32x4 pack_vec(const float (&v)[4], float*) {
+  const f32x4 x = {v[0], v[1], v[2], v[3]};
+  return __builtin_bit_cast(u32x4, x);
+}
+__device__ __forceinline__ u32x4 pack_vec(const float (&v)[8], __bf16*) {
+  bf16x8 x;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = (__bf16)v[e];
+  return __builtin_bit_cast(u32x4, x);
+}
 
 struct DzParams {
   const void* hidden;   // chunk base: [Tc, H]
@@ -53,9 +50,9 @@ struct DzParams {
 };
 
 template <typename T>
-__global__ __launch_bounds__(kHeadThreads) void lmhead_dz_kernel(DzParams p) {
-  using Tile = HeadTile<T>;
-  constexpr int MI = Tile::MI, NI = Tile::NI, WM = Tile::WM, WN = Tile::WN;
+__global__ __launch_bounds__(kHeadThreads, 1) void lmhead_dz_kernel(DzParams p) {
+  using Tile = LogitTile<T>;
+  constexpr int MI = Tile::MI, NI = Tile::NI, VEC = Tile::VEC;
   extern __shared__ __align__(16) char lds[];
 
   const int item = xcd_remap(blockIdx.x, gridDim.x);
@@ -63,98 +60,105 @@ __global__ __launch_bounds__(kHeadThreads) void lmhead_dz_kernel(DzParams p) {
   int vt, tb;
   grouped_tile(item, p.n_vt, p.n_tb, 4, vt, tb);
 
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm = wave % 2, wn = wave / 2;
+  const int la = Tile::wave_m() + Tile::lane_a0(), lb = Tile::wave_n() + Tile::lane_b0();
   const int t0 = tb * 256, v0 = vt * 256;
   const int b_rows = (p.Tc - t0) < 256 ? (p.Tc - t0) : 256;
   const int a_rows = (p.V - v0) < 256 ? (p.V - v0) : 256;
   const T* hidden = static_cast<const T*>(p.hidden) + (int64_t)t0 * p.H;
   const T* weight = static_cast<const T*>(p.weight) + (int64_t)v0 * p.H;
 
-  // Per-token coefficients.  Tokens past the chunk get zero gradient and a huge lse, so p = 0.
-  int lab[NI], tl[NI];
-  float lse2[NI], lse[NI], glp[NI], gent[NI], ent[NI];
+  // A token block whose upstream gradients are all zero (e.g. prompt-only rows) needs no GEMM.
   bool any_grad = false;
 #pragma unroll
-  for (int ni = 0; ni < NI; ++ni) {
-    tl[ni] = t0 + wn * WN + ni * 32 + (lane & 31);
-    const bool ok = tl[ni] < p.Tc;
-    lab[ni] = -1;
-    if (ok) {
-      const int64_t rel = p.labels[tl[ni]] - p.label_offset;   // a label outside these rows matches nothing
-      if (rel >= 0 && rel < p.V) lab[ni] = (int)rel;
-    }
-    lse[ni] = ok ? p.lse[tl[ni]] : 1e30f;
-    lse2[ni] = lse[ni] * kLog2e;
-    glp[ni] = ok ? p.g_lp[tl[ni]] : 0.f;
-    gent[ni] = (ok && p.g_ent) ? p.g_ent[tl[ni]] : 0.f;
-    ent[ni] = (ok && p.g_ent) ? p.entropy[tl[ni]] : 0.f;
-    any_grad |= (glp[ni] != 0.f) | (gent[ni] != 0.f);
+  for (int j = 0; j < NI; ++j) {
+    const int t = t0 + lb + Tile::b_block(j);
+    if (t < p.Tc) any_grad |= (p.g_lp[t] != 0.f) | (p.g_ent != nullptr && p.g_ent[t] != 0.f);
   }
-  // A token block whose upstream gradients are all zero (e.g. prompt-only rows) needs no GEMM.
-  const bool block_live = __syncthreads_or(any_grad);
+  // (the flags pass through the tile's own LDS: all of it is spoken for)
+  int* live = reinterpret_cast<int*>(lds);
+  const bool wave_live = __any(any_grad);
+  if ((threadIdx.x & 63) == 0) live[threadIdx.x >> 6] = wave_live;
+  __syncthreads();
+  const bool block_live = (live[0] | live[1] | live[2] | live[3]) != 0;
+  __syncthreads();
 
-  f32x16 acc[MI][NI];
+  typename Tile::Acc acc;
+  Tile::zero(acc);
+  if (block_live) {
+    Tile core;
+    const int nslab = p.H / Tile::kSlabK;
+    core.start(Tile::Operand::row_major(weight, p.H, a_rows), Tile::Operand::row_major(hidden, p.H, b_rows), nslab, lds);
+    core.run(acc, nslab);
+    Tile::finish();
+  }
+
+  // Per-token coefficients.  Tokens past the chunk get zero gradient and a huge lse, so p = 0.
+  int lab[NI];
+  float lse[NI], glp[NI], gent[NI], ent[NI];
 #pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < NI; ++ni)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
-  if (block_live)
-    Tile::run(acc, Tile::Operand::row_major(weight, p.H, a_rows), Tile::Operand::row_major(hidden, p.H, b_rows), p.H, lds);
+  for (int j = 0; j < NI; ++j) {
+    const int t = t0 + lb + Tile::b_block(j);
+    const bool ok = t < p.Tc;
+    lab[j] = -1;
+    if (ok) {
+      const int64_t rel = p.labels[t] - p.label_offset;   // a label outside these rows matches nothing
+      if (rel >= 0 && rel < p.V) lab[j] = (int)rel;
+    }
+    lse[j] = ok ? p.lse[t] : 1e30f;
+    glp[j] = ok ? p.g_lp[t] : 0.f;
+    gent[j] = (ok && p.g_ent) ? p.g_ent[t] : 0.f;
+    ent[j] = (ok && p.g_ent) ? p.entropy[t] : 0.f;
+  }
 
   T* dz = static_cast<T*>(p.dz);
   T* dzT = static_cast<T*>(p.dzT);
   const float it = p.inv_temperature;
+  constexpr int AG = VEC / 4;                 // blocks along A whose registers make up VEC consecutive vocabulary rows
 #pragma unroll
-  for (int ni = 0; ni < NI; ++ni) {
-    const int rel = lab[ni] - (v0 + wm * WM);
-    const float hot = it * glp[ni];
+  for (int i = 0; i < MI; i += AG) {
+    float d[NI][VEC];
+    const int v = v0 + la + Tile::a_block(i);
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi) {
+    for (int j = 0; j < NI; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        float d[4];
-        const int row0 = wm * WM + mi * 32 + 8 * q + 4 * (lane >> 5);  // tile row of r = 4q
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float zraw = acc[mi][ni][4 * q + j];
-          const float pr = __builtin_amdgcn_exp2f(fmaf(zraw, p.c, -lse2[ni]));
-          const float logp = fmaf(zraw, it, -lse[ni]);
-          // dz = it * ( glp*(1[v==y] - p) - gent * p * (logp + ent) )
-          float v = -it * pr * fmaf(gent[ni], logp + ent[ni], glp[ni]);
-          if (rel == (row0 - wm * WM) + j) v += hot;
-          if (row0 + j >= a_rows || !block_live) v = 0.f;   // vocabulary padding columns / dead block
-          d[j] = v;
-        }
-        const int v_idx = v0 + row0;
-        if (tl[ni] < p.Tc && v_idx < p.ldv) {
-          typedef typename Pack4<T>::type P4;
-          *reinterpret_cast<P4*>(dz + blocked_index<T>(tl[ni], v_idx, p.ldv / Tile::kSlabK)) =
-              Pack4<T>::make(d[0], d[1], d[2], d[3]);
-        }
-        if (tl[ni] < p.ldt) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (v_idx + j < p.V) dzT[blocked_index<T>(v_idx + j, tl[ni], p.ldt / Tile::kSlabK)] = (T)d[j];
-        }
+      for (int e = 0; e < VEC; ++e) {
+        const float zraw = acc_get(acc[i + e / 4][j], e % 4);
+        const float pr = __builtin_amdgcn_exp2f(fmaf(zraw, p.c, -lse[j] * kLog2e));
+        const float logp = fmaf(zraw, it, -lse[j]);
+        // dz = it * ( glp*(1[v==y] - p) - gent * p * (logp + ent) )
+        float x = -it * pr * fmaf(gent[j], logp + ent[j], glp[j]);
+        if (lab[j] == v + e) x += it * glp[j];
+        if (v + e >= p.V || !block_live) x = 0.f;   // vocabulary padding columns / dead block
+        d[j][e] = x;
       }
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const int t = t0 + lb + Tile::b_block(j);
+      if (t < p.Tc && v < p.ldv)
+        *reinterpret_cast<u32x4*>(dz + blocked_index<T>(t, v, p.ldv / Tile::kSlabK)) = pack_vec(d[j], (T*)nullptr);
     }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+#pragma unroll
+      for (int j = 0; j < NI; j += VEC) {
+        float x[VEC];
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) x[k] = d[j + k][e];
+        const int t = t0 + lb + Tile::b_block(j);
+        if (v + e < p.V && t < p.ldt)
+          *reinterpret_cast<u32x4*>(dzT + blocked_index<T>(v + e, t, p.ldt / Tile::kSlabK)) = pack_vec(x, (T*)nullptr);
+      }
   }
 }
 
-// d(logits) from kept logits, in place, plus its transpose.  One workgroup per 32 KB unit of the kept
-// logits (256 token rows x one 128-byte slab of vocabulary, z-native layout, see ZNative): every thread
-// reads its 128 bytes of the unit, forms dz with its rows' coefficients and drops the values into two LDS
-// tiles, [token][vocab] and [vocab][token]; after a barrier the first goes back over the unit as the
-// K-blocked dz operand (the unit's 32 KB are exactly that operand's piece for these rows and this slab)
-// and the second to the K-blocked dzT operand (per 64-token slab one contiguous piece of 64 vocabulary
-// rows).  All global accesses are 16 bytes per lane and contiguous per wavefront.  HBM-bound: reads 1x,
-// writes 2x the chunk.
+// d(logits) from kept logits, in place, plus its transpose.  A unit is 256 token rows x one 128-byte slab of
+// vocabulary: 32 KB of the K-blocked kept logits, which become the same 32 KB of the K-blocked dz operand.
+// A thread takes a square of VEC tokens x VEC vocabulary entries: VEC 16-byte pieces in, VEC pieces of
+// dz back over them, VEC pieces of dzT, the transposition being a choice of registers (no LDS, no barrier
+// between units).  Eight lanes cover a slab row, eight lane groups eight of its token groups, so every access
+// of a wave is whole 128-byte lines.  HBM-bound: reads 1x, writes 2x the chunk.
 struct DzFromZParams {
-  void* z;            // Tc x ldv: in kept logits (z-native, KeptLogit<T>), out dz (K-blocked, T)
+  void* z;            // Tc x ldv: in kept logits (KeptLogit<T>), out dz (T), K-blocked
   void* dzT;          // V x ldt, K-blocked
   const int64_t* labels;
   int64_t label_offset;
@@ -169,127 +173,84 @@ struct DzFromZParams {
 template <typename T>
 __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams p) {
   typedef typename KeptLogit<T>::type ZT;
-  typedef ZNative<ZT> ZL;
   static_assert(sizeof(ZT) == sizeof(T), "d(logits) overwrites the kept logits in place");
-  constexpr int E = ZL::kSlabElems;                 // vocabulary entries of this unit (64 or 32)
+  constexpr int E = Elem<T>::kSlabK;                // vocabulary entries of a unit (64 or 32)
   constexpr int VEC = 16 / (int)sizeof(T);          // elements per 16-byte piece
-  constexpr int kSub = 8 * ZL::VSUB;                // 32x32 sub-blocks per unit
-  constexpr int kSubPerWave = kSub / 4;
-  constexpr int kTPitch = kBlockRows * (int)sizeof(T) + 16;   // bytes per vocabulary row of the transposed tile
-  // one LDS region, used twice: [token R][vocab c] with the 16-byte chunks XOR-swizzled by R % 8 (32 KB),
-  // then [vocab c][token R] with padded rows
-  __shared__ __align__(16) char tile[E * kTPitch > kBlockRows * kRowBytes ? E * kTPitch : kBlockRows * kRowBytes];
-  const int rb = blockIdx.x, ks = blockIdx.y;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int h = lane >> 5, t32 = lane & 31;
+  constexpr int kPasses = kBlockRows / VEC / 32;    // a pass of 256 threads covers 32 token groups
+  __shared__ float s_lse[kBlockRows], s_ent[kBlockRows], s_glp[kBlockRows], s_gen[kBlockRows];
+  __shared__ int s_lab[kBlockRows];
+  const int rb = blockIdx.x;
   const int64_t n_kslab = p.ldv / E;
-  char* unit = static_cast<char*>(p.z) + ((int64_t)rb * n_kslab + ks) * ZL::kUnitBytes;
   const float it = p.inv_temperature;
-
-  u32x4 raw[kSubPerWave][ZL::PIECES];
-#pragma unroll
-  for (int s = 0; s < kSubPerWave; ++s)
-#pragma unroll
-    for (int j = 0; j < ZL::PIECES; ++j)
-      raw[s][j] = *reinterpret_cast<const u32x4*>(unit + (wave + 4 * s) * (ZL::PIECES * 1024) + j * 1024 + lane * 16);
-
-  // this lane's 16 values of each of its sub-blocks, as d(logits) in the operand dtype
-  T dz[kSubPerWave][16];
-#pragma unroll
-  for (int s = 0; s < kSubPerWave; ++s) {
-    const int sb = wave + 4 * s;
-    const int R = (sb / ZL::VSUB) * 32 + t32;       // token row inside the unit
-    const int c0 = (sb % ZL::VSUB) * 32;            // first vocabulary entry of the sub-block inside the unit
-    const int t = rb * kBlockRows + R;
-    float glp = 0.f, gen = 0.f, lse = 0.f, ent = 0.f;
+  {
+    const int t = rb * kBlockRows + threadIdx.x;
+    const bool ok = t < p.Tc;
+    s_glp[threadIdx.x] = ok ? p.g_lp[t] : 0.f;      // rows past the chunk and rows without a gradient give zeros
+    s_gen[threadIdx.x] = (ok && p.g_ent) ? p.g_ent[t] : 0.f;
+    s_lse[threadIdx.x] = ok ? p.lse[t] : 0.f;
+    s_ent[threadIdx.x] = (ok && p.g_ent) ? p.entropy[t] : 0.f;
     int lab = -1;
-    if (t < p.Tc) {
-      glp = p.g_lp[t];
-      gen = p.g_ent ? p.g_ent[t] : 0.f;
-      lse = p.lse[t];
-      ent = p.g_ent ? p.entropy[t] : 0.f;
-      const int64_t rel = p.labels[t] - p.label_offset - ((int64_t)ks * E + c0);   // relative to the sub-block
-      lab = (rel >= 0 && rel < 32) ? (int)rel : -1;
+    if (ok) {
+      const int64_t rel = p.labels[t] - p.label_offset;
+      if (rel >= 0 && rel < p.V) lab = (int)rel;
     }
-    const bool live = glp != 0.f || gen != 0.f;     // rows past the chunk and rows without a gradient give zeros
-    const float lse2 = lse * kLog2e;
+    s_lab[threadIdx.x] = lab;
+  }
+  __syncthreads();
+  const int q = threadIdx.x & 7, cg = threadIdx.x >> 3;   // piece within the slab row, token group
+  T* dzT = static_cast<T*>(p.dzT);
+  const int64_t n_tslab = p.ldt / E;
+  for (int ks = blockIdx.y; ks < (int)n_kslab; ks += gridDim.y) {
+    char* unit = static_cast<char*>(p.z) + ((int64_t)rb * n_kslab + ks) * (kBlockRows * kRowBytes);
+    const int v = ks * E + q * VEC;
 #pragma unroll
-    for (int j = 0; j < ZL::PIECES; ++j) {
-      const ZT* in = reinterpret_cast<const ZT*>(&raw[s][j]);
+    for (int pass = 0; pass < kPasses; ++pass) {
+      const int R = (pass * 32 + cg) * VEC;         // first token row of this thread's square
+      u32x4 raw[VEC];
 #pragma unroll
-      for (int e = 0; e < ZL::kPerPiece; ++e) {
-        const int c32 = ZL::col_of(h, j, e);
-        float d = 0.f;
-        if (live) {
+      for (int k = 0; k < VEC; ++k) raw[k] = *reinterpret_cast<const u32x4*>(unit + (R + k) * kRowBytes + q * 16);
+      float d[VEC][VEC];
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) {
+        const float glp = s_glp[R + k], gen = s_gen[R + k], lse = s_lse[R + k], ent = s_ent[R + k];
+        const int lab = s_lab[R + k] - v;
+        const bool live = glp != 0.f || gen != 0.f;
+        const float lse2 = lse * kLog2e;
+        const ZT* in = reinterpret_cast<const ZT*>(&raw[k]);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
           const float zraw = (float)in[e];
           const float pr = __builtin_amdgcn_exp2f(fmaf(zraw, p.c, -lse2));
           const float logp = fmaf(zraw, it, -lse);
-          d = -it * pr * fmaf(gen, logp + ent, glp);
-          if (c32 == lab) d += it * glp;
-          if (ks * E + c0 + c32 >= p.V) d = 0.f;    // vocabulary padding columns
+          float x = -it * pr * fmaf(gen, logp + ent, glp);
+          if (lab == e) x += it * glp;
+          d[k][e] = (live && v + e < p.V) ? x : 0.f;      // vocabulary padding columns give zeros
         }
-        dz[s][j * ZL::kPerPiece + e] = (T)d;
+      }
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) *reinterpret_cast<u32x4*>(unit + (R + k) * kRowBytes + q * 16) = pack_vec(d[k], (T*)nullptr);
+      const int tok = rb * kBlockRows + R;
+      if (tok < p.ldt) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          float x[VEC];
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) x[k] = d[k][e];
+          if (v + e < p.V) *reinterpret_cast<u32x4*>(dzT + blocked_index<T>(v + e, tok, n_tslab)) = pack_vec(x, (T*)nullptr);
+        }
       }
     }
   }
-
-  // pass 1: [token][vocab] through LDS, back over the unit as the K-blocked dz operand
-#pragma unroll
-  for (int s = 0; s < kSubPerWave; ++s) {
-    const int sb = wave + 4 * s;
-    const int R = (sb / ZL::VSUB) * 32 + t32;
-    const int c0 = (sb % ZL::VSUB) * 32;
-    // registers 4m .. 4m+3 are consecutive vocabulary entries: 4 * sizeof(T) bytes of the token's row
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int byte = (c0 + 8 * m + 4 * h) * (int)sizeof(T);
-      char* dst = tile + R * kRowBytes + (((byte >> 4) ^ (R & 7)) << 4) + (byte & 15);
-      if (sizeof(T) == 2) *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(&dz[s][4 * m]);
-      else *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(&dz[s][4 * m]);
-    }
-  }
-  __syncthreads();     // also: every thread has its part of the unit in registers before anyone overwrites it
-  for (int pc = threadIdx.x; pc < kBlockRows * kChunksPerRow; pc += 256) {
-    const int R = pc >> 3, q = pc & 7;              // row R, 16-byte chunk q of the operand is piece R * 8 + q
-    *reinterpret_cast<u32x4*>(unit + pc * 16) = *reinterpret_cast<const u32x4*>(tile + R * kRowBytes + ((q ^ (R & 7)) << 4));
-  }
-  __syncthreads();
-
-  // pass 2: [vocab][token] through LDS, out to the K-blocked dzT operand (vocabulary row v, token slabs of E)
-#pragma unroll
-  for (int s = 0; s < kSubPerWave; ++s) {
-    const int sb = wave + 4 * s;
-    const int R = (sb / ZL::VSUB) * 32 + t32;
-    const int c0 = (sb % ZL::VSUB) * 32;
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      *reinterpret_cast<T*>(tile + (c0 + 8 * (r >> 2) + 4 * h + (r & 3)) * kTPitch + R * (int)sizeof(T)) = dz[s][r];
-  }
-  __syncthreads();
-  T* dzT = static_cast<T*>(p.dzT);
-  const int64_t n_tslab = p.ldt / E;
-  for (int pc = threadIdx.x; pc < E * (kBlockRows / VEC); pc += 256) {
-    const int sl = pc / (E * kChunksPerRow);        // token slab inside the unit
-    const int c = (pc / kChunksPerRow) % E;         // vocabulary row inside the unit
-    const int q = pc % kChunksPerRow;
-    const int v = ks * E + c;
-    const int tok = rb * kBlockRows + sl * E + q * VEC;
-    if (v < p.V && tok < p.ldt)
-      *reinterpret_cast<u32x4*>(dzT + blocked_index<T>(v, tok, n_tslab)) =
-          *reinterpret_cast<const u32x4*>(tile + c * kTPitch + (sl * E + q * VEC) * (int)sizeof(T));
-  }
 }
 
-// C (+)= A B^T with A [M x K] and B [N x K] K-blocked, C row-major in one of two orientations:
-//   kMContig = false: C[m][n], ld = ldc.  The N index runs along the lanes of an accumulator block
-//     (see gemm_core.hpp), so one store instruction writes whole 128-byte lines (32 lanes x 4 bytes,
-//     two rows): the orientation for fp32 outputs (dW: A = dz^T, B = hidden^T).
-//   kMContig = true:  C[n][m], ld = ldc.  The M index runs along a lane's registers, so a lane owns 4
-//     consecutive elements of a row per register quad: one 8-byte access instead of four 2-byte ones
-//     for 16-bit outputs (dhidden: A = W^T, B = dz).
-// Measured on the Qwen3-8B head: fp32 out, C[n][m] with 16-byte accesses (32 rows x 32 bytes per
-// instruction) is 4 % slower than C[m][n] with 4-byte ones (2 rows x 128 bytes): whole lines matter
-// more than the number of memory instructions; bf16 out gains 2 % from the 8-byte accesses.
+// C (+)= A B^T with A [M x K] and B [N x K] K-blocked, C row-major in one of two orientations; either way
+// a lane's 16-byte pieces lie along C's rows and a store instruction covers runs of at least 64 bytes:
+//   kMContig = false: C[m][n], ld = ldc, fp32 (dW: A = dz^T, B = hidden^T).  A lane holds 4 consecutive n of a row
+//     (GemmTile with BV = 4), 16 lanes 256 contiguous bytes of each of 4 rows.
+//   kMContig = true:  C[n][m], ld = ldc (dhidden: A = W^T, B = dz).  A lane holds VEC consecutive m of a row, the 4
+//     lane groups 64 contiguous bytes of each of 16 rows for 16-bit results.
+template <typename T, bool kMContig> using OutTile = GemmTile<T, kMContig ? 16 / (int)sizeof(T) : 4>;
+
 struct GemmParams {
   const void* A;      // M x K, K-blocked with a_kslabs slabs per row block
   const void* B;      // N x K, K-blocked with b_kslabs slabs per row block
@@ -305,131 +266,108 @@ struct GemmParams {
 };
 
 // Addresses of a 256 x 256 output tile for the accumulator layout: a range-checked buffer descriptor over
-// the tile's valid rows, one per-lane byte offset per 32-wide block of the lane dimension, and an offset
-// per accumulator register (kMContig: per register quad, a compile-time constant; otherwise a uniform
-// multiple of the row pitch, handed to the instruction as its scalar offset).  Along the lane dimension
-// (n) elements outside the tile get a per-lane offset far outside the descriptor: loads of them give 0
-// and stores are dropped.  Along the register dimension (m) nothing relies on the range check, because the
-// scalar offset is not part of it: kMContig skips whole quads (its M extents are multiples of 8), and the
-// other orientation tests every row against the tile's valid rows unless the tile is a full one.
+// the tile's valid rows and one per-lane byte offset per group of BV (kMContig: per block) of the lane dimension.
+// Along the lane dimension (n) elements outside the tile get a per-lane offset far outside the descriptor: loads
+// of them give 0 and stores are dropped.  Along the register dimension (m) nothing relies on the range check:
+// kMContig skips whole 32-row groups (its M extents are multiples of 32), and the other orientation tests
+// every row against the tile's valid rows unless the tile is a full one.
 template <typename T, typename OutT, bool kMContig>
 struct TileAddr {
-  using Tile = HeadTile<T>;
+  using Tile = OutTile<T, kMContig>;
   static constexpr int ES = (int)sizeof(OutT);
+  static constexpr int AG = Tile::VEC / 4;                  // blocks along m whose registers are consecutive
+  static constexpr int kGroups = kMContig ? Tile::NI : Tile::NI / 4;
   __amdgpu_buffer_rsrc_t rsrc;
-  int voff[Tile::NI];
-  int row_bytes, m_first, a_rows;
-  int row_lim;   // valid rows from this lane's first row on: register with row offset dm is inside iff dm < row_lim
+  int voff[kGroups];
+  int row_bytes, a_rows, row_lim;   // row_lim: valid rows from this lane's first row on
   __device__ __forceinline__ TileAddr(OutT* base, int64_t ld, int m0, int n0, int a_rows_, int b_rows) {
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int wm = wave % 2, wn = wave / 2;
     row_bytes = (int)(ld * (int64_t)ES);
-    m_first = wm * Tile::WM;
     a_rows = a_rows_;
-    row_lim = a_rows_ - (m_first + 4 * (lane >> 5));
+    const int m = Tile::wave_m() + Tile::lane_a0();
+    row_lim = a_rows_ - m;
     const int rows = kMContig ? b_rows : a_rows_, cols = kMContig ? a_rows_ : b_rows;
     const int bytes = rows > 0 ? (rows - 1) * row_bytes + cols * ES : 0;
     OutT* origin = kMContig ? base + (int64_t)n0 * ld + m0 : base + (int64_t)m0 * ld + n0;
     rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(origin), 0, bytes, 0x00020000);
 #pragma unroll
-    for (int ni = 0; ni < Tile::NI; ++ni) {
-      const int n = wn * Tile::WN + ni * 32 + (lane & 31);
-      const int m = m_first + 4 * (lane >> 5);
-      voff[ni] = n < b_rows ? (kMContig ? n * row_bytes + m * ES : m * row_bytes + n * ES) : 0x7f000000;
+    for (int k = 0; k < kGroups; ++k) {
+      const int n = Tile::wave_n() + Tile::lane_b0() + Tile::b_block(kMContig ? k : 4 * k);
+      voff[k] = n < b_rows ? (kMContig ? n * row_bytes + m * ES : m * row_bytes + n * ES) : 0x7f000000;
     }
   }
-  // offset of register r of block row mi from voff (rows 8 * (r / 4) + r % 4 of the block, plus the lane half's 4)
-  __device__ __forceinline__ int reg_off(int mi, int r) const {
-    const int dm = mi * 32 + 8 * (r >> 2) + (r & 3);
-    return kMContig ? dm * ES : dm * row_bytes;
-  }
-  __device__ __forceinline__ bool quad_ok(int mi, int q) const { return m_first + mi * 32 + 8 * q < a_rows; }
-  // row of register r of block row mi, relative to this lane's first row
-  __device__ static __forceinline__ int row_delta(int mi, int r) { return mi * 32 + 8 * (r >> 2) + (r & 3); }
+  // kMContig: blocks i .. i + AG - 1 lie inside the tile (uniform over the wave)
+  __device__ __forceinline__ bool group_ok(int i) const { return Tile::wave_m() + (Tile::a_block(i) & ~31) < a_rows; }
   __device__ __forceinline__ bool full_rows() const { return a_rows == Tile::BM; }
 };
 
-__device__ __forceinline__ float elem_load(const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, float*) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, voff, soff, 0));
+// N consecutive elements of a row: 4 or 8 floats, or 8 (T = bf16) 16-bit values.
+template <int N>
+__device__ __forceinline__ void row_load(float (&x)[N], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, float*) {
+#pragma unroll
+  for (int k = 0; k < N; k += 4) {
+    const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff + k * 4, soff, 0));
+    x[k] = v[0]; x[k + 1] = v[1]; x[k + 2] = v[2]; x[k + 3] = v[3];
+  }
 }
-__device__ __forceinline__ float elem_load(const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, __bf16*) {
-  return (float)__builtin_bit_cast(__bf16, __builtin_amdgcn_raw_buffer_load_b16(rsrc, voff, soff, 0));
+__device__ __forceinline__ void row_load(float (&x)[8], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, __bf16*) {
+  const bf16x8 v = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, soff, 0));
+#pragma unroll
+  for (int k = 0; k < 8; ++k) x[k] = (float)v[k];
 }
-__device__ __forceinline__ void elem_store(float v, const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, float*) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), rsrc, voff, soff, 0);
+template <int N>
+__device__ __forceinline__ void row_store(const float (&x)[N], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, float*) {
+#pragma unroll
+  for (int k = 0; k < N; k += 4) {
+    const f32x4 v = {x[k], x[k + 1], x[k + 2], x[k + 3]};
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, voff + k * 4, soff, 0);
+  }
 }
-__device__ __forceinline__ void elem_store(float v, const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, __bf16*) {
-  __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, (__bf16)v), rsrc, voff, soff, 0);
-}
-__device__ __forceinline__ void quad_load(f32x16& a, int q, const __amdgpu_buffer_rsrc_t& rsrc, int voff, float*) {
-  const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, 0, 0));
-  a[4 * q] = v[0]; a[4 * q + 1] = v[1]; a[4 * q + 2] = v[2]; a[4 * q + 3] = v[3];
-}
-__device__ __forceinline__ void quad_load(f32x16& a, int q, const __amdgpu_buffer_rsrc_t& rsrc, int voff, __bf16*) {
-  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-  const bf16x4 v = __builtin_bit_cast(bf16x4, __builtin_amdgcn_raw_buffer_load_b64(rsrc, voff, 0, 0));
-  a[4 * q] = (float)v[0]; a[4 * q + 1] = (float)v[1]; a[4 * q + 2] = (float)v[2]; a[4 * q + 3] = (float)v[3];
-}
-__device__ __forceinline__ void quad_store(const f32x16& a, int q, const __amdgpu_buffer_rsrc_t& rsrc, int voff, float*) {
-  const f32x4 v = {a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, voff, 0, 0);
-}
-__device__ __forceinline__ void quad_store(const f32x16& a, int q, const __amdgpu_buffer_rsrc_t& rsrc, int voff, __bf16*) {
-  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-  const bf16x4 v = {(__bf16)a[4 * q], (__bf16)a[4 * q + 1], (__bf16)a[4 * q + 2], (__bf16)a[4 * q + 3]};
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc, voff, 0, 0);
+__device__ __forceinline__ void row_store(const float (&x)[8], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, __bf16*) {
+  __builtin_amdgcn_raw_buffer_store_b128(pack_vec(x, (__bf16*)nullptr), rsrc, voff, soff, 0);
 }
 
-template <typename T, typename OutT, bool kMContig, typename AccT>
-__device__ __forceinline__ void tile_load(const TileAddr<T, OutT, kMContig>& at, AccT& acc) {
-  using Tile = HeadTile<T>;
-  const bool full = at.full_rows();   // uniform over the workgroup
+// fn(values of one run of a row, per-lane offset, scalar offset), for every run of the tile that lies inside it;
+// kLoad: the values go into the accumulators afterwards.
+template <typename T, typename OutT, bool kMContig, bool kLoad, typename AccT, typename Fn>
+__device__ __forceinline__ void for_rows(const TileAddr<T, OutT, kMContig>& at, AccT& acc, Fn fn) {
+  using Tile = OutTile<T, kMContig>;
+  if constexpr (kMContig) {
+    constexpr int AG = TileAddr<T, OutT, kMContig>::AG, N = 4 * AG;
 #pragma unroll
-  for (int ni = 0; ni < Tile::NI; ++ni)
+    for (int i = 0; i < Tile::MI; i += AG) {
+      if (!at.group_ok(i)) continue;
 #pragma unroll
-    for (int mi = 0; mi < Tile::MI; ++mi)
+      for (int j = 0; j < Tile::NI; ++j) {
+        float x[N] = {};
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (!at.quad_ok(mi, q)) continue;
-        if (kMContig) quad_load(acc[mi][ni], q, at.rsrc, at.voff[ni] + at.reg_off(mi, 4 * q), (OutT*)nullptr);
-        else if (full) {
+        for (int k = 0; k < (kLoad ? 0 : N); ++k) x[k] = acc_get(acc[i + k / 4][j], k % 4);
+        fn(x, at.voff[j] + Tile::a_block(i) * (int)sizeof(OutT), 0);
+        if (kLoad) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            acc[mi][ni][4 * q + i] = elem_load(at.rsrc, at.voff[ni], at.reg_off(mi, 4 * q + i), (OutT*)nullptr);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (at.row_delta(mi, 4 * q + i) < at.row_lim)
-              acc[mi][ni][4 * q + i] = elem_load(at.rsrc, at.voff[ni], at.reg_off(mi, 4 * q + i), (OutT*)nullptr);
+          for (int k = 0; k < N; k += 4) acc_set(acc[i + k / 4][j], x[k], x[k + 1], x[k + 2], x[k + 3]);
         }
       }
-}
-
-template <typename T, typename OutT, bool kMContig, typename AccT>
-__device__ __forceinline__ void tile_store(const TileAddr<T, OutT, kMContig>& at, const AccT& acc) {
-  using Tile = HeadTile<T>;
-  const bool full = at.full_rows();   // uniform over the workgroup
+    }
+  } else {
+    const bool full = at.full_rows();   // uniform over the workgroup
 #pragma unroll
-  for (int ni = 0; ni < Tile::NI; ++ni)
+    for (int i = 0; i < Tile::MI; ++i)
 #pragma unroll
-    for (int mi = 0; mi < Tile::MI; ++mi)
+      for (int j = 0; j < Tile::NI; j += 4) {
+        float x[4][4];                    // [register of the four blocks][block]
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (!at.quad_ok(mi, q)) continue;
-        if (kMContig) quad_store(acc[mi][ni], q, at.rsrc, at.voff[ni] + at.reg_off(mi, 4 * q), (OutT*)nullptr);
-        else if (full) {
+        for (int r = 0; r < 4; ++r) {
+          const int dm = Tile::a_block(i) + r;
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            elem_store(acc[mi][ni][4 * q + i], at.rsrc, at.voff[ni], at.reg_off(mi, 4 * q + i), (OutT*)nullptr);
-        } else {
+          for (int k = 0; k < 4; ++k) x[r][k] = kLoad ? 0.f : acc_get(acc[i][j + k], r);
+          if (full || dm < at.row_lim) fn(x[r], at.voff[j / 4], dm * at.row_bytes);
+        }
+        if (kLoad) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (at.row_delta(mi, 4 * q + i) < at.row_lim)
-              elem_store(acc[mi][ni][4 * q + i], at.rsrc, at.voff[ni], at.reg_off(mi, 4 * q + i), (OutT*)nullptr);
+          for (int k = 0; k < 4; ++k) acc_set(acc[i][j + k], x[0][k], x[1][k], x[2][k], x[3][k]);
         }
       }
+  }
 }
 
 // Accumulators of output tile (m0, n0) before its K loop: zeros, or - when the GEMM adds to C and one
@@ -437,33 +375,28 @@ __device__ __forceinline__ void tile_store(const TileAddr<T, OutT, kMContig>& at
 // in the epilogue puts the loads' latency in front of the K loop, where the first operand slabs are in
 // flight anyway, and leaves the epilogue a pure store.
 template <typename T, typename OutT, bool kMContig>
-__device__ __forceinline__ void gemm_init_tile(const GemmParams& p, f32x16 (&acc)[HeadTile<T>::MI][HeadTile<T>::NI],
-                                               int m0, int n0, int a_rows, int b_rows) {
-  using Tile = HeadTile<T>;
-#pragma unroll
-  for (int mi = 0; mi < Tile::MI; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < Tile::NI; ++ni)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
-  if (p.accumulate && p.k_split == 1) {
+__device__ __forceinline__ void gemm_init_tile(const GemmParams& p, typename OutTile<T, kMContig>::Acc& acc, int m0, int n0,
+                                               int a_rows, int b_rows) {
+  if (kMContig || !p.accumulate || p.k_split > 1) {
+    OutTile<T, kMContig>::zero(acc);
+  } else {
     const TileAddr<T, OutT, kMContig> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows);
-    tile_load(at, acc);
+    for_rows<T, OutT, kMContig, true>(at, acc, [&](auto& x, int voff, int soff) { row_load(x, at.rsrc, voff, soff, (OutT*)nullptr); });
   }
 }
 
 // Output tile from the accumulators: C = acc (the accumulators already hold C's previous contents
 // when the GEMM adds to it, see gemm_init_tile), or the fp32 partial of K range `ks`.
 template <typename T, typename OutT, bool kMContig>
-__device__ __forceinline__ void gemm_store_tile(const GemmParams& p, f32x16 (&acc)[HeadTile<T>::MI][HeadTile<T>::NI],
-                                                int m0, int n0, int a_rows, int b_rows, int ks) {
+__device__ __forceinline__ void gemm_store_tile(const GemmParams& p, typename OutTile<T, kMContig>::Acc& acc, int m0, int n0,
+                                                int a_rows, int b_rows, int ks) {
   if (p.k_split > 1) {
     const TileAddr<T, float, kMContig> at(p.partial + (int64_t)ks * p.M * p.N, kMContig ? p.M : p.N, m0, n0, a_rows, b_rows);
-    tile_store(at, acc);
+    for_rows<T, float, kMContig, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (float*)nullptr); });
     return;
   }
   const TileAddr<T, OutT, kMContig> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows);
-  tile_store(at, acc);
+  for_rows<T, OutT, kMContig, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (OutT*)nullptr); });
 }
 
 // Work item = (walk, fixed tile) when n_walk > 0: the workgroup keeps one operand's tile (A's m tile
@@ -471,58 +404,60 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, f32x16 (&ac
 // K loops stream into each other (the next tile's first slabs are requested while the current tile
 // finishes and is stored).  Otherwise work item = (K range, m tile, n tile), one K loop per workgroup.
 template <typename T, typename OutT, bool kMContig>
-__global__ __launch_bounds__(kHeadThreads) void gemm_nt_kernel(GemmParams p) {
-  using Tile = HeadTile<T>;
-  constexpr int MI = Tile::MI, NI = Tile::NI;
+__global__ __launch_bounds__(kHeadThreads, 1) void gemm_nt_kernel(GemmParams p) {
+  using Tile = OutTile<T, kMContig>;
   constexpr int64_t kSlabElems = (int64_t)kBlockRows * Tile::kSlabK;   // elements of one block's slab
   extern __shared__ __align__(16) char lds[];
 
-  int item = xcd_remap(blockIdx.x, gridDim.x);
-  f32x16 acc[MI][NI];
+  // this workgroup's tiles: (mt, nt) first, then `count - 1` steps along the walked operand; one K range
+  int item = xcd_remap(blockIdx.x, gridDim.x), mt, nt, count = 1, ks = 0, k0 = 0, k_len = p.K;
   if (p.n_walk > 0) {
     const int n_fixed = kMContig ? p.n_mt : p.n_nt;       // tiles of the operand that stays
     const int n_moving = kMContig ? p.n_nt : p.n_mt;      // tiles of the operand that is walked
     if (item >= p.n_walk * n_fixed) return;
     int walk, ft;
     grouped_tile(item, p.n_walk, n_fixed, 4, walk, ft);
-    const int w_begin = (int)((int64_t)walk * n_moving / p.n_walk);
-    const int w_end = (int)((int64_t)(walk + 1) * n_moving / p.n_walk);
-    typename Tile::Stream st;
-    for (int wt = w_begin; wt < w_end; ++wt) {
-      const int mt = kMContig ? ft : wt, nt = kMContig ? wt : ft;
-      const int m0 = mt * 256, n0 = nt * 256;
-      const int a_rows = (p.M - m0) < 256 ? (p.M - m0) : 256;
-      const int b_rows = (p.N - n0) < 256 ? (p.N - n0) : 256;
-      const int moving_left = (kMContig ? p.N : p.M) - (wt + 1) * 256;
-      const int next_rows = moving_left < 256 ? moving_left : 256;
-      const T* A = static_cast<const T*>(p.A) + (int64_t)mt * p.a_kslabs * kSlabElems;
-      const T* B = static_cast<const T*>(p.B) + (int64_t)nt * p.b_kslabs * kSlabElems;
-      const T* next = kMContig ? B + p.b_kslabs * kSlabElems : A + p.a_kslabs * kSlabElems;
-      gemm_init_tile<T, OutT, kMContig>(p, acc, m0, n0, a_rows, b_rows);
-      Tile::run(acc, Tile::Operand::blocked(A, a_rows), Tile::Operand::blocked(B, b_rows), p.K, lds, st,
-                (wt + 1 < w_end) ? next : nullptr, next_rows, true, /*next_is_b=*/kMContig);
-      gemm_store_tile<T, OutT, kMContig>(p, acc, m0, n0, a_rows, b_rows, 0);
-    }
-    return;
+    const int begin = (int)((int64_t)walk * n_moving / p.n_walk);
+    count = (int)((int64_t)(walk + 1) * n_moving / p.n_walk) - begin;
+    mt = kMContig ? ft : begin;
+    nt = kMContig ? begin : ft;
+  } else {
+    if (item >= p.n_mt * p.n_nt * p.k_split) return;
+    ks = item / (p.n_mt * p.n_nt);
+    item -= ks * (p.n_mt * p.n_nt);
+    grouped_tile(item, p.n_mt, p.n_nt, 8, mt, nt);
+    k0 = ks * p.k_per_split;
+    k_len = (p.K - k0) < p.k_per_split ? (p.K - k0) : p.k_per_split;
   }
 
-  if (item >= p.n_mt * p.n_nt * p.k_split) return;
-  const int ks = item / (p.n_mt * p.n_nt);
-  item -= ks * (p.n_mt * p.n_nt);
-  int mt, nt;
-  grouped_tile(item, p.n_mt, p.n_nt, 8, mt, nt);
-  const int m0 = mt * 256, n0 = nt * 256;
-  const int a_rows = (p.M - m0) < 256 ? (p.M - m0) : 256;
-  const int b_rows = (p.N - n0) < 256 ? (p.N - n0) : 256;
-  const int k0 = ks * p.k_per_split;
-  const int k_len = (p.K - k0) < p.k_per_split ? (p.K - k0) : p.k_per_split;
-  gemm_init_tile<T, OutT, kMContig>(p, acc, m0, n0, a_rows, b_rows);
-
+  const int nslab = k_len / Tile::kSlabK;
   const int64_t s0 = k0 / Tile::kSlabK;   // first slab of this K range
-  Tile::run(acc, Tile::Operand::blocked(static_cast<const T*>(p.A) + ((int64_t)mt * p.a_kslabs + s0) * kSlabElems, a_rows),
-            Tile::Operand::blocked(static_cast<const T*>(p.B) + ((int64_t)nt * p.b_kslabs + s0) * kSlabElems, b_rows),
-            k_len, lds);
-  gemm_store_tile<T, OutT, kMContig>(p, acc, m0, n0, a_rows, b_rows, ks);
+  const bool stream = Tile::can_stream(nslab);
+  typename Tile::Acc acc;
+  Tile core;
+  for (int k = 0; k < count; ++k) {
+    const int m0 = mt * 256, n0 = nt * 256;
+    const int a_rows = (p.M - m0) < 256 ? (p.M - m0) : 256;
+    const int b_rows = (p.N - n0) < 256 ? (p.N - n0) : 256;
+    const auto op_a = Tile::Operand::blocked(static_cast<const T*>(p.A) + ((int64_t)mt * p.a_kslabs + s0) * kSlabElems, a_rows);
+    const auto op_b = Tile::Operand::blocked(static_cast<const T*>(p.B) + ((int64_t)nt * p.b_kslabs + s0) * kSlabElems, b_rows);
+    gemm_init_tile<T, OutT, kMContig>(p, acc, m0, n0, a_rows, b_rows);
+    if (k == 0 || !stream) core.start(op_a, op_b, nslab, lds);
+    core.next_a = Tile::hold(op_a, nslab);
+    core.next_b = Tile::hold(op_b, nslab);
+    if (stream && k + 1 < count) {
+      const int left = (kMContig ? p.N - n0 : p.M - m0) - 256;
+      const int next_rows = left < 256 ? left : 256;
+      core.next_a = kMContig ? Tile::cursor(op_a, nslab)
+                             : Tile::cursor(Tile::Operand::blocked(op_a.base + p.a_kslabs * kSlabElems, next_rows), nslab);
+      core.next_b = kMContig ? Tile::cursor(Tile::Operand::blocked(op_b.base + p.b_kslabs * kSlabElems, next_rows), nslab)
+                             : Tile::cursor(op_b, nslab);
+    }
+    core.run(acc, nslab);
+    if (!stream || k + 1 == count) Tile::finish();
+    gemm_store_tile<T, OutT, kMContig>(p, acc, m0, n0, a_rows, b_rows, ks);
+    if (kMContig) ++nt; else ++mt;
+  }
 }
 
 template <typename OutT> __device__ __forceinline__ OutT cvt_out(float v);
@@ -747,7 +682,7 @@ template <typename T, typename OutT, bool kMContig>
 static int launch_gemm_one(const void* A, int64_t a_kslabs, int M, const void* B, int64_t b_kslabs, int N, int K, void* C,
                            int64_t ldc, int accumulate, hipStream_t stream, float* partial, size_t partial_bytes,
                            int k_split_wanted) {
-  using Tile = HeadTile<T>;
+  using Tile = OutTile<T, kMContig>;
   int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_nt_kernel<T, OutT, kMContig>), Tile::kLdsBytes, "gemm_nt_kernel");
   if (rc) return rc;
   GemmParams g;
@@ -796,7 +731,7 @@ template <typename T, typename OutT, bool kMContig>
 static int launch_gemm(const void* A, int64_t a_kslabs, int M, const void* B, int64_t b_kslabs, int N, int K, void* C,
                        int64_t ldc, int accumulate, hipStream_t stream, float* partial = nullptr,
                        size_t partial_bytes = 0) {
-  using Tile = HeadTile<T>;
+  using Tile = OutTile<T, kMContig>;
   constexpr int64_t kSlabElems = (int64_t)kBlockRows * Tile::kSlabK;
   if (!kMContig) {
     // dW: equally long walks over most vocabulary tiles, the rest cut into K ranges (plan_dweight)
@@ -836,7 +771,7 @@ static int launch_transpose(const T* src, int64_t ld_src, T* dst, int64_t ld_dst
 
 template <typename T>
 static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t label_offset) {
-  using Tile = HeadTile<T>;
+  using Tile = LogitTile<T>;
   const int64_t T_ = a->T, H = a->H, V = a->V;
   const bool saved = a->saved_logits != nullptr;
   const bool own_wt = a->weight_t == nullptr;
@@ -881,7 +816,11 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
       q.ldv = (int)ldz;
       q.c = a->inv_temperature * kLog2e;
       q.inv_temperature = a->inv_temperature;
-      dim3 grid((unsigned)((tc + kBlockRows - 1) / kBlockRows), (unsigned)(ldz / Elem<T>::kSlabK));
+      // a workgroup walks units of one token block, so that its coefficients are fetched once; 16 workgroups per CU
+      const int64_t n_tb = (tc + kBlockRows - 1) / kBlockRows, n_units = ldz / Elem<T>::kSlabK;
+      int64_t per_tb = (16 * (int64_t)device_cu_count() + n_tb - 1) / n_tb;
+      if (per_tb > n_units) per_tb = n_units;
+      dim3 grid((unsigned)n_tb, (unsigned)per_tb);
       hipLaunchKernelGGL(dz_from_z_kernel<T>, grid, dim3(256), 0, stream, q);
       rc = check_launch("dz_from_z_kernel");
       if (rc) return rc;

@@ -9,7 +9,7 @@
 // exact rescale and writes logprob / entropy / rowmax / lse.  Logits go to
 // memory only when the caller asks for a chunk's raw logits to be kept for the
 // backward; they then leave straight from the accumulators, 16 bytes per lane,
-// in the accumulators' own order (see ZNative).
+// in the layout of the backward's operand (see KeptLogit).
 //
 // Algorithmic work: 2*T*H*V flop; bytes 2*T*H + 2*V*H (bf16) + 16*T.
 #include "common.hpp"
@@ -20,6 +20,7 @@ namespace clgrpo {
 constexpr int kFwdBM = 256, kFwdBN = 256;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kMaxFwdSplits = 64;   // most vocabulary splits a forward launch uses
+constexpr float kNoLogit = -3.0e38f;   // stands for a vocabulary row past V: finite, so that 0 * kNoLogit is 0
 
 struct FwdParams {
   const void* hidden;
@@ -29,7 +30,7 @@ struct FwdParams {
   int T, H, V;
   int n_tb, n_split, tiles_per_split, n_vt;
   float c;  // inv_temperature * log2(e)
-  void* z_out;   // optional raw logits, z-native layout (see ZNative): rows x ldz entries of KeptLogit<T>
+  void* z_out;   // optional raw logits, K-blocked: rows x ldz entries of KeptLogit<T>
   int64_t ldz;
   const int32_t* z_row_map;  // optional [T]: destination row per token, < 0: not stored
   int z_rows;                // rows of z_out; mapped rows outside [0, z_rows) are not stored
@@ -37,18 +38,17 @@ struct FwdParams {
   int xcd_wgs;   // > 0: launch of several rounds, see xcd_round_remap
 };
 
-// 16 bytes of kept logits from consecutive accumulator registers.
-template <typename ZT> __device__ __forceinline__ u32x4 pack_piece(const f32x16& a, int first);
-template <> __device__ __forceinline__ u32x4 pack_piece<float>(const f32x16& a, int first) {
-  f32x4 v = {a[first], a[first + 1], a[first + 2], a[first + 3]};
-  return __builtin_bit_cast(u32x4, v);
+// 16 bytes of kept logits: consecutive vocabulary entries of one token.
+__device__ __forceinline__ u32x4 pack_kept(const float (&v)[4], float*) {
+  const f32x4 x = {v[0], v[1], v[2], v[3]};
+  return __builtin_bit_cast(u32x4, x);
 }
-template <> __device__ __forceinline__ u32x4 pack_piece<_Float16>(const f32x16& a, int first) {
+__device__ __forceinline__ u32x4 pack_kept(const float (&v)[8], _Float16*) {
   typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-  f16x8 v;
+  f16x8 x;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) v[e] = (_Float16)a[first + e];     // round to nearest even
-  return __builtin_bit_cast(u32x4, v);
+  for (int e = 0; e < 8; ++e) x[e] = (_Float16)v[e];     // round to nearest even
+  return __builtin_bit_cast(u32x4, x);
 }
 
 __device__ __forceinline__ void merge_state(float& m, float& s, float& u, float om, float os,
@@ -62,9 +62,9 @@ __device__ __forceinline__ void merge_state(float& m, float& s, float& u, float 
 }
 
 template <typename T, bool STORE_Z>
-__global__ __launch_bounds__(kHeadThreads) void lmhead_fwd_kernel(FwdParams p) {
-  using Tile = HeadTile<T>;
-  constexpr int MI = Tile::MI, NI = Tile::NI, WM = Tile::WM, WN = Tile::WN;
+__global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p) {
+  using Tile = LogitTile<T>;
+  constexpr int MI = Tile::MI, NI = Tile::NI, VEC = Tile::VEC;
   extern __shared__ __align__(16) char lds[];
 
   const int item = work_item(p.xcd_wgs);
@@ -79,8 +79,9 @@ __global__ __launch_bounds__(kHeadThreads) void lmhead_fwd_kernel(FwdParams p) {
   }
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm = wave % 2, wn = wave / 2;
+  const int wm = Tile::wave_m(), wn = Tile::wave_n();
+  const int la = wm + Tile::lane_a0();               // this lane's first vocabulary row / token of the tile
+  const int lb = wn + Tile::lane_b0();
   const int t0 = tb * kFwdBN;
   const int b_rows = (p.T - t0) < kFwdBN ? (p.T - t0) : kFwdBN;
   const T* hidden = static_cast<const T*>(p.hidden) + (int64_t)t0 * p.H;
@@ -90,174 +91,155 @@ __global__ __launch_bounds__(kHeadThreads) void lmhead_fwd_kernel(FwdParams p) {
   int lab[NI], zrow[NI];
   float m[NI], s[NI], u[NI], zt[NI];
 #pragma unroll
-  for (int ni = 0; ni < NI; ++ni) {
-    const int tok = t0 + wn * WN + ni * 32 + (lane & 31);
-    lab[ni] = -1;
+  for (int j = 0; j < NI; ++j) {
+    const int tok = t0 + lb + Tile::b_block(j);
+    lab[j] = -1;
     if (p.labels != nullptr && tok < p.T) {
       const int64_t rel = p.labels[tok] - p.label_offset;   // a label outside these rows matches nothing
-      if (rel >= 0 && rel < p.V) lab[ni] = (int)rel;
+      if (rel >= 0 && rel < p.V) lab[j] = (int)rel - la;
+      else lab[j] = -0x40000000;
+    } else {
+      lab[j] = -0x40000000;
     }
-    zrow[ni] = (STORE_Z && tok < p.T) ? (p.z_row_map ? p.z_row_map[tok] : tok) : -1;
-    if (zrow[ni] >= p.z_rows) zrow[ni] = -1;
-    m[ni] = -INFINITY;
-    s[ni] = 0.f;
-    u[ni] = 0.f;
-    zt[ni] = 0.f;
+    zrow[j] = (STORE_Z && tok < p.T) ? (p.z_row_map ? p.z_row_map[tok] : tok) : -1;
+    if (zrow[j] >= p.z_rows) zrow[j] = -1;
+    m[j] = -INFINITY;
+    s[j] = 0.f;
+    u[j] = 0.f;
+    zt[j] = 0.f;
   }
 
-  typename Tile::Stream st;
+  Tile core;
+  const int nslab = p.H / Tile::kSlabK;
+  const bool stream = Tile::can_stream(nslab);
+  const auto op_b = Tile::Operand::row_major(hidden, p.H, b_rows);
   const int vt_begin = vs * p.tiles_per_split;
   const int vt_end = (vt_begin + p.tiles_per_split) < p.n_vt ? (vt_begin + p.tiles_per_split) : p.n_vt;
   for (int vt = vt_begin; vt < vt_end; ++vt) {
     const int v0 = vt * kFwdBM;
     const int a_rows = (p.V - v0) < kFwdBM ? (p.V - v0) : kFwdBM;
-    f32x16 acc[MI][NI];
-#pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-      for (int ni = 0; ni < NI; ++ni)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[mi][ni][r] = 0.f;
+    const auto op_a = Tile::Operand::row_major(weight + (int64_t)v0 * p.H, p.H, a_rows);
+    typename Tile::Acc acc;
+    Tile::zero(acc);
+    if (vt == vt_begin || !stream) core.start(op_a, op_b, nslab, lds);
+    if (stream && vt + 1 < vt_end) {
+      const int v1 = v0 + kFwdBM;
+      const int next_rows = (p.V - v1) < kFwdBM ? (p.V - v1) : kFwdBM;
+      core.next_a = Tile::cursor(Tile::Operand::row_major(weight + (int64_t)v1 * p.H, p.H, next_rows), nslab);
+      core.next_b = Tile::cursor(op_b, nslab);
+    } else {
+      core.next_a = Tile::hold(op_a, nslab);
+      core.next_b = Tile::hold(op_b, nslab);
+    }
+    core.run(acc, nslab);
+    if (!stream) Tile::finish();
 
-    // The K loop requests the first slabs of the next vocabulary tile during its last two slab periods.
-    const bool has_next = vt + 1 < vt_end;
-    const int v1 = v0 + kFwdBM;
-    const int next_rows = (p.V - v1) < kFwdBM ? (p.V - v1) : kFwdBM;
-    const T* next_w = weight + (int64_t)v1 * p.H;
-    Tile::run(acc, Tile::Operand::row_major(weight + (int64_t)v0 * p.H, p.H, a_rows),
-              Tile::Operand::row_major(hidden, p.H, b_rows), p.H, lds, st, has_next ? next_w : nullptr, next_rows, true);
-
-    if (STORE_Z) {
-      // Raw logits for the backward, straight from the accumulators: per 32x32 block a lane stores its
-      // 16 values as 16-byte pieces, each piece of the 64 lanes one contiguous KB (z-native layout).
-      // Vocabulary rows past V hold zeros already (the operand loads are range-checked), and the
-      // backward ignores whatever the padding columns hold.
-      typedef typename KeptLogit<T>::type ZT;
-      typedef ZNative<ZT> ZL;
-      char* z = static_cast<char*>(p.z_out);
-      const int64_t n_kslab = p.ldz / ZL::kSlabElems;
+    const bool full = a_rows == kFwdBM;
 #pragma unroll
-      for (int ni = 0; ni < NI; ++ni) {
+    for (int j = 0; j < NI; ++j) {
+      // this token's logits of the lane's vocabulary rows
+      float x[MI * 4];
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[i * 4 + r] = acc_get(acc[i][j], r);
+
+      if (STORE_Z) {
+        // Raw logits for the backward: VEC consecutive vocabulary entries of a token are one 16-byte piece of
+        // the K-blocked layout.  Vocabulary rows past V hold zeros already (the operand loads are
+        // range-checked), and the backward ignores whatever the padding columns hold.
+        typedef typename KeptLogit<T>::type ZT;
+        constexpr int AG = VEC / 4;                     // blocks whose registers make up one piece
         // The row is the same for every vocabulary tile, so the compiler would keep the 64-bit addresses it
         // forms from it alive across the K loops, where registers are scarcest, spill them, and reload them
         // between the stores (a reload waits for the stores issued before it).  Re-deriving them from the
         // 32-bit row costs a handful of instructions per tile.
-        int row = zrow[ni];
+        int row = zrow[j];
         asm volatile("" : "+v"(row));
-        if (row < 0) continue;
+        if (row >= 0) {
+          const int64_t n_kslab = p.ldz / Tile::kSlabK;
+          char* z_row = static_cast<char*>(p.z_out) +
+                        ((int64_t)(row / kBlockRows) * n_kslab * kBlockRows + row % kBlockRows) * kRowBytes;
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi) {
-          const int v_blk = v0 + wm * WM + mi * 32;
-          if (v_blk >= p.ldz) continue;
+          for (int i = 0; i < MI; i += AG) {
+            const int v = v0 + la + Tile::a_block(i);
+            if (!full && v >= p.ldz) continue;
+            float piece[VEC];
 #pragma unroll
-          for (int j = 0; j < ZL::PIECES; ++j)
-            *reinterpret_cast<u32x4*>(z + ZL::piece_offset(row, v_blk >> 5, n_kslab, lane >> 5, j)) =
-                pack_piece<ZT>(acc[mi][ni], j * ZL::kPerPiece);
+            for (int e = 0; e < VEC; ++e) piece[e] = x[i * 4 + e];
+            *reinterpret_cast<u32x4*>(z_row + (int64_t)(v / Tile::kSlabK) * (kBlockRows * kRowBytes) +
+                                      (v % Tile::kSlabK) * (int)sizeof(ZT)) = pack_kept(piece, (ZT*)nullptr);
+          }
         }
       }
-    }
 
-    if (a_rows == kFwdBM) {
+      // Target logit: only a lane whose rows of this tile hold the label looks for it.
+      const int rel = lab[j] - v0;
+      if (__any((unsigned)rel < (unsigned)Tile::WM)) {
 #pragma unroll
-      for (int ni = 0; ni < NI; ++ni) {
-        float tmax = acc[0][ni][0];
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, acc[mi][ni][r]);
-        const float nm = fmaxf(m[ni], tmax);
-        const float scale = exp2f((m[ni] - nm) * c);  // m = -inf on the first tile -> 0
-        const float nb = -nm * c;
-        float ls = 0.f, lu = 0.f;
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float v = acc[mi][ni][r];
-            const float e = __builtin_amdgcn_exp2f(fmaf(v, c, nb));
-            ls += e;
-            lu = fmaf(e, v, lu);
-          }
-        s[ni] = fmaf(s[ni], scale, ls);
-        u[ni] = fmaf(u[ni], scale, lu);
-        m[ni] = nm;
+          for (int r = 0; r < 4; ++r)
+            if (rel == Tile::a_block(i) + r) zt[j] = x[i * 4 + r];
       }
-    } else {
-      // Last, partial vocabulary tile: rows >= a_rows are clamped duplicates and must not count.
-#pragma unroll
-      for (int ni = 0; ni < NI; ++ni) {
-        float tmax = -INFINITY;
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int row = wm * WM + mi * 32 + acc_row(r, lane);
-            if (row < a_rows) tmax = fmaxf(tmax, acc[mi][ni][r]);
-          }
-        const float nm = fmaxf(m[ni], tmax);
-        if (nm == -INFINITY) continue;  // this lane has seen no valid row yet
-        const float scale = exp2f((m[ni] - nm) * c);
-        const float nb = -nm * c;
-        float ls = 0.f, lu = 0.f;
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int row = wm * WM + mi * 32 + acc_row(r, lane);
-            if (row < a_rows) {
-              const float v = acc[mi][ni][r];
-              const float e = __builtin_amdgcn_exp2f(fmaf(v, c, nb));
-              ls += e;
-              lu = fmaf(e, v, lu);
-            }
-          }
-        s[ni] = fmaf(s[ni], scale, ls);
-        u[ni] = fmaf(u[ni], scale, lu);
-        m[ni] = nm;
-      }
-    }
 
-    // Target logit: only the wave whose 128 vocabulary rows hold the label looks for it.
+      if (!full) {
+        // last, partial vocabulary tile: the zeros of rows past V must not count
 #pragma unroll
-    for (int ni = 0; ni < NI; ++ni) {
-      const int rel = lab[ni] - (v0 + wm * WM);
-      const bool in = (unsigned)rel < (unsigned)WM && (lab[ni] < p.V);
-      if (__any(in)) {
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (rel == mi * 32 + acc_row(r, lane)) zt[ni] = acc[mi][ni][r];
+          for (int r = 0; r < 4; ++r)
+            if (la + Tile::a_block(i) + r >= a_rows) x[i * 4 + r] = kNoLogit;
       }
+      float tmax = x[0];
+#pragma unroll
+      for (int k = 1; k < MI * 4; ++k) tmax = fmaxf(tmax, x[k]);
+      if (!full && tmax == kNoLogit && m[j] == -INFINITY) continue;   // this lane has seen no valid row yet
+      const float nm = fmaxf(m[j], tmax);
+      const float scale = exp2f((m[j] - nm) * c);  // m = -inf on the first tile -> 0
+      const float nb = -nm * c;
+      float ls = 0.f, lu = 0.f;
+#pragma unroll
+      for (int k = 0; k < MI * 4; ++k) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(x[k], c, nb));
+        ls += e;
+        lu = fmaf(e, x[k], lu);
+      }
+      s[j] = fmaf(s[j], scale, ls);
+      u[j] = fmaf(u[j], scale, lu);
+      m[j] = nm;
     }
   }
+  if (stream) Tile::finish();
 
-  // Merge the two lane halves (same tokens, different vocabulary rows).
+  // Merge the four lanes that hold the same token's other vocabulary rows.
 #pragma unroll
-  for (int ni = 0; ni < NI; ++ni) {
-    const float om = __shfl_xor(m[ni], 32);
-    const float os = __shfl_xor(s[ni], 32);
-    const float ou = __shfl_xor(u[ni], 32);
-    const float oz = __shfl_xor(zt[ni], 32);
-    merge_state(m[ni], s[ni], u[ni], om, os, ou, c);
-    zt[ni] += oz;
+  for (int j = 0; j < NI; ++j) {
+#pragma unroll
+    for (int off = 16; off < 64; off <<= 1) {
+      const float om = __shfl_xor(m[j], off);
+      const float os = __shfl_xor(s[j], off);
+      const float ou = __shfl_xor(u[j], off);
+      const float oz = __shfl_xor(zt[j], off);
+      merge_state(m[j], s[j], u[j], om, os, ou, c);
+      zt[j] += oz;
+    }
   }
-  // Merge the two waves that share these tokens (wm = 0, 1) through LDS.
+  // Merge the two waves that share these tokens through LDS.
   float4* xch = reinterpret_cast<float4*>(lds);
-  if (wm == 1 && lane < 32) {
+  if (wm != 0 && lane < 16) {
 #pragma unroll
-    for (int ni = 0; ni < NI; ++ni)
-      xch[wn * WN + ni * 32 + lane] = make_float4(m[ni], s[ni], u[ni], zt[ni]);
+    for (int j = 0; j < NI; ++j) xch[lb + Tile::b_block(j)] = make_float4(m[j], s[j], u[j], zt[j]);
   }
   __syncthreads();
-  if (wm == 0 && lane < 32) {
+  if (wm == 0 && lane < 16) {
 #pragma unroll
-    for (int ni = 0; ni < NI; ++ni) {
-      const float4 o = xch[wn * WN + ni * 32 + lane];
-      merge_state(m[ni], s[ni], u[ni], o.x, o.y, o.z, c);
-      zt[ni] += o.w;
-      const int tok = t0 + wn * WN + ni * 32 + lane;
-      if (tok < p.T) p.part[(int64_t)vs * p.T + tok] = make_float4(m[ni], s[ni], u[ni], zt[ni]);
+    for (int j = 0; j < NI; ++j) {
+      const float4 o = xch[lb + Tile::b_block(j)];
+      merge_state(m[j], s[j], u[j], o.x, o.y, o.z, c);
+      zt[j] += o.w;
+      const int tok = t0 + lb + Tile::b_block(j);
+      if (tok < p.T) p.part[(int64_t)vs * p.T + tok] = make_float4(m[j], s[j], u[j], zt[j]);
     }
   }
 }
@@ -335,7 +317,7 @@ static long fwd_single_cost(int n_tb, int n_vt, int cus, int& n_split, int& tile
 
 template <typename T, bool STORE_Z>
 static int launch_fwd(const clgrpo_lmhead_fwd_args* a, hipStream_t stream, int64_t label_offset, float4* record) {
-  using Tile = HeadTile<T>;
+  using Tile = LogitTile<T>;
   FwdParams p;
   p.hidden = a->hidden;
   p.weight = a->weight;

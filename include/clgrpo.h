@@ -43,8 +43,9 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *   2.00 -> 2.01: clgrpo_lmhead_bwd_workspace_bytes sizes the split-K partials by the GEMM's plan (smaller in
  *                 general); clgrpo_lmhead_fwd_launch_plan and clgrpo_lmhead_bwd_dhidden_plan added.
  *   2.01 -> 2.02: clgrpo_lmhead_bwd_workspace_bytes also covers the partials of the dW GEMM's tail launch (a few
- *                 tens of MB more for some shapes); clgrpo_lmhead_bwd_dweight_plan added. */
-#define CLGRPO_VERSION 202
+ *                 tens of MB more for some shapes); clgrpo_lmhead_bwd_dweight_plan added.
+ *   2.02 -> 2.03: kept logits lie in the K-blocked layout that d(logits) takes over (still opaque to callers). */
+#define CLGRPO_VERSION 203
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
 
@@ -73,13 +74,11 @@ typedef struct {
                               clgrpo_lmhead_bwd of the SAME rows that then skips the recomputation.  NULL: nothing
                               is stored.  Callers bound its size by processing a micro-batch in token chunks.
                               The buffer is opaque to the caller: ceil(rows / 256) * 256 rows of ld_saved elements
-                              of sizeof(dtype) bytes.  The forward fills it in the order of its accumulators
-                              (32 KB units of 256 rows x 128 bytes of vocabulary, inside a unit 32 x 32 sub-blocks
-                              stored as 16-byte pieces per lane; 16-bit inputs keep their logits as IEEE half, a raw
-                              logit beyond +-65504 as +-65504: the backward's gradients stay finite, but that
-                              token's probabilities are then formed from the saturated value);
-                              the backward overwrites every unit in place with d(logits) as the K-blocked operand
-                              of its GEMMs: element (row, k) at
+                              of sizeof(dtype) bytes.  The forward fills it with logits (16-bit inputs keep them as
+                              IEEE half, a raw logit beyond +-65504 as +-65504: the backward's gradients stay
+                              finite, but that token's probabilities are then formed from the saturated value), the
+                              backward overwrites it with d(logits), both in the K-blocked layout of the GEMM
+                              operands: element (row, k) at
                               (((row / 256) * (ld_saved / E) + k / E) * 256 + row % 256) * E + k % E,
                               E = 128 / sizeof(dtype). */
   int64_t ld_saved;        /* K extent in elements, a multiple of 64, >= clgrpo_saved_logits_ld(V) */
