@@ -19,7 +19,10 @@ namespace clgrpo {
 
 constexpr int kFwdBM = 256, kFwdBN = 256;
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr int kMaxFwdSplits = 64;   // most vocabulary splits a forward launch uses
+// Most vocabulary splits a forward launch of n_tb token blocks uses: 4096 workgroups in all, 64 splits at least
+// (the partial records of up to 16384 tokens then stay below 17 MB).  A few token blocks need many splits to reach all
+// CUs: with 64 at most, one block of a 152k vocabulary ran on 60 of 256 CUs, three blocks on 180.
+inline int max_fwd_splits(int64_t n_tb) { return n_tb >= 64 ? 64 : (int)(4096 / n_tb); }
 constexpr float kNoLogit = -3.0e38f;   // stands for a vocabulary row past V: finite, so that 0 * kNoLogit is 0
 
 struct FwdParams {
@@ -256,15 +259,47 @@ struct FinalizeParams {
   float4* record;   // non-null: only the merged (max, sum, sum*z, target) record is written
 };
 
-__global__ void lmhead_fwd_finalize_kernel(FinalizeParams p) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= p.T) return;
+// G threads per token, each merging every G-th split, then each other through LDS; a block is 256 / G consecutive
+// tokens wide.  The loop over splits is a chain of merges behind loads: with one thread per token 60 splits
+// took 21 us whatever the number of tokens (four loads are in flight per thread now, and G = 8 cuts the chain).
+constexpr int kFinalizeThreads = 256;
+template <int G>
+__global__ __launch_bounds__(kFinalizeThreads) void lmhead_fwd_finalize_kernel(FinalizeParams p) {
+  constexpr int kTok = kFinalizeThreads / G;
+  const int g = threadIdx.x / kTok, t = blockIdx.x * kTok + threadIdx.x % kTok;
   float m = -INFINITY, s = 0.f, u = 0.f, zt = 0.f;
-  for (int k = 0; k < p.n_split; ++k) {
-    const float4 o = p.part[(int64_t)k * p.T + t];
-    merge_state(m, s, u, o.x, o.y, o.z, p.c);
-    zt += o.w;
+  if (t < p.T) {
+    const float4* part = p.part + t;
+    int k = g;
+    for (; k + 3 * G < p.n_split; k += 4 * G) {
+      float4 o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = part[(int64_t)(k + e * G) * p.T];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        merge_state(m, s, u, o[e].x, o[e].y, o[e].z, p.c);
+        zt += o[e].w;
+      }
+    }
+    for (; k < p.n_split; k += G) {
+      const float4 o = part[(int64_t)k * p.T];
+      merge_state(m, s, u, o.x, o.y, o.z, p.c);
+      zt += o.w;
+    }
   }
+  if (G > 1) {
+    __shared__ float4 sh[kFinalizeThreads];
+    sh[threadIdx.x] = make_float4(m, s, u, zt);
+    __syncthreads();
+    if (g != 0) return;
+#pragma unroll
+    for (int e = 1; e < G; ++e) {
+      const float4 o = sh[e * kTok + threadIdx.x];
+      merge_state(m, s, u, o.x, o.y, o.z, p.c);
+      zt += o.w;
+    }
+  }
+  if (t >= p.T) return;
   if (p.record) {
     p.record[t] = make_float4(m, s, u, zt);
     return;
@@ -279,6 +314,14 @@ __global__ void lmhead_fwd_finalize_kernel(FinalizeParams p) {
     // A label outside [0, V) has no logit; NaN marks it instead of a silent wrong number.
     p.logprob[t] = (lab >= 0 && lab < p.V) ? (zt * p.inv_temperature - lse) : NAN;
   }
+}
+
+static int launch_finalize(const FinalizeParams& f, hipStream_t stream) {
+  if (f.n_split >= 16)
+    hipLaunchKernelGGL(lmhead_fwd_finalize_kernel<8>, dim3((f.T + 31) / 32), dim3(kFinalizeThreads), 0, stream, f);
+  else
+    hipLaunchKernelGGL(lmhead_fwd_finalize_kernel<1>, dim3((f.T + 255) / 256), dim3(kFinalizeThreads), 0, stream, f);
+  return check_launch("lmhead_fwd_finalize_kernel");
 }
 
 // Split of the vocabulary tiles over workgroups.  A workgroup walks ceil(n_vt / n_split) tiles for
@@ -301,7 +344,8 @@ static long fwd_single_cost(int n_tb, int n_vt, int cus, int& n_split, int& tile
   const double xcd_wgs = cus / 8.0, full_block = 4.0 + xcd_wgs / 4.0;
   int best = 1;
   double best_cost = -1.0;
-  for (int sp = 1; sp <= kMaxFwdSplits && sp <= n_vt; ++sp) {
+  const int most = max_fwd_splits(n_tb) < n_vt ? max_fwd_splits(n_tb) : n_vt;
+  for (int sp = 1; sp <= most; ++sp) {
     const int tps = (n_vt + sp - 1) / sp;
     const int eff_sp = (n_vt + tps - 1) / tps;
     const long rounds = ((long)n_tb * eff_sp + cus - 1) / cus;
@@ -356,8 +400,7 @@ static int launch_fwd(const clgrpo_lmhead_fwd_args* a, hipStream_t stream, int64
   f.rowmax = a->rowmax;
   f.lse = a->lse;
   f.record = record;
-  hipLaunchKernelGGL(lmhead_fwd_finalize_kernel, dim3((p.T + 255) / 256), dim3(256), 0, stream, f);
-  return check_launch("lmhead_fwd_finalize_kernel");
+  return launch_finalize(f, stream);
 }
 
 int validate_head_shape(const char* who, int64_t T, int64_t H, int64_t V, int32_t dtype) {
@@ -393,9 +436,9 @@ extern "C" size_t clgrpo_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_
   (void)dtype;
   if (T <= 0 || V <= 0) return 0;
   // one record per token and vocabulary split; the split count depends on the device's CU count and never
-  // exceeds kMaxFwdSplits, so this bound holds on any device
-  const int64_t n_vt = (V + kFwdBM - 1) / kFwdBM;
-  const int64_t splits = n_vt < kMaxFwdSplits ? n_vt : kMaxFwdSplits;
+  // exceeds max_fwd_splits, so this bound holds on any device
+  const int64_t n_vt = (V + kFwdBM - 1) / kFwdBM, most = max_fwd_splits((T + kFwdBN - 1) / kFwdBN);
+  const int64_t splits = n_vt < most ? n_vt : most;
   return (size_t)splits * (size_t)T * sizeof(float4);
 }
 
@@ -463,6 +506,5 @@ extern "C" int clgrpo_lmhead_merge_shards(const void* records, int64_t n_shards,
   f.rowmax = rowmax;
   f.lse = lse;
   f.record = nullptr;
-  hipLaunchKernelGGL(lmhead_fwd_finalize_kernel, dim3((f.T + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream), f);
-  return check_launch("lmhead_fwd_finalize_kernel");
+  return launch_finalize(f, static_cast<hipStream_t>(stream));
 }

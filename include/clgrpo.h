@@ -44,7 +44,8 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *                 general); clgrpo_lmhead_fwd_launch_plan and clgrpo_lmhead_bwd_dhidden_plan added.
  *   2.01 -> 2.02: clgrpo_lmhead_bwd_workspace_bytes also covers the partials of the dW GEMM's tail launch (a few
  *                 tens of MB more for some shapes); clgrpo_lmhead_bwd_dweight_plan added.
- *   2.02 -> 2.03: kept logits lie in the K-blocked layout that d(logits) takes over (still opaque to callers). */
+ *   2.02 -> 2.03: kept logits lie in the K-blocked layout that d(logits) takes over (still opaque to callers);
+ *                 clgrpo_lmhead_fwd_workspace_bytes allows for 4096 / ceil(T / 256) splits where that is more than 64. */
 #define CLGRPO_VERSION 203
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);

@@ -1,0 +1,51 @@
+"""The GEMM tile and the forward's launch plan at the sizes where they can go wrong: K extents of one to five slabs
+(fewer than three do not stream from tile to tile), ragged last tiles in every dimension, several tiles per
+workgroup, and vocabulary splits from one to the most a single token block gets - against float64 on the device."""
+import pytest
+import torch
+
+from tests.util import assert_close_rel
+
+pytestmark = pytest.mark.gpu
+
+# the contract's bounds: bf16 operands are exact here, results pass through at most two bf16 roundings (2^-9 each)
+RTOL = {torch.float32: 1e-5, torch.bfloat16: 1e-2}
+
+
+def _check(dev, T, H, V, dtype, keep, seed):
+    from chatlearn_amd import ops
+    g = torch.Generator(device=dev).manual_seed(seed)
+    h = torch.randn(T, H, generator=g, device=dev).to(dtype)
+    w = (torch.randn(V, H, generator=g, device=dev) * H ** -0.5).to(dtype)
+    y = torch.randint(0, V, (T,), generator=g, device=dev)
+    y[0], y[-1] = 0, V - 1
+    glp, gen = torch.randn(T, generator=g, device=dev), torch.randn(T, generator=g, device=dev) * 0.1
+    zbuf = ops.saved_logits_buffer(T, V, dtype, dev) if keep else None
+    lp, ent, mx, lse = ops.lmhead_forward(h, w, y, 0.9, saved_logits=zbuf)
+    base = torch.randn(V, H, generator=g, device=dev)
+    dh, dw = ops.lmhead_backward(h, w, y, lse, ent, glp, gen, 0.9, saved_logits=zbuf, dweight=base.clone(), accumulate_dweight=True)
+    z = h.double() @ w.double().t() / 0.9
+    rlse = torch.logsumexp(z, 1)
+    p = torch.exp(z - rlse[:, None])
+    rent = rlse - (p * z).sum(1)
+    r = RTOL[dtype]
+    assert_close_rel(lp, z.gather(1, y[:, None])[:, 0] - rlse, r, "logprob")
+    assert_close_rel(ent, rent, r, "entropy")
+    assert_close_rel(mx, z.max(1).values, r, "rowmax")
+    dz = -p * (glp.double()[:, None] + gen.double()[:, None] * (z - rlse[:, None] + rent[:, None]))
+    dz.scatter_add_(1, y[:, None], glp.double()[:, None])
+    dz /= 0.9
+    assert_close_rel(dh, dz @ w.double(), r, "dhidden")
+    assert_close_rel(dw, dz.t() @ h.double() + base.double(), r, "dweight")
+
+
+@pytest.mark.parametrize("keep", [False, True])
+@pytest.mark.parametrize("dtype,H", [(torch.bfloat16, h) for h in (64, 128, 192, 320)] + [(torch.float32, h) for h in (32, 64, 96, 160)])
+def test_k_extents_and_ragged_tiles(dev, dtype, H, keep):
+    _check(dev, 5003, H, 9001, dtype, keep, seed=H)
+
+
+@pytest.mark.parametrize("T", [1, 33, 256, 257, 900])
+@pytest.mark.parametrize("V", [255, 4097, 120001])
+def test_vocabulary_splits(dev, T, V):
+    _check(dev, T, 192, V, torch.bfloat16, True, seed=T + V)
