@@ -41,7 +41,7 @@ class _PolicyLoss(torch.autograd.Function):
 def _adv_tensor(advantages, like):
     # torch.tensor(list) exactly as the reference does (loss_gallery.py:19,53): a list of numpy
     # float64 gives a float64 tensor, a list of Python floats a float32 one.
-    return torch.tensor(advantages).to(like.device)
+    return ops.upload(torch.tensor(advantages), like.device)
 
 
 def calculate_grpo_loss(

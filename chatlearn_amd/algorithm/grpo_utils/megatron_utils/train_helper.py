@@ -71,7 +71,7 @@ def get_batch_packed(data_b: Dict[str, Any], is_training: bool, *, eod: int, tp_
         if "loss_mask" in data_b:
             loss_mask = data_b['loss_mask'].to(device).to(torch.int32).contiguous()
         else:
-            as_i32 = lambda x: torch.as_tensor(x, dtype=torch.int32).to(device)
+            as_i32 = lambda x: ops.upload(torch.as_tensor(x, dtype=torch.int32), device)
             _, loss_mask, _ = ops.build_masks(as_i32(data_b["prompt_token_length"]),
                                               as_i32(data_b["response_token_length"]), seqlen,
                                               want_position_ids=False)
@@ -175,7 +175,7 @@ def _loss_dict(module_args, logprob: torch.Tensor, entropy: torch.Tensor,
                training_inputs: Dict[str, Any]) -> Dict[str, torch.Tensor]:
     """The loss dict from the [b, s] logprob (carrying the gradient) and the detached [b, s] entropy."""
     gspo = bool(module_args.use_group_sequence_policy)
-    adv = torch.tensor(training_inputs["advantages"]).to(logprob.device)      # dtype rule of loss_gallery.py:19,53
+    adv = ops.upload(torch.tensor(training_inputs["advantages"]), logprob.device)      # dtype rule of loss_gallery.py:19,53
     clips = {k: getattr(module_args, k) for k in ("diff_clip_ratio", "pos_clip_ratio", "neg_clip_ratio",
                                                   "final_clip_ratio")}
     surrogate, kl, *flags = _TokenLosses.apply(logprob, training_inputs["old_logprobs"],
@@ -197,9 +197,11 @@ def _compute_all_losses(module_args, model, all_token_logits: torch.Tensor, labe
     sample-averaged by ``loss_func``).  ``model`` is unused: the reference only reaches through it for the
     cross entropy, which here is the softmax-statistics kernel on the given logits."""
     del model
-    logprob = _batch_rows(language_model_logprob(labels, all_token_logits), module_args, training_inputs)
-    entropy = _batch_rows(entropy_from_tensor_parallel_logits(all_token_logits).permute(1, 0), module_args,
-                          training_inputs)
+    # language_model_logprob and entropy_from_tensor_parallel_logits in one pass over the logits
+    s, b, V = all_token_logits.shape
+    lp, ent = _StatsFromLogits.apply(all_token_logits.reshape(s * b, V), labels.transpose(0, 1).reshape(-1), True, True)
+    logprob = _batch_rows(lp.reshape(s, b).transpose(0, 1).contiguous(), module_args, training_inputs)
+    entropy = _batch_rows(ent.detach().reshape(s, b).permute(1, 0), module_args, training_inputs)
     return _loss_dict(module_args, logprob, entropy, training_inputs)
 
 

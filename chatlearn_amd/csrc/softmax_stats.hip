@@ -1,9 +1,13 @@
 // Softmax statistics (logprob, entropy, lse) from materialised logits and the
 // matching d(logits), for call sites that already hold [R, V] logits.
-// One 256-thread block per row, 16 bytes per lane and four loads in flight per thread; the row is
-// streamed once for the statistics (online max / sum / weighted sum, fp32).  The backward reads
-// it once more and writes d(logits), taking lse / entropy from the forward when the caller kept
-// them.  HBM-bound: V*sizeof(dtype) bytes per row read (+ the same written).
+// One block per row, 16 bytes per lane and four loads in flight per thread; the row is streamed once for the
+// statistics (online max / sum / weighted sum, fp32).  The backward reads it once more and writes
+// d(logits), taking lse / entropy from the forward when the caller kept them.  HBM-bound:
+// V*sizeof(dtype) bytes per row read (+ the same written).  A row may start anywhere: what lies before its first
+// and behind its last 16-byte boundary goes element by element, the rest in 16-byte pieces (519 rows of 32003 fp32,
+// three quarters of them misaligned: 48 -> 16 us, gradients 73 -> 28 us; as bf16 47 -> 13 and 46 -> 17.5 us).
+// 2048 rows of the 152k vocabulary, bf16: statistics 116 us = 5.4 TB/s, gradients 239 us = 5.2 TB/s, where a copy of
+// 1 GB reaches 5.0 TB/s on this card.
 #include "common.hpp"
 
 namespace clgrpo {
@@ -64,64 +68,90 @@ __device__ __forceinline__ void rs_update(RowStats& st, const float (&z)[N]) {
   }
 }
 
-// Rows whose start and length are multiples of 16 bytes are streamed 16 bytes per lane, four
-// independent loads in flight per thread; other rows element by element.
+// A row of V elements from `row`: elements before the first 16-byte boundary, whole pieces, the rest.
 template <typename T>
-__device__ __forceinline__ bool rows_vectorizable(const void* base, int64_t ld, int64_t V) {
-  constexpr int N = Vec16<T>::N;
-  return (reinterpret_cast<uintptr_t>(base) % 16 == 0) && (ld % N == 0) && (V % N == 0);
-}
+struct RowSpan {
+  static constexpr int N = Vec16<T>::N;
+  int head, tail;
+  int64_t pieces;
+  const u32x4_t* vec;
+  __device__ __forceinline__ RowSpan(const T* row, int64_t V) {
+    head = (int)((16 - (reinterpret_cast<uintptr_t>(row) & 15)) & 15) / (int)sizeof(T);
+    if (head > V) head = (int)V;
+    pieces = (V - head) / N;
+    tail = (int)(V - head - pieces * N);
+    vec = reinterpret_cast<const u32x4_t*>(row + head);
+  }
+  // the element outside the pieces that thread `tid` takes, or -1 (head and tail have at most 7 each)
+  __device__ __forceinline__ int64_t loose(int tid) const {
+    if (tid < head) return tid;
+    if (tid >= 32 && tid - 32 < tail) return head + pieces * N + (tid - 32);
+    return -1;
+  }
+};
 
-template <typename T>
-__device__ RowStats row_stats(const T* row, int64_t V, bool vec) {
+template <typename T, int BLOCK>
+__device__ RowStats row_stats(const T* row, int64_t V) {
   constexpr int N = Vec16<T>::N;
   RowStats st{-INFINITY, 0.f, 0.f};
-  if (vec) {
-    const u32x4_t* rv = reinterpret_cast<const u32x4_t*>(row);
-    const int64_t nvec = V / N;
-    int64_t i = threadIdx.x;
-    // two independent running states per thread (merged below): the update is a dependent chain
-    RowStats st2{-INFINITY, 0.f, 0.f};
-    for (; i + 3 * 256 < nvec; i += 4 * 256) {
-      const u32x4_t r0 = rv[i], r1 = rv[i + 256], r2 = rv[i + 512], r3 = rv[i + 768];
-      float z[N], y[N];
-      Vec16<T>::unpack(r0, z); Vec16<T>::unpack(r1, y);
-      rs_update<N>(st, z); rs_update<N>(st2, y);
-      Vec16<T>::unpack(r2, z); Vec16<T>::unpack(r3, y);
-      rs_update<N>(st, z); rs_update<N>(st2, y);
+  const RowSpan<T> span(row, V);
+  const u32x4_t* rv = span.vec;
+  int64_t i = threadIdx.x;
+  // two independent running states per thread (merged below): the update is a dependent chain; the next four pieces
+  // are requested before the current four are worked on
+  RowStats st2{-INFINITY, 0.f, 0.f};
+  auto four = [&](const u32x4_t (&r)[4]) {
+    float z[N], y[N];
+    Vec16<T>::unpack(r[0], z); Vec16<T>::unpack(r[1], y);
+    rs_update<N>(st, z); rs_update<N>(st2, y);
+    Vec16<T>::unpack(r[2], z); Vec16<T>::unpack(r[3], y);
+    rs_update<N>(st, z); rs_update<N>(st2, y);
+  };
+  if (i + 3 * BLOCK < span.pieces) {
+    u32x4_t cur[4], nxt[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) cur[k] = rv[i + k * BLOCK];
+    for (i += 4 * BLOCK; i + 3 * BLOCK < span.pieces; i += 4 * BLOCK) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) nxt[k] = rv[i + k * BLOCK];
+      __builtin_amdgcn_sched_barrier(0);
+      four(cur);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) cur[k] = nxt[k];
     }
-    rs_merge(st, st2);
-    for (; i < nvec; i += 256) {
-      float z[N];
-      Vec16<T>::unpack(rv[i], z);
-      rs_update<N>(st, z);
-    }
-  } else {
-    for (int64_t v = threadIdx.x; v < V; v += 256) {
-      const float z[1] = {to_f32<T>(row[v])};
-      rs_update<1>(st, z);
-    }
+    four(cur);
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    RowStats o{__shfl_xor(st.m, off), __shfl_xor(st.s, off), __shfl_xor(st.u, off)};
-    rs_merge(st, o);
+  for (; i < span.pieces; i += BLOCK) {
+    float z[N];
+    Vec16<T>::unpack(rv[i], z);
+    rs_update<N>(st, z);
   }
-  __shared__ RowStats sh[4];
+  const int64_t loose = span.loose(threadIdx.x);
+  if (loose >= 0) {
+    const float z[1] = {to_f32<T>(row[loose])};
+    rs_update<1>(st2, z);
+  }
+  rs_merge(st, st2);
+  auto fold = [&](int from) {
+    for (int off = from; off > 0; off >>= 1) {
+      RowStats o{__shfl_xor(st.m, off), __shfl_xor(st.s, off), __shfl_xor(st.u, off)};
+      rs_merge(st, o);
+    }
+  };
+  fold(32);
+  __shared__ RowStats sh[BLOCK / 64];
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = st;
   __syncthreads();
-  RowStats t = sh[0];
-  rs_merge(t, sh[1]);
-  rs_merge(t, sh[2]);
-  rs_merge(t, sh[3]);
-  __syncthreads();
-  return t;
+  st = sh[threadIdx.x % (BLOCK / 64)];     // every wave folds all waves' results
+  fold(BLOCK / 128);
+  return st;
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void softmax_stats_kernel(clgrpo_softmax_stats_args a) {
+template <typename T, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void softmax_stats_kernel(clgrpo_softmax_stats_args a) {
   const int64_t r = blockIdx.x;
   const T* row = static_cast<const T*>(a.logits) + r * a.ld;
-  const RowStats st = row_stats<T>(row, a.V, rows_vectorizable<T>(a.logits, a.ld, a.V));
+  const RowStats st = row_stats<T, BLOCK>(row, a.V);
   if (threadIdx.x == 0) {
     const float lse = st.m + logf(st.s);
     if (a.lse) a.lse[r] = lse;
@@ -135,19 +165,18 @@ __global__ __launch_bounds__(256) void softmax_stats_kernel(clgrpo_softmax_stats
 
 // d(logits) of one row: with the row's lse (and entropy, when it carries a gradient) from the forward the
 // row is read once and written once; without them the statistics are rebuilt by one more pass over it.
-template <typename T>
-__global__ __launch_bounds__(256) void softmax_stats_bwd_kernel(clgrpo_softmax_stats_bwd_args a) {
+template <typename T, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void softmax_stats_bwd_kernel(clgrpo_softmax_stats_bwd_args a) {
   constexpr int N = Vec16<T>::N;
   const int64_t r = blockIdx.x;
   const T* row = static_cast<const T*>(a.logits) + r * a.ld;
   T* out = static_cast<T*>(a.dlogits) + r * a.V;
-  const bool vec = rows_vectorizable<T>(a.logits, a.ld, a.V) && (reinterpret_cast<uintptr_t>(a.dlogits) % 16 == 0);
   float lse, ent;
   if (a.lse != nullptr && (a.g_entropy == nullptr || a.entropy != nullptr)) {
     lse = a.lse[r];
     ent = a.g_entropy ? a.entropy[r] : 0.f;
   } else {
-    const RowStats st = row_stats<T>(row, a.V, vec);
+    const RowStats st = row_stats<T, BLOCK>(row, a.V);
     lse = st.m + logf(st.s);
     ent = lse - st.u / st.s;
   }
@@ -161,27 +190,35 @@ __global__ __launch_bounds__(256) void softmax_stats_bwd_kernel(clgrpo_softmax_s
     if (v == y) d += glp;
     return d;
   };
-  if (vec) {
-    const u32x4_t* rv = reinterpret_cast<const u32x4_t*>(row);
-    u32x4_t* ov = reinterpret_cast<u32x4_t*>(out);
-    const int64_t nvec = a.V / N;
+  if (((reinterpret_cast<uintptr_t>(row) ^ reinterpret_cast<uintptr_t>(out)) & 15) == 0) {
+    const RowSpan<T> span(row, a.V);
+    const u32x4_t* rv = span.vec;
+    u32x4_t* ov = reinterpret_cast<u32x4_t*>(out + span.head);
     auto one = [&](const u32x4_t& raw, int64_t i) {
       float z[N], d[N];
       Vec16<T>::unpack(raw, z);
 #pragma unroll
-      for (int k = 0; k < N; ++k) d[k] = dz(z[k], i * N + k);
+      for (int k = 0; k < N; ++k) d[k] = dz(z[k], span.head + i * N + k);
       ov[i] = Vec16<T>::pack(d);
     };
     int64_t i = threadIdx.x;
-    for (; i + 3 * 256 < nvec; i += 4 * 256) {
-      const u32x4_t r0 = rv[i], r1 = rv[i + 256], r2 = rv[i + 512], r3 = rv[i + 768];
-      one(r0, i); one(r1, i + 256); one(r2, i + 512); one(r3, i + 768);
+    for (; i + 3 * BLOCK < span.pieces; i += 4 * BLOCK) {
+      const u32x4_t r0 = rv[i], r1 = rv[i + BLOCK], r2 = rv[i + 2 * BLOCK], r3 = rv[i + 3 * BLOCK];
+      one(r0, i); one(r1, i + BLOCK); one(r2, i + 2 * BLOCK); one(r3, i + 3 * BLOCK);
     }
-    for (; i < nvec; i += 256) one(rv[i], i);
+    for (; i < span.pieces; i += BLOCK) one(rv[i], i);
+    const int64_t loose = span.loose(threadIdx.x);
+    if (loose >= 0) out[loose] = (T)dz(to_f32<T>(row[loose]), loose);
   } else {
-    for (int64_t v = threadIdx.x; v < a.V; v += 256) out[v] = (T)dz(to_f32<T>(row[v]), v);
+    // rows a stride apart that shifts them against the packed result
+    for (int64_t v = threadIdx.x; v < a.V; v += BLOCK) out[v] = (T)dz(to_f32<T>(row[v]), v);
   }
 }
+
+// Threads per row.  Measured with 256 / 512 / 1024 (us): statistics of 48 bf16 rows of the 152k vocabulary 15.6 / 13.9 /
+// 14.5, of 600 42 / 46 / 60, of 2048 116 / 125 / 155 - a wider block waits longer for its slowest wave's reduction; gradients
+// of 48 24 / 19 / 18, of 2048 249 / 239 / 237, of 519 fp32 rows of 32003 28.5 / 28.0 / 31.0.
+constexpr int kStatsThreads = 256, kStatsBwdThreads = 512;
 
 }  // namespace clgrpo
 
@@ -196,8 +233,8 @@ extern "C" int clgrpo_softmax_stats(const clgrpo_softmax_stats_args* a, void* st
   CLGRPO_REQUIRE_PTR(a->logits, "logits");
   if (a->logprob) CLGRPO_REQUIRE_PTR(a->labels, "labels");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (a->dtype == CLGRPO_BF16) hipLaunchKernelGGL(softmax_stats_kernel<__bf16>, dim3((unsigned)a->R), dim3(256), 0, s, *a);
-  else hipLaunchKernelGGL(softmax_stats_kernel<float>, dim3((unsigned)a->R), dim3(256), 0, s, *a);
+  if (a->dtype == CLGRPO_BF16) hipLaunchKernelGGL((softmax_stats_kernel<__bf16, kStatsThreads>), dim3((unsigned)a->R), dim3(kStatsThreads), 0, s, *a);
+  else hipLaunchKernelGGL((softmax_stats_kernel<float, kStatsThreads>), dim3((unsigned)a->R), dim3(kStatsThreads), 0, s, *a);
   return check_launch("softmax_stats_kernel");
 }
 
@@ -210,7 +247,7 @@ extern "C" int clgrpo_softmax_stats_bwd(const clgrpo_softmax_stats_bwd_args* a, 
   CLGRPO_REQUIRE_PTR(a->dlogits, "dlogits");
   if (a->g_logprob) CLGRPO_REQUIRE_PTR(a->labels, "labels");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (a->dtype == CLGRPO_BF16) hipLaunchKernelGGL(softmax_stats_bwd_kernel<__bf16>, dim3((unsigned)a->R), dim3(256), 0, s, *a);
-  else hipLaunchKernelGGL(softmax_stats_bwd_kernel<float>, dim3((unsigned)a->R), dim3(256), 0, s, *a);
+  if (a->dtype == CLGRPO_BF16) hipLaunchKernelGGL((softmax_stats_bwd_kernel<__bf16, kStatsBwdThreads>), dim3((unsigned)a->R), dim3(kStatsBwdThreads), 0, s, *a);
+  else hipLaunchKernelGGL((softmax_stats_bwd_kernel<float, kStatsBwdThreads>), dim3((unsigned)a->R), dim3(kStatsBwdThreads), 0, s, *a);
   return check_launch("softmax_stats_bwd_kernel");
 }

@@ -55,39 +55,6 @@ def _nonzero_rows(mask: torch.Tensor) -> torch.Tensor:
     return live
 
 
-class _PinnedStaging:
-    """Host-side staging for small index arrays that go to the device without stalling the host: two pinned
-    buffers used in turn, each guarded by an event so that it is not rewritten while its copy is in flight."""
-
-    def __init__(self):
-        self.slots = [None, None]
-        self.events = [None, None]
-        self.turn = 0
-
-    def upload(self, host: torch.Tensor, device) -> torch.Tensor:
-        i = self.turn
-        self.turn ^= 1
-        nbytes = host.numel() * host.element_size()
-        if self.events[i] is not None:
-            self.events[i].synchronize()
-        if self.slots[i] is None or self.slots[i].numel() < nbytes:
-            self.slots[i] = torch.empty(max(nbytes, 1 << 16), dtype=torch.uint8, pin_memory=True)
-        stage = self.slots[i][:nbytes].view(host.dtype)
-        stage.copy_(host.reshape(-1))
-        out = stage.to(device, non_blocking=True)
-        self.events[i] = torch.cuda.Event()
-        self.events[i].record()
-        return out.reshape(host.shape)
-
-
-_staging = {}
-
-
-def _upload(host: torch.Tensor, device) -> torch.Tensor:
-    key = (torch.device(device).index or 0, host.dtype)
-    return _staging.setdefault(key, _PinnedStaging()).upload(host, device)
-
-
 def _live_rows_from_host_mask(mask_host: torch.Tensor, chunks, device):
     """Per token chunk: (positions of the unmasked rows inside the chunk, int64; row map int32 with the
     rank of each unmasked row or -1), built on the host from a host copy of the loss mask and sent
@@ -104,8 +71,8 @@ def _live_rows_from_host_mask(mask_host: torch.Tensor, chunks, device):
         local[a:b] -= lo
         row_map[live_all[a:b]] = np.arange(b - a, dtype=np.int32)
         counts.append((a, b))
-    local_d = _upload(torch.from_numpy(local), device) if local.size else torch.empty(0, dtype=torch.int64, device=device)
-    map_d = _upload(torch.from_numpy(row_map), device)
+    local_d = ops.upload(torch.from_numpy(local), device) if local.size else torch.empty(0, dtype=torch.int64, device=device)
+    map_d = ops.upload(torch.from_numpy(row_map), device)
     return [(local_d[a:b], map_d[lo:hi]) for (a, b), (lo, hi) in zip(counts, chunks)]
 
 
@@ -134,7 +101,7 @@ class _FusedHead(torch.autograd.Function):
             if mask_host is not None:
                 live_h = _host_live_rows(mask_host, T)          # no device value is read back
                 n_live = int(live_h.size)
-                live = _upload(torch.from_numpy(live_h), dev) if n_live else torch.empty(0, dtype=torch.int64, device=dev)
+                live = ops.upload(torch.from_numpy(live_h), dev) if n_live else torch.empty(0, dtype=torch.int64, device=dev)
             elif row_mask is not None:
                 live = _nonzero_rows(row_mask)                  # one host round trip for the count
                 n_live = int(live.numel())

@@ -46,6 +46,15 @@ def _stream(t: torch.Tensor):
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
+def upload(host: torch.Tensor, device) -> torch.Tensor:
+    """Device copy of a CPU tensor that does not stall the host: an ordinary copy from pageable memory waits for
+    everything queued on the stream before it.  The pinned block in between comes from torch's caching host
+    allocator, which hands it out again only once the copy is done, whatever thread or stream asks."""
+    if host.numel() == 0:
+        return host.to(device)
+    return host.contiguous().pin_memory().to(device, non_blocking=True)
+
+
 # --------------------------------------------------------------------------- fused lm_head
 
 def _round_up(x: int, m: int) -> int:
@@ -593,7 +602,7 @@ def thd_pack(tokens: torch.Tensor, prompt_len, response_len, align: int, pad_tok
     total, max_padded = sum(padded), max(padded)
     dev = tokens.device
     i32 = dict(dtype=torch.int32, device=dev)
-    lens = torch.tensor([pl, rl], dtype=torch.int32).to(dev)
+    lens = upload(torch.tensor([pl, rl], dtype=torch.int32), dev)
     cu, seqlens, seqlens_padded = torch.empty(B + 1, **i32), torch.empty(B, **i32), torch.empty(B, **i32)
     stats, status = torch.empty(3, **i32), torch.empty(1, **i32)
     per_rank = total // cp_size
