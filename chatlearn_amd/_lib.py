@@ -69,6 +69,20 @@ class MaskedSumsArgs(C.Structure):
                 ("mask", vp), ("out", vp), ("count", vp)]
 
 
+class HeadStepArgs(C.Structure):
+    _fields_ = [("hidden", vp), ("weight", vp), ("labels", vp), ("old_logprob", vp), ("ref_logprob", vp),
+                ("advantages", vp), ("cu_seqlens", vp), ("loss_mask", vp), ("row_order", vp),
+                ("T", i64), ("n_live", i64), ("H", i64), ("V", i64), ("B", i64), ("token_offset", i64), ("chunk", i64),
+                ("dtype", i32), ("compute_dtype", i32), ("mode", i32), ("forward_live_only", i32),
+                ("accumulate_dweight", i32), ("weight_t_ready", i32), ("stages", i32), ("inv_temperature", f32),
+                ("diff_clip_ratio", f64), ("pos_clip_ratio", f64), ("neg_clip_ratio", f64), ("final_clip_ratio", f64),
+                ("kl_coef", f64), ("entropy_coef", f64), ("grad_scale", f64),
+                ("logprob", vp), ("entropy", vp), ("lse", vp), ("g_logprob", vp), ("loss", vp), ("kl", vp),
+                ("sums", vp), ("flags", vp), ("result", vp), ("dhidden", vp), ("dweight", vp),
+                ("workspace", vp), ("workspace_bytes", sz), ("recompute_cap", sz), ("saved_logits", vp),
+                ("ld_saved", i64), ("saved_rows", i64), ("weight_t", vp)]
+
+
 class GroupAdvantageArgs(C.Structure):
     _fields_ = [("n_samples", i64), ("n_groups", i64), ("rewards", vp), ("group_of", vp), ("pool", vp),
                 ("pool_offsets", vp), ("eps", f64), ("advantages", vp), ("all_zeros", vp), ("all_ones", vp)]
@@ -125,6 +139,9 @@ SIGNATURES = {
     "clgrpo_policy_loss_static_max_sequences": (i64, []),
     "clgrpo_masked_sums": (C.c_int, [C.POINTER(MaskedSumsArgs), vp]),
     "clgrpo_masked_sums_bwd": (C.c_int, [i64, vp, vp, vp, i32, vp]),
+    "clgrpo_head_step_workspace_bytes": (sz, [i64, i64, i64, i64, i64, i32, i32, sz]),
+    "clgrpo_head_step_max_ordered_bytes": (i64, []),
+    "clgrpo_head_step": (C.c_int, [C.POINTER(HeadStepArgs), vp]),
     "clgrpo_group_advantage": (C.c_int, [C.POINTER(GroupAdvantageArgs), vp]),
     "clgrpo_build_masks": (C.c_int, [C.POINTER(BuildMasksArgs), vp]),
     "clgrpo_shift_labels": (C.c_int, [C.POINTER(ShiftLabelsArgs), vp]),

@@ -18,6 +18,7 @@ SOURCES = [
     "common.hip",
     "lmhead_fwd.hip",
     "lmhead_bwd.hip",
+    "head_step.hip",
     "loss_kernels.hip",
     "index_kernels.hip",
     "advantage.hip",

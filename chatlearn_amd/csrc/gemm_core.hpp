@@ -189,11 +189,11 @@ struct GemmTile {
   };
 
   int slab_a, slab_b, shrink_a, shrink_b;     // address step and size step per slab
-  int pass_a, pass_b;                         // bytes between the rows of two loads of a slab
+  int pass_a;                                 // bytes between the rows of two loads of a slab
   Cursor a, b, next_a, next_b;
   lds_char* lds;
   __amdgpu_buffer_rsrc_t rsrc_a, rsrc_b;
-  int voff_a, voff_b[2];
+  int voff_a, voff_b[8];
   u32x4 af[2][MI], bf[2][NI];
   uint32_t a0, b0;                            // this lane's fragment address in slot 0 of either ring
   uint32_t ra, rb, na, nb;                    // the same in the slab being read and in the one after it
@@ -209,10 +209,12 @@ struct GemmTile {
   }
   // Load p (0 .. 7) of the slab at the cursor: 8 rows per wave, 32 per workgroup.
   __device__ __forceinline__ void load_a(int p) {
+    int voff_a = this->voff_a;
+    asm volatile("" : "+v"(voff_a));      // one addition per load instead of eight registers across the loop
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, lds + da + p * 4096, 16, voff_a + p * pass_a, 0, 0, 0);
   }
   __device__ __forceinline__ void load_b(int p) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, lds + db + p * 4096, 16, voff_b[BV == 8 ? (p & 1) : 0] + p * pass_b, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, lds + db + p * 4096, 16, voff_b[p], 0, 0, 0);
   }
   __device__ __forceinline__ void step_a() { step_a1(); step_a2(); step_a3(); }
   // in pieces, to be placed between matrix instructions; masks, because a select would become a branch
@@ -258,21 +260,26 @@ struct GemmTile {
   }
 
   // First tile of a workgroup (or of a run that does not stream): nothing is in flight, LDS is free.
-  __device__ __forceinline__ void start(const Operand& A, const Operand& B, int nslab, char* shared) {
+  // b_order: row r of the B tile is row b_order[r] of B.base (B.rows: rows of the whole array; b_rows of them used).
+  __device__ __forceinline__ void start(const Operand& A, const Operand& B, int nslab, char* shared,
+                                        const int32_t* b_order = nullptr, int b_rows = 0) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     lds = (lds_char*)shared;
     slab_a = A.slab_bytes; slab_b = B.slab_bytes;
     shrink_a = A.slab_bytes == kRowBytes ? kRowBytes : 0;
     shrink_b = B.slab_bytes == kRowBytes ? kRowBytes : 0;
-    pass_a = 32 * A.row_bytes; pass_b = 32 * B.row_bytes;
+    pass_a = 32 * A.row_bytes;
     w0 = __builtin_amdgcn_readfirstlane(wave) * 1024;
     // A wave's load fills 1 KB of LDS in lane order: 8 rows x 8 chunks.  The lane that lands on (row, slot)
-    // fetches chunk slot ^ swz(row); load p of a slab starts 32 p rows further down, which leaves a_swz and
-    // b_swz<4> as they are and moves b_swz<8> by 4 p, so odd loads have an offset of their own.
+    // fetches chunk slot ^ swz(row); load p of a slab starts 32 p rows further down, which leaves a_swz as it is.
     const int row = wave * 8 + (lane >> 3), chunk = lane & 7;
     voff_a = row * A.row_bytes + (chunk ^ a_swz(row)) * 16;
-    voff_b[0] = row * B.row_bytes + (chunk ^ b_swz(row)) * 16;
-    voff_b[1] = row * B.row_bytes + (chunk ^ b_swz(row + 32)) * 16;
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+      const int r = row + 32 * p;
+      const int off = b_order == nullptr ? r * B.row_bytes : (r < b_rows ? b_order[r] * B.row_bytes : 0x7fffff00);
+      voff_b[p] = off + (chunk ^ b_swz(r)) * 16;
+    }
     const int g = lane >> 4, c = lane & 15;
     const int fa = a_lane(c), fb = c * BV;
     a0 = (wave_m() + fa) * kRowBytes + (g ^ a_swz(fa)) * 16;

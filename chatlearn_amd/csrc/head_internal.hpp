@@ -1,0 +1,27 @@
+// What the whole-step entry point shares with the entry points of its stages.
+#pragma once
+#include "common.hpp"
+
+namespace clgrpo {
+
+// A choice of rows of a [total, H] array: row n of a kernel's compact problem is row order[n] of the array
+// (and entry order[n] of every per-token array); order == nullptr: row n itself.  The kernels that take one put
+// the row into a 32-bit offset, so total * H * sizeof(dtype) stays within kMaxOrderedBytes.
+struct RowOrder {
+  const int32_t* order;
+  int64_t total;
+};
+constexpr int64_t kMaxOrderedBytes = 0x7f000000;
+
+// Forward of the a->T rows of `rows`; per-token outputs and labels are indexed by order[n], kept logits by n.
+int head_forward(const char* who, const clgrpo_lmhead_fwd_args* a, int64_t vocab_begin, void* record, const RowOrder& rows,
+                 hipStream_t stream);
+// Backward of the a->T rows of `rows`; hidden, per-token arrays and dhidden are indexed by order[n] (dhidden rows outside
+// `rows` are left alone), kept logits by n.  An order needs kept logits.
+int head_backward(const char* who, const clgrpo_lmhead_bwd_args* a, int64_t vocab_begin, const RowOrder& rows,
+                  hipStream_t stream);
+// clgrpo_policy_loss with the scratch memory named apart.
+int head_policy_loss(const char* who, const clgrpo_policy_loss_args* a, void* workspace, size_t workspace_bytes,
+                     hipStream_t stream);
+
+}  // namespace clgrpo

@@ -9,7 +9,7 @@
 // Every contraction runs through the same K-contiguous MFMA tile (gemm_core.hpp).
 //
 // Algorithmic work: 4*T*H*V flop (dhidden + dW); the z recomputation (2*T*H*V) is overhead.
-#include "common.hpp"
+#include "head_internal.hpp"
 #include "gemm_core.hpp"
 
 namespace clgrpo {
@@ -166,6 +166,7 @@ struct DzFromZParams {
   const float* entropy;
   const float* g_lp;
   const float* g_ent;
+  const int32_t* order;   // optional [Tc]: row n is token order[n] of the per-token arrays
   int Tc, ldt, V, ldv;
   float c, inv_temperature;
 };
@@ -183,8 +184,9 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams p) {
   const int64_t n_kslab = p.ldv / E;
   const float it = p.inv_temperature;
   {
-    const int t = rb * kBlockRows + threadIdx.x;
-    const bool ok = t < p.Tc;
+    const int n = rb * kBlockRows + threadIdx.x;
+    const bool ok = n < p.Tc;
+    const int t = ok && p.order ? p.order[n] : n;
     s_glp[threadIdx.x] = ok ? p.g_lp[t] : 0.f;      // rows past the chunk and rows without a gradient give zeros
     s_gen[threadIdx.x] = (ok && p.g_ent) ? p.g_ent[t] : 0.f;
     s_lse[threadIdx.x] = ok ? p.lse[t] : 0.f;
@@ -263,6 +265,8 @@ struct GemmParams {
   int k_per_split;    // K extent of one range, a multiple of the slab
   int n_walk;         // > 0: workgroups walk runs of tiles (see gemm_nt_kernel); needs k_split == 1
   float* partial;     // [k_split] copies of C's shape in fp32, densely packed (row stride N or M)
+  const int32_t* order;   // kMContig, optional [N]: row n of the result is row order[n] of the `total` rows of C
+  int64_t total;
 };
 
 // Addresses of a 256 x 256 output tile for the accumulator layout: a range-checked buffer descriptor over
@@ -280,19 +284,23 @@ struct TileAddr {
   __amdgpu_buffer_rsrc_t rsrc;
   int voff[kGroups];
   int row_bytes, a_rows, row_lim;   // row_lim: valid rows from this lane's first row on
-  __device__ __forceinline__ TileAddr(OutT* base, int64_t ld, int m0, int n0, int a_rows_, int b_rows) {
+  __device__ __forceinline__ TileAddr(OutT* base, int64_t ld, int m0, int n0, int a_rows_, int b_rows,
+                                      const int32_t* order = nullptr, int64_t total = 0) {
     row_bytes = (int)(ld * (int64_t)ES);
     a_rows = a_rows_;
     const int m = Tile::wave_m() + Tile::lane_a0();
     row_lim = a_rows_ - m;
     const int rows = kMContig ? b_rows : a_rows_, cols = kMContig ? a_rows_ : b_rows;
-    const int bytes = rows > 0 ? (rows - 1) * row_bytes + cols * ES : 0;
-    OutT* origin = kMContig ? base + (int64_t)n0 * ld + m0 : base + (int64_t)m0 * ld + n0;
+    const bool ordered = kMContig && order != nullptr;
+    const int bytes = ordered ? (int)(total * row_bytes) - m0 * ES : (rows > 0 ? (rows - 1) * row_bytes + cols * ES : 0);
+    OutT* origin = kMContig ? base + (ordered ? 0 : (int64_t)n0 * ld) + m0 : base + (int64_t)m0 * ld + n0;
     rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(origin), 0, bytes, 0x00020000);
 #pragma unroll
     for (int k = 0; k < kGroups; ++k) {
       const int n = Tile::wave_n() + Tile::lane_b0() + Tile::b_block(kMContig ? k : 4 * k);
-      voff[k] = n < b_rows ? (kMContig ? n * row_bytes + m * ES : m * row_bytes + n * ES) : 0x7f000000;
+      if (n >= b_rows) voff[k] = 0x7f000000;
+      else if (kMContig) voff[k] = (ordered ? order[n0 + n] : n) * row_bytes + m * ES;
+      else voff[k] = m * row_bytes + n * ES;
     }
   }
   // kMContig: blocks i .. i + AG - 1 lie inside the tile (uniform over the wave)
@@ -395,7 +403,7 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, typename Ou
     for_rows<T, float, kMContig, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (float*)nullptr); });
     return;
   }
-  const TileAddr<T, OutT, kMContig> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows);
+  const TileAddr<T, OutT, kMContig> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows, p.order, p.total);
   for_rows<T, OutT, kMContig, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (OutT*)nullptr); });
 }
 
@@ -467,23 +475,24 @@ template <> __device__ __forceinline__ __bf16 cvt_out<__bf16>(float v) { return 
 // C (+)= sum over splits of partial[s], each a dense copy of C's shape with `cols` elements per row
 template <typename OutT>
 __global__ void splitk_reduce_kernel(const float* __restrict__ partial, int k_split, int64_t MN, int cols, OutT* C,
-                                     int64_t ldc, int accumulate) {
+                                     int64_t ldc, int accumulate, const int32_t* __restrict__ order) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < MN; i += (int64_t)gridDim.x * blockDim.x) {
     float v = 0.f;
     for (int s = 0; s < k_split; ++s) v += partial[(int64_t)s * MN + i];
     const int64_t row = i / cols, col = i - row * cols;
-    OutT* dst = C + row * ldc + col;
+    OutT* dst = C + (order ? order[row] : row) * ldc + col;
     if (accumulate) v += (float)*dst;
     *dst = cvt_out<OutT>(v);
   }
 }
 
-// dst(c, r) = src[r][c] for r < R, c < C and 0 for R <= r < ld_dst, where dst is the K-blocked
+// dst(c, r) = src[r][c] (src[order[r]][c] with an order) for r < R, c < C and 0 for R <= r < ld_dst, where dst is the K-blocked
 // operand with C rows and ld_dst K elements (see blocked_index).  64x64 tiles, 16-byte accesses on
 // both sides (C and ld_src are multiples of 32 elements here, so a 16-byte piece never straddles an edge).
 template <typename T>
 __global__ __launch_bounds__(256) void transpose_block_kernel(const T* __restrict__ src, int64_t ld_src,
-                                                              T* __restrict__ dst, int64_t ld_dst, int R, int C) {
+                                                              T* __restrict__ dst, int64_t ld_dst, int R, int C,
+                                                              const int32_t* __restrict__ order) {
   constexpr int VEC = 16 / (int)sizeof(T);       // elements per 16-byte access
   constexpr int CPR = 64 / VEC;                  // accesses per 64-wide tile row
   constexpr int RPP = 256 / CPR;                 // tile rows covered per pass
@@ -496,7 +505,7 @@ __global__ __launch_bounds__(256) void transpose_block_kernel(const T* __restric
     alignas(16) T vals[VEC];
 #pragma unroll
     for (int j = 0; j < VEC; ++j) vals[j] = (T)0.f;
-    if (r < R && c < C) *reinterpret_cast<u32x4*>(vals) = *reinterpret_cast<const u32x4*>(src + (int64_t)r * ld_src + c);
+    if (r < R && c < C) *reinterpret_cast<u32x4*>(vals) = *reinterpret_cast<const u32x4*>(src + (int64_t)(order ? order[r] : r) * ld_src + c);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) tile[q * VEC + j][rr] = vals[j];
   }
@@ -681,7 +690,7 @@ static int64_t chunk_for_workspace(int64_t T, int64_t H, int64_t V, size_t es, s
 template <typename T, typename OutT, bool kMContig>
 static int launch_gemm_one(const void* A, int64_t a_kslabs, int M, const void* B, int64_t b_kslabs, int N, int K, void* C,
                            int64_t ldc, int accumulate, hipStream_t stream, float* partial, size_t partial_bytes,
-                           int k_split_wanted) {
+                           int k_split_wanted, const RowOrder& rows = RowOrder{nullptr, 0}) {
   using Tile = OutTile<T, kMContig>;
   int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_nt_kernel<T, OutT, kMContig>), Tile::kLdsBytes, "gemm_nt_kernel");
   if (rc) return rc;
@@ -690,6 +699,7 @@ static int launch_gemm_one(const void* A, int64_t a_kslabs, int M, const void* B
   g.M = M; g.N = N; g.K = K;
   g.n_mt = (M + 255) / 256; g.n_nt = (N + 255) / 256;
   g.accumulate = accumulate;
+  g.order = rows.order; g.total = rows.total;
   const int slab = Tile::kSlabK;
   const int cus = device_cu_count();
   g.k_split = (partial && partial_bytes) ? k_split_wanted : 1;
@@ -722,7 +732,7 @@ static int launch_gemm_one(const void* A, int64_t a_kslabs, int M, const void* B
   const int64_t MN = (int64_t)M * N;
   int blocks = (int)((MN + 255) / 256 < 4096 ? (MN + 255) / 256 : 4096);
   hipLaunchKernelGGL(splitk_reduce_kernel<OutT>, dim3(blocks), dim3(256), 0, stream, partial, g.k_split, MN, kMContig ? M : N,
-                     static_cast<OutT*>(C), ldc, accumulate);
+                     static_cast<OutT*>(C), ldc, accumulate, rows.order);
   return check_launch("splitk_reduce_kernel");
 }
 
@@ -730,7 +740,7 @@ static int launch_gemm_one(const void* A, int64_t a_kslabs, int M, const void* B
 template <typename T, typename OutT, bool kMContig>
 static int launch_gemm(const void* A, int64_t a_kslabs, int M, const void* B, int64_t b_kslabs, int N, int K, void* C,
                        int64_t ldc, int accumulate, hipStream_t stream, float* partial = nullptr,
-                       size_t partial_bytes = 0) {
+                       size_t partial_bytes = 0, const RowOrder& rows = RowOrder{nullptr, 0}) {
   using Tile = OutTile<T, kMContig>;
   constexpr int64_t kSlabElems = (int64_t)kBlockRows * Tile::kSlabK;
   if (!kMContig) {
@@ -747,30 +757,32 @@ static int launch_gemm(const void* A, int64_t a_kslabs, int M, const void* B, in
                                               dw.k_split > 1 ? partial : nullptr, dw.k_split > 1 ? partial_bytes : 0, dw.k_split);
   }
   if (!(partial && partial_bytes))
-    return launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, M, B, b_kslabs, N, K, C, ldc, accumulate, stream, nullptr, 0, 1);
+    return launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, M, B, b_kslabs, N, K, C, ldc, accumulate, stream, nullptr, 0, 1, rows);
   const DhPlan pl = plan_dhidden(N, M, K, Tile::kSlabK, device_cu_count(), partial_bytes);
   if (pl.bulk_nt == 0)
     return launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, M, B, b_kslabs, N, K, C, ldc, accumulate, stream, partial,
-                                              partial_bytes, pl.k_split);
+                                              partial_bytes, pl.k_split, rows);
   const int bulk_rows = pl.bulk_nt * 256;
   int rc = launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, M, B, b_kslabs, bulk_rows, K, C, ldc, accumulate, stream,
-                                              nullptr, 0, 1);
+                                              nullptr, 0, 1, rows);
   if (rc) return rc;
   const T* b_tail = static_cast<const T*>(B) + (int64_t)pl.bulk_nt * b_kslabs * kSlabElems;
-  OutT* c_tail = static_cast<OutT*>(C) + (int64_t)bulk_rows * ldc;
+  OutT* c_tail = static_cast<OutT*>(C) + (rows.order ? 0 : (int64_t)bulk_rows * ldc);
+  const RowOrder tail{rows.order ? rows.order + bulk_rows : nullptr, rows.total};
   return launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, M, b_tail, b_kslabs, N - bulk_rows, K, c_tail, ldc, accumulate,
-                                            stream, partial, partial_bytes, pl.k_split);
+                                            stream, partial, partial_bytes, pl.k_split, tail);
 }
 
 template <typename T>
-static int launch_transpose(const T* src, int64_t ld_src, T* dst, int64_t ld_dst, int R, int C, hipStream_t stream) {
+static int launch_transpose(const T* src, int64_t ld_src, T* dst, int64_t ld_dst, int R, int C, hipStream_t stream,
+                            const int32_t* order = nullptr) {
   dim3 grid((C + 63) / 64, (int)((ld_dst + 63) / 64));
-  hipLaunchKernelGGL(transpose_block_kernel<T>, grid, dim3(256), 0, stream, src, ld_src, dst, ld_dst, R, C);
+  hipLaunchKernelGGL(transpose_block_kernel<T>, grid, dim3(256), 0, stream, src, ld_src, dst, ld_dst, R, C, order);
   return check_launch("transpose_block_kernel");
 }
 
 template <typename T>
-static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t label_offset) {
+static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t label_offset, const RowOrder& rows) {
   using Tile = LogitTile<T>;
   const int64_t T_ = a->T, H = a->H, V = a->V;
   const bool saved = a->saved_logits != nullptr;
@@ -800,16 +812,20 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
     const int64_t tc = (T_ - c0) < chunk ? (T_ - c0) : chunk;
     const int64_t ldt = round_up64(tc, 64);
     T* dz = saved ? static_cast<T*>(a->saved_logits) + c0 * ldz : dz_ws;
+    // with an order the chunk's tokens are looked up from the start of the arrays, without they follow one another
+    const int64_t t0 = rows.order ? 0 : c0;
+    const int32_t* order = rows.order ? rows.order + c0 : nullptr;
     if (saved) {
       DzFromZParams q;
       q.z = dz;
       q.dzT = dzt;
-      q.labels = a->labels + c0;
+      q.labels = a->labels + t0;
       q.label_offset = label_offset;
-      q.lse = a->lse + c0;
-      q.entropy = a->g_entropy ? a->entropy + c0 : nullptr;
-      q.g_lp = a->g_logprob + c0;
-      q.g_ent = a->g_entropy ? a->g_entropy + c0 : nullptr;
+      q.lse = a->lse + t0;
+      q.entropy = a->g_entropy ? a->entropy + t0 : nullptr;
+      q.g_lp = a->g_logprob + t0;
+      q.g_ent = a->g_entropy ? a->g_entropy + t0 : nullptr;
+      q.order = order;
       q.Tc = (int)tc;
       q.ldt = (int)ldt;
       q.V = (int)V;
@@ -853,13 +869,13 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
     if (a->dhidden) {
       // dhidden[chunk][h] = sum_v WT[h][v] dz[t][v]   (M = H, N = tokens, C[n][m])
       rc = launch_gemm<T, T, true>(wt, pl.ldv / Tile::kSlabK, (int)H, dz, ldz / Tile::kSlabK, (int)tc, (int)pl.ldv,
-                             static_cast<T*>(a->dhidden) + c0 * H, H, 0, stream,
-                             reinterpret_cast<float*>(ws + pl.off_part), pl.part_bytes);
+                             static_cast<T*>(a->dhidden) + t0 * H, H, 0, stream,
+                             reinterpret_cast<float*>(ws + pl.off_part), pl.part_bytes, RowOrder{order, rows.total});
       if (rc) return rc;
     }
     if (a->dweight) {
       // hidT(h, t) = hidden[c0 + t][h], zero for tc <= t < ldt, K-blocked;  dW[v][h] (+)= sum_t dzT(v, t) hidT(h, t)   (M = V, N = H, C[m][n])
-      rc = launch_transpose<T>(hidden + c0 * H, H, hidt, ldt, (int)tc, (int)H, stream);
+      rc = launch_transpose<T>(hidden + t0 * H, H, hidt, ldt, (int)tc, (int)H, stream, order);
       if (rc) return rc;
       rc = launch_gemm<T, float, false>(dzt, ldt / Tile::kSlabK, (int)V, hidt, ldt / Tile::kSlabK, (int)H, (int)ldt, a->dweight, H,
                                         (a->accumulate_dweight || c0 > 0) ? 1 : 0, stream,
@@ -899,7 +915,8 @@ extern "C" int clgrpo_lmhead_bwd_dweight_plan(int64_t rows, int64_t H, int64_t V
   return CLGRPO_OK;
 }
 
-static int bwd_entry(const char* who, const clgrpo_lmhead_bwd_args* a, int64_t vocab_begin, void* stream) {
+int clgrpo::head_backward(const char* who, const clgrpo_lmhead_bwd_args* a, int64_t vocab_begin, const RowOrder& rows,
+                          hipStream_t s) {
   CLGRPO_REQUIRE_PTR(a, "args");
   int rc = validate_head_shape(who, a->T, a->H, a->V, a->dtype);
   if (rc) return rc;
@@ -919,14 +936,19 @@ static int bwd_entry(const char* who, const clgrpo_lmhead_bwd_args* a, int64_t v
   if (a->saved_logits != nullptr && a->saved_rows < round_up64(a->T, 256))
     return fail(CLGRPO_ESHAPE, "%s: saved_rows=%lld, but the kept-logits buffer must hold %lld rows (T rounded up to 256)", who,
                 (long long)a->saved_rows, (long long)round_up64(a->T, 256));
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  return a->dtype == CLGRPO_BF16 ? run_bwd<__bf16>(a, s, vocab_begin) : run_bwd<float>(a, s, vocab_begin);
+  if (rows.order != nullptr && (a->saved_logits == nullptr || rows.total < a->T ||
+                                rows.total * a->H * (int64_t)dtype_bytes(a->dtype) > kMaxOrderedBytes))
+    return fail(CLGRPO_ESHAPE, "%s: a row order needs kept logits and at most %lld bytes of hidden states", who,
+                (long long)kMaxOrderedBytes);
+  return a->dtype == CLGRPO_BF16 ? run_bwd<__bf16>(a, s, vocab_begin, rows) : run_bwd<float>(a, s, vocab_begin, rows);
 }
 
 extern "C" int clgrpo_lmhead_bwd(const clgrpo_lmhead_bwd_args* a, void* stream) {
-  return bwd_entry("clgrpo_lmhead_bwd", a, 0, stream);
+  CLGRPO_REQUIRE_PTR(a, "args");
+  return head_backward("clgrpo_lmhead_bwd", a, 0, RowOrder{nullptr, a->T}, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int clgrpo_lmhead_bwd_shard(const clgrpo_lmhead_bwd_args* a, int64_t vocab_begin, void* stream) {
-  return bwd_entry("clgrpo_lmhead_bwd_shard", a, vocab_begin, stream);
+  CLGRPO_REQUIRE_PTR(a, "args");
+  return head_backward("clgrpo_lmhead_bwd_shard", a, vocab_begin, RowOrder{nullptr, a->T}, static_cast<hipStream_t>(stream));
 }

@@ -12,7 +12,7 @@
 // in the layout of the backward's operand (see KeptLogit).
 //
 // Algorithmic work: 2*T*H*V flop; bytes 2*T*H + 2*V*H (bf16) + 16*T.
-#include "common.hpp"
+#include "head_internal.hpp"
 #include "gemm_core.hpp"
 
 namespace clgrpo {
@@ -39,6 +39,8 @@ struct FwdParams {
   int z_rows;                // rows of z_out; mapped rows outside [0, z_rows) are not stored
   float4* part;  // [n_split][T]: (max raw, sum 2^{(z-max) c}, sum 2^{(z-max) c} z raw, target raw)
   int xcd_wgs;   // > 0: launch of several rounds, see xcd_round_remap
+  const int32_t* order;   // optional [T]: row n is token order[n] of `total` (see RowOrder); kept logits go by n
+  int total;
 };
 
 // 16 bytes of kept logits: consecutive vocabulary entries of one token.
@@ -87,7 +89,6 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
   const int lb = wn + Tile::lane_b0();
   const int t0 = tb * kFwdBN;
   const int b_rows = (p.T - t0) < kFwdBN ? (p.T - t0) : kFwdBN;
-  const T* hidden = static_cast<const T*>(p.hidden) + (int64_t)t0 * p.H;
   const T* weight = static_cast<const T*>(p.weight);
   const float c = p.c;
 
@@ -98,7 +99,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
     const int tok = t0 + lb + Tile::b_block(j);
     lab[j] = -1;
     if (p.labels != nullptr && tok < p.T) {
-      const int64_t rel = p.labels[tok] - p.label_offset;   // a label outside these rows matches nothing
+      const int64_t rel = p.labels[p.order ? p.order[tok] : tok] - p.label_offset;   // a label outside these rows matches nothing
       if (rel >= 0 && rel < p.V) lab[j] = (int)rel - la;
       else lab[j] = -0x40000000;
     } else {
@@ -115,7 +116,9 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
   Tile core;
   const int nslab = p.H / Tile::kSlabK;
   const bool stream = Tile::can_stream(nslab);
-  const auto op_b = Tile::Operand::row_major(hidden, p.H, b_rows);
+  const int32_t* order = p.order ? p.order + t0 : nullptr;
+  const auto op_b = Tile::Operand::row_major(static_cast<const T*>(p.hidden) + (order ? 0 : (int64_t)t0 * p.H), p.H,
+                                             order ? p.total : b_rows);
   const int vt_begin = vs * p.tiles_per_split;
   const int vt_end = (vt_begin + p.tiles_per_split) < p.n_vt ? (vt_begin + p.tiles_per_split) : p.n_vt;
   for (int vt = vt_begin; vt < vt_end; ++vt) {
@@ -124,7 +127,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
     const auto op_a = Tile::Operand::row_major(weight + (int64_t)v0 * p.H, p.H, a_rows);
     typename Tile::Acc acc;
     Tile::zero(acc);
-    if (vt == vt_begin || !stream) core.start(op_a, op_b, nslab, lds);
+    if (vt == vt_begin || !stream) core.start(op_a, op_b, nslab, lds, order, b_rows);
     if (stream && vt + 1 < vt_end) {
       const int v1 = v0 + kFwdBM;
       const int next_rows = (p.V - v1) < kFwdBM ? (p.V - v1) : kFwdBM;
@@ -257,6 +260,7 @@ struct FinalizeParams {
   float* rowmax;
   float* lse;
   float4* record;   // non-null: only the merged (max, sum, sum*z, target) record is written
+  const int32_t* order;   // optional: row n writes to and takes its label from token order[n]
 };
 
 // G threads per token, each merging every G-th split, then each other through LDS; a block is 256 / G consecutive
@@ -304,15 +308,16 @@ __global__ __launch_bounds__(kFinalizeThreads) void lmhead_fwd_finalize_kernel(F
     p.record[t] = make_float4(m, s, u, zt);
     return;
   }
+  const int tok = p.order ? p.order[t] : t;
   const float mx = m * p.inv_temperature;
   const float lse = mx + logf(s);
-  p.lse[t] = lse;
-  if (p.rowmax) p.rowmax[t] = mx;
-  if (p.entropy) p.entropy[t] = lse - p.inv_temperature * u / s;
+  p.lse[tok] = lse;
+  if (p.rowmax) p.rowmax[tok] = mx;
+  if (p.entropy) p.entropy[tok] = lse - p.inv_temperature * u / s;
   if (p.logprob) {
-    const int64_t lab = p.labels[t];
+    const int64_t lab = p.labels[tok];
     // A label outside [0, V) has no logit; NaN marks it instead of a silent wrong number.
-    p.logprob[t] = (lab >= 0 && lab < p.V) ? (zt * p.inv_temperature - lse) : NAN;
+    p.logprob[tok] = (lab >= 0 && lab < p.V) ? (zt * p.inv_temperature - lse) : NAN;
   }
 }
 
@@ -360,7 +365,8 @@ static long fwd_single_cost(int n_tb, int n_vt, int cus, int& n_split, int& tile
 }
 
 template <typename T, bool STORE_Z>
-static int launch_fwd(const clgrpo_lmhead_fwd_args* a, hipStream_t stream, int64_t label_offset, float4* record) {
+static int launch_fwd(const clgrpo_lmhead_fwd_args* a, hipStream_t stream, int64_t label_offset, float4* record,
+                      const RowOrder& rows) {
   using Tile = LogitTile<T>;
   FwdParams p;
   p.hidden = a->hidden;
@@ -379,6 +385,8 @@ static int launch_fwd(const clgrpo_lmhead_fwd_args* a, hipStream_t stream, int64
   p.ldz = a->ld_saved;
   p.z_row_map = a->saved_row_map;
   p.z_rows = (int)a->saved_rows;
+  p.order = rows.order;
+  p.total = (int)rows.total;
   constexpr int lds_bytes = Tile::kLdsBytes;
   int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&lmhead_fwd_kernel<T, STORE_Z>), lds_bytes, "lmhead_fwd_kernel");
   if (rc) return rc;
@@ -400,6 +408,7 @@ static int launch_fwd(const clgrpo_lmhead_fwd_args* a, hipStream_t stream, int64
   f.rowmax = a->rowmax;
   f.lse = a->lse;
   f.record = record;
+  f.order = rows.order;
   return launch_finalize(f, stream);
 }
 
@@ -442,9 +451,10 @@ extern "C" size_t clgrpo_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_
   return (size_t)splits * (size_t)T * sizeof(float4);
 }
 
-// Shared by the whole-vocabulary entry point (record == nullptr) and the shard one.
-static int run_fwd(const char* who, const clgrpo_lmhead_fwd_args* a, int64_t vocab_begin, float4* record,
-                   void* stream) {
+// Shared by the whole-vocabulary entry point (record == nullptr), the shard one and the whole step.
+int clgrpo::head_forward(const char* who, const clgrpo_lmhead_fwd_args* a, int64_t vocab_begin, void* record_ptr,
+                         const RowOrder& rows, hipStream_t s) {
+  float4* record = static_cast<float4*>(record_ptr);
   CLGRPO_REQUIRE_PTR(a, "args");
   int rc = validate_head_shape(who, a->T, a->H, a->V, a->dtype);
   if (rc) return rc;
@@ -465,22 +475,26 @@ static int run_fwd(const char* who, const clgrpo_lmhead_fwd_args* a, int64_t voc
                 (long long)a->ld_saved, (long long)clgrpo_saved_logits_ld(a->V));
   if (a->saved_logits != nullptr && (a->saved_rows <= 0 || a->saved_rows >= (1LL << 31)))
     return fail(CLGRPO_EINVAL, "%s: saved_rows=%lld", who, (long long)a->saved_rows);
-  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (rows.order != nullptr && (rows.total < a->T || rows.total * a->H * (int64_t)dtype_bytes(a->dtype) > kMaxOrderedBytes))
+    return fail(CLGRPO_ESHAPE, "%s: %lld rows of %lld elements are too large for a row order", who, (long long)rows.total,
+                (long long)a->H);
   if (a->saved_logits != nullptr)
-    return a->dtype == CLGRPO_BF16 ? launch_fwd<__bf16, true>(a, s, vocab_begin, record)
-                                   : launch_fwd<float, true>(a, s, vocab_begin, record);
-  return a->dtype == CLGRPO_BF16 ? launch_fwd<__bf16, false>(a, s, vocab_begin, record)
-                                 : launch_fwd<float, false>(a, s, vocab_begin, record);
+    return a->dtype == CLGRPO_BF16 ? launch_fwd<__bf16, true>(a, s, vocab_begin, record, rows)
+                                   : launch_fwd<float, true>(a, s, vocab_begin, record, rows);
+  return a->dtype == CLGRPO_BF16 ? launch_fwd<__bf16, false>(a, s, vocab_begin, record, rows)
+                                 : launch_fwd<float, false>(a, s, vocab_begin, record, rows);
 }
 
 extern "C" int clgrpo_lmhead_fwd(const clgrpo_lmhead_fwd_args* a, void* stream) {
-  return run_fwd("clgrpo_lmhead_fwd", a, 0, nullptr, stream);
+  CLGRPO_REQUIRE_PTR(a, "args");
+  return head_forward("clgrpo_lmhead_fwd", a, 0, nullptr, RowOrder{nullptr, a->T}, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int clgrpo_lmhead_fwd_shard(const clgrpo_lmhead_fwd_args* a, int64_t vocab_begin, void* record,
                                        void* stream) {
   CLGRPO_REQUIRE_PTR(record, "record");
-  return run_fwd("clgrpo_lmhead_fwd_shard", a, vocab_begin, static_cast<float4*>(record), stream);
+  CLGRPO_REQUIRE_PTR(a, "args");
+  return head_forward("clgrpo_lmhead_fwd_shard", a, vocab_begin, record, RowOrder{nullptr, a->T}, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int clgrpo_lmhead_merge_shards(const void* records, int64_t n_shards, int64_t T, const int64_t* labels,
@@ -506,5 +520,6 @@ extern "C" int clgrpo_lmhead_merge_shards(const void* records, int64_t n_shards,
   f.rowmax = rowmax;
   f.lse = lse;
   f.record = nullptr;
+  f.order = nullptr;
   return launch_finalize(f, static_cast<hipStream_t>(stream));
 }

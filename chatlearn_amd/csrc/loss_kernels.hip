@@ -16,7 +16,7 @@
 // dtype rules follow what torch does in the reference: logprob arithmetic,
 // exp, clamp and the KL stay fp32; the product with the advantages (and the
 // final cap) is carried in the advantages' dtype, fp32 or fp64.
-#include "common.hpp"
+#include "head_internal.hpp"
 #include <mutex>
 
 namespace clgrpo {
@@ -381,7 +381,7 @@ extern "C" size_t clgrpo_policy_loss_workspace_bytes(int64_t n, int64_t B) {
 }
 
 // Validation and launches shared by the entry points; `ws` is the scratch memory they differ in.
-static int run_policy_loss(const char* who, const clgrpo_policy_loss_args* a, void* ws_ptr, size_t ws_bytes, void* stream) {
+int clgrpo::head_policy_loss(const char* who, const clgrpo_policy_loss_args* a, void* ws_ptr, size_t ws_bytes, hipStream_t s) {
   CLGRPO_REQUIRE_PTR(a, "args");
   if (a->mode != CLGRPO_LOSS_GRPO && a->mode != CLGRPO_LOSS_GSPO)
     return fail(CLGRPO_EINVAL, "%s: mode %d", who, a->mode);
@@ -405,7 +405,6 @@ static int run_policy_loss(const char* who, const clgrpo_policy_loss_args* a, vo
   const size_t need = clgrpo_policy_loss_workspace_bytes(a->n, a->B);
   if (ws_bytes < need)
     return fail(CLGRPO_EWORKSPACE, "%s: workspace %zu < %zu bytes", who, ws_bytes, need);
-  hipStream_t s = static_cast<hipStream_t>(stream);
 
   LossParams p;
   p.mode = a->mode;
@@ -453,7 +452,7 @@ static int run_policy_loss(const char* who, const clgrpo_policy_loss_args* a, vo
 
 extern "C" int clgrpo_policy_loss(const clgrpo_policy_loss_args* a, void* stream) {
   CLGRPO_REQUIRE_PTR(a, "args");
-  return run_policy_loss("clgrpo_policy_loss", a, a->workspace, a->workspace_bytes, stream);
+  return head_policy_loss("clgrpo_policy_loss", a, a->workspace, a->workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 // ---- the entry point that allocates nothing ---------------------------------------------------
@@ -498,7 +497,7 @@ extern "C" int clgrpo_policy_loss_static(const clgrpo_policy_loss_args* a, void*
   void* ptr = nullptr;
   int rc = static_scratch_address(&ptr);
   if (rc) return rc;
-  return run_policy_loss("clgrpo_policy_loss_static", a, ptr, kStaticScratchBytes, stream);
+  return head_policy_loss("clgrpo_policy_loss_static", a, ptr, kStaticScratchBytes, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int clgrpo_policy_loss_launches(int64_t n, int32_t mode) {

@@ -18,7 +18,7 @@ from typing import Optional
 import numpy as np
 import torch
 
-from . import ops
+from . import _lib, ops
 from ._lib import LOSS_GRPO, LOSS_GSPO
 
 
@@ -53,27 +53,6 @@ def _nonzero_rows(mask: torch.Tensor) -> torch.Tensor:
         mask = torch.nn.functional.pad(mask, (0, 64 - n % 64))
     live, _, _, _ = ops.unpad_indices(mask.reshape(-1, 64))
     return live
-
-
-def _live_rows_from_host_mask(mask_host: torch.Tensor, chunks, device):
-    """Per token chunk: (positions of the unmasked rows inside the chunk, int64; row map int32 with the
-    rank of each unmasked row or -1), built on the host from a host copy of the loss mask and sent
-    over in two asynchronous copies, so that no device value has to be read back.  The index work is
-    numpy's (single-threaded): a few microseconds, and no thread pool to wake on the step's critical path."""
-    flat = mask_host.reshape(-1).numpy() != 0
-    live_all = np.flatnonzero(flat).astype(np.int64)
-    bounds = np.searchsorted(live_all, [lo for lo, _ in chunks] + [chunks[-1][1]])
-    local = live_all.copy()
-    row_map = np.full(flat.shape[0], -1, dtype=np.int32)
-    counts = []
-    for k, (lo, hi) in enumerate(chunks):
-        a, b = int(bounds[k]), int(bounds[k + 1])
-        local[a:b] -= lo
-        row_map[live_all[a:b]] = np.arange(b - a, dtype=np.int32)
-        counts.append((a, b))
-    local_d = ops.upload(torch.from_numpy(local), device) if local.size else torch.empty(0, dtype=torch.int64, device=device)
-    map_d = ops.upload(torch.from_numpy(row_map), device)
-    return [(local_d[a:b], map_d[lo:hi]) for (a, b), (lo, hi) in zip(counts, chunks)]
 
 
 def _host_live_rows(mask_host, T):
@@ -373,7 +352,7 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     this many rows (one [chunk, V] buffer of 16-bit or fp32 elements, reused chunk after chunk) so that
     the backward does not recompute them; ``"auto"`` (the default) bounds that buffer at
     ``DEFAULT_KEEP_LOGITS_BYTES``.  Every token counts as a row, except that with
-    ``skip_masked_rows`` and ``loss_mask_host`` only the unmasked tokens do (only they are kept).  ``None`` keeps nothing: the
+    ``skip_masked_rows`` only the unmasked tokens do (only they are kept).  ``None`` keeps nothing: the
     backward then recomputes the logit tiles from ``hidden`` and ``weight``.  The sequence-level
     loss needs chunks that end on sequence boundaries, so it reads ``cu_seqlens_host`` (or copies
     ``cu_seqlens`` to the host once).
@@ -388,9 +367,9 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     instead of the values the reference computes and then ignores; ``rows_projected_fwd`` counts
     the rows the forward ran on.
 
-    ``loss_mask_host``: a host copy of ``loss_mask`` (the trainer builds the mask on the host anyway).  With
-    it the unmasked rows of every chunk are found on the host and sent over asynchronously; without it
-    they are found on the device, which costs one host round trip per chunk for their count.
+    ``loss_mask_host``: a host copy of ``loss_mask`` (the trainer builds the mask on the host anyway).  The
+    unmasked rows are found on the host and their order is sent over asynchronously; without the copy the mask is
+    read back once.
 
     ``chunk_hidden_bytes``: a chunk's hidden states are also kept below this many bytes (``None``, the
     default: no such bound).  It paid at H = 7168 (two chunks of 16384 tokens against one of 32768) only while
@@ -409,164 +388,140 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     ``stage_hook(name)`` is called on the host at "forward", "loss", "backward", "end" boundaries
     of every chunk (a benchmark records stream events there).
     """
-    hook = stage_hook or (lambda name: None)
-    T = hidden.shape[0]
+    hidden = ops._dev(hidden, "hidden")
+    weight = ops._dev(weight, "weight", hidden.dtype)
+    T, H = hidden.shape
     V = weight.shape[0]
+    dev, es = hidden.device, hidden.element_size()
     keep_logits_chunk = _resolve_keep(keep_logits_chunk, V, hidden.dtype)
     scale = float(fsdp_size) / float(n_tokens_total)
-    mode = LOSS_GSPO if use_group_sequence_policy else LOSS_GRPO
-    skip = keep_logits_chunk is not None and loss_mask is not None and skip_masked_rows
+    skip = keep_logits_chunk is not None and loss_mask is not None and skip_masked_rows and T > 0
     if loss_mask_host is not None and (loss_mask_host.is_cuda or loss_mask_host.numel() != T):
         raise ValueError(f"loss_mask_host must be a CPU copy of loss_mask with {T} entries")
-    chunks = head_step_chunks(T, keep_logits_chunk, use_group_sequence_policy,
-                              cu_seqlens_host if cu_seqlens_host is not None else cu_seqlens,
-                              loss_mask_host if skip else None, shape=(hidden.shape[1], V), dtype=hidden.dtype,
-                              chunk_hidden_bytes=chunk_hidden_bytes if keep_logits_chunk is not None else None)
-    zbuf = None
-    rows_of = None
-    if skip and loss_mask_host is not None and T > 0:
-        rows_of = _live_rows_from_host_mask(loss_mask_host, chunks, hidden.device)
-    longest = max(hi - lo for lo, hi in chunks)
-    cache = workspace_cache if workspace_cache is not None else {}
 
-    def scratch(name, nbytes):
-        buf = cache.get(name)
-        if buf is None or buf.numel() < nbytes or buf.device != hidden.device:
-            buf = cache[name] = torch.empty(nbytes, dtype=torch.uint8, device=hidden.device)
-        return buf
+    # which rows carry a gradient, and the token chunks
+    live = None
+    mask_h = None
+    if skip:
+        mask_h = loss_mask_host if loss_mask_host is not None else loss_mask.cpu()
+        live = np.flatnonzero(mask_h.reshape(-1).numpy())
+    rows_total = T if live is None else live.size
+    ordered_bytes = _lib.lib().clgrpo_head_step_max_ordered_bytes()
+    if live is not None and live.size < T and T * H * es > ordered_bytes:
+        chunk_hidden_bytes = min(chunk_hidden_bytes or ordered_bytes, ordered_bytes)
+    hidden_bound = chunk_hidden_bytes if keep_logits_chunk is not None else None
+    if (keep_logits_chunk is None or keep_logits_chunk >= rows_total) and not (hidden_bound and T * H * es > hidden_bound):
+        chunks = [(0, T)]
+    else:
+        chunks = head_step_chunks(T, keep_logits_chunk, use_group_sequence_policy,
+                                  cu_seqlens_host if cu_seqlens_host is not None else cu_seqlens, mask_h, shape=(H, V),
+                                  dtype=hidden.dtype, chunk_hidden_bytes=hidden_bound)
+    # per chunk: (first token, tokens, rows with a gradient, whether they are picked by an order); the orders are
+    # relative to the chunk and travel in one copy
+    parts, order = [], None
+    if live is None or live.size == T:
+        parts = [(lo, hi - lo, hi - lo, False) for lo, hi in chunks]
+    else:
+        dead = np.flatnonzero(mask_h.reshape(-1).numpy() == 0)
+        order_h = np.empty(T, dtype=np.int32)
+        for lo, hi in chunks:
+            a, b = np.searchsorted(live, (lo, hi))
+            c, d = np.searchsorted(dead, (lo, hi))
+            n_live = int(b - a)
+            order_h[lo:lo + n_live] = live[a:b] - lo
+            order_h[lo + n_live:hi] = dead[c:d] - lo
+            pick = n_live < hi - lo and (hi - lo) * H * es <= ordered_bytes     # one longer sequence may be beyond an order
+            parts.append((lo, hi - lo, n_live if pick else hi - lo, pick))
+        order = ops.upload(torch.from_numpy(order_h), dev)
 
-    if keep_logits_chunk is not None and T > 0:
-        kept = longest if rows_of is None else max(int(live.numel()) for live, _ in rows_of)
-        zbuf = cache.get("kept_logits")
-        if zbuf is None or zbuf.shape[0] < kept or zbuf.dtype != hidden.dtype or zbuf.device != hidden.device \
-                or zbuf.shape[1] != ops.saved_logits_ld(V):
-            zbuf = cache["kept_logits"] = ops.saved_logits_buffer(kept, V, hidden.dtype, hidden.device)
-    # scratch memory of the forward and the backward, shared by all chunks of this call
-    H = hidden.shape[1]
-    fwd_ws = scratch("forward", max(ops.lmhead_forward_workspace_bytes(longest, H, V, hidden.dtype), 16)) if T > 0 else None
-    bwd_rows = longest if zbuf is None else min(longest, zbuf.shape[0])
-    bwd_ws = None
-    f = dict(dtype=torch.float32, device=hidden.device)
-    lp_all, ent_all, lse_all, glp_all = (torch.empty(T, **f) for _ in range(4))
-    loss_all = torch.empty(T, dtype=advantages.dtype, device=hidden.device)
-    kl_all = torch.empty(T, **f) if ref_logprob is not None else None
+    f = dict(dtype=torch.float32, device=dev)
+    per_token = torch.empty(5, T, **f)
+    lp_all, ent_all, lse_all, glp_all, kl_all = per_token.unbind(0)
+    if ref_logprob is None:
+        kl_all = None
+    loss_all = torch.empty(T, dtype=advantages.dtype, device=dev)
     dh_all = torch.empty_like(hidden) if need_dhidden else None
-    sums = torch.zeros(8, dtype=torch.float64, device=hidden.device)
-    flags = torch.zeros(1, dtype=torch.int32, device=hidden.device)
-    dw = dweight
-    acc_dw = accumulate_dweight
-    rows_projected_bwd = 0
-    rows_projected_fwd = 0
+    n_chunks = len(chunks)
+    scratch = torch.empty(14 + 9 * n_chunks, dtype=torch.float64, device=dev)
+    result, sums_buf, flags_buf = scratch[:14], scratch[14:14 + 8 * n_chunks], scratch[14 + 8 * n_chunks:]
+    dw, acc_dw = dweight, accumulate_dweight
+    if dw is None:
+        dw = torch.empty(V, H, dtype=torch.float32, device=dev)
+        acc_dw = False
+    else:
+        dw = ops._dev(dw, "dweight", torch.float32)
+        if tuple(dw.shape) != (V, H) or not dw.is_contiguous() or dw.data_ptr() != dweight.data_ptr():
+            raise ValueError("dweight must be a contiguous fp32 [V,H] tensor")
     wt, wt_ready = None, False
     if need_dhidden and weight_t_cache is not None:
-        wt, wt_ready = weight_t_cache.get("weight_t"), weight_t_cache.get("weight_t") is not None
-    if need_dhidden and wt is None and (len(chunks) > 1 or weight_t_cache is not None):
+        wt = weight_t_cache.get("weight_t")
+        wt_ready = wt is not None
+    if need_dhidden and wt is None and (n_chunks > 1 or weight_t_cache is not None):
         wt = ops.weight_t_buffer(weight)
-    if zbuf is not None:
-        bwd_ws = scratch("backward", ops.lmhead_backward_workspace_bytes(bwd_rows, H, V, hidden.dtype, True, wt is not None))
-    kl_c = kl_coef if kl_coef > 0 else 0.0
-    en_c = entropy_coef if entropy_coef > 0 else 0.0
-    for k, (lo, hi) in enumerate(chunks):
-        sl = slice(lo, hi)
-        n = hi - lo
-        live = row_map = None
-        if skip and n > 0:
-            # Rows whose loss mask is zero get a zero upstream gradient whatever the logits are:
-            # keep logits only for the others and run the backward on that compact set of rows.
-            if rows_of is not None:
-                live, row_map = rows_of[k]
+    if wt is not None:
+        ops.check_weight_t(wt, weight)
+    zbuf = ws = None
+    B = cu_seqlens.numel() - 1
+    if T > 0:
+        cache = workspace_cache if workspace_cache is not None else {}
+        if keep_logits_chunk is not None:
+            kept = max(n for _, _, n, _ in parts)
+            zbuf = cache.get("kept_logits")
+            if zbuf is None or zbuf.shape[0] < kept or zbuf.dtype != hidden.dtype or zbuf.device != dev \
+                    or zbuf.shape[1] != ops.saved_logits_ld(V):
+                zbuf = cache["kept_logits"] = ops.saved_logits_buffer(kept, V, hidden.dtype, dev)
+        need = max(ops.head_step_workspace_bytes(n, n_live, H, V, B, hidden.dtype, zbuf is not None, wt is not None)
+                   for _, n, n_live, _ in parts)
+        ws = cache.get("head_step")
+        if ws is None or ws.numel() < need or ws.device != dev:
+            ws = cache["head_step"] = torch.empty(need, dtype=torch.uint8, device=dev)
+    rows_projected_bwd = rows_projected_fwd = 0
+    if T > 0:
+        step = ops.HeadStep(hidden, weight, labels, old_logprob, ref_logprob, advantages, cu_seqlens, loss_mask, order,
+                            mode=LOSS_GSPO if use_group_sequence_policy else LOSS_GRPO, temperature=temperature,
+                            diff_clip_ratio=diff_clip_ratio, pos_clip_ratio=pos_clip_ratio, neg_clip_ratio=neg_clip_ratio,
+                            final_clip_ratio=final_clip_ratio, kl_coef=max(kl_coef, 0.0), entropy_coef=max(entropy_coef, 0.0),
+                            grad_scale=scale, logprob=lp_all, entropy=ent_all, lse=lse_all, g_logprob=glp_all, loss=loss_all,
+                            kl=kl_all, sums=sums_buf, flags=flags_buf, result=result, dhidden=dh_all, dweight=dw,
+                            workspace=ws, saved_logits=zbuf, weight_t=wt)
+        for k, (lo, n, n_live, pick) in enumerate(parts):
+            live_only = bool(skip_masked_forward and pick and n_live > 0)
+            chunk = dict(lo=lo, n=n, n_live=n_live, ordered=pick, chunk=k, forward_live_only=live_only, accumulate=acc_dw,
+                         weight_t_ready=wt_ready)
+            if stage_hook is None:
+                step.enqueue(7, **chunk)
             else:
-                live = _nonzero_rows(loss_mask[sl])
-                row_map = torch.full((n,), -1, dtype=torch.int32, device=hidden.device)
-                row_map[live] = torch.arange(live.numel(), dtype=torch.int32, device=hidden.device)
-        hook("forward")
-        h_c = lab_c = None
-        if live is not None and skip_masked_forward and live.numel() > 0:
-            # forward on the compact set of unmasked rows; results scattered back, zeros elsewhere
-            h_c, lab_c = ops.gather_rows(hidden[sl], live), ops.gather_rows(labels[sl].reshape(n, 1), live).reshape(-1)
-            lp_c, ent_c, _, lse_c = ops.lmhead_forward(h_c, weight, lab_c, temperature, need_entropy=True,
-                                                       saved_logits=zbuf, workspace=fwd_ws)
-            spread = lambda x: ops.scatter_rows(x.reshape(-1, 1), live, n).reshape(-1)
-            lp, ent, lse = spread(lp_c), spread(ent_c), spread(lse_c)
-            rows_projected_fwd += int(live.numel())
-        else:
-            lp, ent, _, lse = ops.lmhead_forward(hidden[sl], weight, labels[sl], temperature, need_entropy=True,
-                                                 saved_logits=zbuf, saved_row_map=row_map, workspace=fwd_ws)
-            rows_projected_fwd += n
-        hook("loss")
-        res = ops.policy_loss(
-            lp, old_logprob[sl], advantages, mode=mode, cu_seqlens=cu_seqlens,
-            ref_logprob=None if ref_logprob is None else ref_logprob[sl], entropy=ent,
-            loss_mask=None if loss_mask is None else loss_mask[sl], diff_clip_ratio=diff_clip_ratio,
-            pos_clip_ratio=pos_clip_ratio, neg_clip_ratio=neg_clip_ratio, final_clip_ratio=final_clip_ratio,
-            kl_coef=kl_c, entropy_coef=en_c, grad_scale=scale, want_dloss=False, want_upstream=True,
-            token_offset=lo)
-        hook("backward")
-        if live is None:
-            dh, dw = ops.lmhead_backward(hidden[sl], weight, labels[sl], lse, ent, res.g_logprob, res.g_entropy,
-                                         temperature, need_dhidden=need_dhidden, need_dweight=True, dweight=dw,
-                                         accumulate_dweight=acc_dw, saved_logits=zbuf, weight_t=wt,
-                                         weight_t_ready=wt_ready, workspace=bwd_ws)
-            wt_ready = True
-        elif live.numel() == 0:
-            dh = torch.zeros_like(hidden[sl]) if need_dhidden else None
-            if not acc_dw:
-                dw = torch.zeros(V, hidden.shape[1], dtype=torch.float32, device=hidden.device) if dw is None \
-                    else dw.zero_()
-            rows_projected_bwd -= n
-        else:
-            pick = lambda x: None if x is None else ops.gather_rows(x.reshape(n, -1), live).reshape(-1)
-            if h_c is None:
-                h_c, lab_c = ops.gather_rows(hidden[sl], live), pick(labels[sl])
-            dh_c, dw = ops.lmhead_backward(
-                h_c, weight, lab_c, pick(lse), pick(ent),
-                pick(res.g_logprob), pick(res.g_entropy), temperature, need_dhidden=need_dhidden,
-                need_dweight=True, dweight=dw, accumulate_dweight=acc_dw, saved_logits=zbuf, weight_t=wt,
-                weight_t_ready=wt_ready, workspace=bwd_ws)
-            wt_ready = True
-            dh = ops.scatter_rows(dh_c, live, n) if need_dhidden else None
-            rows_projected_bwd += int(live.numel()) - n
-        rows_projected_bwd += n
-        hook("end")
-        acc_dw = True
+                for name, bit in (("forward", 1), ("loss", 2), ("backward", 4)):
+                    stage_hook(name)
+                    step.enqueue(bit, **chunk)
+                stage_hook("end")
+            rows_projected_fwd += n_live if live_only else n
+            rows_projected_bwd += n_live
+            wt_ready = wt_ready or n_live > 0
+            acc_dw = True
         if weight_t_cache is not None and wt_ready:
             weight_t_cache["weight_t"] = wt
-        lp_all[sl], ent_all[sl], lse_all[sl], glp_all[sl], loss_all[sl] = lp, ent, lse, res.g_logprob, res.loss
-        if kl_all is not None:
-            kl_all[sl] = res.kl
-        if need_dhidden:
-            dh_all[sl] = dh
-        sums += res.sums
-        flags |= res.flags
+    else:
+        scratch.zero_()
+        if not acc_dw:
+            dw.zero_()
     if check_flags:
         # one read-back for the reference's three assertions and the host mask's consistency
-        fl, n_masked = (int(x) for x in torch.stack([flags[0].double(), sums[3]]).tolist())
+        fl, n_masked = (int(x) for x in result[12:].tolist())
         assert not fl & 1, "pg loss is nan"
         assert not fl & 2, "kl loss ratio has inf values"
         assert not fl & 4, "kl loss ratio has nan values"
-        if rows_of is not None and loss_mask is not None:
+        if skip and loss_mask_host is not None:
             n_host = int(loss_mask_host.sum())
             if n_host != n_masked:
                 raise ValueError(f"loss_mask_host sums to {n_host}, the device loss_mask to {n_masked}: "
                                  "the host copy is stale or laid out differently")
-    pg = sums[0] * scale
-    kl = sums[1] * scale
-    en = sums[2] * scale
-    total = pg
-    if entropy_coef > 0:
-        total = total - entropy_coef * en
-    if kl_coef > 0:
-        total = total + kl_coef * kl
-    return {"logprob": lp_all, "entropy": ent_all, "lse": lse_all, "pg_loss_mean": pg, "kl_loss_mean": kl,
-            "entropy_loss_mean": en, "total_loss": total, "num_masked": sums[3],
+    return {"logprob": lp_all, "entropy": ent_all, "lse": lse_all, "pg_loss_mean": result[8], "kl_loss_mean": result[9],
+            "entropy_loss_mean": result[10], "total_loss": result[11], "num_masked": result[3],
             "per_token_loss": loss_all, "per_token_kl": kl_all, "dhidden": dh_all, "dweight": dw,
             "g_logprob": glp_all, "rows_projected_bwd": rows_projected_bwd,
-            "rows_projected_fwd": rows_projected_fwd, "sums": sums, "token_chunks": chunks,
+            "rows_projected_fwd": rows_projected_fwd, "sums": result[:8], "token_chunks": chunks,
             # device memory this call held beyond its inputs and outputs: kept logits (they become d(logits) in
-            # place), the backward's operands (d(logits)^T, hidden^T, W^T unless the caller's cache holds it,
-            # split-K partials) and the forward's per-split records
-            "scratch_bytes": sum(t.numel() * t.element_size() for t in (zbuf, fwd_ws, bwd_ws) if t is not None)
-                             + (wt.numel() * wt.element_size() if wt is not None else 0)
-                             + (0 if (zbuf is not None or T == 0) else min(
-                                 ops.lmhead_backward_workspace_bytes(longest, H, V, hidden.dtype, False, wt is not None),
-                                 ops.DEFAULT_BWD_WORKSPACE_BYTES))}
+            # place), the workspace (d(logits)^T, hidden^T, W^T unless the caller's cache holds it, split-K partials;
+            # the forward's per-split records before that) and the caller's W^T
+            "scratch_bytes": sum(t.numel() * t.element_size() for t in (zbuf, ws, wt) if t is not None)}

@@ -316,6 +316,86 @@ def lmhead_backward(hidden, weight, labels, lse, entropy, g_logprob, g_entropy=N
     return dhidden, dweight
 
 
+def check_weight_t(weight_t: torch.Tensor, weight: torch.Tensor) -> None:
+    V, H = weight.shape
+    if weight_t.dtype != weight.dtype or tuple(weight_t.shape) != (_round_up(H, 256), saved_logits_ld(V)) or \
+            not weight_t.is_contiguous():
+        raise ValueError("weight_t must come from weight_t_buffer(weight)")
+
+
+def head_step_workspace_bytes(T: int, n_live: int, H: int, V: int, B: int, dtype, with_saved_logits: bool,
+                              caller_keeps_weight_t: bool) -> int:
+    """Bytes of scratch one token chunk of a head step needs (see ``HeadStep``)."""
+    flags = (1 if with_saved_logits else 0) | (2 if caller_keeps_weight_t else 0)
+    return int(_lib.lib().clgrpo_head_step_workspace_bytes(T, n_live, H, V, B, BF16 if dtype == torch.bfloat16 else F32, flags,
+                                                           DEFAULT_BWD_WORKSPACE_BYTES))
+
+
+class HeadStep:
+    """The token chunks of one micro-batch through clgrpo_head_step: the tensors of the whole micro-batch, checked
+    once; ``enqueue`` launches one chunk (or one stage of it) on the current stream."""
+
+    def __init__(self, hidden, weight, labels, old_logprob, ref_logprob, advantages, cu_seqlens, loss_mask, order, *, mode,
+                 temperature, diff_clip_ratio, pos_clip_ratio, neg_clip_ratio, final_clip_ratio, kl_coef, entropy_coef,
+                 grad_scale, logprob, entropy, lse, g_logprob, loss, kl, sums, flags, result, dhidden, dweight, workspace,
+                 saved_logits, weight_t):
+        T, H = hidden.shape
+        V = weight.shape[0]
+        labels = _dev(labels, "labels", torch.int64)
+        old_logprob = _dev(old_logprob, "old_logprob", torch.float32)
+        advantages = _dev(advantages, "advantages")
+        cu_seqlens = _dev(cu_seqlens, "cu_seqlens", torch.int32)
+        if ref_logprob is not None:
+            ref_logprob = _dev(ref_logprob, "ref_logprob", torch.float32)
+        if loss_mask is not None:
+            loss_mask = _dev(loss_mask if loss_mask.dtype == torch.int32 else loss_mask.to(torch.int32), "loss_mask", torch.int32)
+        for name, t in (("labels", labels), ("old_logprob", old_logprob), ("ref_logprob", ref_logprob), ("loss_mask", loss_mask)):
+            if t is not None and t.numel() != T:
+                raise ValueError(f"{name} must have {T} elements, got {t.numel()}")
+        B = cu_seqlens.numel() - 1
+        cdt = _dtype_enum(advantages)
+        if cdt not in (F32, F64):
+            raise TypeError("advantages must be fp32 or fp64")
+        if advantages.numel() != B:
+            raise ValueError(f"advantages must have {B} elements, got {advantages.numel()}")
+        if weight.shape[1] != H:
+            raise ValueError(f"hidden [T,H] / weight [V,H] expected, got {tuple(hidden.shape)} / {tuple(weight.shape)}")
+        self.tensors = (hidden, weight, labels, old_logprob, ref_logprob, advantages, cu_seqlens, loss_mask, order, logprob,
+                        entropy, lse, g_logprob, loss, kl, sums, flags, result, dhidden, dweight, workspace, saved_logits,
+                        weight_t)                      # alive as long as launches may name them
+        self.row_bytes = {"hidden": H * hidden.element_size(), "labels": 8, "old_logprob": 4, "ref_logprob": 4, "loss_mask": 4,
+                          "row_order": 4, "logprob": 4, "entropy": 4, "lse": 4, "g_logprob": 4,
+                          "loss": loss.element_size(), "kl": 4, "dhidden": H * hidden.element_size()}
+        self.base = {"hidden": _ptr(hidden), "labels": _ptr(labels), "old_logprob": _ptr(old_logprob),
+                     "ref_logprob": _ptr(ref_logprob), "loss_mask": _ptr(loss_mask), "row_order": _ptr(order),
+                     "logprob": _ptr(logprob), "entropy": _ptr(entropy), "lse": _ptr(lse), "g_logprob": _ptr(g_logprob),
+                     "loss": _ptr(loss), "kl": _ptr(kl), "dhidden": _ptr(dhidden)}
+        a = self.args = _lib.HeadStepArgs()
+        a.weight, a.advantages, a.cu_seqlens = _ptr(weight), _ptr(advantages), _ptr(cu_seqlens)
+        a.H, a.V, a.B, a.dtype, a.compute_dtype, a.mode = H, V, B, _dtype_enum(hidden), cdt, mode
+        a.inv_temperature = 1.0 / float(temperature)
+        a.diff_clip_ratio, a.pos_clip_ratio, a.neg_clip_ratio = float(diff_clip_ratio), float(pos_clip_ratio), float(neg_clip_ratio)
+        a.final_clip_ratio, a.kl_coef, a.entropy_coef = float(final_clip_ratio), float(kl_coef), float(entropy_coef)
+        a.grad_scale = float(grad_scale)
+        a.sums, a.flags, a.result, a.dweight = _ptr(sums), _ptr(flags), _ptr(result), _ptr(dweight)
+        a.workspace, a.workspace_bytes, a.recompute_cap = _ptr(workspace), workspace.numel(), DEFAULT_BWD_WORKSPACE_BYTES
+        if saved_logits is not None:
+            a.saved_logits, a.ld_saved, a.saved_rows = _ptr(saved_logits), saved_logits.shape[1], saved_logits.shape[0]
+        a.weight_t = _ptr(weight_t)
+        self.device = hidden.device
+
+    def enqueue(self, stages, *, lo, n, n_live, ordered, chunk, forward_live_only, accumulate, weight_t_ready):
+        a = self.args
+        for name, base in self.base.items():
+            setattr(a, name, None if base is None else base + lo * self.row_bytes[name])
+        if not ordered:
+            a.row_order = None
+        a.T, a.n_live, a.token_offset, a.chunk = n, n_live, lo, chunk
+        a.forward_live_only, a.accumulate_dweight, a.weight_t_ready = int(forward_live_only), int(accumulate), int(weight_t_ready)
+        a.stages = stages
+        _lib.call("clgrpo_head_step", a, torch.cuda.current_stream(self.device).cuda_stream)
+
+
 # --------------------------------------------------------------------------- stats from logits
 
 def softmax_stats(logits2d: torch.Tensor, labels: Optional[torch.Tensor], need_entropy=True, need_logprob=True):

@@ -45,7 +45,8 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *   2.01 -> 2.02: clgrpo_lmhead_bwd_workspace_bytes also covers the partials of the dW GEMM's tail launch (a few
  *                 tens of MB more for some shapes); clgrpo_lmhead_bwd_dweight_plan added.
  *   2.02 -> 2.03: kept logits lie in the K-blocked layout that d(logits) takes over (still opaque to callers);
- *                 clgrpo_lmhead_fwd_workspace_bytes allows for 4096 / ceil(T / 256) splits where that is more than 64. */
+ *                 clgrpo_lmhead_fwd_workspace_bytes allows for 4096 / ceil(T / 256) splits where that is more than 64;
+ *                 clgrpo_head_step added. */
 #define CLGRPO_VERSION 203
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
@@ -296,6 +297,60 @@ typedef struct {
 int clgrpo_masked_sums(const clgrpo_masked_sums_args* a, void* stream);
 /* dst[i] = g[0] * mask[i] in `dtype` (CLGRPO_F32 / CLGRPO_F64); g is a device scalar. */
 int clgrpo_masked_sums_bwd(int64_t n, const float* g, const int32_t* mask, void* dst, int32_t dtype, void* stream);
+
+/* ------------------------------------------------------------------ *
+ * One token chunk of a training step of the head: forward, policy loss, backward, enqueued by one call.
+ * Replaces: the head's share of a micro-batch of the trainer's loop (policy_trainer.py:216-286).
+ * ------------------------------------------------------------------ */
+typedef struct {
+  const void* hidden;            /* [T, H] of the chunk */
+  const void* weight;            /* [V, H] */
+  const int64_t* labels;         /* [T] */
+  const float* old_logprob;      /* [T] */
+  const float* ref_logprob;      /* [T] or NULL */
+  const void* advantages;        /* [B], compute_dtype */
+  const int32_t* cu_seqlens;     /* [B + 1], of the whole micro-batch */
+  const int32_t* loss_mask;      /* [T] or NULL */
+  const int32_t* row_order;      /* [T] or NULL: a permutation of the rows, first the n_live ones that carry a
+                                    gradient.  Only they keep their logits and enter the backward; the others' loss
+                                    mask must be zero.  Needs saved_logits and T * H * sizeof(dtype) <=
+                                    clgrpo_head_step_max_ordered_bytes() */
+  int64_t T, n_live, H, V, B;
+  int64_t token_offset;          /* position of the chunk's first token within cu_seqlens */
+  int64_t chunk;                 /* index of the chunk: its sums go to sums[8 * chunk ..], its flags to flags[chunk] */
+  int32_t dtype, compute_dtype, mode;
+  int32_t forward_live_only;     /* leave the other rows out of the forward too: their logprob / entropy / lse are 0 */
+  int32_t accumulate_dweight;
+  int32_t weight_t_ready;
+  int32_t stages;                /* 1 forward | 2 loss | 4 backward: which of them this call enqueues (7: all) */
+  float inv_temperature;
+  double diff_clip_ratio, pos_clip_ratio, neg_clip_ratio, final_clip_ratio, kl_coef, entropy_coef, grad_scale;
+  float* logprob;                /* [T] out */
+  float* entropy;                /* [T] out */
+  float* lse;                    /* [T] out */
+  float* g_logprob;              /* [T] out: upstream gradient of logprob */
+  void* loss;                    /* [T] out, compute_dtype */
+  float* kl;                     /* [T] out, required with ref_logprob */
+  double* sums;                  /* out, see clgrpo_policy_loss_args */
+  int32_t* flags;                /* out */
+  double* result;                /* [14] out or NULL, written by the loss stage: the sums of chunks 0 .. chunk added up [0..7],
+                                    times grad_scale: surrogate [8], KL [9], entropy [10]; total loss [11]; flags
+                                    of all chunks [12]; masked tokens [13] */
+  void* dhidden;                 /* [T, H] out or NULL */
+  float* dweight;                /* [V, H] out */
+  void* workspace;
+  size_t workspace_bytes;        /* clgrpo_head_step_workspace_bytes */
+  size_t recompute_cap;          /* without saved_logits: bound on the backward's share of the workspace */
+  void* saved_logits;            /* see clgrpo_lmhead_fwd_args; NULL: the backward recomputes them */
+  int64_t ld_saved, saved_rows;
+  void* weight_t;                /* see clgrpo_lmhead_bwd_args */
+} clgrpo_head_step_args;
+
+/* flags: 1 = with saved_logits, 2 = the caller keeps weight_t */
+size_t clgrpo_head_step_workspace_bytes(int64_t T, int64_t n_live, int64_t H, int64_t V, int64_t B, int32_t dtype, int32_t flags,
+                                        size_t recompute_cap);
+int64_t clgrpo_head_step_max_ordered_bytes(void);
+int clgrpo_head_step(const clgrpo_head_step_args* a, void* stream);
 
 /* ------------------------------------------------------------------ *
  * Group-wise reward -> advantage: adv = (r - mean(pool_g)) / (std(pool_g) + eps),
