@@ -209,8 +209,6 @@ struct GemmTile {
   }
   // Load p (0 .. 7) of the slab at the cursor: 8 rows per wave, 32 per workgroup.
   __device__ __forceinline__ void load_a(int p) {
-    int voff_a = this->voff_a;
-    asm volatile("" : "+v"(voff_a));      // one addition per load instead of eight registers across the loop
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, lds + da + p * 4096, 16, voff_a + p * pass_a, 0, 0, 0);
   }
   __device__ __forceinline__ void load_b(int p) {
