@@ -13,12 +13,12 @@ gradient clipping stay with the caller.
 """
 from typing import Any, Callable, Dict, List, Optional
 
+import numpy as np
 import torch
 
 from ... import ops
 from ...fused import AUTO, grpo_head_step
-from .trainer_utils import (batching, generate_loss_mask_position_ids, split_and_unpadding, split_microbatch,
-                            unpad_input)
+from .trainer_utils import batching, generate_loss_mask_position_ids, split_microbatch, unpad_input
 
 _DEFAULT_ARGS = {"entropy_coef": 0.0, "kl_coef": 0.0, "pos_clip_ratio": 0.2, "neg_clip_ratio": 0.2,
                  "diff_clip_ratio": 10, "final_clip_ratio": 3, "use_group_sequence_policy": False}
@@ -69,8 +69,8 @@ class PolicyStep:
     def preprocess_data_list(self, data_list: List[Dict[str, Any]], training: bool):
         """Split into micro-batches, batch, build masks / position ids / labels, pack when asked
         (policy_trainer.py:80-172).  The all-reduce of the response-token count is the identity here."""
-        response_token_length_total = torch.tensor(
-            sum(data["response_token_length"] for data in data_list), device=self.device) / 1
+        response_token_length_total = ops.upload(
+            torch.tensor(sum(data["response_token_length"] for data in data_list)), self.device) / 1
         if self.packing:
             microbatch_list = split_microbatch(data_list=data_list, max_train_token=self.max_token_in_seq,
                                                packing=self.packing)
@@ -81,18 +81,22 @@ class PolicyStep:
         for data_b in (batching(mb) for mb in microbatch_list):
             tokens_ = data_b["all_tokens"].long()
             ori_batch_size, ori_seq_len = tokens_.size()
+            plen, rlen = list(data_b["prompt_token_length"]), list(data_b["response_token_length"])
+            text = 'position_ids' not in data_b and self.model_type != "vlm"
+            if text:
+                # the masks stay on the device: nothing the host needs of them cannot be had from the lengths
+                tokens_ = self._put(tokens_)
             # vision-language samples carry their prompt's three position channels and the image tensors
             attn_mask, loss_mask, position_ids = generate_loss_mask_position_ids(
-                tokens_, data_b["prompt_token_length"], data_b["response_token_length"], data_b.get("position_ids", None))
+                tokens_, plen, rlen, data_b.get("position_ids", None))
             if 'loss_mask' in data_b:
                 loss_mask = data_b['loss_mask']
             indices = cu_seqlens = None
-            if self.packing and 'position_ids' not in data_b and self.model_type != "vlm":
+            if self.packing and text:
                 # unpad_input of tokens and position ids plus the label roll (policy_trainer.py:143-162) in
                 # one device pass driven by the length lists; no device value is read back
-                packed = ops.thd_pack(tokens_.to(self.device), data_b["prompt_token_length"],
-                                      data_b["response_token_length"], align=1, pad_token=0,
-                                      want_loss_mask=False, want_position_ids=True, verify_on_device=False)
+                packed = ops.thd_pack(tokens_, plen, rlen, align=1, pad_token=0, want_loss_mask=False,
+                                      want_position_ids=True, verify_on_device=False)
                 tokens = packed["tokens"].unsqueeze(0)
                 position_ids = packed["position_ids"].unsqueeze(0)
                 labels = packed["labels"].unsqueeze(0)
@@ -115,25 +119,16 @@ class PolicyStep:
                         position_ids = position_ids.permute(1, 0)
                 tokens = tokens_
                 # labels roll along the (packed or padded) token row (policy_trainer.py:135,160)
-                labels, _ = ops.shift_labels(tokens.to(self.device).contiguous(), None, zero_last=False)
+                labels, _ = ops.shift_labels(self._put(tokens).contiguous(), None, zero_last=False)
             # the training mask rolls along the padded rows and loses its last column (policy_trainer.py:161-162)
             shifted = shifted_host = None
             if training:
-                _, shifted = ops.shift_labels(None, loss_mask.to(self.device).to(torch.int32).contiguous(),
-                                              zero_last=True)
-                # the same shift on the host copy, flattened the way the kernels see the tokens: it tells the
-                # head step which rows carry a gradient without reading anything back from the device
-                shifted_host = torch.roll(loss_mask.cpu().to(torch.int32), shifts=-1, dims=1)
-                shifted_host[:, -1] = 0
-                if self.packing:
-                    lens = [p + r for p, r in zip(data_b["prompt_token_length"], data_b["response_token_length"])]
-                    shifted_host = torch.cat([shifted_host[i, :n] for i, n in enumerate(lens)])
-                else:
-                    shifted_host = shifted_host.reshape(-1)
+                _, shifted = ops.shift_labels(None, self._put(loss_mask).to(torch.int32).contiguous(), zero_last=True)
+                shifted_host = self._shifted_mask_host(data_b.get('loss_mask', None), plen, rlen, ori_seq_len)
             data_obj = {"all_tokens": tokens, "position_ids": position_ids, "labels": labels,
                         "ori_seq_len": ori_seq_len, "indices": indices, "cu_seqlens": cu_seqlens,
                         "ori_batch_size": ori_batch_size, "sample_ids": data_b["id_in_list"],
-                        "attention_mask": attn_mask, "pad_size": 0}
+                        "attention_mask": attn_mask, "pad_size": 0, "sample_lengths": [p + r for p, r in zip(plen, rlen)]}
             if self.model_type == "vlm":
                 data_obj.update({"pixel_values": data_b.get("pixel_values", None),
                                  "image_grid_thw": data_b.get("image_grid_thw", None)})
@@ -144,8 +139,24 @@ class PolicyStep:
             data_after_process.append(data_obj)
         return response_token_length_total, data_after_process
 
+    def _shifted_mask_host(self, given, plen, rlen, width):
+        """The shifted training mask on the host, flattened the way the kernels see the tokens: it tells the head
+        step which rows carry a gradient without reading anything back from the device."""
+        rows = np.zeros((len(plen), width), dtype=np.int32)
+        if given is not None:
+            rows[:, :-1] = given.cpu().to(torch.int32).numpy()[:, 1:]
+        else:
+            for row, p, r in zip(rows, plen, rlen):       # response positions p .. p + r - 1, one to the left
+                row[max(p - 1, 0):min(p + r - 1, width - 1)] = 1
+        if self.packing:
+            return torch.from_numpy(np.concatenate([row[:p + r] for row, p, r in zip(rows, plen, rlen)]))
+        return torch.from_numpy(rows.reshape(-1))
+
+    def _put(self, t):
+        return t if t.is_cuda else ops.upload(t, self.device)
+
     def _to_device(self, inputs):
-        return {k: (v.to(self.device) if isinstance(v, torch.Tensor) and not k.endswith("_host") else v)
+        return {k: (self._put(v) if isinstance(v, torch.Tensor) and not k.endswith("_host") else v)
                 for k, v in inputs.items()}
 
     def _backbone(self, inputs):
@@ -171,8 +182,9 @@ class PolicyStep:
         optimizer).  Gradients reach the backbone through ``hidden.backward`` and the lm_head weight
         through ``dweight_buffer`` (fp32, accumulated) or ``lm_head_weight.grad``."""
         args = self.module_args
-        n_tok, data_list = self.preprocess_data_list(data_list=data_list, training=True)
-        n_tok_f = float(n_tok.item())
+        # the same fp32 value that preprocess_data_list leaves on the device
+        n_tok_f = float(np.float32(sum(data["response_token_length"] for data in data_list)))
+        _, data_list = self.preprocess_data_list(data_list=data_list, training=True)
         sums = torch.zeros(8, dtype=torch.float64, device=self.device)
         dw = self.dweight_buffer
         accumulate = dw is not None
@@ -182,7 +194,7 @@ class PolicyStep:
             inputs = self._to_device(inputs)
             hidden = self._backbone(inputs)
             flat, cu, pick = self._flat_view(inputs, hidden)
-            adv = torch.tensor(inputs["advantages"]).to(self.device)
+            adv = ops.upload(torch.tensor(inputs["advantages"]), self.device)
             out = grpo_head_step(
                 flat.detach(), self.weight.detach(), inputs["labels"].reshape(-1), pick(inputs["old_logprobs"].float()),
                 pick(inputs["ref_logprobs"].float()), adv, cu, pick(inputs["loss_mask"]), n_tokens_total=n_tok_f,
@@ -223,12 +235,13 @@ class PolicyStep:
                 hidden = self._backbone(inputs)
                 lp, *_ = ops.lmhead_forward(hidden.reshape(-1, hidden.shape[-1]), self.weight,
                                             inputs["labels"].reshape(-1), self.temperature, need_entropy=False)
-                B, S = inputs["ori_batch_size"], inputs["ori_seq_len"]
+                # sample i's tokens are a run of the packed row, or the start of row i
+                lens = inputs["sample_lengths"]
                 if self.packing:
-                    lp = ops.scatter_rows(lp.reshape(-1, 1), inputs["indices"], B * S).reshape(B, S)
+                    logprobs = lp.split(lens)
                 else:
-                    lp = lp.reshape(B, S)
-            for sample_id, logprob in zip(inputs['sample_ids'], split_and_unpadding(lp, inputs['attention_mask'])):
+                    logprobs = [row[:n] for row, n in zip(lp.reshape(inputs["ori_batch_size"], inputs["ori_seq_len"]), lens)]
+            for sample_id, logprob in zip(inputs['sample_ids'], logprobs):
                 data[sample_id].update({tag: logprob})
         return data
 
