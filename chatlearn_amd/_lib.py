@@ -37,7 +37,7 @@ class LmheadBwdArgs(C.Structure):
     _fields_ = [("hidden", vp), ("weight", vp), ("labels", vp), ("lse", vp), ("entropy", vp),
                 ("g_logprob", vp), ("g_entropy", vp), ("T", i64), ("H", i64), ("V", i64),
                 ("dtype", i32), ("inv_temperature", f32), ("dhidden", vp), ("dweight", vp),
-                ("accumulate_dweight", i32), ("workspace", vp), ("workspace_bytes", sz),
+                ("accumulate_dweight", i32), ("dweight_bf16", i32), ("workspace", vp), ("workspace_bytes", sz),
                 ("saved_logits", vp), ("ld_saved", i64), ("weight_t", vp), ("weight_t_ready", i32),
                 ("saved_rows", i64)]
 
@@ -80,7 +80,13 @@ class HeadStepArgs(C.Structure):
                 ("logprob", vp), ("entropy", vp), ("lse", vp), ("g_logprob", vp), ("loss", vp), ("kl", vp),
                 ("sums", vp), ("flags", vp), ("result", vp), ("dhidden", vp), ("dweight", vp),
                 ("workspace", vp), ("workspace_bytes", sz), ("recompute_cap", sz), ("saved_logits", vp),
-                ("ld_saved", i64), ("saved_rows", i64), ("weight_t", vp)]
+                ("ld_saved", i64), ("saved_rows", i64), ("weight_t", vp),
+                ("kept_dzt", vp), ("kept_hidt", vp), ("kept_ld", i64), ("kept_k", i64)]
+
+
+class DweightArgs(C.Structure):
+    _fields_ = [("dzt", vp), ("hidt", vp), ("ld", i64), ("k", i64), ("H", i64), ("V", i64), ("dtype", i32), ("accumulate", i32),
+                ("dweight", vp), ("dweight_bf16", i32), ("workspace", vp), ("workspace_bytes", sz)]
 
 
 class GroupAdvantageArgs(C.Structure):
@@ -142,6 +148,8 @@ SIGNATURES = {
     "clgrpo_head_step_workspace_bytes": (sz, [i64, i64, i64, i64, i64, i32, i32, sz]),
     "clgrpo_head_step_max_ordered_bytes": (i64, []),
     "clgrpo_head_step": (C.c_int, [C.POINTER(HeadStepArgs), vp]),
+    "clgrpo_dweight_workspace_bytes": (sz, [i64, i64, i64, i32]),
+    "clgrpo_dweight": (C.c_int, [C.POINTER(DweightArgs), vp]),
     "clgrpo_group_advantage": (C.c_int, [C.POINTER(GroupAdvantageArgs), vp]),
     "clgrpo_build_masks": (C.c_int, [C.POINTER(BuildMasksArgs), vp]),
     "clgrpo_shift_labels": (C.c_int, [C.POINTER(ShiftLabelsArgs), vp]),

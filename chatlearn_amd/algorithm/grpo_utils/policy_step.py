@@ -17,7 +17,7 @@ import numpy as np
 import torch
 
 from ... import ops
-from ...fused import AUTO, grpo_head_step
+from ...fused import AUTO, grpo_head_step, keep_rows_bound
 from .trainer_utils import batching, generate_loss_mask_position_ids, split_microbatch, unpad_input
 
 _DEFAULT_ARGS = {"entropy_coef": 0.0, "kl_coef": 0.0, "pos_clip_ratio": 0.2, "neg_clip_ratio": 0.2,
@@ -188,6 +188,12 @@ class PolicyStep:
         sums = torch.zeros(8, dtype=torch.float64, device=self.device)
         dw = self.dweight_buffer
         accumulate = dw is not None
+        # with kept logits dW is contracted over the micro-batches together, as many rows at a time as keep their logits
+        keep = keep_rows_bound(self.keep_logits_chunk, self.weight.shape[0], self.weight.dtype)
+        dw_sum = None
+        if keep is not None and data_list:
+            rows = sum(int(np.count_nonzero(inputs["loss_mask_host"].numpy())) + 64 for inputs in data_list)
+            dw_sum = ops.DweightSum(self.weight.detach(), rows, keep, dw)
         wt_cache = {}   # the weight does not change between the micro-batches of this step
         ws_cache = {}   # kept logits and head scratch memory, shared by the micro-batches of this step
         for inputs in data_list:
@@ -201,16 +207,18 @@ class PolicyStep:
                 fsdp_size=self.fsdp_size, use_group_sequence_policy=args["use_group_sequence_policy"],
                 pos_clip_ratio=args["pos_clip_ratio"], neg_clip_ratio=args["neg_clip_ratio"],
                 diff_clip_ratio=args["diff_clip_ratio"], final_clip_ratio=args["final_clip_ratio"],
-                kl_coef=args["kl_coef"], entropy_coef=args["entropy_coef"], temperature=self.temperature, dweight=dw,
-                accumulate_dweight=accumulate, need_dhidden=flat.requires_grad,
+                kl_coef=args["kl_coef"], entropy_coef=args["entropy_coef"], temperature=self.temperature,
+                dweight=dw if dw_sum is None else None, accumulate_dweight=accumulate, need_dhidden=flat.requires_grad,
                 keep_logits_chunk=self.keep_logits_chunk,
                 # only masked sums leave this method, so rows outside the loss mask need no forward either
                 skip_masked_forward=True, weight_t_cache=wt_cache, loss_mask_host=inputs["loss_mask_host"],
-                workspace_cache=ws_cache)
+                workspace_cache=ws_cache, _dweight_sum=dw_sum)
             dw, accumulate = out["dweight"], True
             if flat.requires_grad:
                 hidden.backward(out["dhidden"].reshape(hidden.shape))
             sums += out["sums"]
+        if dw_sum is not None and (self.dweight_buffer is not None or self.weight.requires_grad):
+            dw = dw_sum.finish(self.weight.dtype)
         if self.dweight_buffer is None and dw is not None and self.weight.requires_grad:
             g = dw.to(self.weight.dtype)
             self.weight.grad = g if self.weight.grad is None else self.weight.grad + g

@@ -104,7 +104,9 @@ extern "C" int clgrpo_head_step(const clgrpo_head_step_args* a, void* stream) {
   CLGRPO_REQUIRE_PTR(a->labels, "labels");
   CLGRPO_REQUIRE_PTR(a->g_logprob, "g_logprob");
   const bool saved = a->saved_logits != nullptr;
-  const int32_t flags = (saved ? 1 : 0) | (a->weight_t ? 2 : 0);
+  const bool keep_dw = a->kept_dzt != nullptr;
+  if (keep_dw) CLGRPO_REQUIRE_PTR(a->kept_hidt, "kept_hidt");
+  const int32_t flags = (saved ? 1 : 0) | (a->weight_t ? 2 : 0) | (keep_dw ? 4 : 0);
   const StepPlan pl = step_plan(a->T, a->n_live, a->H, a->V, a->B, a->dtype, flags, a->recompute_cap);
   if (a->workspace_bytes < pl.total)
     return fail(CLGRPO_EWORKSPACE, "%s: workspace %zu < %zu bytes", who, a->workspace_bytes, pl.total);
@@ -165,9 +167,10 @@ extern "C" int clgrpo_head_step(const clgrpo_head_step_args* a, void* stream) {
       b.workspace = ws + pl.off_big; b.workspace_bytes = pl.big_bytes;
       b.saved_logits = a->saved_logits; b.ld_saved = a->ld_saved; b.saved_rows = a->saved_rows;
       b.weight_t = a->weight_t; b.weight_t_ready = a->weight_t_ready;
-      return head_backward(who, &b, 0, rows, s);
+      const DwOperands kept{a->kept_dzt, a->kept_hidt, a->kept_ld, a->kept_k};
+      return head_backward(who, &b, 0, rows, s, keep_dw ? &kept : nullptr);
     }
-    if (a->dweight && !a->accumulate_dweight) {
+    if (a->dweight && !a->accumulate_dweight && !keep_dw) {
       hipLaunchKernelGGL(zero_floats_kernel, dim3(4096), dim3(256), 0, s, a->dweight, a->V * a->H);
       return check_launch("zero_floats_kernel");
     }

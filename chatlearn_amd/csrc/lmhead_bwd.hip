@@ -159,7 +159,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_dz_kernel(DzParams p) 
 // of a wave is whole 128-byte lines.  HBM-bound: reads 1x, writes 2x the chunk.
 struct DzFromZParams {
   void* z;            // Tc x ldv: in kept logits (KeptLogit<T>), out dz (T), K-blocked
-  void* dzT;          // V x ldt, K-blocked
+  void* dzT;          // V rows, K-blocked: the slab of the chunk's first token
   const int64_t* labels;
   int64_t label_offset;
   const float* lse;
@@ -167,7 +167,8 @@ struct DzFromZParams {
   const float* g_lp;
   const float* g_ent;
   const int32_t* order;   // optional [Tc]: row n is token order[n] of the per-token arrays
-  int Tc, ldt, V, ldv;
+  int Tc, ldt, V, ldv;    // ldt: tokens of dzT to write, Tc rounded up to 64
+  int64_t t_slabs;        // slabs per row of dzT, of which these tokens are the first ldt / E
   float c, inv_temperature;
 };
 
@@ -201,7 +202,6 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams p) {
   __syncthreads();
   const int q = threadIdx.x & 7, cg = threadIdx.x >> 3;   // piece within the slab row, token group
   T* dzT = static_cast<T*>(p.dzT);
-  const int64_t n_tslab = p.ldt / E;
   for (int ks = blockIdx.y; ks < (int)n_kslab; ks += gridDim.y) {
     char* unit = static_cast<char*>(p.z) + ((int64_t)rb * n_kslab + ks) * (kBlockRows * kRowBytes);
     const int v = ks * E + q * VEC;
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams p) {
           float x[VEC];
 #pragma unroll
           for (int k = 0; k < VEC; ++k) x[k] = d[k][e];
-          if (v + e < p.V) *reinterpret_cast<u32x4*>(dzT + blocked_index<T>(v + e, tok, n_tslab)) = pack_vec(x, (T*)nullptr);
+          if (v + e < p.V) *reinterpret_cast<u32x4*>(dzT + blocked_index<T>(v + e, tok, p.t_slabs)) = pack_vec(x, (T*)nullptr);
         }
       }
     }
@@ -247,8 +247,8 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams p) {
 
 // C (+)= A B^T with A [M x K] and B [N x K] K-blocked, C row-major in one of two orientations; either way
 // a lane's 16-byte pieces lie along C's rows and a store instruction covers runs of at least 64 bytes:
-//   kMContig = false: C[m][n], ld = ldc, fp32 (dW: A = dz^T, B = hidden^T).  A lane holds 4 consecutive n of a row
-//     (GemmTile with BV = 4), 16 lanes 256 contiguous bytes of each of 4 rows.
+//   kMContig = false: C[m][n], ld = ldc, fp32 or 16-bit (dW: A = dz^T, B = hidden^T).  A lane holds 4 consecutive n of
+//     a row (GemmTile with BV = 4), 16 lanes 256 contiguous bytes of each of 4 rows for fp32, 128 for 16-bit results.
 //   kMContig = true:  C[n][m], ld = ldc (dhidden: A = W^T, B = dz).  A lane holds VEC consecutive m of a row, the 4
 //     lane groups 64 contiguous bytes of each of 16 rows for 16-bit results.
 template <typename T, bool kMContig> using OutTile = GemmTile<T, kMContig ? 16 / (int)sizeof(T) : 4>;
@@ -334,6 +334,13 @@ __device__ __forceinline__ void row_store(const float (&x)[8], const __amdgpu_bu
   __builtin_amdgcn_raw_buffer_store_b128(pack_vec(x, (__bf16*)nullptr), rsrc, voff, soff, 0);
 }
 
+__device__ __forceinline__ void row_store(const float (&x)[4], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, __bf16*) {
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const bf16x4 v = {(__bf16)x[0], (__bf16)x[1], (__bf16)x[2], (__bf16)x[3]};
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc, voff, soff, 0);
+}
+
 // fn(values of one run of a row, per-lane offset, scalar offset), for every run of the tile that lies inside it;
 // kLoad: the values go into the accumulators afterwards.
 template <typename T, typename OutT, bool kMContig, bool kLoad, typename AccT, typename Fn>
@@ -385,9 +392,10 @@ __device__ __forceinline__ void for_rows(const TileAddr<T, OutT, kMContig>& at, 
 template <typename T, typename OutT, bool kMContig>
 __device__ __forceinline__ void gemm_init_tile(const GemmParams& p, typename OutTile<T, kMContig>::Acc& acc, int m0, int n0,
                                                int a_rows, int b_rows) {
-  if (kMContig || !p.accumulate || p.k_split > 1) {
-    OutTile<T, kMContig>::zero(acc);
-  } else {
+  constexpr bool kAdds = !kMContig && sizeof(OutT) == 4;    // only an fp32 C is ever added to
+  if (!kAdds || !p.accumulate || p.k_split > 1) OutTile<T, kMContig>::zero(acc);
+  if constexpr (kAdds) {
+    if (!p.accumulate || p.k_split > 1) return;
     const TileAddr<T, OutT, kMContig> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows);
     for_rows<T, OutT, kMContig, true>(at, acc, [&](auto& x, int voff, int soff) { row_load(x, at.rsrc, voff, soff, (OutT*)nullptr); });
   }
@@ -486,12 +494,12 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ partial, int k_sp
   }
 }
 
-// dst(c, r) = src[r][c] (src[order[r]][c] with an order) for r < R, c < C and 0 for R <= r < ld_dst, where dst is the K-blocked
-// operand with C rows and ld_dst K elements (see blocked_index).  64x64 tiles, 16-byte accesses on
+// dst(c, r) = src[r][c] (src[order[r]][c] with an order) for r < R, c < C and 0 for R <= r < r_dst, where dst is the K-blocked
+// operand with C rows and ld_dst K elements (see blocked_index), of which the first r_dst are written.  64x64 tiles, 16-byte accesses on
 // both sides (C and ld_src are multiples of 32 elements here, so a 16-byte piece never straddles an edge).
 template <typename T>
 __global__ __launch_bounds__(256) void transpose_block_kernel(const T* __restrict__ src, int64_t ld_src,
-                                                              T* __restrict__ dst, int64_t ld_dst, int R, int C,
+                                                              T* __restrict__ dst, int64_t ld_dst, int64_t r_dst, int R, int C,
                                                               const int32_t* __restrict__ order) {
   constexpr int VEC = 16 / (int)sizeof(T);       // elements per 16-byte access
   constexpr int CPR = 64 / VEC;                  // accesses per 64-wide tile row
@@ -512,7 +520,7 @@ __global__ __launch_bounds__(256) void transpose_block_kernel(const T* __restric
   __syncthreads();
   for (int cc = row; cc < 64; cc += RPP) {
     const int c = c0 + cc, r = r0 + q * VEC;
-    if (c < C && r < ld_dst)
+    if (c < C && r < r_dst)
       *reinterpret_cast<u32x4*>(dst + blocked_index<T>(c, r, ld_dst / kE)) = *reinterpret_cast<const u32x4*>(&tile[cc][q * VEC]);
   }
 }
@@ -649,7 +657,7 @@ struct BwdPlan {
 };
 
 static BwdPlan bwd_plan(int64_t T, int64_t H, int64_t V, size_t es, int64_t chunk_tokens, bool saved = false,
-                        bool own_wt = true) {
+                        bool own_wt = true, bool own_dw = true) {
   BwdPlan pl;
   pl.ldv = round_up64(V, 64);
   int64_t chunk = (chunk_tokens <= 0 || chunk_tokens >= T) ? T : round_up64(chunk_tokens, 256);
@@ -660,15 +668,15 @@ static BwdPlan bwd_plan(int64_t T, int64_t H, int64_t V, size_t es, int64_t chun
   // K-blocked operands: whole blocks of 256 rows
   const size_t Hb = (size_t)round_up64(H, 256), Cb = (size_t)round_up64(chunk, 256), Vb = (size_t)round_up64(V, 256);
   pl.off_wt = off;   off += own_wt ? align_up(Hb * pl.ldv * es, 256) : 0;
-  pl.off_hidt = off; off += align_up(Hb * pl.ldt * es, 256);
+  pl.off_hidt = off; off += own_dw ? align_up(Hb * pl.ldt * es, 256) : 0;
   pl.off_dz = off;   off += saved ? 0 : align_up(Cb * pl.ldv * es, 256);
-  pl.off_dzt = off;  off += align_up(Vb * pl.ldt * es, 256);
+  pl.off_dzt = off;  off += own_dw ? align_up(Vb * pl.ldt * es, 256) : 0;
   // split-K partials of the dhidden GEMM and of the dW GEMM's tail (used one after the other): what a full chunk and
   // the shorter last chunk want
   const int slab = (int)(kRowBytes / es);
   size_t part = 0;
   for (size_t b : {dhidden_partial_bytes(chunk, H, pl.ldv, slab), dhidden_partial_bytes(T % chunk, H, pl.ldv, slab),
-                   dweight_partial_bytes(chunk, H, V, slab), dweight_partial_bytes(T % chunk, H, V, slab)})
+                   own_dw ? dweight_partial_bytes(chunk, H, V, slab) : 0, own_dw ? dweight_partial_bytes(T % chunk, H, V, slab) : 0})
     if (b > part) part = b;
   pl.part_bytes = align_up(part, 256);
   pl.off_part = off; off += pl.part_bytes;
@@ -677,12 +685,12 @@ static BwdPlan bwd_plan(int64_t T, int64_t H, int64_t V, size_t es, int64_t chun
 }
 
 // Largest chunk (multiple of 256, or T itself) whose plan fits into `bytes`; 0 if none does.
-static int64_t chunk_for_workspace(int64_t T, int64_t H, int64_t V, size_t es, size_t bytes, bool saved, bool own_wt) {
-  if (bwd_plan(T, H, V, es, T, saved, own_wt).total <= bytes) return T;
+static int64_t chunk_for_workspace(int64_t T, int64_t H, int64_t V, size_t es, size_t bytes, bool saved, bool own_wt, bool own_dw) {
+  if (bwd_plan(T, H, V, es, T, saved, own_wt, own_dw).total <= bytes) return T;
   int64_t lo = 0, hi = T / 256;   // in units of 256 tokens
   while (lo < hi) {
     const int64_t mid = (lo + hi + 1) / 2;
-    if (bwd_plan(T, H, V, es, mid * 256, saved, own_wt).total <= bytes) lo = mid; else hi = mid - 1;
+    if (bwd_plan(T, H, V, es, mid * 256, saved, own_wt, own_dw).total <= bytes) lo = mid; else hi = mid - 1;
   }
   return lo * 256;
 }
@@ -774,30 +782,46 @@ static int launch_gemm(const void* A, int64_t a_kslabs, int M, const void* B, in
 }
 
 template <typename T>
-static int launch_transpose(const T* src, int64_t ld_src, T* dst, int64_t ld_dst, int R, int C, hipStream_t stream,
-                            const int32_t* order = nullptr) {
-  dim3 grid((C + 63) / 64, (int)((ld_dst + 63) / 64));
-  hipLaunchKernelGGL(transpose_block_kernel<T>, grid, dim3(256), 0, stream, src, ld_src, dst, ld_dst, R, C, order);
+static int launch_transpose(const T* src, int64_t ld_src, T* dst, int64_t r_dst, int R, int C, hipStream_t stream,
+                            const int32_t* order = nullptr, int64_t ld_dst = 0) {
+  dim3 grid((C + 63) / 64, (int)((r_dst + 63) / 64));
+  hipLaunchKernelGGL(transpose_block_kernel<T>, grid, dim3(256), 0, stream, src, ld_src, dst, ld_dst ? ld_dst : r_dst, r_dst, R, C, order);
   return check_launch("transpose_block_kernel");
 }
 
 template <typename T>
-static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t label_offset, const RowOrder& rows) {
+static int run_dweight(const T* dzt, const T* hidt, int64_t ld, int64_t k, int64_t V, int64_t H, void* dweight, bool to_bf16,
+                       bool accumulate, void* partial, size_t partial_bytes, hipStream_t stream) {
+  // dW[v][h] (+)= sum_t dzT(v, t) hidT(h, t)   (M = V, N = H, K = the first k of ld tokens, C[m][n])
+  constexpr int slab = GemmTile<T, 4>::kSlabK;
+  if constexpr (sizeof(T) == 2) {
+    if (to_bf16)
+      return launch_gemm<T, __bf16, false>(dzt, ld / slab, (int)V, hidt, ld / slab, (int)H, (int)k, dweight, H, 0, stream,
+                                           static_cast<float*>(partial), partial_bytes);
+  }
+  return launch_gemm<T, float, false>(dzt, ld / slab, (int)V, hidt, ld / slab, (int)H, (int)k, dweight, H, accumulate ? 1 : 0, stream,
+                                      static_cast<float*>(partial), partial_bytes);
+}
+
+template <typename T>
+static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t label_offset, const RowOrder& rows,
+                   const DwOperands* kept) {
   using Tile = LogitTile<T>;
   const int64_t T_ = a->T, H = a->H, V = a->V;
   const bool saved = a->saved_logits != nullptr;
   const bool own_wt = a->weight_t == nullptr;
-  const int64_t chunk = chunk_for_workspace(T_, H, V, sizeof(T), a->workspace_bytes, saved, own_wt);
+  const bool own_dw = kept == nullptr;
+  const int64_t chunk = chunk_for_workspace(T_, H, V, sizeof(T), a->workspace_bytes, saved, own_wt, own_dw);
   if (chunk <= 0)
     return fail(CLGRPO_EWORKSPACE, "clgrpo_lmhead_bwd: workspace %zu bytes cannot hold a 256-token chunk (%zu needed)",
-                a->workspace_bytes, bwd_plan(T_, H, V, sizeof(T), 256, saved, own_wt).total);
-  const BwdPlan pl = bwd_plan(T_, H, V, sizeof(T), chunk, saved, own_wt);
+                a->workspace_bytes, bwd_plan(T_, H, V, sizeof(T), 256, saved, own_wt, own_dw).total);
+  if (a->dweight_bf16 && chunk < T_)
+    return fail(CLGRPO_EWORKSPACE, "clgrpo_lmhead_bwd: a 16-bit dweight needs a workspace for all %lld tokens at once", (long long)T_);
+  const BwdPlan pl = bwd_plan(T_, H, V, sizeof(T), chunk, saved, own_wt, own_dw);
   const int64_t ldz = saved ? a->ld_saved : pl.ldv;
   char* ws = static_cast<char*>(a->workspace);
   T* wt = a->weight_t ? static_cast<T*>(a->weight_t) : reinterpret_cast<T*>(ws + pl.off_wt);
-  T* hidt = reinterpret_cast<T*>(ws + pl.off_hidt);
   T* dz_ws = reinterpret_cast<T*>(ws + pl.off_dz);
-  T* dzt = reinterpret_cast<T*>(ws + pl.off_dzt);
   const T* hidden = static_cast<const T*>(a->hidden);
   const T* weight = static_cast<const T*>(a->weight);
 
@@ -811,6 +835,11 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
   for (int64_t c0 = 0; c0 < T_; c0 += chunk) {
     const int64_t tc = (T_ - c0) < chunk ? (T_ - c0) : chunk;
     const int64_t ldt = round_up64(tc, 64);
+    // the operands of dW: this chunk's own, or its place among the ones that the caller contracts later
+    constexpr int64_t kSlabElems = (int64_t)kBlockRows * Tile::kSlabK;
+    const int64_t k0 = kept ? kept->k + c0 : 0, ld_dw = kept ? kept->ld : ldt;
+    T* dzt = (kept ? static_cast<T*>(kept->dzt) : reinterpret_cast<T*>(ws + pl.off_dzt)) + k0 / Tile::kSlabK * kSlabElems;
+    T* hidt = (kept ? static_cast<T*>(kept->hidt) : reinterpret_cast<T*>(ws + pl.off_hidt)) + k0 / Tile::kSlabK * kSlabElems;
     T* dz = saved ? static_cast<T*>(a->saved_logits) + c0 * ldz : dz_ws;
     // with an order the chunk's tokens are looked up from the start of the arrays, without they follow one another
     const int64_t t0 = rows.order ? 0 : c0;
@@ -828,6 +857,7 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
       q.order = order;
       q.Tc = (int)tc;
       q.ldt = (int)ldt;
+      q.t_slabs = ld_dw / Tile::kSlabK;
       q.V = (int)V;
       q.ldv = (int)ldz;
       q.c = a->inv_temperature * kLog2e;
@@ -873,13 +903,14 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
                              reinterpret_cast<float*>(ws + pl.off_part), pl.part_bytes, RowOrder{order, rows.total});
       if (rc) return rc;
     }
-    if (a->dweight) {
-      // hidT(h, t) = hidden[c0 + t][h], zero for tc <= t < ldt, K-blocked;  dW[v][h] (+)= sum_t dzT(v, t) hidT(h, t)   (M = V, N = H, C[m][n])
-      rc = launch_transpose<T>(hidden + t0 * H, H, hidt, ldt, (int)tc, (int)H, stream, order);
+    if (a->dweight || kept) {
+      // hidT(h, t) = hidden[c0 + t][h], zero for tc <= t < ldt, K-blocked
+      rc = launch_transpose<T>(hidden + t0 * H, H, hidt, ldt, (int)tc, (int)H, stream, order, ld_dw);
       if (rc) return rc;
-      rc = launch_gemm<T, float, false>(dzt, ldt / Tile::kSlabK, (int)V, hidt, ldt / Tile::kSlabK, (int)H, (int)ldt, a->dweight, H,
-                                        (a->accumulate_dweight || c0 > 0) ? 1 : 0, stream,
-                                        reinterpret_cast<float*>(ws + pl.off_part), pl.part_bytes);
+    }
+    if (a->dweight && !kept) {
+      rc = run_dweight<T>(dzt, hidt, ldt, ldt, V, H, a->dweight, a->dweight_bf16 != 0, a->accumulate_dweight || c0 > 0,
+                          ws + pl.off_part, pl.part_bytes, stream);
       if (rc) return rc;
     }
   }
@@ -893,7 +924,8 @@ using namespace clgrpo;
 extern "C" size_t clgrpo_lmhead_bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int32_t dtype,
                                                     int64_t chunk_tokens, int32_t with_saved_logits) {
   if (T <= 0 || H <= 0 || V <= 0 || (dtype != CLGRPO_BF16 && dtype != CLGRPO_F32)) return 0;
-  return bwd_plan(T, H, V, dtype_bytes(dtype), chunk_tokens, (with_saved_logits & 1) != 0, (with_saved_logits & 2) == 0).total;
+  return bwd_plan(T, H, V, dtype_bytes(dtype), chunk_tokens, (with_saved_logits & 1) != 0, (with_saved_logits & 2) == 0,
+                  (with_saved_logits & 4) == 0).total;
 }
 
 extern "C" int clgrpo_lmhead_bwd_dhidden_plan(int64_t rows, int64_t H, int64_t V, int32_t dtype, int32_t cus, int32_t* out) {
@@ -915,8 +947,37 @@ extern "C" int clgrpo_lmhead_bwd_dweight_plan(int64_t rows, int64_t H, int64_t V
   return CLGRPO_OK;
 }
 
+extern "C" size_t clgrpo_dweight_workspace_bytes(int64_t k, int64_t H, int64_t V, int32_t dtype) {
+  if (k <= 0 || H <= 0 || V <= 0 || (dtype != CLGRPO_BF16 && dtype != CLGRPO_F32)) return 0;
+  return align_up(dweight_partial_bytes(k, H, V, (int)(kRowBytes / dtype_bytes(dtype))), 256);
+}
+
+extern "C" int clgrpo_dweight(const clgrpo_dweight_args* a, void* stream) {
+  static const char* who = "clgrpo_dweight";
+  CLGRPO_REQUIRE_PTR(a, "args");
+  int rc = validate_head_shape(who, a->k, a->H, a->V, a->dtype);
+  if (rc) return rc;
+  if (a->k % 64 != 0 || a->ld % 64 != 0 || a->ld < a->k)
+    return fail(CLGRPO_ESHAPE, "%s: k=%lld of ld=%lld must be multiples of 64", who, (long long)a->k, (long long)a->ld);
+  CLGRPO_REQUIRE_PTR(a->dzt, "dzt");
+  CLGRPO_REQUIRE_PTR(a->hidt, "hidt");
+  CLGRPO_REQUIRE_PTR(a->dweight, "dweight");
+  if (a->dweight_bf16 && (a->accumulate || a->dtype != CLGRPO_BF16))
+    return fail(CLGRPO_EINVAL, "%s: a 16-bit dweight needs 16-bit operands and is not added to", who);
+  const size_t need = clgrpo_dweight_workspace_bytes(a->k, a->H, a->V, a->dtype);
+  if (need > 0) CLGRPO_REQUIRE_PTR(a->workspace, "workspace");
+  if (a->workspace_bytes < need)
+    return fail(CLGRPO_EWORKSPACE, "%s: workspace %zu < %zu bytes", who, a->workspace_bytes, need);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (a->dtype == CLGRPO_BF16)
+    return run_dweight<__bf16>(static_cast<const __bf16*>(a->dzt), static_cast<const __bf16*>(a->hidt), a->ld, a->k, a->V, a->H,
+                               a->dweight, a->dweight_bf16 != 0, a->accumulate != 0, a->workspace, a->workspace_bytes, s);
+  return run_dweight<float>(static_cast<const float*>(a->dzt), static_cast<const float*>(a->hidt), a->ld, a->k, a->V, a->H,
+                            a->dweight, false, a->accumulate != 0, a->workspace, a->workspace_bytes, s);
+}
+
 int clgrpo::head_backward(const char* who, const clgrpo_lmhead_bwd_args* a, int64_t vocab_begin, const RowOrder& rows,
-                          hipStream_t s) {
+                          hipStream_t s, const DwOperands* kept) {
   CLGRPO_REQUIRE_PTR(a, "args");
   int rc = validate_head_shape(who, a->T, a->H, a->V, a->dtype);
   if (rc) return rc;
@@ -926,7 +987,14 @@ int clgrpo::head_backward(const char* who, const clgrpo_lmhead_bwd_args* a, int6
   CLGRPO_REQUIRE_PTR(a->lse, "lse");
   CLGRPO_REQUIRE_PTR(a->g_logprob, "g_logprob");
   if (a->g_entropy != nullptr) CLGRPO_REQUIRE_PTR(a->entropy, "entropy");
-  if (a->dhidden == nullptr && a->dweight == nullptr) return fail(CLGRPO_ENULL, "%s: both dhidden and dweight are NULL", who);
+  if (a->dhidden == nullptr && a->dweight == nullptr && kept == nullptr)
+    return fail(CLGRPO_ENULL, "%s: both dhidden and dweight are NULL", who);
+  if (a->dweight_bf16 && (a->accumulate_dweight || a->dtype != CLGRPO_BF16))
+    return fail(CLGRPO_EINVAL, "%s: a 16-bit dweight needs 16-bit operands and is not added to", who);
+  if (kept != nullptr && (a->saved_logits == nullptr || kept->k < 0 || kept->k % 64 != 0 || kept->ld % 64 != 0 ||
+                          kept->k + round_up64(a->T, 64) > kept->ld))
+    return fail(CLGRPO_ESHAPE, "%s: %lld tokens do not fit behind the %lld of %lld kept for dweight", who, (long long)a->T,
+                (long long)kept->k, (long long)kept->ld);
   if (vocab_begin < 0) return fail(CLGRPO_EINVAL, "%s: vocab_begin=%lld", who, (long long)vocab_begin);
   if (!(a->inv_temperature > 0.f)) return fail(CLGRPO_EINVAL, "%s: inv_temperature must be > 0", who);
   CLGRPO_REQUIRE_PTR(a->workspace, "workspace");
@@ -940,7 +1008,7 @@ int clgrpo::head_backward(const char* who, const clgrpo_lmhead_bwd_args* a, int6
                                 rows.total * a->H * (int64_t)dtype_bytes(a->dtype) > kMaxOrderedBytes))
     return fail(CLGRPO_ESHAPE, "%s: a row order needs kept logits and at most %lld bytes of hidden states", who,
                 (long long)kMaxOrderedBytes);
-  return a->dtype == CLGRPO_BF16 ? run_bwd<__bf16>(a, s, vocab_begin, rows) : run_bwd<float>(a, s, vocab_begin, rows);
+  return a->dtype == CLGRPO_BF16 ? run_bwd<__bf16>(a, s, vocab_begin, rows, kept) : run_bwd<float>(a, s, vocab_begin, rows, kept);
 }
 
 extern "C" int clgrpo_lmhead_bwd(const clgrpo_lmhead_bwd_args* a, void* stream) {

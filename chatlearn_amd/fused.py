@@ -38,7 +38,8 @@ def default_keep_rows(V: int, dtype) -> int:
     return max(256, rows // 256 * 256)
 
 
-def _resolve_keep(keep, V, dtype):
+def keep_rows_bound(keep, V, dtype):
+    """Rows that may keep their logits under a ``keep_logits_rows`` / ``keep_logits_chunk`` argument, None for none."""
     return default_keep_rows(V, dtype) if isinstance(keep, str) and keep == AUTO else keep
 
 
@@ -134,9 +135,13 @@ class _FusedHead(torch.autograd.Function):
             else:
                 idx = live[lo:hi]
                 pick = lambda x: None if x is None else ops.gather_rows(x.reshape(T, -1), idx).reshape((hi - lo,) + x.shape[1:])
+            # one contraction over all live rows is rounded to the weight's type as it is written (151936 x 2048: no 0.3 ms
+            # pass that converts, half the bytes written)
+            whole = dweight is None and hi - lo == n_live
             return ops.lmhead_backward(pick(hidden), weight, pick(labels), pick(lse), pick(ent), pick(g_lp), pick(g_ent),
                                        ctx.temperature, need_dhidden=need_h, need_dweight=need_w, dweight=dweight,
-                                       accumulate_dweight=accumulate, saved_logits=saved)
+                                       accumulate_dweight=accumulate, saved_logits=saved,
+                                       dweight_dtype=weight.dtype if whole else torch.float32)
 
         dw, acc = dw_buf, dw_buf is not None
         pieces = []
@@ -185,7 +190,7 @@ def fused_linear_logprob_entropy(hidden: torch.Tensor, weight: torch.Tensor, lab
     lead = labels.shape
     h2 = hidden.reshape(-1, hidden.shape[-1])
     needs_grad = torch.is_grad_enabled() and (hidden.requires_grad or weight.requires_grad)
-    keep = _resolve_keep(keep_logits_rows, weight.shape[0], hidden.dtype) if needs_grad else None
+    keep = keep_rows_bound(keep_logits_rows, weight.shape[0], hidden.dtype) if needs_grad else None
     mask = host = None
     if needs_grad:                 # the masks only matter to the backward (and to which rows keep their logits)
         host = loss_mask_host
@@ -340,7 +345,8 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
                    keep_logits_chunk=AUTO, cu_seqlens_host=None,
                    skip_masked_rows=True, skip_masked_forward=False, weight_t_cache: Optional[dict] = None,
                    stage_hook=None, loss_mask_host: Optional[torch.Tensor] = None,
-                   workspace_cache: Optional[dict] = None, chunk_hidden_bytes: Optional[int] = None):
+                   workspace_cache: Optional[dict] = None, chunk_hidden_bytes: Optional[int] = None,
+                   _dweight_sum: Optional[ops.DweightSum] = None):
     """Forward + loss + backward of the head for one packed micro-batch, no autograd graph.
 
     Mirrors policy_trainer.py:216-286 on packed rows: returns a dict with the
@@ -387,13 +393,16 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
 
     ``stage_hook(name)`` is called on the host at "forward", "loss", "backward", "end" boundaries
     of every chunk (a benchmark records stream events there).
+
+    ``_dweight_sum`` (needs kept logits): the operands of dW go there in the place of being contracted, ``dweight``
+    in the result is None.
     """
     hidden = ops._dev(hidden, "hidden")
     weight = ops._dev(weight, "weight", hidden.dtype)
     T, H = hidden.shape
     V = weight.shape[0]
     dev, es = hidden.device, hidden.element_size()
-    keep_logits_chunk = _resolve_keep(keep_logits_chunk, V, hidden.dtype)
+    keep_logits_chunk = keep_rows_bound(keep_logits_chunk, V, hidden.dtype)
     scale = float(fsdp_size) / float(n_tokens_total)
     skip = keep_logits_chunk is not None and loss_mask is not None and skip_masked_rows and T > 0
     if loss_mask_host is not None and (loss_mask_host.is_cuda or loss_mask_host.numel() != T):
@@ -445,7 +454,10 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     scratch = torch.empty(14 + 9 * n_chunks, dtype=torch.float64, device=dev)
     result, sums_buf, flags_buf = scratch[:14], scratch[14:14 + 8 * n_chunks], scratch[14 + 8 * n_chunks:]
     dw, acc_dw = dweight, accumulate_dweight
-    if dw is None:
+    if _dweight_sum is not None:
+        if keep_logits_chunk is None or dw is not None:
+            raise ValueError("a dW sum needs kept logits and takes the place of dweight")
+    elif dw is None:
         dw = torch.empty(V, H, dtype=torch.float32, device=dev)
         acc_dw = False
     else:
@@ -470,7 +482,8 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
             if zbuf is None or zbuf.shape[0] < kept or zbuf.dtype != hidden.dtype or zbuf.device != dev \
                     or zbuf.shape[1] != ops.saved_logits_ld(V):
                 zbuf = cache["kept_logits"] = ops.saved_logits_buffer(kept, V, hidden.dtype, dev)
-        need = max(ops.head_step_workspace_bytes(n, n_live, H, V, B, hidden.dtype, zbuf is not None, wt is not None)
+        need = max(ops.head_step_workspace_bytes(n, n_live, H, V, B, hidden.dtype, zbuf is not None, wt is not None,
+                                                 _dweight_sum is not None)
                    for _, n, n_live, _ in parts)
         ws = cache.get("head_step")
         if ws is None or ws.numel() < need or ws.device != dev:
@@ -483,7 +496,7 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
                             final_clip_ratio=final_clip_ratio, kl_coef=max(kl_coef, 0.0), entropy_coef=max(entropy_coef, 0.0),
                             grad_scale=scale, logprob=lp_all, entropy=ent_all, lse=lse_all, g_logprob=glp_all, loss=loss_all,
                             kl=kl_all, sums=sums_buf, flags=flags_buf, result=result, dhidden=dh_all, dweight=dw,
-                            workspace=ws, saved_logits=zbuf, weight_t=wt)
+                            workspace=ws, saved_logits=zbuf, weight_t=wt, dweight_sum=_dweight_sum)
         for k, (lo, n, n_live, pick) in enumerate(parts):
             live_only = bool(skip_masked_forward and pick and n_live > 0)
             chunk = dict(lo=lo, n=n, n_live=n_live, ordered=pick, chunk=k, forward_live_only=live_only, accumulate=acc_dw,
@@ -503,7 +516,7 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
             weight_t_cache["weight_t"] = wt
     else:
         scratch.zero_()
-        if not acc_dw:
+        if dw is not None and not acc_dw:
             dw.zero_()
     if check_flags:
         # one read-back for the reference's three assertions and the host mask's consistency

@@ -46,8 +46,10 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *                 tens of MB more for some shapes); clgrpo_lmhead_bwd_dweight_plan added.
  *   2.02 -> 2.03: kept logits lie in the K-blocked layout that d(logits) takes over (still opaque to callers);
  *                 clgrpo_lmhead_fwd_workspace_bytes allows for 4096 / ceil(T / 256) splits where that is more than 64;
- *                 clgrpo_head_step added. */
-#define CLGRPO_VERSION 203
+ *                 clgrpo_head_step added.
+ *   2.03 -> 2.04: clgrpo_lmhead_bwd_args gained dweight_bf16 (in former padding); clgrpo_head_step_args gained kept_dzt,
+ *                 kept_hidt, kept_ld, kept_k; clgrpo_dweight added. */
+#define CLGRPO_VERSION 204
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
 
@@ -123,8 +125,10 @@ typedef struct {
   int32_t dtype;
   float inv_temperature;
   void* dhidden;            /* [T, H] out, `dtype`; NULL => skipped */
-  float* dweight;           /* [V, H] out, fp32; NULL => skipped */
+  void* dweight;            /* [V, H] out, fp32 (bf16 with dweight_bf16); NULL => skipped */
   int32_t accumulate_dweight; /* nonzero: dweight += ; zero: dweight = */
+  int32_t dweight_bf16;     /* nonzero: round dweight to bf16 once, on its way out; needs bf16 inputs, a workspace for all
+                               T tokens and no accumulation */
   void* workspace;
   size_t workspace_bytes;   /* sets the token chunk: see clgrpo_lmhead_bwd_workspace_bytes */
   void* saved_logits;       /* optional in/out: logits stored by clgrpo_lmhead_fwd for these rows (the same opaque
@@ -344,13 +348,34 @@ typedef struct {
   void* saved_logits;            /* see clgrpo_lmhead_fwd_args; NULL: the backward recomputes them */
   int64_t ld_saved, saved_rows;
   void* weight_t;                /* see clgrpo_lmhead_bwd_args */
+  void* kept_dzt;                /* optional: leave both operands of dW here and compute none; needs saved_logits.  K-blocked
+                                    (see saved_logits of clgrpo_lmhead_fwd_args), rows = V and H rounded up to 256, K =
+                                    kept_ld tokens.  This chunk's rows take the place [kept_k, kept_k + ceil64(n_live)) */
+  void* kept_hidt;
+  int64_t kept_ld, kept_k;       /* multiples of 64 */
 } clgrpo_head_step_args;
 
-/* flags: 1 = with saved_logits, 2 = the caller keeps weight_t */
+/* flags: 1 = with saved_logits, 2 = the caller keeps weight_t, 4 = with kept_dzt */
 size_t clgrpo_head_step_workspace_bytes(int64_t T, int64_t n_live, int64_t H, int64_t V, int64_t B, int32_t dtype, int32_t flags,
                                         size_t recompute_cap);
 int64_t clgrpo_head_step_max_ordered_bytes(void);
 int clgrpo_head_step(const clgrpo_head_step_args* a, void* stream);
+
+/* dW (+)= dzT hidT^T over the operands that clgrpo_head_step calls have kept: one contraction over the tokens of several
+ * micro-batches in the place of one per micro-batch, each of which would read and write dW. */
+typedef struct {
+  const void* dzt;               /* see kept_dzt, kept_hidt, kept_ld */
+  const void* hidt;
+  int64_t ld, k;                 /* tokens per row and how many of them count, multiples of 64 */
+  int64_t H, V;
+  int32_t dtype, accumulate;
+  void* dweight;                 /* [V, H] out, fp32 or bf16 */
+  int32_t dweight_bf16;          /* as in clgrpo_lmhead_bwd_args */
+  void* workspace;
+  size_t workspace_bytes;        /* clgrpo_dweight_workspace_bytes */
+} clgrpo_dweight_args;
+size_t clgrpo_dweight_workspace_bytes(int64_t k, int64_t H, int64_t V, int32_t dtype);
+int clgrpo_dweight(const clgrpo_dweight_args* a, void* stream);
 
 /* ------------------------------------------------------------------ *
  * Group-wise reward -> advantage: adv = (r - mean(pool_g)) / (std(pool_g) + eps),
