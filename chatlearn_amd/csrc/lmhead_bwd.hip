@@ -480,18 +480,38 @@ template <typename OutT> __device__ __forceinline__ OutT cvt_out(float v);
 template <> __device__ __forceinline__ float cvt_out<float>(float v) { return v; }
 template <> __device__ __forceinline__ __bf16 cvt_out<__bf16>(float v) { return (__bf16)v; }
 
-// C (+)= sum over splits of partial[s], each a dense copy of C's shape with `cols` elements per row
+// C (+)= sum over splits of partial[s], each a dense copy of C's shape with `cols` elements per row (a multiple of 32).
+// A thread takes 4 consecutive columns of one row, a block's row is uniform.  HBM-bound: reads the partials once.
+// 16 ranges of 1064 rows at H = 4096 (279 MB): 82.7 -> 57.4 us = 4.9 TB/s, 7 of 5428 at 2048 85.5 -> 54.8 us; with one element
+// per thread the index arithmetic (a 64-bit division each) was what took the time.
 template <typename OutT>
-__global__ void splitk_reduce_kernel(const float* __restrict__ partial, int k_split, int64_t MN, int cols, OutT* C,
-                                     int64_t ldc, int accumulate, const int32_t* __restrict__ order) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < MN; i += (int64_t)gridDim.x * blockDim.x) {
-    float v = 0.f;
-    for (int s = 0; s < k_split; ++s) v += partial[(int64_t)s * MN + i];
-    const int64_t row = i / cols, col = i - row * cols;
-    OutT* dst = C + (order ? order[row] : row) * ldc + col;
-    if (accumulate) v += (float)*dst;
-    *dst = cvt_out<OutT>(v);
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ partial, int k_split, int64_t MN, int cols,
+                                                            OutT* C, int64_t ldc, int accumulate,
+                                                            const int32_t* __restrict__ order) {
+  const int64_t row = blockIdx.x;
+  const int col = (int)(blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  if (col >= cols) return;
+  const f32x4* src = reinterpret_cast<const f32x4*>(partial + row * cols + col);
+  const int64_t step = MN / 4;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+  int s = 0;
+  for (; s + 4 <= k_split; s += 4) {          // four ranges in flight, added in their order
+    const f32x4 x0 = src[s * step], x1 = src[(s + 1) * step], x2 = src[(s + 2) * step], x3 = src[(s + 3) * step];
+    v += x0; v += x1; v += x2; v += x3;
   }
+  for (; s < k_split; ++s) v += src[s * step];
+  OutT* dst = C + (order ? order[row] : row) * ldc + col;
+  struct alignas(4 * sizeof(OutT)) Four { OutT x[4]; };
+  const bool aligned = (reinterpret_cast<uintptr_t>(dst) & (4 * sizeof(OutT) - 1)) == 0;   // the caller's result may start anywhere
+  Four out;
+  if (accumulate) {
+    if (aligned) out = *reinterpret_cast<const Four*>(dst);
+    else for (int k = 0; k < 4; ++k) out.x[k] = dst[k];
+    for (int k = 0; k < 4; ++k) v[k] += (float)out.x[k];
+  }
+  for (int k = 0; k < 4; ++k) out.x[k] = cvt_out<OutT>(v[k]);
+  if (aligned) *reinterpret_cast<Four*>(dst) = out;
+  else for (int k = 0; k < 4; ++k) dst[k] = out.x[k];
 }
 
 // dst(c, r) = src[r][c] (src[order[r]][c] with an order) for r < R, c < C and 0 for R <= r < r_dst, where dst is the K-blocked
@@ -527,12 +547,15 @@ __global__ __launch_bounds__(256) void transpose_block_kernel(const T* __restric
 
 // K ranges per tile that fill `cus` CUs best (1 = no split): work items = tiles x ranges, and a launch
 // takes ceil(items / cus) rounds.  At most kMaxKSplit ranges, each at least 8 slabs long and none empty,
-// and at most what `partial_bytes` can hold of fp32 partial tiles.
+// and at most what `partial_bytes` can hold of fp32 partial tiles.  Fewer tiles than cus / kMaxKSplit may use twice as
+// many ranges: a range is a chain of slabs on one CU while most of the others stand idle (143 rows at H = 1024, V = 32000:
+// 4 tiles, 16 -> 32 ranges 44.8 -> 29.9 us, the sum over the ranges 6 us either way).
 constexpr int kMaxKSplit = 16;
 static int pick_k_split(int tiles, int M, int N, int K, int slab, size_t partial_bytes, int cus) {
   int best = 1;
   double best_eff = 0.0;
-  for (int s = 1; s <= kMaxKSplit; ++s) {
+  const int most = tiles * kMaxKSplit < cus ? 2 * kMaxKSplit : kMaxKSplit;
+  for (int s = 1; s <= most; ++s) {
     if (s > 1) {
       if ((size_t)s * M * N * sizeof(float) > partial_bytes || K / s < 8 * slab) break;
       const int64_t per = round_up64((K + s - 1) / s, slab);
@@ -738,9 +761,10 @@ static int launch_gemm_one(const void* A, int64_t a_kslabs, int M, const void* B
   rc = check_launch("gemm_nt_kernel");
   if (rc || g.k_split == 1) return rc;
   const int64_t MN = (int64_t)M * N;
-  int blocks = (int)((MN + 255) / 256 < 4096 ? (MN + 255) / 256 : 4096);
-  hipLaunchKernelGGL(splitk_reduce_kernel<OutT>, dim3(blocks), dim3(256), 0, stream, partial, g.k_split, MN, kMContig ? M : N,
-                     static_cast<OutT*>(C), ldc, accumulate, rows.order);
+  const int cols = kMContig ? M : N, rows_out = kMContig ? N : M;
+  const int threads = cols / 4 >= 256 ? 256 : (cols / 4 + 63) / 64 * 64;
+  hipLaunchKernelGGL(splitk_reduce_kernel<OutT>, dim3(rows_out, (cols / 4 + threads - 1) / threads), dim3(threads), 0, stream,
+                     partial, g.k_split, MN, cols, static_cast<OutT*>(C), ldc, accumulate, rows.order);
   return check_launch("splitk_reduce_kernel");
 }
 
