@@ -194,7 +194,8 @@ class PolicyStep:
         if keep is not None and data_list:
             rows = sum(int(np.count_nonzero(inputs["loss_mask_host"].numpy())) + 64 for inputs in data_list)
             dw_sum = ops.DweightSum(self.weight.detach(), rows, keep, dw)
-        wt_cache = {}   # the weight does not change between the micro-batches of this step
+        # the weight does not change between the micro-batches of this step; a single one decides itself whether to transpose it
+        wt_cache = {} if len(data_list) > 1 else None
         ws_cache = {}   # kept logits and head scratch memory, shared by the micro-batches of this step
         for inputs in data_list:
             inputs = self._to_device(inputs)

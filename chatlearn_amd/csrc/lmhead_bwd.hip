@@ -672,6 +672,133 @@ static size_t dweight_partial_bytes(int64_t rows, int64_t H, int64_t V, int slab
   return rows > 0 ? plan_dweight(V, H, round_up64(rows, 64), slab, 256, (size_t)1 << 30).partial_bytes : 0;
 }
 
+// dhidden of few rows straight from W [V, H], without W^T.  Building W^T reads and writes the weight once each (V = 151936,
+// H = 4096: 465 us), more than a contraction over a few hundred rows takes.  A wave owns 128 columns of H, 128 rows and
+// a K range.  Lane 16 g + c reads 8 vocabulary rows (k = 8 g ..) x 8 columns (8 c ..) of W, 16 bytes per row, and
+// transposes the square between registers: the result is its A fragment of 8 blocks of 16 columns each, block i
+// holding columns 8 c + i.  B fragments are 16-byte pieces of the K-blocked dz.  No LDS and no barriers: the
+// four waves of a workgroup (512 columns) meet in the L1 on the dz pieces.  Bound by reading W as long as one or
+// two blocks of 128 rows share it; with more rows the matrix work takes over, at a lower rate than the tile of
+// gemm_core.hpp (the limit and both sides' times: kFewRows).
+struct FewRowsParams {
+  const __bf16* dz;       // K-blocked, whole blocks of 256 rows
+  const __bf16* weight;
+  float* partial;         // [k_split][rows][H]
+  int64_t n_kslab;
+  int rows, H, V;
+  int n_h, n_t, k_split, slabs_per_split;
+};
+
+__global__ __launch_bounds__(256, 1) void dhidden_few_rows_kernel(FewRowsParams p) {
+  const int item = xcd_remap(blockIdx.x, gridDim.x);
+  if (item >= p.n_h * p.n_t * p.k_split) return;
+  const int tt = item % p.n_t, ks = item / p.n_t / p.n_h;
+  const int h0 = ((item / p.n_t % p.n_h) * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * 128;
+  if (h0 >= p.H) return;
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int s0 = ks * p.slabs_per_split;
+  const int n_slab = p.n_kslab - s0 < p.slabs_per_split ? (int)(p.n_kslab - s0) : p.slabs_per_split;
+  const int last = 2 * n_slab - 1;                                // steps of 32 vocabulary rows
+  const int col = h0 + 8 * c < p.H ? h0 + 8 * c : p.H - 8;        // columns past H: any, they are not stored
+  const __bf16* z = p.dz + (((int64_t)(tt >> 1) * p.n_kslab + s0) * kBlockRows + (tt & 1) * 128 + c) * 64 + 8 * g;
+
+  // Range-checked loads from a descriptor over the step's valid rows: rows past V read as zero, and no branch stands
+  // between a request and the matrix instructions it is to overlap.
+  const int row_bytes = p.H * 2, voff = 8 * g * row_bytes + col * 2;
+  auto load_a = [&](u32x4 (&raw)[8], int n) __attribute__((always_inline)) {
+    const int v0 = s0 * 64 + (n < last ? n : last) * 32;
+    const int rows = p.V - v0 < 32 ? (p.V > v0 ? p.V - v0 : 0) : 32;
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p.weight) + (int64_t)v0 * p.H, 0, rows * row_bytes, 0x00020000);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) raw[e] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, e * row_bytes, 0);
+  };
+  auto load_b = [&](u32x4 (&b)[8], int n) __attribute__((always_inline)) {
+    const int m = n < last ? n : last;
+    const __bf16* at = z + (int64_t)(m >> 1) * (kBlockRows * 64) + (m & 1) * 32;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) b[j] = *reinterpret_cast<const u32x4*>(at + j * 16 * 64);
+  };
+  f32x4 acc[8][8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc_set(acc[i][j], 0.f, 0.f, 0.f, 0.f);
+  u32x4 raw0[8], raw1[8], b0[8], b1[8];
+  // one step: the fragments of `raw`, the requests for the step after next into it, the products with `b`
+  auto step = [&](u32x4 (&raw)[8], const u32x4 (&b)[8], int n) __attribute__((always_inline)) {
+    u32x4 a[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        a[i][q] = __builtin_amdgcn_perm(raw[2 * q + 1][i / 2], raw[2 * q][i / 2], i % 2 ? 0x07060302u : 0x05040100u);
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(raw, n + 2);
+    GemmTile<__bf16, 8>::settle();     // vector results on their way into matrix instructions
+    each<64>([&](auto m) __attribute__((always_inline)) { Mma<__bf16>::slot(acc, a, b, decltype(m)::value); });
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  load_a(raw0, 0);
+  load_b(b0, 0);
+  load_a(raw1, 1);
+  for (int s = 0; s < n_slab; ++s) {
+    load_b(b1, 2 * s + 1);
+    step(raw0, b0, 2 * s);
+    load_b(b0, 2 * s + 2);
+    step(raw1, b1, 2 * s + 1);
+  }
+  GemmTile<__bf16, 8>::settle();
+  // register r of block (i, j): column 8 (4 g + r) + i, row 16 j + c
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int t = tt * 128 + 16 * j + c;
+    if (t >= p.rows) continue;
+    float* row = p.partial + ((int64_t)ks * p.rows + t) * p.H;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int h = h0 + 8 * (4 * g + r);
+      if (h >= p.H) continue;
+      f32x4 lo, hi;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) { lo[i] = acc_get(acc[i][j], r); hi[i] = acc_get(acc[4 + i][j], r); }
+      *reinterpret_cast<f32x4*>(row + h) = lo;
+      *reinterpret_cast<f32x4*>(row + h + 4) = hi;
+    }
+  }
+}
+
+// K ranges: one workgroup per CU, none empty, at least 8 slabs each; fewer the more rows their partial sums have (384
+// rows at H = 1024, V = 32000: whole step 284 us with 32 ranges, 295 with 42).
+// Up to three blocks of 128 rows: whole training steps with W^T / without it, us, V = 151936 (H = 7168: 129280):
+//   H = 2048: 100 rows 1030 / 809, 200 1165 / 983, 384 1298 / 1183, 512 1368 / 1317, 700 1634 / 1682
+//   H = 4096: 100 rows 1669 / 1235, 200 1875 / 1556, 384 2235 / 2021, 512 2385 / 2317, 700 2997 / 3036
+//   H = 7168: 100 rows 2351 / 1704, 200 2629 / 2213, 384 3289 / 2867, 480 3505 / 3590
+constexpr int64_t kFewRows = 384;
+struct FewRowsPlan {
+  int n_h, n_t, k_split, slabs_per_split;
+  size_t partial_bytes;
+};
+static FewRowsPlan plan_few_rows(int64_t rows, int64_t H, int64_t ldv, int cus, size_t partial_cap) {
+  FewRowsPlan pl;
+  pl.n_h = (int)((H + 511) / 512);
+  pl.n_t = (int)((rows + 127) / 128);
+  const int64_t n_slab = ldv / 64;
+  int64_t s = cus / (pl.n_h * pl.n_t);
+  const int64_t most = (int64_t)(partial_cap / ((size_t)rows * H * sizeof(float)));
+  if (s > 64) s = 64;
+  if (s > 96 / pl.n_t) s = 96 / pl.n_t;
+  if (s > n_slab / 8) s = n_slab / 8;
+  if (s > most) s = most;
+  if (s < 1) s = 1;
+  pl.slabs_per_split = (int)((n_slab + s - 1) / s);
+  pl.k_split = (int)((n_slab + pl.slabs_per_split - 1) / pl.slabs_per_split);
+  pl.partial_bytes = (size_t)pl.k_split * rows * H * sizeof(float);
+  return pl;
+}
+static bool few_rows(int64_t rows, int64_t T, size_t es, bool saved, bool own_wt) {
+  return es == 2 && saved && own_wt && rows == T && rows <= kFewRows;
+}
+
 struct BwdPlan {
   int64_t ldv;        // K extent of dz / WT (V rounded up to 64)
   int64_t chunk;      // tokens per chunk (multiple of 256 unless >= T)
@@ -690,7 +817,8 @@ static BwdPlan bwd_plan(int64_t T, int64_t H, int64_t V, size_t es, int64_t chun
   size_t off = 0;
   // K-blocked operands: whole blocks of 256 rows
   const size_t Hb = (size_t)round_up64(H, 256), Cb = (size_t)round_up64(chunk, 256), Vb = (size_t)round_up64(V, 256);
-  pl.off_wt = off;   off += own_wt ? align_up(Hb * pl.ldv * es, 256) : 0;
+  const bool few = few_rows(chunk, T, es, saved, own_wt);       // reads W itself
+  pl.off_wt = off;   off += own_wt && !few ? align_up(Hb * pl.ldv * es, 256) : 0;
   pl.off_hidt = off; off += own_dw ? align_up(Hb * pl.ldt * es, 256) : 0;
   pl.off_dz = off;   off += saved ? 0 : align_up(Cb * pl.ldv * es, 256);
   pl.off_dzt = off;  off += own_dw ? align_up(Vb * pl.ldt * es, 256) : 0;
@@ -701,6 +829,10 @@ static BwdPlan bwd_plan(int64_t T, int64_t H, int64_t V, size_t es, int64_t chun
   for (size_t b : {dhidden_partial_bytes(chunk, H, pl.ldv, slab), dhidden_partial_bytes(T % chunk, H, pl.ldv, slab),
                    own_dw ? dweight_partial_bytes(chunk, H, V, slab) : 0, own_dw ? dweight_partial_bytes(T % chunk, H, V, slab) : 0})
     if (b > part) part = b;
+  if (few) {
+    const size_t b = plan_few_rows(chunk, H, pl.ldv, 256, (size_t)1 << 30).partial_bytes;
+    if (b > part) part = b;
+  }
   pl.part_bytes = align_up(part, 256);
   pl.off_part = off; off += pl.part_bytes;
   pl.total = off;
@@ -716,6 +848,15 @@ static int64_t chunk_for_workspace(int64_t T, int64_t H, int64_t V, size_t es, s
     if (bwd_plan(T, H, V, es, mid * 256, saved, own_wt, own_dw).total <= bytes) lo = mid; else hi = mid - 1;
   }
   return lo * 256;
+}
+
+template <typename OutT>
+static int launch_splitk_reduce(const float* partial, int k_split, int rows, int cols, OutT* C, int64_t ldc, int accumulate,
+                                const int32_t* order, hipStream_t stream) {
+  const int threads = cols / 4 >= 256 ? 256 : (cols / 4 + 63) / 64 * 64;
+  hipLaunchKernelGGL(splitk_reduce_kernel<OutT>, dim3(rows, (cols / 4 + threads - 1) / threads), dim3(threads), 0, stream,
+                     partial, k_split, (int64_t)rows * cols, cols, C, ldc, accumulate, order);
+  return check_launch("splitk_reduce_kernel");
 }
 
 template <typename T, typename OutT, bool kMContig>
@@ -760,12 +901,8 @@ static int launch_gemm_one(const void* A, int64_t a_kslabs, int M, const void* B
   hipLaunchKernelGGL((gemm_nt_kernel<T, OutT, kMContig>), dim3(grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
   rc = check_launch("gemm_nt_kernel");
   if (rc || g.k_split == 1) return rc;
-  const int64_t MN = (int64_t)M * N;
-  const int cols = kMContig ? M : N, rows_out = kMContig ? N : M;
-  const int threads = cols / 4 >= 256 ? 256 : (cols / 4 + 63) / 64 * 64;
-  hipLaunchKernelGGL(splitk_reduce_kernel<OutT>, dim3(rows_out, (cols / 4 + threads - 1) / threads), dim3(threads), 0, stream,
-                     partial, g.k_split, MN, cols, static_cast<OutT*>(C), ldc, accumulate, rows.order);
-  return check_launch("splitk_reduce_kernel");
+  return launch_splitk_reduce<OutT>(partial, g.k_split, kMContig ? N : M, kMContig ? M : N, static_cast<OutT*>(C), ldc, accumulate,
+                                    rows.order, stream);
 }
 
 // C (+)= A B^T under the launch plan of its orientation: plan_dhidden (C[n][m], with `partial`) or plan_dweight (C[m][n]).
@@ -851,7 +988,8 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
 
   int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&lmhead_dz_kernel<T>), Tile::kLdsBytes, "lmhead_dz_kernel");
   if (rc) return rc;
-  if (a->dhidden && !(a->weight_t && a->weight_t_ready)) {
+  const bool few = few_rows(chunk, T_, sizeof(T), saved, own_wt);
+  if (a->dhidden && !few && !(a->weight_t && a->weight_t_ready)) {
     // WT(h, v) = W[v][h], zero for V <= v < ldv, K-blocked
     rc = launch_transpose<T>(weight, H, wt, pl.ldv, (int)V, (int)H, stream);
     if (rc) return rc;
@@ -920,7 +1058,21 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
       rc = check_launch("lmhead_dz_kernel");
       if (rc) return rc;
     }
-    if (a->dhidden) {
+    if (a->dhidden && few) {
+      const FewRowsPlan fp = plan_few_rows(tc, H, pl.ldv, device_cu_count(), pl.part_bytes);
+      FewRowsParams q;
+      q.dz = reinterpret_cast<const __bf16*>(dz);
+      q.weight = reinterpret_cast<const __bf16*>(weight);
+      q.partial = reinterpret_cast<float*>(ws + pl.off_part);
+      q.n_kslab = ldz / 64;
+      q.rows = (int)tc; q.H = (int)H; q.V = (int)V;
+      q.n_h = fp.n_h; q.n_t = fp.n_t; q.k_split = fp.k_split; q.slabs_per_split = fp.slabs_per_split;
+      hipLaunchKernelGGL(dhidden_few_rows_kernel, dim3((fp.n_h * fp.n_t * fp.k_split + 7) / 8 * 8), dim3(256), 0, stream, q);
+      rc = check_launch("dhidden_few_rows_kernel");
+      if (rc) return rc;
+      rc = launch_splitk_reduce<T>(q.partial, fp.k_split, (int)tc, (int)H, static_cast<T*>(a->dhidden) + t0 * H, H, 0, order, stream);
+      if (rc) return rc;
+    } else if (a->dhidden) {
       // dhidden[chunk][h] = sum_v WT[h][v] dz[t][v]   (M = H, N = tokens, C[n][m])
       rc = launch_gemm<T, T, true>(wt, pl.ldv / Tile::kSlabK, (int)H, dz, ldz / Tile::kSlabK, (int)tc, (int)pl.ldv,
                              static_cast<T*>(a->dhidden) + t0 * H, H, 0, stream,

@@ -49,3 +49,11 @@ def test_k_extents_and_ragged_tiles(dev, dtype, H, keep):
 @pytest.mark.parametrize("V", [255, 4097, 120001])
 def test_vocabulary_splits(dev, T, V):
     _check(dev, T, 192, V, torch.bfloat16, True, seed=T + V)
+
+
+@pytest.mark.parametrize("H,V", [(64, 4097), (192, 33000), (448, 9001), (576, 20064), (1088, 9001)])
+@pytest.mark.parametrize("T", [1, 16, 127, 128, 129, 257, 384, 385])
+def test_dhidden_of_few_rows(dev, T, H, V):
+    """Up to 384 rows with kept logits read W itself (128 columns per wave, 512 per workgroup, 128 rows, K ranges of at least
+    8 slabs); H beyond a whole number of either, a vocabulary that ends inside a slab, rows on both sides of a block and of the limit."""
+    _check(dev, T, H, V, torch.bfloat16, True, seed=T + H)
