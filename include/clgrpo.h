@@ -50,8 +50,10 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *   2.03 -> 2.04: clgrpo_lmhead_bwd_args gained dweight_bf16 (in former padding); clgrpo_head_step_args gained kept_dzt,
  *                 kept_hidt, kept_ld, kept_k; clgrpo_dweight added.
  *   2.04 -> 2.05: clgrpo_lmhead_bwd_workspace_bytes leaves W^T out where it is not built: up to 384 bf16 rows with kept
- *                 logits, all at once and without the caller's weight_t. */
-#define CLGRPO_VERSION 205
+ *                 logits, all at once and without the caller's weight_t.
+ *   2.05 -> 3.00: no change but the number: a caller built against 2.02 may have left the padding unset that is
+ *                 dweight_bf16 since 2.04. */
+#define CLGRPO_VERSION 300
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
 
