@@ -444,11 +444,13 @@ extern "C" size_t clgrpo_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_
   (void)H;
   (void)dtype;
   if (T <= 0 || V <= 0) return 0;
-  // one record per token and vocabulary split; the split count depends on the device's CU count and never
-  // exceeds max_fwd_splits, so this bound holds on any device
-  const int64_t n_vt = (V + kFwdBM - 1) / kFwdBM, most = max_fwd_splits((T + kFwdBN - 1) / kFwdBN);
-  const int64_t splits = n_vt < most ? n_vt : most;
-  return (size_t)splits * (size_t)T * sizeof(float4);
+  // One record per token and vocabulary split; the split count depends on the device's CU count and never
+  // exceeds max_fwd_splits, so this bound holds on any device.  Fewer tokens may take more splits (2200 tokens 455,
+  // 2600 372), so it is the largest over all launches of up to T tokens: below 64 blocks of 256, splits x tokens is at
+  // most 4096 x 256.  A caller may size scratch memory for its longest call and use it for any shorter one.
+  const int64_t n_vt = (V + kFwdBM - 1) / kFwdBM;
+  const int64_t few_blocks = n_vt * T < 4096 * kFwdBN ? n_vt * T : 4096 * kFwdBN, many_blocks = (n_vt < 64 ? n_vt : 64) * T;
+  return (size_t)(few_blocks > many_blocks ? few_blocks : many_blocks) * sizeof(float4);
 }
 
 // Shared by the whole-vocabulary entry point (record == nullptr), the shard one and the whole step.

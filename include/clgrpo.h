@@ -52,8 +52,10 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *   2.04 -> 2.05: clgrpo_lmhead_bwd_workspace_bytes leaves W^T out where it is not built: up to 384 bf16 rows with kept
  *                 logits, all at once and without the caller's weight_t.
  *   2.05 -> 3.00: no change but the number: a caller built against 2.02 may have left the padding unset that is
- *                 dweight_bf16 since 2.04. */
-#define CLGRPO_VERSION 300
+ *                 dweight_bf16 since 2.04.
+ *   3.00 -> 3.01: clgrpo_lmhead_fwd_workspace_bytes never shrinks as T grows (up to 16 MB more for fewer than 64 blocks of
+ *                 256 tokens): between 2.03 and 3.00 scratch memory sized for a longer call could be too small for a shorter one. */
+#define CLGRPO_VERSION 301
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
 

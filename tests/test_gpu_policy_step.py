@@ -158,6 +158,30 @@ def test_host_copy_of_the_training_mask_equals_the_device_mask(dev, packing):
         assert torch.equal(pick(inputs["loss_mask"]).cpu(), inputs["loss_mask_host"])
 
 
+def test_train_step_whose_live_rows_take_more_splits_than_all_rows(dev):
+    """Two padded micro-batches of 33 token blocks of which 31 carry a gradient: the forward runs on those alone, in more
+    vocabulary splits than 33 blocks would get, in scratch memory where nothing else of the step is larger (W^T
+    and the dW operands are kept over the micro-batches).  Against keeping 2048 rows at a time: the same rows, other chunks."""
+    from chatlearn_amd.algorithm.grpo_utils.policy_step import PolicyStep
+    n, p, r, Hd, V = 8, 72, 1977, 2048, 33000
+    g = torch.Generator(device=dev).manual_seed(5)
+    weight = (torch.randn(V, Hd, generator=g, device=dev) * Hd ** -0.5).bfloat16().requires_grad_(True)
+    table = torch.randn(512, Hd, generator=g, device=dev)
+    data = [{"all_tokens": torch.randint(0, 512, (p + r,), generator=g, device=dev).cpu(), "prompt_token_length": p,
+             "response_token_length": r, "old_logprobs": torch.full((p + r,), -10.9), "ref_logprobs": torch.full((p + r,), -10.9),
+             "advantages": float(i % 3 - 1)} for i in range(n)]
+    out = []
+    for keep in ("auto", 2048):
+        weight.grad, tok = None, table.clone().requires_grad_(True)
+        step = PolicyStep(lambda ids, pos: tok[ids].bfloat16(), weight, train_micro_batch_size=4, keep_logits_chunk=keep)
+        out.append((step.train_step(copy.deepcopy(data)), tok.grad, weight.grad))
+    for k in ("pg_loss", "kl_loss", "entropy_loss"):
+        assert out[0][0][k] == pytest.approx(out[1][0][k], rel=1e-5, abs=1e-7), k
+    # fp32 sums in another order, then dhidden and dW are rounded to bf16 once (2^-8 between neighbours)
+    assert_close_rel(out[0][1], out[1][1], 2 ** -8, "token-embedding grad")
+    assert_close_rel(out[0][2], out[1][2], 2 ** -8, "lm_head grad")
+
+
 def test_stale_host_mask_is_refused(dev):
     """A host mask that does not match the device mask would silently drop gradients: the head step
     compares the two sums in the read-back it does anyway for the reference's assertions."""
