@@ -81,7 +81,7 @@ class PolicyStep:
         for data_b in (batching(mb) for mb in microbatch_list):
             tokens_ = data_b["all_tokens"].long()
             ori_batch_size, ori_seq_len = tokens_.size()
-            plen, rlen = list(data_b["prompt_token_length"]), list(data_b["response_token_length"])
+            plen, rlen = ([int(x) for x in data_b[key]] for key in ("prompt_token_length", "response_token_length"))
             text = 'position_ids' not in data_b and self.model_type != "vlm"
             if text:
                 # the masks stay on the device: nothing the host needs of them cannot be had from the lengths
@@ -183,7 +183,7 @@ class PolicyStep:
         through ``dweight_buffer`` (fp32, accumulated) or ``lm_head_weight.grad``."""
         args = self.module_args
         # the same fp32 value that preprocess_data_list leaves on the device
-        n_tok_f = float(np.float32(sum(data["response_token_length"] for data in data_list)))
+        n_tok_f = float(np.float32(float(sum(data["response_token_length"] for data in data_list))))
         _, data_list = self.preprocess_data_list(data_list=data_list, training=True)
         sums = torch.zeros(8, dtype=torch.float64, device=self.device)
         dw = self.dweight_buffer

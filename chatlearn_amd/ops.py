@@ -49,8 +49,9 @@ def _stream(t: torch.Tensor):
 def upload(host: torch.Tensor, device) -> torch.Tensor:
     """Device copy of a CPU tensor that does not stall the host: an ordinary copy from pageable memory waits for
     everything queued on the stream before it.  The pinned block in between comes from torch's caching host
-    allocator, which hands it out again only once the copy is done, whatever thread or stream asks."""
-    if host.numel() == 0 or host.is_pinned():        # a caller's pinned tensor may change once this returns
+    allocator, which hands it out again only once the copy is done, whatever thread or stream asks.  What lists
+    and numbers are mostly given as may also arrive in a device tensor, which goes to ``device`` as it is."""
+    if host.device.type != "cpu" or host.numel() == 0 or host.is_pinned():  # a caller's pinned tensor may change once this returns
         return host.to(device)
     return host.contiguous().pin_memory().to(device, non_blocking=True)
 
