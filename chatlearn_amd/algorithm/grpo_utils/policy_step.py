@@ -153,7 +153,8 @@ class PolicyStep:
         return torch.from_numpy(rows.reshape(-1))
 
     def _put(self, t):
-        return t if t.is_cuda else ops.upload(t, self.device)
+        """On the weight's device: records may hold tensors of another one (a reference policy's)."""
+        return t if t.device == self.device else ops.upload(t, self.device)
 
     def _to_device(self, inputs):
         return {k: (self._put(v) if isinstance(v, torch.Tensor) and not k.endswith("_host") else v)
