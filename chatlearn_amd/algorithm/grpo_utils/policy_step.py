@@ -147,7 +147,7 @@ class PolicyStep:
             rows[:, :-1] = given.cpu().to(torch.int32).numpy()[:, 1:]
         else:
             for row, p, r in zip(rows, plen, rlen):       # response positions p .. p + r - 1, one to the left
-                row[max(p - 1, 0):min(p + r - 1, width - 1)] = 1
+                row[max(p - 1, 0):max(min(p + r - 1, width - 1), 0)] = 1
         if self.packing:
             return torch.from_numpy(np.concatenate([row[:p + r] for row, p, r in zip(rows, plen, rlen)]))
         return torch.from_numpy(rows.reshape(-1))

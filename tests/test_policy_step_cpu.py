@@ -1,4 +1,5 @@
 """Host side of PolicyStep, without a device."""
+import pytest
 import torch
 
 
@@ -17,3 +18,19 @@ def test_tensors_of_another_device_are_moved():
         moved = step._to_device({"old_logprobs": there, "loss_mask_host": torch.empty(3), "n": 2})
         assert moved["old_logprobs"].device == torch.device("cuda:0")
         assert moved["loss_mask_host"].device == torch.device("cpu") and moved["n"] == 2
+
+
+@pytest.mark.parametrize("packing", [False, True])
+def test_host_mask_is_the_rolled_response_mask(packing):
+    """All prompt and response lengths up to the row's end, empty ones among them, against a roll of the mask itself."""
+    width = 5
+    pairs = [(p, r) for p in range(width + 1) for r in range(width + 1 - p)]
+    mask = torch.zeros(len(pairs), width, dtype=torch.int32)
+    for row, (p, r) in zip(mask, pairs):
+        row[p:p + r] = 1
+    want = torch.roll(mask, -1, 1)
+    want[:, -1] = 0
+    want = torch.cat([row[:p + r] for row, (p, r) in zip(want, pairs)]) if packing else want.reshape(-1)
+    plen, rlen = zip(*pairs)
+    for given in (None, mask):
+        assert torch.equal(_step(packing=packing)._shifted_mask_host(given, plen, rlen, width), want)
