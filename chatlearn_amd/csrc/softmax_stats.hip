@@ -59,7 +59,9 @@ __device__ __forceinline__ void rs_update(RowStats& st, const float (&z)[N]) {
     st.u *= f;
     st.m = vmax;
   }
-  const float nb = (st.m == -INFINITY) ? 0.f : -st.m * kLog2e;   // only -inf so far (masked entries): every term is 0
+  // Only -inf so far: every term is 0, and so it is for what lies below -2e38 (entries masked with the type's lowest
+  // value), where -m log2(e) overflows and an infinite sum would outlive the rescale to the first ordinary entry.
+  const float nb = (st.m == -INFINITY) ? 0.f : -fmaxf(st.m, -2e38f) * kLog2e;
 #pragma unroll
   for (int k = 0; k < N; ++k) {
     const float e = __builtin_amdgcn_exp2f(fmaf(z[k], kLog2e, nb));   // one hardware exp2 per element
