@@ -412,7 +412,8 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     live = None
     mask_h = None
     if skip:
-        mask_h = loss_mask_host if loss_mask_host is not None else loss_mask.cpu()
+        # as the loss reads it: of any type, a fraction is no token
+        mask_h = (loss_mask_host if loss_mask_host is not None else loss_mask.detach().cpu()).to(torch.int32)
         live = np.flatnonzero(mask_h.reshape(-1).numpy())
     rows_total = T if live is None else live.size
     ordered_bytes = _lib.lib().clgrpo_head_step_max_ordered_bytes()

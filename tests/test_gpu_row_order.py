@@ -46,3 +46,22 @@ def test_step_with_an_order_equals_the_step_without(dev, n_live, keep, dtype):
         assert_close_rel(got["dhidden"], full["dhidden"], tol, "dhidden")
         assert_close_rel(got["dweight"], full["dweight"], 1e-5 if dtype == torch.float32 else 1e-3, "dweight")
         assert float(got["total_loss"]) == pytest.approx(float(full["total_loss"]), rel=1e-5, abs=1e-7)
+
+
+@pytest.mark.parametrize("host", [False, True])
+@pytest.mark.parametrize("mask_dtype", [torch.bool, torch.int64, torch.bfloat16, torch.float32])
+def test_mask_of_any_type(dev, mask_dtype, host):
+    from chatlearn_amd.fused import grpo_head_step
+    g = torch.Generator().manual_seed(1)
+    mask = (torch.rand(T, generator=g) < 0.4).int()
+    hidden, weight = torch.randn(T, H, generator=g).to(dev), (torch.randn(V, H, generator=g) * 0.07).to(dev)
+    old = (torch.randn(T, generator=g) * 0.1 - 7.5).to(dev)
+    cu = torch.tensor([0, 100, 300, T], dtype=torch.int32)
+    out = []
+    for m in (mask, mask.to(mask_dtype)):
+        out.append(grpo_head_step(hidden, weight, torch.zeros(T, dtype=torch.int64, device=dev), old, old, torch.ones(3, device=dev),
+                                  cu.to(dev), m.to(dev), n_tokens_total=float(mask.sum()), keep_logits_chunk=256,
+                                  cu_seqlens_host=cu.tolist(), loss_mask_host=m if host else None))
+    assert out[0]["rows_projected_bwd"] == out[1]["rows_projected_bwd"] == int(mask.sum())
+    for k in ("total_loss", "dhidden", "dweight"):
+        assert torch.equal(out[0][k], out[1][k])
