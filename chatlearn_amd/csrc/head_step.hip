@@ -105,14 +105,38 @@ extern "C" int clgrpo_head_step(const clgrpo_head_step_args* a, void* stream) {
   CLGRPO_REQUIRE_PTR(a->g_logprob, "g_logprob");
   const bool saved = a->saved_logits != nullptr;
   const bool keep_dw = a->kept_dzt != nullptr;
+  const int64_t n_fwd = a->forward_live_only ? a->n_live : a->T;
+  // What a stage would refuse only behind the launches of the ones before it, or not at all.
+  if ((a->stages & 5) && saved && a->n_live > 0 && a->saved_rows < round_up64(a->n_live, 256))
+    return fail(CLGRPO_ESHAPE, "%s: saved_rows=%lld, but %lld rows keep their logits (rounded up to 256)", who,
+                (long long)a->saved_rows, (long long)a->n_live);
+  if ((a->stages & 1) && n_fwd < a->T) {       // the other rows' outputs are cleared
+    CLGRPO_REQUIRE_PTR(a->logprob, "logprob");
+    CLGRPO_REQUIRE_PTR(a->entropy, "entropy");
+    CLGRPO_REQUIRE_PTR(a->lse, "lse");
+  }
+  if (a->stages & 2) {
+    CLGRPO_REQUIRE_PTR(a->cu_seqlens, "cu_seqlens");
+    CLGRPO_REQUIRE_PTR(a->sums, "sums");
+    CLGRPO_REQUIRE_PTR(a->flags, "flags");
+    if (a->chunk < 0) return fail(CLGRPO_EINVAL, "%s: chunk=%lld", who, (long long)a->chunk);
+  }
   if (keep_dw) CLGRPO_REQUIRE_PTR(a->kept_hidt, "kept_hidt");
+  if ((a->stages & 4) && a->n_live > 0) {
+    if (!saved && (a->row_order != nullptr || keep_dw))
+      return fail(CLGRPO_ESHAPE, "%s: a row order and kept dweight operands need kept logits", who);
+    if (keep_dw && (a->kept_k < 0 || a->kept_k % 64 != 0 || a->kept_ld % 64 != 0 || a->kept_k + round_up64(a->n_live, 64) > a->kept_ld))
+      return fail(CLGRPO_ESHAPE, "%s: %lld tokens do not fit behind the %lld of %lld kept for dweight", who, (long long)a->n_live,
+                  (long long)a->kept_k, (long long)a->kept_ld);
+    if (a->dhidden == nullptr && a->dweight == nullptr && !keep_dw)
+      return fail(CLGRPO_ENULL, "%s: both dhidden and dweight are NULL", who);
+  }
   const int32_t flags = (saved ? 1 : 0) | (a->weight_t ? 2 : 0) | (keep_dw ? 4 : 0);
   const StepPlan pl = step_plan(a->T, a->n_live, a->H, a->V, a->B, a->dtype, flags, a->recompute_cap);
   if (a->workspace_bytes < pl.total)
     return fail(CLGRPO_EWORKSPACE, "%s: workspace %zu < %zu bytes", who, a->workspace_bytes, pl.total);
   char* ws = static_cast<char*>(a->workspace);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t n_fwd = a->forward_live_only ? a->n_live : a->T;
   const RowOrder rows{a->row_order, a->T};
   float* g_entropy = a->entropy_coef > 0 ? reinterpret_cast<float*>(ws + pl.off_gent) : nullptr;
 
@@ -147,7 +171,6 @@ extern "C" int clgrpo_head_step(const clgrpo_head_step_args* a, void* stream) {
     p.grad_scale = a->grad_scale;
     p.loss = a->loss; p.kl = a->ref_logprob ? a->kl : nullptr; p.g_logprob = a->g_logprob; p.g_entropy = g_entropy;
     p.sums = a->sums + 8 * a->chunk; p.flags = a->flags + a->chunk; p.token_offset = a->token_offset;
-    CLGRPO_REQUIRE_PTR(a->cu_seqlens, "cu_seqlens");
     int rc = head_policy_loss(who, &p, ws + pl.off_loss, pl.off_gent - pl.off_loss, s);
     if (rc) return rc;
     if (a->result) {

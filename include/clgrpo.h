@@ -54,7 +54,8 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *   2.05 -> 3.00: no change but the number: a caller built against 2.02 may have left the padding unset that is
  *                 dweight_bf16 since 2.04.
  *   3.00 -> 3.01: clgrpo_lmhead_fwd_workspace_bytes never shrinks as T grows (up to 16 MB more for fewer than 64 blocks of
- *                 256 tokens): between 2.03 and 3.00 scratch memory sized for a longer call could be too small for a shorter one. */
+ *                 256 tokens): between 2.03 and 3.00 scratch memory sized for a longer call could be too small for a shorter one.
+ *                 clgrpo_head_step refuses what a later stage would refuse (or overrun) before it enqueues anything. */
 #define CLGRPO_VERSION 301
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
@@ -352,7 +353,7 @@ typedef struct {
   size_t workspace_bytes;        /* clgrpo_head_step_workspace_bytes */
   size_t recompute_cap;          /* without saved_logits: bound on the backward's share of the workspace */
   void* saved_logits;            /* see clgrpo_lmhead_fwd_args; NULL: the backward recomputes them */
-  int64_t ld_saved, saved_rows;
+  int64_t ld_saved, saved_rows;  /* saved_rows: at least n_live rounded up to 256 */
   void* weight_t;                /* see clgrpo_lmhead_bwd_args */
   void* kept_dzt;                /* optional: leave both operands of dW here and compute none; needs saved_logits.  K-blocked
                                     (see saved_logits of clgrpo_lmhead_fwd_args), rows = V and H rounded up to 256, K =
