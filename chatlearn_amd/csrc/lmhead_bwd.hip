@@ -703,14 +703,15 @@ __global__ __launch_bounds__(256, 1) void dhidden_few_rows_kernel(FewRowsParams 
   const __bf16* z = p.dz + (((int64_t)(tt >> 1) * p.n_kslab + s0) * kBlockRows + (tt & 1) * 128 + c) * 64 + 8 * g;
 
   // Range-checked loads from a descriptor over the step's valid rows: rows past V read as zero, and no branch stands
-  // between a request and the matrix instructions it is to overlap.
+  // between a request and the matrix instructions it is to overlap.  What is checked is the per-lane offset, so the row
+  // is part of it (a scalar offset is outside the check by the builtin's contract).
   const int row_bytes = p.H * 2, voff = 8 * g * row_bytes + col * 2;
   auto load_a = [&](u32x4 (&raw)[8], int n) __attribute__((always_inline)) {
     const int v0 = s0 * 64 + (n < last ? n : last) * 32;
     const int rows = p.V - v0 < 32 ? (p.V > v0 ? p.V - v0 : 0) : 32;
     const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p.weight) + (int64_t)v0 * p.H, 0, rows * row_bytes, 0x00020000);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) raw[e] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, e * row_bytes, 0);
+    for (int e = 0; e < 8; ++e) raw[e] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff + e * row_bytes, 0, 0);
   };
   auto load_b = [&](u32x4 (&b)[8], int n) __attribute__((always_inline)) {
     const int m = n < last ? n : last;

@@ -57,3 +57,27 @@ def test_dhidden_of_few_rows(dev, T, H, V):
     """Up to 384 rows with kept logits read W itself (128 columns per wave, 512 per workgroup, 128 rows, K ranges of at least
     8 slabs); H beyond a whole number of either, a vocabulary that ends inside a slab, rows on both sides of a block and of the limit."""
     _check(dev, T, H, V, torch.bfloat16, True, seed=T + H)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("V", [4097, 9001, 9020])
+@pytest.mark.parametrize("T", [100, 385])
+def test_what_lies_behind_the_operands_does_not_matter(dev, T, V, dtype):
+    """W and the hidden states cut from the front of larger arrays that are not finite behind them; vocabularies that end
+    inside a group of 8 rows, inside a step of 32 and inside a slab."""
+    from chatlearn_amd import ops
+    H = 192
+    g = torch.Generator(device=dev).manual_seed(V)
+    h, w = torch.randn(T, H, generator=g, device=dev).to(dtype), (torch.randn(V, H, generator=g, device=dev) * H ** -0.5).to(dtype)
+    y = torch.randint(0, V, (T,), generator=g, device=dev)
+    glp = torch.randn(T, generator=g, device=dev)
+    behind = torch.full((256, H), float("nan"), dtype=dtype, device=dev)
+    cut = (torch.cat([h, behind])[:T], torch.cat([w, behind])[:V])
+    for keep in (True, False):
+        out = []
+        for hidden, weight in ((h, w), cut):
+            z = ops.saved_logits_buffer(T, V, dtype, dev) if keep else None
+            lp, ent, _, lse = ops.lmhead_forward(hidden, weight, y, saved_logits=z)
+            out.append((lp, ent) + ops.lmhead_backward(hidden, weight, y, lse, None, glp, saved_logits=z))
+        for a, b in zip(*out):
+            assert a.isfinite().all() and torch.equal(a, b)
