@@ -142,7 +142,7 @@ class PolicyStep:
     def _shifted_mask_host(self, given, plen, rlen, width):
         """The shifted training mask on the host, flattened the way the kernels see the tokens: it tells the head
         step which rows carry a gradient without reading anything back from the device."""
-        rows = np.zeros((len(plen), width), dtype=np.int32)
+        rows = np.zeros((len(plen), width) if given is None else tuple(given.shape), dtype=np.int32)
         if given is not None:
             rows[:, :-1] = given.cpu().to(torch.int32).numpy()[:, 1:]
         else:

@@ -34,3 +34,12 @@ def test_host_mask_is_the_rolled_response_mask(packing):
     plen, rlen = zip(*pairs)
     for given in (None, mask):
         assert torch.equal(_step(packing=packing)._shifted_mask_host(given, plen, rlen, width), want)
+
+
+@pytest.mark.parametrize("packing", [False, True])
+@pytest.mark.parametrize("extra", [-2, 0, 3])
+def test_host_mask_of_a_record_has_the_record_s_width(packing, extra):
+    """One sample whose tokens are padded wider than its own loss mask, or less wide: the device mask keeps the record's width."""
+    given = torch.tensor([[0, 0, 1, 1, 0, 1]], dtype=torch.int32)
+    want = torch.tensor([0, 1, 1, 0, 1, 0], dtype=torch.int32)[:5 if packing else None]
+    assert torch.equal(_step(packing=packing)._shifted_mask_host(given, [2], [3], given.shape[1] + extra), want)
