@@ -192,7 +192,8 @@ class PolicyStep:
         # with kept logits dW is contracted over the micro-batches together, as many rows at a time as keep their logits
         keep = keep_rows_bound(self.keep_logits_chunk, self.weight.shape[0], self.weight.dtype)
         dw_sum = None
-        if keep is not None and data_list:
+        need_dw = dw is not None or self.weight.requires_grad
+        if need_dw and keep is not None and data_list:
             rows = sum(int(np.count_nonzero(inputs["loss_mask_host"].numpy())) + 64 for inputs in data_list)
             dw_sum = ops.DweightSum(self.weight.detach(), rows, keep, dw)
         # the weight does not change between the micro-batches of this step; a single one decides itself whether to transpose it
@@ -214,12 +215,12 @@ class PolicyStep:
                 keep_logits_chunk=self.keep_logits_chunk,
                 # only masked sums leave this method, so rows outside the loss mask need no forward either
                 skip_masked_forward=True, weight_t_cache=wt_cache, loss_mask_host=inputs["loss_mask_host"],
-                workspace_cache=ws_cache, _dweight_sum=dw_sum)
+                workspace_cache=ws_cache, _dweight_sum=dw_sum, _need_dweight=need_dw)
             dw, accumulate = out["dweight"], True
             if flat.requires_grad:
                 hidden.backward(out["dhidden"].reshape(hidden.shape))
             sums += out["sums"]
-        if dw_sum is not None and (self.dweight_buffer is not None or self.weight.requires_grad):
+        if dw_sum is not None:
             dw = dw_sum.finish(self.weight.dtype)
         if self.dweight_buffer is None and dw is not None and self.weight.requires_grad:
             g = dw.to(self.weight.dtype)

@@ -346,7 +346,7 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
                    skip_masked_rows=True, skip_masked_forward=False, weight_t_cache: Optional[dict] = None,
                    stage_hook=None, loss_mask_host: Optional[torch.Tensor] = None,
                    workspace_cache: Optional[dict] = None, chunk_hidden_bytes: Optional[int] = None,
-                   _dweight_sum: Optional[ops.DweightSum] = None):
+                   _dweight_sum: Optional[ops.DweightSum] = None, _need_dweight: bool = True):
     """Forward + loss + backward of the head for one packed micro-batch, no autograd graph.
 
     Mirrors policy_trainer.py:216-286 on packed rows: returns a dict with the
@@ -395,7 +395,7 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     of every chunk (a benchmark records stream events there).
 
     ``_dweight_sum`` (needs kept logits): the operands of dW go there in the place of being contracted, ``dweight``
-    in the result is None.
+    in the result is None.  Without ``_need_dweight`` dW is not computed (a frozen weight), ``dweight`` is None as well.
     """
     hidden = ops._dev(hidden, "hidden")
     weight = ops._dev(weight, "weight", hidden.dtype)
@@ -458,6 +458,8 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     if _dweight_sum is not None:
         if keep_logits_chunk is None or dw is not None:
             raise ValueError("a dW sum needs kept logits and takes the place of dweight")
+    elif not _need_dweight:
+        dw = None
     elif dw is None:
         dw = torch.empty(V, H, dtype=torch.float32, device=dev)
         acc_dw = False
@@ -498,16 +500,17 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
                             grad_scale=scale, logprob=lp_all, entropy=ent_all, lse=lse_all, g_logprob=glp_all, loss=loss_all,
                             kl=kl_all, sums=sums_buf, flags=flags_buf, result=result, dhidden=dh_all, dweight=dw,
                             workspace=ws, saved_logits=zbuf, weight_t=wt, dweight_sum=_dweight_sum)
+        stages = 7 if need_dhidden or dw is not None or _dweight_sum is not None else 3       # without a result no backward
         for k, (lo, n, n_live, pick) in enumerate(parts):
             live_only = bool(skip_masked_forward and pick and n_live > 0)
             chunk = dict(lo=lo, n=n, n_live=n_live, ordered=pick, chunk=k, forward_live_only=live_only, accumulate=acc_dw,
                          weight_t_ready=wt_ready)
             if stage_hook is None:
-                step.enqueue(7, **chunk)
+                step.enqueue(stages, **chunk)
             else:
                 for name, bit in (("forward", 1), ("loss", 2), ("backward", 4)):
                     stage_hook(name)
-                    step.enqueue(bit, **chunk)
+                    step.enqueue(bit & stages, **chunk)
                 stage_hook("end")
             rows_projected_fwd += n_live if live_only else n
             rows_projected_bwd += n_live

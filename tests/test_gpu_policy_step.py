@@ -182,6 +182,32 @@ def test_train_step_whose_live_rows_take_more_splits_than_all_rows(dev):
     assert_close_rel(out[0][2], out[1][2], 2 ** -8, "lm_head grad")
 
 
+@pytest.mark.parametrize("keep", ["auto", 64, None])
+@pytest.mark.parametrize("packing", [False, True])
+def test_frozen_weight_keeps_and_contracts_nothing_for_dweight(dev, packing, keep, monkeypatch):
+    """A frozen lm_head without a gradient buffer: the backbone's gradients and the statistics of a trainable one, no operands
+    of dW kept over the micro-batches, no dW; and, with nothing that takes a gradient at all, the statistics alone."""
+    from chatlearn_amd import ops
+    from chatlearn_amd.algorithm.grpo_utils.policy_step import PolicyStep
+    data = _samples(9, 11, True)
+    g = torch.Generator().manual_seed(4)
+    weight = (torch.randn(VOCAB, H, generator=g) * 0.1).to(dev)
+    made, new_sum = [], ops.DweightSum
+    monkeypatch.setattr(ops, "DweightSum", lambda *a: made.append(a) or new_sum(*a))
+    out = []
+    for train_weight, train_backbone in ((True, True), (False, True), (False, False)):
+        bb = _Backbone(torch.float32).to(dev).requires_grad_(train_backbone)
+        w = weight.clone().requires_grad_(train_weight)
+        made.clear()
+        step = PolicyStep(bb, w, packing=packing, max_token_in_seq=200, train_micro_batch_size=2, keep_logits_chunk=keep)
+        stats = step.train_step(copy.deepcopy(data))
+        assert bool(made) == (train_weight and keep is not None) and (w.grad is None) != train_weight
+        out.append((stats, bb.tok.grad))
+    for stats, _ in out[1:]:
+        assert stats == out[0][0]
+    assert torch.equal(out[0][1], out[1][1]) and out[2][1] is None
+
+
 def test_stale_host_mask_is_refused(dev):
     """A host mask that does not match the device mask would silently drop gradients: the head step
     compares the two sums in the read-back it does anyway for the reference's assertions."""
