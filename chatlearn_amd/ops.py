@@ -363,7 +363,7 @@ class DweightSum:
     def place(self, rows: int) -> None:
         """Make room for the operands of ``rows`` more tokens."""
         rows = _round_up(rows, 64)
-        if self.used + rows > self.capacity:
+        if self.used > 0 and self.used + rows > self.capacity:
             self._contract(torch.float32)
         if rows > self.capacity:                 # one chunk beyond the limit
             self.capacity, self.dzt, self.hidt = rows, None, None
