@@ -32,13 +32,15 @@ class PolicyStep:
                  train_micro_batch_size: int = 1, generate_micro_batch_size: int = 1, trainable: bool = True,
                  fsdp_size: int = 1, temperature: float = 1.0, dweight_buffer: Optional[torch.Tensor] = None,
                  keep_logits_chunk=AUTO, model_type: str = "llm",
-                 prepend_text_position_channel: Optional[bool] = None):
+                 prepend_text_position_channel: Optional[bool] = None, dweight_sum_rows=AUTO):
         """``backbone(input_ids, position_ids)`` returns the final hidden states ``[b, s, H]``; with
         ``model_type='vlm'`` it is called as ``backbone(input_ids, position_ids, pixel_values=...,
         image_grid_thw=...)`` (policy_trainer.py:206-214).  ``prepend_text_position_channel``: packed
         vision-language position ids get the first channel repeated in front, which the reference does for
         transformers >= 4.55 (policy_trainer.py:124-125); ``None`` decides the same way from the installed
-        transformers, if there is one."""
+        transformers, if there is one.  ``dweight_sum_rows``: rows whose operands of dW ``train_step`` holds beside the
+        kept logits, to contract several micro-batches together - 2 (V + H) bytes each in bf16, ``"auto"`` as many as
+        ``keep_logits_chunk`` (10 GiB, or what the mini-batch needs); ``None`` contracts every micro-batch by itself."""
         self.backbone = backbone
         self.weight = lm_head_weight
         self.module_args = dict(_DEFAULT_ARGS)
@@ -52,6 +54,7 @@ class PolicyStep:
         self.temperature = temperature
         self.dweight_buffer = dweight_buffer
         self.keep_logits_chunk = keep_logits_chunk
+        self.dweight_sum_rows = dweight_sum_rows
         self.model_type = model_type
         if prepend_text_position_channel is None and model_type == "vlm":
             try:
@@ -152,6 +155,16 @@ class PolicyStep:
             return torch.from_numpy(np.concatenate([row[:p + r] for row, p, r in zip(rows, plen, rlen)]))
         return torch.from_numpy(rows.reshape(-1))
 
+    def _dweight_sum(self, data_list):
+        """Where the operands of dW wait over the micro-batches, None where each is contracted by itself (always
+        without kept logits)."""
+        keep = keep_rows_bound(self.keep_logits_chunk, self.weight.shape[0], self.weight.dtype)
+        limit = keep if isinstance(self.dweight_sum_rows, str) and self.dweight_sum_rows == AUTO else self.dweight_sum_rows
+        if keep is None or not limit:
+            return None
+        rows = sum(int(np.count_nonzero(inputs["loss_mask_host"].numpy())) + 64 for inputs in data_list)
+        return ops.DweightSum(self.weight.detach(), rows, limit, self.dweight_buffer)
+
     def _put(self, t):
         """On the weight's device: records may hold tensors of another one (a reference policy's)."""
         return t if t.device == self.device else ops.upload(t, self.device)
@@ -189,13 +202,8 @@ class PolicyStep:
         sums = torch.zeros(8, dtype=torch.float64, device=self.device)
         dw = self.dweight_buffer
         accumulate = dw is not None
-        # with kept logits dW is contracted over the micro-batches together, as many rows at a time as keep their logits
-        keep = keep_rows_bound(self.keep_logits_chunk, self.weight.shape[0], self.weight.dtype)
-        dw_sum = None
         need_dw = dw is not None or self.weight.requires_grad
-        if need_dw and keep is not None and data_list:
-            rows = sum(int(np.count_nonzero(inputs["loss_mask_host"].numpy())) + 64 for inputs in data_list)
-            dw_sum = ops.DweightSum(self.weight.detach(), rows, keep, dw)
+        dw_sum = self._dweight_sum(data_list) if need_dw and data_list else None
         # the weight does not change between the micro-batches of this step; a single one decides itself whether to transpose it
         wt_cache = {} if len(data_list) > 1 else None
         ws_cache = {}   # kept logits and head scratch memory, shared by the micro-batches of this step

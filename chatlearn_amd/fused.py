@@ -540,5 +540,6 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
             "rows_projected_fwd": rows_projected_fwd, "sums": result[:8], "token_chunks": chunks,
             # device memory this call held beyond its inputs and outputs: kept logits (they become d(logits) in
             # place), the workspace (d(logits)^T, hidden^T, W^T unless the caller's cache holds it, split-K partials;
-            # the forward's per-split records before that) and the caller's W^T
-            "scratch_bytes": sum(t.numel() * t.element_size() for t in (zbuf, ws, wt) if t is not None)}
+            # the forward's per-split records before that), the caller's W^T and the operands of dW that wait in a sum
+            "scratch_bytes": sum(t.numel() * t.element_size() for t in (zbuf, ws, wt) if t is not None)
+                             + (_dweight_sum.bytes if _dweight_sum is not None else 0)}

@@ -360,6 +360,11 @@ class DweightSum:
         self.dzt = self.hidt = None
         self.used = 0
 
+    @property
+    def bytes(self) -> int:
+        """Device memory the operands take (not the sum itself)."""
+        return sum(t.numel() * t.element_size() for t in (self.dzt, self.hidt) if t is not None)
+
     def place(self, rows: int) -> None:
         """Make room for the operands of ``rows`` more tokens."""
         rows = _round_up(rows, 64)

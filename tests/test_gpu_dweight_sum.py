@@ -41,6 +41,7 @@ def test_sum_over_micro_batches(dev, dtype, H, V, limit, with_buffer):
         a = grpo_head_step(*args, loss_mask_host=mask, cu_seqlens_host=cu, dweight=want, accumulate_dweight=True, **kw)
         b = grpo_head_step(*args, loss_mask_host=mask, cu_seqlens_host=cu, _dweight_sum=total, **kw)
         assert b["dweight"] is None and torch.equal(a["dhidden"], b["dhidden"])
+        assert b["scratch_bytes"] >= total.bytes > 0
     got = total.finish(dtype)
     assert got.dtype == (torch.float32 if with_buffer else dtype) and (buffer is None or got is buffer)
     # the order of fp32 sums differs; a bf16 result is rounded once (2^-9 of each entry)

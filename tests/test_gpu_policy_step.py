@@ -208,6 +208,24 @@ def test_frozen_weight_keeps_and_contracts_nothing_for_dweight(dev, packing, kee
     assert torch.equal(out[0][1], out[1][1]) and out[2][1] is None
 
 
+@pytest.mark.parametrize("with_buffer", [False, True])
+def test_bound_on_the_rows_that_wait_for_dweight(dev, with_buffer):
+    """Micro-batches contracted by themselves, a few rows at a time or all together: the same dW but for the order of
+    fp32 sums, and each step's memory as it is reported."""
+    from chatlearn_amd.algorithm.grpo_utils import policy_step as ps
+    data = _samples(9, 21, True)
+    g = torch.Generator().manual_seed(4)
+    weight, base = (torch.randn(VOCAB, H, generator=g) * 0.1).to(dev), torch.randn(VOCAB, H, generator=g).to(dev)
+    out = []
+    for rows in (None, 64, "auto"):
+        bb, w, buf = _Backbone(torch.float32).to(dev), weight.clone().requires_grad_(True), base.clone() if with_buffer else None
+        step = ps.PolicyStep(bb, w, train_micro_batch_size=2, dweight_buffer=buf, dweight_sum_rows=rows)
+        out.append((step.train_step(copy.deepcopy(data)), bb.tok.grad, buf if with_buffer else w.grad))
+    for stats, tok, dw in out[1:]:
+        assert stats == out[0][0] and torch.equal(tok, out[0][1])
+        assert_close_rel(dw, out[0][2], 1e-5, "dweight")
+
+
 def test_stale_host_mask_is_refused(dev):
     """A host mask that does not match the device mask would silently drop gradients: the head step
     compares the two sums in the read-back it does anyway for the reference's assertions."""
