@@ -334,7 +334,8 @@ static int launch_finalize(const FinalizeParams& f, hipStream_t stream) {
 // ceil(n_tb * n_split / CUs) rounds, so its cost in tile periods is rounds * tiles-per-workgroup.
 // Many splits and several rounds are fine (65 token blocks: 35 splits of 17 tiles, 9 rounds = 153 tile
 // periods against the ideal 151), so the plan stays within a few per cent of n_tb * n_vt / CUs tile periods
-// from about 7 token blocks on.  Two smaller terms, both measured on launches of equal tile periods:
+// from about 7 token blocks on.  Two smaller terms, both measured on launches of equal tile periods, with a core of eight
+// waves per tile that the present one has replaced (not measured again since):
 //  - the splits are handed out in groups of 4 (the workgroups of an XCD then form a block of 4 splits x
 //    CUs/32 token blocks that shares operand slabs in the XCD's L2: 4 + 8 = 12 slabs per step for 32 tiles).
 //    A last group of w < 4 splits makes blocks of w x 32/w, w + 32/w slabs per step; the time grows by about
