@@ -131,7 +131,8 @@ class PolicyStep:
             data_obj = {"all_tokens": tokens, "position_ids": position_ids, "labels": labels,
                         "ori_seq_len": ori_seq_len, "indices": indices, "cu_seqlens": cu_seqlens,
                         "ori_batch_size": ori_batch_size, "sample_ids": data_b["id_in_list"],
-                        "attention_mask": attn_mask, "pad_size": 0, "sample_lengths": [p + r for p, r in zip(plen, rlen)]}
+                        "attention_mask": attn_mask, "pad_size": 0,
+                        "sample_lengths": [min(p + r, ori_seq_len) for p, r in zip(plen, rlen)]}   # as many as attn_mask marks
             if self.model_type == "vlm":
                 data_obj.update({"pixel_values": data_b.get("pixel_values", None),
                                  "image_grid_thw": data_b.get("image_grid_thw", None)})

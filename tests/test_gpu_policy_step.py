@@ -389,3 +389,24 @@ def test_vision_language_inputs_reach_the_backbone_and_train(dev, packing, prepe
     recs = step.forward_step(copy.deepcopy(data))
     for a, b in zip(recs, centred):
         assert_close_rel(a["old_logprobs"], b["old_logprobs"], 1e-5, "per-sample logprobs (vlm)")
+
+
+def test_vision_language_records_of_a_sample_cut_short(dev):
+    """Tokens cut below prompt + response: the records are as long as the tokens, packed as padded."""
+    from chatlearn_amd.algorithm.grpo_utils.policy_step import PolicyStep
+    g = torch.Generator().manual_seed(5)
+    data = _samples(4, 31, False)
+    for s in data:
+        p = s["prompt_token_length"]
+        s["all_tokens"] = s["all_tokens"][:40]
+        s["response_token_length"] = s["all_tokens"].numel() - p + (20 if s["all_tokens"].numel() == 40 else 0)
+        s["position_ids"] = [sorted(torch.randint(0, p, (p,), generator=g).tolist()) for _ in range(3)]
+        s["pixel_values"], s["image_grid_thw"] = torch.randn(2, 6, generator=g), torch.tensor([[1, 1, 2]])
+    bb, weight = _VLBackbone(torch.float32).to(dev), (torch.randn(VOCAB, H, generator=g) * 0.05).to(dev)
+    out = [PolicyStep(bb, weight, packing=packing, max_token_in_seq=10 ** 6, generate_micro_batch_size=4, model_type="vlm",
+                      prepend_text_position_channel=False).forward_step(copy.deepcopy(data)) for packing in (False, True)]
+    for padded, packed in zip(*out):
+        n = packed["all_tokens"].numel()
+        assert packed["old_logprobs"].numel() == padded["old_logprobs"].numel() == n
+        # the last token's label is the next sample's first token or the padding
+        assert_close_rel(packed["old_logprobs"][:n - 1], padded["old_logprobs"][:n - 1], 1e-5, "per-sample logprobs")
