@@ -335,7 +335,6 @@ def gemm_kernels(w, keep, reps=3):
     row_map = torch.full((n,), -1, dtype=torch.int32, device=dev)
     row_map[live] = torch.arange(rows, dtype=torch.int32, device=dev)
     zbuf = ops.saved_logits_buffer(rows, cfg.V, cfg.dtype, dev)
-    wt = ops.weight_t_buffer(w.weight)
     hidden, labels = w.hidden[lo:hi], w.labels[lo:hi]
     state = {}
 
@@ -355,9 +354,7 @@ def gemm_kernels(w, keep, reps=3):
     def bwd(need_h, need_w):
         ops.lmhead_backward(h_c, w.weight, lab_c, state["lse"], state["ent"] if g_en is not None else None, g_lp, g_en,
                             cfg.temperature, need_dhidden=need_h, need_dweight=need_w, dweight=dwbuf if need_w else None,
-                            accumulate_dweight=False, saved_logits=zbuf, weight_t=wt, weight_t_ready=True)
-    ops.lmhead_backward(h_c, w.weight, lab_c, state["lse"], None, g_lp, None, cfg.temperature, need_dweight=False,
-                        saved_logits=zbuf, weight_t=wt, weight_t_ready=False)          # fills W^T once
+                            accumulate_dweight=False, saved_logits=zbuf)
     t_fwd = _events(fwd, reps)
     t_both = _events(lambda: bwd(True, True), reps, setup=fwd_and_pick)
     t_dh_only = _events(lambda: bwd(True, False), reps, setup=fwd_and_pick)
@@ -371,8 +368,8 @@ def gemm_kernels(w, keep, reps=3):
                 "frac": round(tf / peak, 4)}
     return {"chunk_tokens": n,
             "forward": rec("lmhead_fwd_kernel (+ finalize)", n, t_fwd),
-            "dhidden": rec("gemm_nt_kernel<16-bit out> (+ split-K reduce)", rows, t_both - t_dw_only),
-            "dweight": rec("gemm_nt_kernel<fp32 out>", rows, t_both - t_dh_only),
+            "dhidden": rec("gemm_kernel<W across> (+ split-K reduce)", rows, t_both - t_dw_only),
+            "dweight": rec("gemm_kernel<d(logits) across> (+ split-K tail)", rows, t_both - t_dh_only),
             "rest_of_backward_ms": round(t_dh_only + t_dw_only - t_both, 3)}
 
 
@@ -540,7 +537,7 @@ def autograd_seam(w, steps):
 def sweep(cfg, device, weight, keep):
     """Every micro-batch of the configuration's mini-batch: the sample population regrouped by the library's
     bin packing (split_microbatch with packing, rows 6-8 of the path) into micro-batches of at most cfg.T
-    tokens, each run through the head step; dW accumulates across them and W^T is built once."""
+    tokens, each run through the head step; dW accumulates across them."""
     from chatlearn_amd.algorithm.grpo_utils.trainer_utils import split_microbatch
     pop = synthetic.sample_population(cfg, synthetic.generator_for(cfg))
     adv_all = advantages_for(pop, device, group=cfg.group)
@@ -566,15 +563,14 @@ def sweep(cfg, device, weight, keep):
         w.adv = adv_all[torch.tensor([s["sample_index"] for s in mb], device=device)]
         works.append(w.finish())
     dweight = torch.zeros(cfg.V, cfg.H, dtype=torch.float32, device=device)
-    cache, ws_cache = {}, {}
+    ws_cache = {}
     for w in works[:2]:                                    # warm-up
-        head_step(w, keep, dweight, accumulate=True, weight_t_cache=cache, n_tok=n_tok_total, workspace_cache=ws_cache)
-    cache.clear()
+        head_step(w, keep, dweight, accumulate=True, n_tok=n_tok_total, workspace_cache=ws_cache)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     rows_bwd = launches = 0
     for i, w in enumerate(works):
-        o = head_step(w, keep, dweight, accumulate=i > 0, weight_t_cache=cache, n_tok=n_tok_total, workspace_cache=ws_cache)
+        o = head_step(w, keep, dweight, accumulate=i > 0, n_tok=n_tok_total, workspace_cache=ws_cache)
         rows_bwd += o["rows_projected_bwd"]
         launches += len(o["token_chunks"])
     torch.cuda.synchronize()
@@ -586,7 +582,7 @@ def sweep(cfg, device, weight, keep):
             "tokens_per_micro_batch_min_max": [min(w.T for w in works), max(w.T for w in works)],
             "ms_total": dt * 1e3, "tokens_per_s": tokens / dt, "host_bin_packing_ms": round(packing_ms, 2),
             "host_bin_packing_library_calls_ms": round(packing_calls_ms, 3),
-            "note": "bin-packed micro-batches of the whole mini-batch, dW accumulated, W^T built once"}
+            "note": "bin-packed micro-batches of the whole mini-batch, dW accumulated"}
 
 
 def other_config(name, device, steps, warmup):

@@ -205,8 +205,6 @@ class PolicyStep:
         accumulate = dw is not None
         need_dw = dw is not None or self.weight.requires_grad
         dw_sum = self._dweight_sum(data_list) if need_dw and data_list else None
-        # the weight does not change between the micro-batches of this step; a single one decides itself whether to transpose it
-        wt_cache = {} if len(data_list) > 1 else None
         ws_cache = {}   # kept logits and head scratch memory, shared by the micro-batches of this step
         for inputs in data_list:
             inputs = self._to_device(inputs)
@@ -223,7 +221,7 @@ class PolicyStep:
                 dweight=dw if dw_sum is None else None, accumulate_dweight=accumulate, need_dhidden=flat.requires_grad,
                 keep_logits_chunk=self.keep_logits_chunk,
                 # only masked sums leave this method, so rows outside the loss mask need no forward either
-                skip_masked_forward=True, weight_t_cache=wt_cache, loss_mask_host=inputs["loss_mask_host"],
+                skip_masked_forward=True, loss_mask_host=inputs["loss_mask_host"],
                 workspace_cache=ws_cache, _dweight_sum=dw_sum, _need_dweight=need_dw)
             dw, accumulate = out["dweight"], True
             if flat.requires_grad:

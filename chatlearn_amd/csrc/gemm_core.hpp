@@ -1,5 +1,5 @@
-// NT-GEMM workgroup tile for gfx950 (CDNA4): C^[256 x 256] = A[256 x K] * B[256 x K]^T,
-// both operands K-contiguous in memory, fp32 accumulation on the matrix cores.
+// GEMM workgroup tile for gfx950 (CDNA4): C^[256 x 256] = A[256 x K] * B[256 x K]^T, B K-contiguous in memory, A either
+// way round, fp32 accumulation on the matrix cores.
 //
 // One workgroup of 2 x 2 wavefronts (64 lanes each, one per SIMD of a CU) owns a 256 x 256 tile; a wave
 // owns 128 x 128 of it as 8 x 8 blocks of 16 x 16.  K is walked in slabs of 128 bytes per row (64 bf16 or 32
@@ -10,34 +10,35 @@
 //  - 128 x 128 per wave reads 16 fragments per 64 matrix instructions; the 128 x 64 of eight waves read 12 per 32.
 //  - v_mfma 16x16x32 against 32x32x16 on the same operands: 2 % more rate out of registers (1870 against 1827
 //    TFLOP/s), 6 % in this loop.
-//  - every instruction's place is fixed in the source: a fragment read of the next half after every second
-//    matrix instruction, an operand load after every eighth (more often and the loads back up behind the
-//    vector memory path, which takes a wave's kilobyte per 16 cycles, and the wave with them), scalar address
-//    work one piece at a time in between.  With one wave per SIMD nothing else would fill a gap.
-// Measured on operands of M = 4096, N = 12288, K = 32768 (bf16): 1493 TFLOP/s row-major, 1505 K-blocked; the
-// eight-wave 32x32x16 form of this tile with two 64 KB stages ran 1310.
+//  - every instruction's place is fixed in the source (see the schedule): with one wave per SIMD nothing else would
+//    fill a gap.
+// At 12288 tokens, H = 4096, V = 151936 (bf16, counters): matrix cores busy 0.865 of the cycles at 1.64 GHz, 1.50 - 1.54
+// PFLOP/s for either contraction of the backward.  With the barriers and load waits left out (wrong results) they are busy
+// 0.88 and the clock falls: 0.5 % less time.  The eight-wave 32x32x16 form of this tile with two 64 KB stages ran
+// 13 % slower.
 //
 // Operand slabs travel HBM/L2 -> LDS directly (buffer loads with an LDS destination; no registers, no LDS
 // store instructions) into two rings of 32 KB slots, three for A and two for B: all 160 KB.  While the matrix
 // cores work on slab s, B(s+1) and A(s+1), A(s+2) land; a slot is requested again right after the barrier
 // behind its last fragment read.  The third A slot is what makes the loads of a slab early enough: with two
-// 64 KB stages (same loop) the row-major rate is 1398.  One barrier per slab, preceded by an explicit
+// 64 KB stages (same loop) the rate was 6 % lower.  One barrier per slab, preceded by an explicit
 // wait for this wave's own loads, because a barrier alone does not wait for loads whose destination is LDS; the
 // youngest eight (the A slab after next) stay outstanding.
 //
 // A load fills LDS in lane order, so rows are 128 bytes apart with no padding; bank conflicts are
-// avoided by an XOR swizzle of the 16-byte K-chunks within a row, applied on the global side of the load and
-// undone by the fragment reads (0 conflict cycles).
+// avoided by which 16-byte chunk and row a lane fetches, undone by the fragment reads (0 conflict cycles, see Bank conflicts).
 //
-// Operands are either row-major (the caller's hidden states and weight) or K-blocked (the library's own
-// intermediates: per tile and slab one contiguous 32 KB piece, see Operand).  Consecutive tiles of a
-// workgroup stream into each other: requests that run past a tile's last slab continue with the next
-// tile's first ones, whose first fragments are in registers when the tile ends.
+// Operands are row-major (the caller's hidden states and weight), K-blocked (hidden^T, a caller's W^T: per tile and
+// slab one contiguous 32 KB piece, see Operand) or kept logits / d(logits) (units, see unit_index).  A may also lie the
+// other way round, with the contracted dimension along its rows (see Side): d(logits) has tokens as rows and
+// serves both contractions of the backward, and W is read as it is for dhidden.  Neither has a transposed copy.
+// Consecutive tiles of a workgroup stream into each other: requests that run past a tile's last slab continue
+// with the next tile's first ones, whose first fragments are in registers when the tile ends.
 //
 // Accumulators (v_mfma_f32_16x16x*): lane l = 16 g + c holds, in register r of block (i, j), the product of
-//     A row a_row(i, 4 g + r)   and   B row b_row(j, c).
+//     A row lane_a0() + a_off(i, r)   and   B row lane_b0() + b_block(j)   of the wave's 128.
 // Which rows of the wave's 128 make up a block is free, because it only decides where a fragment is read
-// from.  a_row gives a lane VEC = 16 / sizeof(T) consecutive A rows (bf16: over a pair of blocks), b_row BV
+// from.  a_off gives a lane VEC = 16 / sizeof(T) consecutive A rows (bf16: over a pair of blocks), b_block BV
 // consecutive B rows over BV blocks, so that 16-byte pieces of either orientation of the result are in one
 // lane and leave without a shuffle.  The callers put the dimension they reduce over (vocabulary, for the
 // softmax statistics) on A, which makes that reduction mostly lane-local.
@@ -68,9 +69,18 @@ __host__ __device__ __forceinline__ int64_t blocked_index(int64_t row, int64_t k
   return (((row / kBlockRows) * n_kslab + k / E) * kBlockRows + (row % kBlockRows)) * E + (k % E);
 }
 
-// Kept logits: the forward leaves a chunk's raw logits for the backward in the K-blocked layout (rows =
-// tokens, K = vocabulary) that the d(logits) operand will have, so that the kernel that turns one into the
-// other works in place.  16-bit inputs keep their logits as IEEE half (10 mantissa bits against bf16's 7: the
+// Element (token, v) of kept logits and of d(logits) with `n_kslab` slabs per token: units of one slab's 128 bytes of
+// vocabulary by as many tokens as a slab has elements (64 x 64 of 16 bits, 32 x 32 of fp32), the units of a row of units one
+// after another.  A 256-wide tile of either orientation and one slab of the other dimension are then whole units: 256 / E
+// pieces of E * 128 bytes, one 32 KB run where the tile lies along the vocabulary.
+template <typename T>
+__host__ __device__ __forceinline__ int64_t unit_index(int64_t token, int64_t v, int64_t n_kslab) {
+  constexpr int E = kRowBytes / (int)sizeof(T);
+  return ((token / E * n_kslab + v / E) * E + token % E) * E + v % E;
+}
+
+// Kept logits: the forward leaves a chunk's raw logits for the backward in the layout (see unit_index) that the
+// d(logits) operand will have, so that the kernel that turns one into the other works in place.  16-bit inputs keep their logits as IEEE half (10 mantissa bits against bf16's 7: the
 // softmax the backward rebuilds from them is 8x closer to the fp32 one), fp32 inputs as fp32.
 template <typename T> struct KeptLogit;
 template <> struct KeptLogit<__bf16> { typedef _Float16 type; };
@@ -84,6 +94,7 @@ template <> struct KeptLogit<float> { typedef float type; };
 // acc_get / acc_set for the same reason.
 template <typename T> struct Mma;
 template <> struct Mma<__bf16> {
+  template <bool kAcross = false>
   __device__ static __forceinline__ void slot(f32x4 (&acc)[8][8], const u32x4 (&a)[8], const u32x4 (&b)[8], int m) {
     const int i = m / 8, j = (i & 1) ? 7 - m % 8 : m % 8;
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(a[i]), "v"(b[j]));
@@ -92,12 +103,16 @@ template <> struct Mma<__bf16> {
 template <> struct Mma<float> {
   // 16 bytes hold four K=4 steps: lane group g, element e stands for k = 4g + e in both operands.  A slot takes
   // step m % 8 / 2 of four blocks of row i, so that an accumulator comes up again eight instructions later.
+  // kAcross: a[4 q + e] holds k = 4g + e of the four blocks 4 q .. 4 q + 3 (an A with K along its rows): the
+  // transposition of a 4 x 4 square of single registers is a choice of registers.
+  template <bool kAcross = false>
   __device__ static __forceinline__ void slot(f32x4 (&acc)[8][8], const u32x4 (&a)[8], const u32x4 (&b)[8], int m) {
     const int i = m / 8, e = m % 8 / 2;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int j = (m % 2) * 4 + k;
-      asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(a[i][e]), "v"(b[j][e]));
+      const uint32_t av = kAcross ? a[i / 4 * 4 + e][i % 4] : a[i][e];
+      asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(av), "v"(b[j][e]));
     }
   }
 };
@@ -124,8 +139,23 @@ __device__ __forceinline__ void each(Fn fn, std::integer_sequence<int, M...>) { 
 template <int N, typename Fn>
 __device__ __forceinline__ void each(Fn fn) { each(fn, std::make_integer_sequence<int, N>{}); }
 
-// BV: consecutive B rows a lane holds (see above), 8 or 4.
-template <typename T, int BV>
+// Where the contracted dimension K of operand A lies.
+//   kRows:    along the rows of memory (row-major or K-blocked, see Operand): a fragment is 16 bytes of an A row.
+//   kWeight:  across them, in a row-major matrix [K][M] (W for dhidden: K = vocabulary, M = H).
+//   kLogits:  across them, in units (d(logits) for dW: K = tokens, M = vocabulary).
+// Across: a slab is kSlabK rows of 256 columns, in LDS kSub pieces of kSlabK rows x 128 bytes.  A lane reads VEC
+// rows (k = VEC g ..) of 16 bytes and transposes that square between registers.  bf16: 32 v_perm_b32 for the 8
+// fragments of a half, half of a 4-cycle instruction per matrix instruction of 16 cycles, no LDS access more than
+// reading rows takes; fp32: a choice of registers.  It costs 1.5 - 2 % of a contraction (12288 tokens, H = 4096, V = 151936:
+// dhidden 9.9 -> 10.05 ms, dW the same within the runs); the transposed copies cost more: W^T 0.46 ms, dz^T 0.75 - 1.1 ms of
+// the d(logits) pass and as much memory as the logits.  16384 tokens at H = 4096, whole step: 38.6 -> 37.3 ms, 32768 at
+// 2048: 46.9 -> 45.2, 6400 at 2048: 10.0 -> 9.4.  ds_read_b64_tr_b16 in its place needs twice the LDS reads (dW 14 % slower).
+// Up to 384 rows a kernel without LDS read W directly; this tile is faster from the first row on (dhidden and the
+// d(logits) pass, 256 rows at H = 4096: 471 -> 312 us, 32 rows 271 -> 242).
+enum class Side { kRows, kWeight, kLogits };
+
+// BV: consecutive B rows a lane holds (see above), 8 or 4.  kUnitsB: B is d(logits) in units (see unit_index).
+template <typename T, int BV, Side kSideA = Side::kRows, bool kUnitsB = false>
 struct GemmTile {
   static constexpr int BM = 256, BN = 256, WM = 128, WN = 128;
   static constexpr int MI = 8, NI = 8;                 // 16 x 16 blocks per wave along A / B
@@ -136,45 +166,81 @@ struct GemmTile {
   static constexpr int kSlabK = Elem<T>::kSlabK;
   static constexpr int VEC = 16 / (int)sizeof(T);      // elements per 16-byte piece
   static constexpr int kBB = kASlots * kSlotBytes;     // LDS offset of the B ring
+  static constexpr bool kAcross = kSideA != Side::kRows;
+  static constexpr bool kPerm = kAcross && VEC == 8;   // fragments are made from what is read
+  static constexpr int kUnitBytes = kSlabK * kRowBytes;     // a unit of d(logits); a piece of a slab read across
+  static constexpr int kSub = 256 / kSlabK;                 // of them per 256-wide slab
+  static constexpr uint32_t kHalf = kAcross ? (uint32_t)kUnitBytes / 2 : 64u;   // from a slab's first half to its second in LDS
   static_assert(BV == 8 || BV == 4, "B rows per lane");
 
   typedef f32x4 Acc[MI][NI];
   typedef __attribute__((address_space(3))) char lds_char;
   typedef __attribute__((address_space(3))) const u32x4 lds_vec;
 
-  // This lane's rows within the wave's 128: a_row(i, r) of register r of blocks i, b_row(j) of blocks j.
+  // This lane's rows within the wave's 128: lane_a0() + a_off(i, r) for register r of blocks i, lane_b0() + b_block(j)
+  // of blocks j.
   __device__ static __forceinline__ constexpr int a_block(int i) {
     return VEC == 8 ? (i >> 1) * 32 + (i & 1) * 4 : i * 16;
+  }
+  __device__ static __forceinline__ constexpr int a_off(int i, int r) {
+    return kAcross ? i / VEC * 16 * VEC + 4 * VEC * r + i % VEC : a_block(i) + r;
   }
   __device__ static __forceinline__ int a_lane(int rho) { return VEC == 8 ? (rho >> 2) * 8 + (rho & 3) : rho; }
   __device__ static __forceinline__ constexpr int b_block(int j) { return (j / BV) * 16 * BV + j % BV; }
   __device__ static __forceinline__ int lane_a0() {     // first A row of this lane (block 0, register 0)
     const int g = (threadIdx.x & 63) >> 4;
-    return VEC == 8 ? g * 8 : g * 4;
+    return VEC * g;
   }
   __device__ static __forceinline__ int lane_b0() { return (threadIdx.x & 15) * BV; }
   __device__ static __forceinline__ int wave_m() { return ((threadIdx.x >> 6) & 1) * WM; }
   __device__ static __forceinline__ int wave_n() { return (threadIdx.x >> 7) * WN; }
 
-  // Swizzle of LDS row R's chunks: eight rows that one fragment read takes together get eight values.
+  // Bank conflicts.  LDS has 64 banks of 4 bytes, two rows of a slab wide; a wave's 16-byte read takes lanes 0-3, 12-15,
+  // 20-27 in one cycle, 4-11, 16-19, 28-31 in the next, and so on 32 lanes further (counted with pairs of lanes on
+  // one bank).  In lanes (c, g): eight c's of lane group g and the other eight of g + 1.  These sixteen must fall on
+  // eight chunks of either parity of rows.
+  //   A rows: the swizzle of a row's chunks is enough, its rows differ in parity.
+  //   B rows (row BV c + j): all of one parity, so rows are exchanged in pairs where c is odd (b_row), and the chunks
+  //     are swizzled by the rest of c.  Without the exchange every B read took 4 cycles more (half of SQ_LDS_BANK_CONFLICT per read).
+  //   A across: chunks of one row over two pieces of a slab; the odd pieces have their rows exchanged in pairs.
+  // A lane reads an exchanged row at the other address of its pair: odd rows go by addresses of their own (odd_a, odd_b).
   __device__ static __forceinline__ int a_swz(int row) { return VEC == 8 ? (row & 3) | ((row >> 3) & 1) << 2 : row & 7; }
-  __device__ static __forceinline__ int b_swz(int row) { return (BV == 8 ? row >> 3 : row >> 2) & 7; }
+  __device__ static __forceinline__ int b_swz(int row) { return row / (2 * BV) & 7; }
+  __device__ static __forceinline__ int b_row(int row) { return row ^ (row / BV & 1); }     // its own inverse
 
   // Where an operand's tile lives in memory: `rows` valid rows starting at `base`, consecutive
   // rows `row_bytes` apart, consecutive 128-byte K slabs of a row `slab_bytes` apart.
   //   row-major [rows][ld]:                  row_bytes = ld * sizeof(T), slab_bytes = 128
   //   K-blocked [row block][K slab][256][128 B]: row_bytes = 128, slab_bytes = 256 * 128 (one
   //   contiguous 32 KB piece per tile and slab)
+  //   units (as B): row_bytes = 128, slab_bytes = one unit, rows of units `unit_row` bytes apart
+  // Across (as A) `rows` counts the valid columns of the tile, and `k_left` the valid rows from the K range's first on:
+  //   kWeight: row_bytes = ld * sizeof(T), slab_bytes = kSlabK rows, sub_bytes = 128, front = bytes in front of base in its row
+  //   kLogits: row_bytes = 128, slab_bytes = a row of units, sub_bytes = one unit
   struct Operand {
     const T* base;
     int row_bytes;
-    int slab_bytes;
+    int64_t slab_bytes;
     int rows;
+    int sub_bytes;
+    int k_left;
+    int front;
+    int64_t unit_row;
     __device__ static __forceinline__ Operand row_major(const T* base, int64_t ld, int rows) {
-      return Operand{base, (int)(ld * (int64_t)sizeof(T)), kRowBytes, rows};
+      return Operand{base, (int)(ld * (int64_t)sizeof(T)), kRowBytes, rows, 0, 0, 0, 0};
     }
     __device__ static __forceinline__ Operand blocked(const T* block_base, int rows) {
-      return Operand{block_base, kRowBytes, kBlockRows * kRowBytes, rows};
+      return Operand{block_base, kRowBytes, kBlockRows * kRowBytes, rows, 0, 0, 0, 0};
+    }
+    __device__ static __forceinline__ Operand units(const T* base, int64_t n_kslab, int rows) {
+      return Operand{base, kRowBytes, kUnitBytes, rows, 0, 0, 0, n_kslab * kUnitBytes};
+    }
+    __device__ static __forceinline__ Operand across_weight(const T* base, int64_t ld, int col0, int cols, int k_left) {
+      const int row = (int)(ld * (int64_t)sizeof(T));
+      return Operand{base, row, (int64_t)kSlabK * row, cols, kRowBytes, k_left, col0 * (int)sizeof(T), 0};
+    }
+    __device__ static __forceinline__ Operand across_units(const T* base, int64_t n_kslab, int cols) {
+      return Operand{base, kRowBytes, n_kslab * kUnitBytes, cols, kUnitBytes, 0, 0, 0};
     }
   };
 
@@ -182,79 +248,163 @@ struct GemmTile {
   // exactly the valid rows, so rows past them read as zero and nothing outside the operands is touched: the
   // row offset is in the per-lane part, which is what the hardware checks, the K-slab offset in the base
   // address, and the size is what is left of the valid rows from there.
+  //   kWeight: `bytes` covers the slab's valid rows of `k_left`; columns past the tile's get an offset outside of it
+  //   kLogits: `bytes` covers the units of the tile that exist
+  //   kUnitsB: `bytes` counts the tile's rows of units that hold any valid row; the others read as zero
   struct Cursor {
     const char* p;
     int bytes;
     int left;       // slabs of this tile from here on
+    int k_left;
+    int64_t step;
   };
 
-  int slab_a, slab_b, shrink_a, shrink_b;     // address step and size step per slab
+  int64_t slab_a, slab_b;                     // address step per slab
+  int shrink_a, shrink_b;                     // size step per slab
+  int64_t jump_a, jump_b;                     // address step behind a tile's last slab
   int pass_a;                                 // bytes between the rows of two loads of a slab
+  int row_a, front_a;
+  int64_t unit_row_b;
   Cursor a, b, next_a, next_b;
-  lds_char* lds;
   __amdgpu_buffer_rsrc_t rsrc_a, rsrc_b;
-  int voff_a, voff_b[8];
+  const char* unit_b;                         // this slab's unit of the next load
+  int voff_a[8], voff_b[8];
+  u32x4 raw[8];                               // kPerm: a half of A as it is read
   u32x4 af[2][MI], bf[2][NI];
-  uint32_t a0, b0;                            // this lane's fragment address in slot 0 of either ring
-  uint32_t ra, rb, na, nb;                    // the same in the slab being read and in the one after it
-  uint32_t da, db;                            // where the next requested slab goes
-  uint32_t w0;
+  uint32_t a0, b0;                            // this lane's fragment addresses in slot 0 of either ring, first half of a slab
+  uint32_t odd_a, odd_b;                      // added to them for odd rows
+  uint32_t sa, sb;                            // slots of the slab that is read (bytes); B's other slot is sb ^ kSlotBytes
+  uint32_t sa1;                               // A's slot after sa
+  uint32_t da;                                // slot of the A slab that is requested
+  uint32_t w0;                                // this wave's place in a load
 
   __device__ static __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
   __device__ __forceinline__ void make_a() {
     rsrc_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.p), 0, a.bytes, 0x00020000);
   }
   __device__ __forceinline__ void make_b() {
-    rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(b.p), 0, b.bytes, 0x00020000);
+    if constexpr (kUnitsB) { next_unit(0, 0); next_unit(1, 0); }
+    else rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(b.p), 0, b.bytes, 0x00020000);
   }
-  // Load p (0 .. 7) of the slab at the cursor: 8 rows per wave, 32 per workgroup.
+  // Load p (0 .. 7) of the slab at the cursor: 8 rows per wave, 32 per workgroup (across: 8 rows of one piece).
   __device__ __forceinline__ void load_a(int p) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, lds + da + p * 4096, 16, voff_a + p * pass_a, 0, 0, 0);
+    if constexpr (kAcross)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_char*)(uintptr_t)(w0 + da + p * 4096), 16, voff_a[p], 0, 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_char*)(uintptr_t)(w0 + da + p * 4096), 16, voff_a[0] + p * pass_a, 0, 0, 0);
   }
-  __device__ __forceinline__ void load_b(int p) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, lds + db + p * 4096, 16, voff_b[p], 0, 0, 0);
+  static constexpr int kUnitLoads = kSlabK / 32;       // loads per unit
+  __device__ __forceinline__ void next_unit(int part, int u) {     // the descriptor of the slab's unit u
+    if (part == 0) unit_b = u == 0 ? b.p : unit_b + unit_row_b;
+    else rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(unit_b), 0, u < b.bytes ? kUnitBytes : 0, 0x00020000);
   }
-  __device__ __forceinline__ void step_a() { step_a1(); step_a2(); step_a3(); }
-  // in pieces, to be placed between matrix instructions; masks, because a select would become a branch
-  __device__ __forceinline__ void step_a1() { a.left -= 1; }
-  __device__ __forceinline__ void step_a2() {
-    const int64_t sw = -(int64_t)(a.left == 0);
-    a.p += ((next_a.p - a.p) & sw) | (slab_a & ~sw);
+  __device__ __forceinline__ void load_b(int p, uint32_t slot) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_char*)(uintptr_t)(w0 + kBB + slot + p * 4096), 16, voff_b[p], 0, 0, 0);
   }
-  __device__ __forceinline__ void step_a3() {
-    const int sw = -(int)(a.left == 0);
-    a.bytes += ((next_a.bytes - a.bytes) & sw) | (-shrink_a & ~sw);
-    a.left |= next_a.left & sw;
+  __device__ __forceinline__ void load_b(uint32_t slot) {
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+      if (kUnitsB && p > 0 && p % kUnitLoads == 0) { next_unit(0, p / kUnitLoads); next_unit(1, p / kUnitLoads); }
+      load_b(p, slot);
+    }
   }
-  __device__ __forceinline__ void step_b() { step_b1(); step_b2(); step_b3(); }
-  // in pieces, to be placed between matrix instructions; masks, because a select would become a branch
-  __device__ __forceinline__ void step_b1() { b.left -= 1; }
-  __device__ __forceinline__ void step_b2() {
-    const int64_t sw = -(int64_t)(b.left == 0);
-    b.p += ((next_b.p - b.p) & sw) | (slab_b & ~sw);
+  // left == 0 ? x : y of scalar values.  As assembly, because the compiler may make a branch of it, and a branch in the slab
+  // loop ends the schedule: dW of 12288 tokens at H = 4096 then takes 11.9 ms for 10.3.
+  __device__ static __forceinline__ int if_zero(int left, int x, int y) {
+    int r;
+    asm("s_cmp_eq_u32 %1, 0\n\ts_cselect_b32 %0, %2, %3" : "=s"(r) : "s"(left), "s"(x), "s"(y) : "scc");
+    return r;
   }
-  __device__ __forceinline__ void step_b3() {
-    const int sw = -(int)(b.left == 0);
-    b.bytes += ((next_b.bytes - b.bytes) & sw) | (-shrink_b & ~sw);
-    b.left |= next_b.left & sw;
+  __device__ static __forceinline__ int64_t if_zero(int left, int64_t x, int64_t y) {
+    int64_t r;
+    asm("s_cmp_eq_u32 %1, 0\n\ts_cselect_b64 %0, %2, %3" : "=s"(r) : "s"(left), "s"(x), "s"(y) : "scc");
+    return r;
   }
-  __device__ __forceinline__ void slot_a() { const uint32_t t = da + kSlotBytes; da = t >= (uint32_t)kBB ? t - kBB : t; }
-  __device__ __forceinline__ void slot_b() { db = 2 * (kBB + w0) + kSlotBytes - db; }
-  // Fragment read n (0 .. 15) of a half: the first A fragment, all of B, the rest of A.
+  // The cursors' step to the next slab, in pieces of at most three scalar instructions: what a matrix instruction covers.
+  static constexpr int kSteps = 6;
+  __device__ static __forceinline__ void advance(int n, Cursor& c, const Cursor& next, int64_t slab, int64_t jump, int shrink) {
+    if (n == 0) c.left -= 1;
+    if (n == 1) c.step = if_zero(c.left, jump, slab);
+    if (n == 2) c.p += c.step;
+    if (n == 3) c.bytes = if_zero(c.left, next.bytes, c.bytes - shrink);
+    if (n == 4) c.left = if_zero(c.left, next.left, c.left);
+  }
+  __device__ __forceinline__ void step_a(int n) {
+    if constexpr (kSideA == Side::kWeight) {
+      if (n == 3) a.k_left = if_zero(a.left, next_a.k_left, a.k_left - kSlabK);
+      else advance(n, a, next_a, slab_a, jump_a, 0);
+      if (n == 5) a.bytes = weight_bytes(a.k_left, row_a, front_a);
+    } else {
+      advance(n, a, next_a, slab_a, jump_a, shrink_a);
+    }
+  }
+  __device__ __forceinline__ void step_b(int n) { advance(n, b, next_b, slab_b, jump_b, shrink_b); }
+  __device__ __forceinline__ void step_a() { for (int n = 0; n < kSteps; ++n) step_a(n); }
+  __device__ __forceinline__ void step_b() { for (int n = 0; n < kSteps; ++n) step_b(n); }
+  __device__ static __forceinline__ uint32_t next_slot(uint32_t slot) { return slot == (kASlots - 1) * kSlotBytes ? 0 : slot + kSlotBytes; }
+  __device__ __forceinline__ void read_b(int set, uint32_t pb, int j) {
+    bf[set][j] = *(lds_vec*)(uintptr_t)((j % 2 ? pb + odd_b : pb) + b_block(j) * kRowBytes);
+  }
+  // Fragment read n (0 .. 15) of a half: the first A fragment, all of B, the rest of A; across: all of A, all of B.
   __device__ __forceinline__ void read(int set, uint32_t pa, uint32_t pb, int n) {
-    if (n == 0) af[set][0] = *(lds_vec*)(lds + pa);
-    else if (n <= NI) bf[set][n - 1] = *(lds_vec*)(lds + pb + b_block(n - 1) * kRowBytes);
-    else af[set][n - NI] = *(lds_vec*)(lds + pa + a_block(n - NI) * kRowBytes);
+    if constexpr (kAcross) {
+      if (n >= MI) read_b(set, pb, n - MI);
+      else if constexpr (kPerm) raw[n] = *(lds_vec*)(uintptr_t)((n % 2 ? pa + odd_a : pa) + n * kRowBytes);
+      else af[set][n] = *(lds_vec*)(uintptr_t)((n % 2 ? pa + odd_a : pa) + n / VEC * 2 * kUnitBytes + n % VEC * kRowBytes);
+    } else {
+      if (n == 0) af[set][0] = *(lds_vec*)(uintptr_t)(pa);
+      else if (n <= NI) read_b(set, pb, n - 1);
+      else af[set][n - NI] = *(lds_vec*)(uintptr_t)(pa + a_block(n - NI) * kRowBytes);
+    }
+  }
+  // Register n (0 .. 31) of a half's fragments: rows 2 q, 2 q + 1 of column i of the square.
+  __device__ __forceinline__ void perm(int set, int n) {
+    const int i = n / 4, q = n % 4;
+    af[set][i][q] = __builtin_amdgcn_perm(raw[2 * q + 1][i / 2], raw[2 * q][i / 2],
+                                          i % 2 ? 0x07060302u : 0x05040100u);
   }
 
+  // Bytes of a kWeight slab of which k_left rows are valid, from the tile's first column on.
+  __device__ static __forceinline__ int weight_bytes(int k_left, int row, int front) {
+    const int rows = k_left < kSlabK ? k_left : kSlabK;
+    const int bytes = rows * row - front;
+    return bytes > 0 ? bytes : 0;
+  }
   __device__ static __forceinline__ Cursor cursor(const Operand& o, int nslab) {
-    return Cursor{reinterpret_cast<const char*>(o.base), o.rows * o.row_bytes, nslab};
+    return Cursor{reinterpret_cast<const char*>(o.base), o.rows * o.row_bytes, nslab, 0, 0};
+  }
+  __device__ static __forceinline__ Cursor cursor_a(const Operand& o, int nslab) {
+    if constexpr (kSideA == Side::kRows) return cursor(o, nslab);
+    const int bytes = kSideA == Side::kWeight ? weight_bytes(o.k_left, o.row_bytes, o.front)
+                                              : (o.rows + kSlabK - 1) / kSlabK * kUnitBytes;
+    return Cursor{reinterpret_cast<const char*>(o.base), bytes, nslab, o.k_left, 0};
+  }
+  __device__ static __forceinline__ Cursor cursor_b(const Operand& o, int nslab) {
+    if constexpr (!kUnitsB) return cursor(o, nslab);
+    return Cursor{reinterpret_cast<const char*>(o.base), (o.rows + kSlabK - 1) / kSlabK, nslab, 0, 0};
   }
   // What the cursor does behind the last slab of the last tile: request that slab again.
-  __device__ static __forceinline__ Cursor hold(const Operand& o, int nslab) {
-    const int shrink = o.slab_bytes == kRowBytes ? kRowBytes : 0;
-    return Cursor{reinterpret_cast<const char*>(o.base) + (int64_t)(nslab - 1) * o.slab_bytes,
-                  o.rows * o.row_bytes - (nslab - 1) * shrink, 1};
+  __device__ static __forceinline__ Cursor held(Cursor c, const Operand& o, int nslab, int shrink) {
+    c.p += (int64_t)(nslab - 1) * o.slab_bytes;
+    c.bytes -= (nslab - 1) * shrink;
+    c.left = 1;
+    return c;
+  }
+  __device__ static __forceinline__ Cursor hold_a(const Operand& o, int nslab) {
+    Cursor c = held(cursor_a(o, nslab), o, nslab, shrink(o));
+    if constexpr (kSideA == Side::kWeight) {
+      c.k_left -= (nslab - 1) * kSlabK;
+      c.bytes = weight_bytes(c.k_left, o.row_bytes, o.front);
+    }
+    return c;
+  }
+  __device__ static __forceinline__ Cursor hold_b(const Operand& o, int nslab) { return held(cursor_b(o, nslab), o, nslab, shrink(o)); }
+  __device__ static __forceinline__ int shrink(const Operand& o) { return o.slab_bytes == kRowBytes ? kRowBytes : 0; }
+  // What follows the tile whose operands are A and B: a call per tile, behind start().
+  __device__ __forceinline__ void follow(const Operand& A, const Operand& B, int nslab, const Cursor& na, const Cursor& nb) {
+    next_a = na; next_b = nb;
+    jump_a = na.p - (reinterpret_cast<const char*>(A.base) + (int64_t)(nslab - 1) * A.slab_bytes);
+    jump_b = nb.p - (reinterpret_cast<const char*>(B.base) + (int64_t)(nslab - 1) * B.slab_bytes);
   }
 
   // First tile of a workgroup (or of a run that does not stream): nothing is in flight, LDS is free.
@@ -262,45 +412,87 @@ struct GemmTile {
   __device__ __forceinline__ void start(const Operand& A, const Operand& B, int nslab, char* shared,
                                         const int32_t* b_order = nullptr, int b_rows = 0) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    lds = (lds_char*)shared;
+    const uint32_t lds = (uint32_t)(uintptr_t)(lds_char*)shared;
     slab_a = A.slab_bytes; slab_b = B.slab_bytes;
-    shrink_a = A.slab_bytes == kRowBytes ? kRowBytes : 0;
-    shrink_b = B.slab_bytes == kRowBytes ? kRowBytes : 0;
+    shrink_a = kAcross ? 0 : shrink(A);
+    shrink_b = shrink(B);
     pass_a = 32 * A.row_bytes;
-    w0 = __builtin_amdgcn_readfirstlane(wave) * 1024;
+    row_a = A.row_bytes; front_a = A.front;
+    unit_row_b = B.unit_row;
+    w0 = lds + __builtin_amdgcn_readfirstlane(wave) * 1024;
     // A wave's load fills 1 KB of LDS in lane order: 8 rows x 8 chunks.  The lane that lands on (row, slot)
     // fetches chunk slot ^ swz(row); load p of a slab starts 32 p rows further down, which leaves a_swz as it is.
     const int row = wave * 8 + (lane >> 3), chunk = lane & 7;
-    voff_a = row * A.row_bytes + (chunk ^ a_swz(row)) * 16;
+    if constexpr (kAcross) {
+#pragma unroll
+      for (int p = 0; p < 8; ++p) {
+        const int sub = p * 32 / kSlabK, k = (p * 32 % kSlabK + row) ^ (sub & 1);
+        const bool valid = kSideA == Side::kLogits || sub * kSlabK < A.rows;
+        voff_a[p] = valid ? sub * A.sub_bytes + k * A.row_bytes + chunk * 16 : 0x7fffff00;
+      }
+    } else {
+      voff_a[0] = row * A.row_bytes + (chunk ^ a_swz(row)) * 16;
+    }
 #pragma unroll
     for (int p = 0; p < 8; ++p) {
-      const int r = row + 32 * p;
-      const int off = b_order == nullptr ? r * B.row_bytes : (r < b_rows ? b_order[r] * B.row_bytes : 0x7fffff00);
+      const int r = b_row(row + 32 * p);
+      const int off = kUnitsB ? r % kSlabK * kRowBytes
+                              : (b_order == nullptr ? r * B.row_bytes : (r < b_rows ? b_order[r] * B.row_bytes : 0x7fffff00));
       voff_b[p] = off + (chunk ^ b_swz(r)) * 16;
     }
     const int g = lane >> 4, c = lane & 15;
     const int fa = a_lane(c), fb = c * BV;
-    a0 = (wave_m() + fa) * kRowBytes + (g ^ a_swz(fa)) * 16;
-    b0 = kBB + (wave_n() + fb) * kRowBytes + (g ^ b_swz(fb)) * 16;
-    a = cursor(A, nslab); b = cursor(B, nslab);
-    next_a = hold(A, nslab); next_b = hold(B, nslab);
+    if constexpr (kAcross) {
+      const int pc = (c & 3) * 4 + (c >> 2), sub = wave_m() / kSlabK + (pc >> 3);    // chunk of the wave's first 16
+      a0 = lds + sub * kUnitBytes + (VEC * g + (sub & 1)) * kRowBytes + (pc & 7) * 16;
+      odd_a = -2 * (sub & 1) * kRowBytes;
+    } else {
+      a0 = lds + (wave_m() + fa) * kRowBytes + (g ^ a_swz(fa)) * 16;
+    }
+    b0 = lds + kBB + (wave_n() + fb + (c & 1)) * kRowBytes + (g ^ b_swz(fb)) * 16;
+    odd_b = -2 * (c & 1) * kRowBytes;
+    a = cursor_a(A, nslab); b = cursor_b(B, nslab);
+    follow(A, B, nslab, hold_a(A, nslab), hold_b(B, nslab));
     make_a(); make_b();
-    da = w0; db = kBB + w0;
+    da = sa = sb = 0;
 #pragma unroll
     for (int p = 0; p < 8; ++p) load_a(p);
-#pragma unroll
-    for (int p = 0; p < 8; ++p) load_b(p);
-    step_a(); step_b(); make_a(); make_b(); slot_a(); slot_b();
+    load_b(0u);
+    step_a(); step_b(); make_a(); make_b(); da = kSlotBytes;
 #pragma unroll
     for (int p = 0; p < 8; ++p) load_a(p);
-    step_a(); make_a(); slot_a();
+    step_a(); make_a(); da = 2 * kSlotBytes;
     __builtin_amdgcn_s_waitcnt(0x0F78);    // all but the youngest eight loads
     __syncthreads();
-    ra = a0; rb = b0; na = a0 + kSlotBytes; nb = b0 + kSlotBytes;
 #pragma unroll
-    for (int n = 0; n < 16; ++n) read(0, ra, rb, n);
+    for (int n = 0; n < 16; ++n) read(0, a0, b0, n);
+    if constexpr (kPerm) {
 #pragma unroll
-    for (int p = 0; p < 8; ++p) load_b(p);
+      for (int n = 0; n < 4 * MI; ++n) perm(0, n);
+    }
+    load_b((uint32_t)kSlotBytes);
+  }
+
+  // The schedule of a half of a slab: 64 slots of one matrix instruction (fp32: four) each.  It takes 16 cycles and its issue 4, so
+  // three more instructions fit behind it, and every one beyond that is a gap in the matrix cores' work: the same
+  // instructions with up to nine scalar ones in a slot were 5 % slower in the contraction that has the most of them.  Fragment
+  // reads take even slots of the first 32, a load every eighth (three instructions by itself, its LDS address goes through
+  // m0), scalar steps the odd slots left over, the second 32 slots the transposition.  Loads every 4 or 6 slots: no faster.
+  static constexpr int load_at(int m) { return m % 8 == 1 ? m / 8 : -1; }
+  static constexpr int unit_at(int m) {                // unit that begins with slot m's load of B
+    return kUnitsB && load_at(m) > 0 && load_at(m) % kUnitLoads == 0 ? load_at(m) / kUnitLoads : -1;
+  }
+  static constexpr int step_at(int m, bool units) {    // scalar step of slot m; a unit's descriptor is made in the two slots before its load
+    if (m % 2 == 0 || load_at(m) >= 0 || (units && unit_at(m + 2) > 0)) return -1;
+    int n = 0;
+    for (int k = 1; k < m; k += 2) n += load_at(k) < 0 && !(units && unit_at(k + 2) > 0);
+    return n;
+  }
+  static constexpr int perm_from(int m) {              // registers transposed in front of slot m: none behind a load, two in the first slots
+    int n = 0, twice = 4;
+    for (int k = 32; k < m; ++k)
+      if (load_at(k) < 0) n += twice > 0 ? (--twice, 2) : 1;
+    return n;
   }
 
   // One tile's K loop of `nslab` slabs; acc must be initialised by the caller.  Between tiles of a
@@ -309,16 +501,18 @@ struct GemmTile {
     settle();
     for (int s = 0; s < nslab; ++s) {
       each<MI * NI>([&](auto c) __attribute__((always_inline)) {            // first half of the slab
-        constexpr int m = decltype(c)::value;
-        Mma<T>::slot(acc, af[0], bf[0], m);
+        constexpr int m = decltype(c)::value, n = step_at(m, false);
+        Mma<T>::template slot<kAcross>(acc, af[0], bf[0], m);
         fence();
-        if constexpr (m % 2 == 0 && m < 32) { read(1, ra ^ 64, rb ^ 64, m / 2); fence(); }
-        if constexpr (m % 8 == 1) { load_a(m / 8); fence(); }
-        if constexpr (m == 35) { step_b1(); fence(); }
-        if constexpr (m == 37) { step_b2(); fence(); }
-        if constexpr (m == 43) { step_b3(); fence(); }
-        if constexpr (m == 45) { make_b(); fence(); }
-        if constexpr (m == 47) { slot_b(); fence(); }
+        if constexpr (m % 2 == 0 && m < 32) { read(1, half_a() + sa, (b0 ^ 64) + sb, m / 2); fence(); }
+        if constexpr (load_at(m) >= 0) { load_a(load_at(m)); fence(); }
+        if constexpr (n >= 0 && n < kSteps) { step_b(n); fence(); }
+        if constexpr (n == kSteps) { make_b(); fence(); }
+        if constexpr (n == kSteps + 1) { sa1 = next_slot(sa); fence(); }
+        if constexpr (kPerm) {
+#pragma unroll
+          for (int k = perm_from(m); k < perm_from(m + 1); ++k) { perm(1, k); fence(); }
+        }
       });
       fence();
       // every wave has the last fragments of this slab, and the next one's loads have landed
@@ -326,23 +520,27 @@ struct GemmTile {
       __builtin_amdgcn_s_barrier();
       fence();
       each<MI * NI>([&](auto c) __attribute__((always_inline)) {            // second half, while the next slab's first fragments come in
-        constexpr int m = decltype(c)::value;
-        Mma<T>::slot(acc, af[1], bf[1], m);
+        constexpr int m = decltype(c)::value, n = step_at(m, kUnitsB);
+        Mma<T>::template slot<kAcross>(acc, af[1], bf[1], m);
         fence();
-        if constexpr (m % 2 == 0 && m < 32) { read(0, na, nb, m / 2); fence(); }
-        if constexpr (m % 8 == 1) { load_b(m / 8); fence(); }
-        if constexpr (m == 35) { step_a1(); fence(); }
-        if constexpr (m == 37) { step_a2(); fence(); }
-        if constexpr (m == 43) { step_a3(); fence(); }
-        if constexpr (m == 45) { make_a(); fence(); }
-        if constexpr (m == 47) { slot_a(); fence(); }
-        if constexpr (m == 51) { ra = na; rb = nb; fence(); }
-        if constexpr (m == 53) { const uint32_t t = na + kSlotBytes; na = t >= (uint32_t)kBB ? t - kBB : t; fence(); }
-        if constexpr (m == 55) { nb = 2 * b0 + kSlotBytes - nb; fence(); }
+        if constexpr (m % 2 == 0 && m < 32) { read(0, a0 + sa1, b0 + (sb ^ kSlotBytes), m / 2); fence(); }
+        if constexpr (load_at(m) >= 0) { load_b(load_at(m), sb); fence(); }
+        if constexpr (unit_at(m + 2) > 0) { next_unit(0, unit_at(m + 2)); fence(); }
+        if constexpr (unit_at(m + 1) > 0) { next_unit(1, unit_at(m + 1)); fence(); }
+        if constexpr (n >= 0 && n < kSteps) { step_a(n); fence(); }
+        if constexpr (n == kSteps) { make_a(); fence(); }
+        if constexpr (n == kSteps + 1) { da = next_slot(da); fence(); }
+        if constexpr (kPerm) {
+#pragma unroll
+          for (int k = perm_from(m); k < perm_from(m + 1); ++k) { perm(0, k); fence(); }
+        }
       });
+      sa = sa1; sb ^= kSlotBytes;
     }
     settle();
   }
+
+  __device__ __forceinline__ uint32_t half_a() const { return kAcross ? a0 + kUnitBytes / 2 : a0 ^ 64; }
 
   // Wait states between matrix instructions and other accesses to the accumulators, in either direction: at most
   // 19 (result of a 16-pass instruction read by the vector unit).

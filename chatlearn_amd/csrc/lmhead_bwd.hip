@@ -1,12 +1,13 @@
 // Backward of the fused lm_head + log-softmax statistics.
 //
 // Per chunk of tokens (the chunk length is set by the workspace the caller gives):
-//   1. dz kernel: recompute a z^T tile [256 vocab x 256 tokens] on the matrix cores
-//      exactly as the forward does, turn it into d(logits) with the stored lse,
-//      and write it in both orientations, dz[token][vocab] and dzT[vocab][token].
-//   2. dhidden[chunk] = dz * W        as an NT GEMM against WT = W^T (built once per call)
-//   3. dW (+)= dzT * hidden[chunk]    as an NT GEMM against hidT = hidden[chunk]^T, fp32 out
-// Every contraction runs through the same K-contiguous MFMA tile (gemm_core.hpp).
+//   1. d(logits) in place of the chunk's kept logits, or by recomputing a z^T tile [256 vocab x 256 tokens] on the
+//      matrix cores exactly as the forward does.
+//   2. dhidden[chunk] = dz * W        K = vocabulary, which runs across the rows of W
+//   3. dW (+)= dz^T * hidden[chunk]   K = tokens, which run across the rows of dz, against hidT = hidden[chunk]^T; fp32 out
+// Both contractions run through the MFMA tile of gemm_core.hpp, which turns an operand that lies across on its way
+// from LDS into the matrix cores (see Side): neither W^T nor dz^T is formed.  Measured against NT products of transposed
+// copies: see Side.
 //
 // Algorithmic work: 4*T*H*V flop (dhidden + dW); the z recomputation (2*T*H*V) is overhead.
 #include "head_internal.hpp"
@@ -40,13 +41,12 @@ struct DzParams {
   const float* g_lp;
   const float* g_ent;     // or nullptr
   int Tc;       // valid tokens in the chunk
-  int ldt;      // K extent of dzT = Tc rounded up to 64
+  int ldt;      // tokens of dz to write = Tc rounded up to 64 (zeros past Tc)
   int H, V;
-  int ldv;      // K extent of dz = V rounded up to 64
+  int ldv;      // vocabulary extent of dz = V rounded up to 64
   int n_tb, n_vt;
   float c, inv_temperature;
-  void* dz;     // Tc x ldv, K-blocked (see blocked_index)
-  void* dzT;    // V x ldt, K-blocked
+  void* dz;     // ldt x ldv, in units (see unit_index)
 };
 
 template <typename T>
@@ -111,15 +111,14 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_dz_kernel(DzParams p) 
   }
 
   T* dz = static_cast<T*>(p.dz);
-  T* dzT = static_cast<T*>(p.dzT);
   const float it = p.inv_temperature;
   constexpr int AG = VEC / 4;                 // blocks along A whose registers make up VEC consecutive vocabulary rows
 #pragma unroll
   for (int i = 0; i < MI; i += AG) {
-    float d[NI][VEC];
     const int v = v0 + la + Tile::a_block(i);
 #pragma unroll
-    for (int j = 0; j < NI; ++j)
+    for (int j = 0; j < NI; ++j) {
+      float d[VEC];
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         const float zraw = acc_get(acc[i + e / 4][j], e % 4);
@@ -129,37 +128,23 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_dz_kernel(DzParams p) 
         float x = -it * pr * fmaf(gent[j], logp + ent[j], glp[j]);
         if (lab[j] == v + e) x += it * glp[j];
         if (v + e >= p.V || !block_live) x = 0.f;   // vocabulary padding columns / dead block
-        d[j][e] = x;
+        d[e] = x;
       }
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
       const int t = t0 + lb + Tile::b_block(j);
-      if (t < p.Tc && v < p.ldv)
-        *reinterpret_cast<u32x4*>(dz + blocked_index<T>(t, v, p.ldv / Tile::kSlabK)) = pack_vec(d[j], (T*)nullptr);
+      if (t < p.ldt && v < p.ldv)
+        *reinterpret_cast<u32x4*>(dz + unit_index<T>(t, v, p.ldv / Tile::kSlabK)) = pack_vec(d, (T*)nullptr);
     }
-#pragma unroll
-    for (int e = 0; e < VEC; ++e)
-#pragma unroll
-      for (int j = 0; j < NI; j += VEC) {
-        float x[VEC];
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) x[k] = d[j + k][e];
-        const int t = t0 + lb + Tile::b_block(j);
-        if (v + e < p.V && t < p.ldt)
-          *reinterpret_cast<u32x4*>(dzT + blocked_index<T>(v + e, t, p.ldt / Tile::kSlabK)) = pack_vec(x, (T*)nullptr);
-      }
   }
 }
 
-// d(logits) from kept logits, in place, plus its transpose.  A unit is 256 token rows x one 128-byte slab of
-// vocabulary: 32 KB of the K-blocked kept logits, which become the same 32 KB of the K-blocked dz operand.
-// A thread takes a square of VEC tokens x VEC vocabulary entries: VEC 16-byte pieces in, VEC pieces of
-// dz back over them, VEC pieces of dzT, the transposition being a choice of registers (no LDS, no barrier
-// between units).  Eight lanes cover a slab row, eight lane groups eight of its token groups, so every access
-// of a wave is whole 128-byte lines.  HBM-bound: reads 1x, writes 2x the chunk.
+// d(logits) from kept logits: in place, or into the operands of dW that the caller keeps.  HBM-bound: reads and writes the
+// chunk once.  A thread owns one 16-byte piece of one or two tokens in every unit that its workgroup walks: their
+// coefficients stay in registers, the loads of kAhead units are in flight together, and a wave's access is one kilobyte.
+// 12126 rows of the 152k vocabulary: 2.25 -> 1.49 ms, 32768 rows 5.92 -> 3.57 ms (5.6 TB/s), against a pass that also wrote the
+// transpose.
 struct DzFromZParams {
-  void* z;            // Tc x ldv: in kept logits (KeptLogit<T>), out dz (T), K-blocked
-  void* dzT;          // V rows, K-blocked: the slab of the chunk's first token
+  const void* z;      // kept logits (KeptLogit<T>): z_kslab units per row of units
+  void* dz;           // d(logits) (T): dz_kslab units per row of units
   const int64_t* labels;
   int64_t label_offset;
   const float* lse;
@@ -167,103 +152,113 @@ struct DzFromZParams {
   const float* g_lp;
   const float* g_ent;
   const int32_t* order;   // optional [Tc]: row n is token order[n] of the per-token arrays
-  int Tc, ldt, V, ldv;    // ldt: tokens of dzT to write, Tc rounded up to 64
-  int64_t t_slabs;        // slabs per row of dzT, of which these tokens are the first ldt / E
+  int64_t z_kslab, dz_kslab;
+  int Tc, V, n_units;     // n_units: units of dz per row of units
   float c, inv_temperature;
 };
 
-template <typename T>
+template <typename T, bool kEntropy>
 __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams p) {
   typedef typename KeptLogit<T>::type ZT;
   static_assert(sizeof(ZT) == sizeof(T), "d(logits) overwrites the kept logits in place");
-  constexpr int E = Elem<T>::kSlabK;                // vocabulary entries of a unit (64 or 32)
+  constexpr int E = Elem<T>::kSlabK;                // tokens and vocabulary entries of a unit (64 or 32)
   constexpr int VEC = 16 / (int)sizeof(T);          // elements per 16-byte piece
-  constexpr int kPasses = kBlockRows / VEC / 32;    // a pass of 256 threads covers 32 token groups
-  __shared__ float s_lse[kBlockRows], s_ent[kBlockRows], s_glp[kBlockRows], s_gen[kBlockRows];
-  __shared__ int s_lab[kBlockRows];
-  const int rb = blockIdx.x;
-  const int64_t n_kslab = p.ldv / E;
+  constexpr int kRows = E / 32;                     // tokens per thread
+  constexpr int kAhead = 4;                         // units in flight
+  const int q = threadIdx.x & 7, row = threadIdx.x >> 3;
   const float it = p.inv_temperature;
-  {
-    const int n = rb * kBlockRows + threadIdx.x;
-    const bool ok = n < p.Tc;
+  float lse[kRows], lse2[kRows], glp[kRows], gen[kRows], ent[kRows];
+  int lab[kRows];
+  bool live[kRows];
+#pragma unroll
+  for (int h = 0; h < kRows; ++h) {
+    const int n = blockIdx.x * E + h * 32 + row;
+    const bool ok = n < p.Tc;                       // rows past the chunk and rows without a gradient give zeros
     const int t = ok && p.order ? p.order[n] : n;
-    s_glp[threadIdx.x] = ok ? p.g_lp[t] : 0.f;      // rows past the chunk and rows without a gradient give zeros
-    s_gen[threadIdx.x] = (ok && p.g_ent) ? p.g_ent[t] : 0.f;
-    s_lse[threadIdx.x] = ok ? p.lse[t] : 0.f;
-    s_ent[threadIdx.x] = (ok && p.g_ent) ? p.entropy[t] : 0.f;
-    int lab = -1;
+    glp[h] = ok ? p.g_lp[t] : 0.f;
+    gen[h] = kEntropy && ok ? p.g_ent[t] : 0.f;
+    lse[h] = ok ? p.lse[t] : 0.f;
+    ent[h] = kEntropy && ok ? p.entropy[t] : 0.f;
+    lse2[h] = lse[h] * kLog2e;
+    live[h] = glp[h] != 0.f || gen[h] != 0.f;
+    lab[h] = -1;
     if (ok) {
       const int64_t rel = p.labels[t] - p.label_offset;
-      if (rel >= 0 && rel < p.V) lab = (int)rel;
+      if (rel >= 0 && rel < p.V) lab[h] = (int)rel;
     }
-    s_lab[threadIdx.x] = lab;
   }
-  __syncthreads();
-  const int q = threadIdx.x & 7, cg = threadIdx.x >> 3;   // piece within the slab row, token group
-  T* dzT = static_cast<T*>(p.dzT);
-  for (int ks = blockIdx.y; ks < (int)n_kslab; ks += gridDim.y) {
-    char* unit = static_cast<char*>(p.z) + ((int64_t)rb * n_kslab + ks) * (kBlockRows * kRowBytes);
-    const int v = ks * E + q * VEC;
+  const int at = row * kRowBytes + q * 16;          // byte of this thread's first piece within a unit
+  const char* z = static_cast<const char*>(p.z) + (int64_t)blockIdx.x * p.z_kslab * (E * kRowBytes) + at;
+  char* dz = static_cast<char*>(p.dz) + (int64_t)blockIdx.x * p.dz_kslab * (E * kRowBytes) + at;
+  const int step = gridDim.y;
+  for (int k0 = blockIdx.y; k0 < p.n_units; k0 += kAhead * step) {
+    u32x4 raw[kAhead][kRows];
 #pragma unroll
-    for (int pass = 0; pass < kPasses; ++pass) {
-      const int R = (pass * 32 + cg) * VEC;         // first token row of this thread's square
-      u32x4 raw[VEC];
+    for (int u = 0; u < kAhead; ++u) {
+      const int ks = k0 + u * step < p.n_units ? k0 + u * step : k0;
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) raw[k] = *reinterpret_cast<const u32x4*>(unit + (R + k) * kRowBytes + q * 16);
-      float d[VEC][VEC];
+      for (int h = 0; h < kRows; ++h)
+        raw[u][h] = *reinterpret_cast<const u32x4*>(z + (int64_t)ks * (E * kRowBytes) + h * 32 * kRowBytes);
+    }
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) {
-        const float glp = s_glp[R + k], gen = s_gen[R + k], lse = s_lse[R + k], ent = s_ent[R + k];
-        const int lab = s_lab[R + k] - v;
-        const bool live = glp != 0.f || gen != 0.f;
-        const float lse2 = lse * kLog2e;
-        const ZT* in = reinterpret_cast<const ZT*>(&raw[k]);
+    for (int u = 0; u < kAhead; ++u) {
+      const int ks = k0 + u * step;
+      if (ks >= p.n_units) break;
+      const int v = ks * E + q * VEC;
+#pragma unroll
+      for (int h = 0; h < kRows; ++h) {
+        const ZT* in = reinterpret_cast<const ZT*>(&raw[u][h]);
+        float d[VEC];
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
           const float zraw = (float)in[e];
-          const float pr = __builtin_amdgcn_exp2f(fmaf(zraw, p.c, -lse2));
-          const float logp = fmaf(zraw, it, -lse);
-          float x = -it * pr * fmaf(gen, logp + ent, glp);
-          if (lab == e) x += it * glp;
-          d[k][e] = (live && v + e < p.V) ? x : 0.f;      // vocabulary padding columns give zeros
+          const float pr = __builtin_amdgcn_exp2f(fmaf(zraw, p.c, -lse2[h]));
+          float up = glp[h];
+          if (kEntropy) up = fmaf(gen[h], fmaf(zraw, it, -lse[h]) + ent[h], up);
+          d[e] = -it * pr * up;
         }
-      }
+        if ((unsigned)(lab[h] - v) < (unsigned)VEC) {
 #pragma unroll
-      for (int k = 0; k < VEC; ++k) *reinterpret_cast<u32x4*>(unit + (R + k) * kRowBytes + q * 16) = pack_vec(d[k], (T*)nullptr);
-      const int tok = rb * kBlockRows + R;
-      if (tok < p.ldt) {
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-          float x[VEC];
-#pragma unroll
-          for (int k = 0; k < VEC; ++k) x[k] = d[k][e];
-          if (v + e < p.V) *reinterpret_cast<u32x4*>(dzT + blocked_index<T>(v + e, tok, p.t_slabs)) = pack_vec(x, (T*)nullptr);
+          for (int e = 0; e < VEC; ++e)
+            if (lab[h] - v == e) d[e] += it * glp[h];
         }
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) d[e] = live[h] ? d[e] : 0.f;
+        if (v + VEC > p.V) {                        // vocabulary padding columns give zeros
+#pragma unroll
+          for (int e = 0; e < VEC; ++e)
+            if (v + e >= p.V) d[e] = 0.f;
+        }
+        *reinterpret_cast<u32x4*>(dz + (int64_t)ks * (E * kRowBytes) + h * 32 * kRowBytes) = pack_vec(d, (T*)nullptr);
       }
     }
   }
 }
 
-// C (+)= A B^T with A [M x K] and B [N x K] K-blocked, C row-major in one of two orientations; either way
+// C (+)= A B^T with A [M x K] and B [N x K], C row-major in one of two orientations; either way
 // a lane's 16-byte pieces lie along C's rows and a store instruction covers runs of at least 64 bytes:
-//   kMContig = false: C[m][n], ld = ldc, fp32 or 16-bit (dW: A = dz^T, B = hidden^T).  A lane holds 4 consecutive n of
-//     a row (GemmTile with BV = 4), 16 lanes 256 contiguous bytes of each of 4 rows for fp32, 128 for 16-bit results.
-//   kMContig = true:  C[n][m], ld = ldc (dhidden: A = W^T, B = dz).  A lane holds VEC consecutive m of a row, the 4
-//     lane groups 64 contiguous bytes of each of 16 rows for 16-bit results.
-template <typename T, bool kMContig> using OutTile = GemmTile<T, kMContig ? 16 / (int)sizeof(T) : 4>;
+//   dW (side kLogits):  C[m][n], ld = ldc, fp32 or 16-bit, A = dz^T (dz in units), B = hidden^T (K-blocked).  A lane holds
+//     4 consecutive n of a row (GemmTile with BV = 4), 16 lanes 256 contiguous bytes of each of 4 rows for fp32, 128 for
+//     16-bit results.
+//   dhidden (kMContig): C[n][m], ld = ldc, A = W^T (kWeight: W itself; kRows: the caller's K-blocked W^T), B = dz (in
+//     units).  A lane holds VEC consecutive m of a row, the 4 lane groups 64 contiguous bytes of each of 16 rows for 16-bit results.
+template <Side S> constexpr bool kMContig = S != Side::kLogits;
+template <typename T, Side S> using OutTile = GemmTile<T, kMContig<S> ? 16 / (int)sizeof(T) : 4, S, kMContig<S>>;
 
 struct GemmParams {
-  const void* A;      // M x K, K-blocked with a_kslabs slabs per row block
-  const void* B;      // N x K, K-blocked with b_kslabs slabs per row block
+  const void* A;
+  const void* B;
   void* C;
-  int64_t a_kslabs, b_kslabs, ldc;
+  int64_t a_step, b_step;   // A: slabs per row block (kRows), row stride in elements (kWeight), units per row of units (kLogits);
+                            // B: units per row of units (kMContig), slabs per row block
+  int64_t ldc;
   int M, N, K;
+  int k_valid;              // kWeight: rows of W; the rest of K reads as zero
   int n_mt, n_nt;
   int accumulate;
   int k_split;        // > 1: work item = (tile, K range); fp32 partial tiles go to `partial`
   int k_per_split;    // K extent of one range, a multiple of the slab
-  int n_walk;         // > 0: workgroups walk runs of tiles (see gemm_nt_kernel); needs k_split == 1
+  int n_walk;         // > 0: workgroups walk runs of tiles (see gemm_kernel); needs k_split == 1
   float* partial;     // [k_split] copies of C's shape in fp32, densely packed (row stride N or M)
   const int32_t* order;   // kMContig, optional [N]: row n of the result is row order[n] of the `total` rows of C
   int64_t total;
@@ -275,12 +270,17 @@ struct GemmParams {
 // of them give 0 and stores are dropped.  Along the register dimension (m) nothing relies on the range check:
 // kMContig skips whole 32-row groups (its M extents are multiples of 32), and the other orientation tests
 // every row against the tile's valid rows unless the tile is a full one.
-template <typename T, typename OutT, bool kMContig>
+template <typename T, typename OutT, Side S>
 struct TileAddr {
-  using Tile = OutTile<T, kMContig>;
+  using Tile = OutTile<T, S>;
+  static constexpr bool kMContig = clgrpo::kMContig<S>;
   static constexpr int ES = (int)sizeof(OutT);
-  static constexpr int AG = Tile::VEC / 4;                  // blocks along m whose registers are consecutive
+  static constexpr int kPieces = Tile::MI * 4 / Tile::VEC;  // kMContig: runs of VEC consecutive m per lane and block j
   static constexpr int kGroups = kMContig ? Tile::NI : Tile::NI / 4;
+  // element k of piece n: its block and register
+  static constexpr int block(int n, int k) { return Tile::kAcross ? n / 4 * Tile::VEC + k : n * (Tile::VEC / 4) + k / 4; }
+  static constexpr int reg(int n, int k) { return Tile::kAcross ? n % 4 : k % 4; }
+  static constexpr int piece_off(int n) { return Tile::a_off(block(n, 0), reg(n, 0)); }
   __amdgpu_buffer_rsrc_t rsrc;
   int voff[kGroups];
   int row_bytes, a_rows, row_lim;   // row_lim: valid rows from this lane's first row on
@@ -303,8 +303,8 @@ struct TileAddr {
       else voff[k] = m * row_bytes + n * ES;
     }
   }
-  // kMContig: blocks i .. i + AG - 1 lie inside the tile (uniform over the wave)
-  __device__ __forceinline__ bool group_ok(int i) const { return Tile::wave_m() + (Tile::a_block(i) & ~31) < a_rows; }
+  // kMContig: piece n lies inside the tile (uniform over the wave)
+  __device__ __forceinline__ bool piece_ok(int n) const { return Tile::wave_m() + (piece_off(n) & ~31) < a_rows; }
   __device__ __forceinline__ bool full_rows() const { return a_rows == Tile::BM; }
 };
 
@@ -342,25 +342,22 @@ __device__ __forceinline__ void row_store(const float (&x)[4], const __amdgpu_bu
 }
 
 // fn(values of one run of a row, per-lane offset, scalar offset), for every run of the tile that lies inside it;
-// kLoad: the values go into the accumulators afterwards.
-template <typename T, typename OutT, bool kMContig, bool kLoad, typename AccT, typename Fn>
-__device__ __forceinline__ void for_rows(const TileAddr<T, OutT, kMContig>& at, AccT& acc, Fn fn) {
-  using Tile = OutTile<T, kMContig>;
-  if constexpr (kMContig) {
-    constexpr int AG = TileAddr<T, OutT, kMContig>::AG, N = 4 * AG;
+// kLoad (dW only): the values go into the accumulators afterwards.
+template <typename T, typename OutT, Side S, bool kLoad, typename AccT, typename Fn>
+__device__ __forceinline__ void for_rows(const TileAddr<T, OutT, S>& at, AccT& acc, Fn fn) {
+  using Tile = OutTile<T, S>;
+  using Addr = TileAddr<T, OutT, S>;
+  if constexpr (kMContig<S>) {
+    static_assert(!kLoad, "dhidden is never added to");
 #pragma unroll
-    for (int i = 0; i < Tile::MI; i += AG) {
-      if (!at.group_ok(i)) continue;
+    for (int n = 0; n < Addr::kPieces; ++n) {
+      if (!at.piece_ok(n)) continue;
 #pragma unroll
       for (int j = 0; j < Tile::NI; ++j) {
-        float x[N] = {};
+        float x[Tile::VEC];
 #pragma unroll
-        for (int k = 0; k < (kLoad ? 0 : N); ++k) x[k] = acc_get(acc[i + k / 4][j], k % 4);
-        fn(x, at.voff[j] + Tile::a_block(i) * (int)sizeof(OutT), 0);
-        if (kLoad) {
-#pragma unroll
-          for (int k = 0; k < N; k += 4) acc_set(acc[i + k / 4][j], x[k], x[k + 1], x[k + 2], x[k + 3]);
-        }
+        for (int k = 0; k < Tile::VEC; ++k) x[k] = acc_get(acc[Addr::block(n, k)][j], Addr::reg(n, k));
+        fn(x, at.voff[j] + Addr::piece_off(n) * (int)sizeof(OutT), 0);
       }
     }
   } else {
@@ -372,7 +369,7 @@ __device__ __forceinline__ void for_rows(const TileAddr<T, OutT, kMContig>& at, 
         float x[4][4];                    // [register of the four blocks][block]
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int dm = Tile::a_block(i) + r;
+          const int dm = Tile::a_off(i, r);
 #pragma unroll
           for (int k = 0; k < 4; ++k) x[r][k] = kLoad ? 0.f : acc_get(acc[i][j + k], r);
           if (full || dm < at.row_lim) fn(x[r], at.voff[j / 4], dm * at.row_bytes);
@@ -389,54 +386,56 @@ __device__ __forceinline__ void for_rows(const TileAddr<T, OutT, kMContig>& at, 
 // workgroup owns the whole K range of the tile - the tile's current contents.  Reading C here instead of
 // in the epilogue puts the loads' latency in front of the K loop, where the first operand slabs are in
 // flight anyway, and leaves the epilogue a pure store.
-template <typename T, typename OutT, bool kMContig>
-__device__ __forceinline__ void gemm_init_tile(const GemmParams& p, typename OutTile<T, kMContig>::Acc& acc, int m0, int n0,
+template <typename T, typename OutT, Side S>
+__device__ __forceinline__ void gemm_init_tile(const GemmParams& p, typename OutTile<T, S>::Acc& acc, int m0, int n0,
                                                int a_rows, int b_rows) {
-  constexpr bool kAdds = !kMContig && sizeof(OutT) == 4;    // only an fp32 C is ever added to
-  if (!kAdds || !p.accumulate || p.k_split > 1) OutTile<T, kMContig>::zero(acc);
+  constexpr bool kAdds = !kMContig<S> && sizeof(OutT) == 4;    // only an fp32 C is ever added to
+  if (!kAdds || !p.accumulate || p.k_split > 1) OutTile<T, S>::zero(acc);
   if constexpr (kAdds) {
     if (!p.accumulate || p.k_split > 1) return;
-    const TileAddr<T, OutT, kMContig> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows);
-    for_rows<T, OutT, kMContig, true>(at, acc, [&](auto& x, int voff, int soff) { row_load(x, at.rsrc, voff, soff, (OutT*)nullptr); });
+    const TileAddr<T, OutT, S> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows);
+    for_rows<T, OutT, S, true>(at, acc, [&](auto& x, int voff, int soff) { row_load(x, at.rsrc, voff, soff, (OutT*)nullptr); });
   }
 }
 
 // Output tile from the accumulators: C = acc (the accumulators already hold C's previous contents
 // when the GEMM adds to it, see gemm_init_tile), or the fp32 partial of K range `ks`.
-template <typename T, typename OutT, bool kMContig>
-__device__ __forceinline__ void gemm_store_tile(const GemmParams& p, typename OutTile<T, kMContig>::Acc& acc, int m0, int n0,
+template <typename T, typename OutT, Side S>
+__device__ __forceinline__ void gemm_store_tile(const GemmParams& p, typename OutTile<T, S>::Acc& acc, int m0, int n0,
                                                 int a_rows, int b_rows, int ks) {
   if (p.k_split > 1) {
-    const TileAddr<T, float, kMContig> at(p.partial + (int64_t)ks * p.M * p.N, kMContig ? p.M : p.N, m0, n0, a_rows, b_rows);
-    for_rows<T, float, kMContig, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (float*)nullptr); });
+    const TileAddr<T, float, S> at(p.partial + (int64_t)ks * p.M * p.N, kMContig<S> ? p.M : p.N, m0, n0, a_rows, b_rows);
+    for_rows<T, float, S, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (float*)nullptr); });
     return;
   }
-  const TileAddr<T, OutT, kMContig> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows, p.order, p.total);
-  for_rows<T, OutT, kMContig, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (OutT*)nullptr); });
+  const TileAddr<T, OutT, S> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows, p.order, p.total);
+  for_rows<T, OutT, S, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (OutT*)nullptr); });
 }
 
 // Work item = (walk, fixed tile) when n_walk > 0: the workgroup keeps one operand's tile (A's m tile
 // when C is [n][m], B's n tile when C is [m][n]) and walks a contiguous run of tiles of the other, so the
 // K loops stream into each other (the next tile's first slabs are requested while the current tile
 // finishes and is stored).  Otherwise work item = (K range, m tile, n tile), one K loop per workgroup.
-template <typename T, typename OutT, bool kMContig>
-__global__ __launch_bounds__(kHeadThreads, 1) void gemm_nt_kernel(GemmParams p) {
-  using Tile = OutTile<T, kMContig>;
-  constexpr int64_t kSlabElems = (int64_t)kBlockRows * Tile::kSlabK;   // elements of one block's slab
+template <typename T, typename OutT, Side S>
+__global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
+  using Tile = OutTile<T, S>;
+  constexpr bool kMC = kMContig<S>;
+  constexpr int E = Tile::kSlabK;
+  constexpr int64_t kSlabElems = (int64_t)kBlockRows * E;   // elements of a K-blocked block's slab, and of a 256-wide row of units
   extern __shared__ __align__(16) char lds[];
 
   // this workgroup's tiles: (mt, nt) first, then `count - 1` steps along the walked operand; one K range
   int item = xcd_remap(blockIdx.x, gridDim.x), mt, nt, count = 1, ks = 0, k0 = 0, k_len = p.K;
   if (p.n_walk > 0) {
-    const int n_fixed = kMContig ? p.n_mt : p.n_nt;       // tiles of the operand that stays
-    const int n_moving = kMContig ? p.n_nt : p.n_mt;      // tiles of the operand that is walked
+    const int n_fixed = kMC ? p.n_mt : p.n_nt;       // tiles of the operand that stays
+    const int n_moving = kMC ? p.n_nt : p.n_mt;      // tiles of the operand that is walked
     if (item >= p.n_walk * n_fixed) return;
     int walk, ft;
     grouped_tile(item, p.n_walk, n_fixed, 4, walk, ft);
     const int begin = (int)((int64_t)walk * n_moving / p.n_walk);
     count = (int)((int64_t)(walk + 1) * n_moving / p.n_walk) - begin;
-    mt = kMContig ? ft : begin;
-    nt = kMContig ? begin : ft;
+    mt = kMC ? ft : begin;
+    nt = kMC ? begin : ft;
   } else {
     if (item >= p.n_mt * p.n_nt * p.k_split) return;
     ks = item / (p.n_mt * p.n_nt);
@@ -446,33 +445,40 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_nt_kernel(GemmParams p) 
     k_len = (p.K - k0) < p.k_per_split ? (p.K - k0) : p.k_per_split;
   }
 
-  const int nslab = k_len / Tile::kSlabK;
-  const int64_t s0 = k0 / Tile::kSlabK;   // first slab of this K range
+  const int nslab = k_len / E;
+  const int64_t s0 = k0 / E;   // first slab of this K range
   const bool stream = Tile::can_stream(nslab);
+  const T* A = static_cast<const T*>(p.A);
+  const T* B = static_cast<const T*>(p.B);
+  auto operand_a = [&](int m_tile, int rows) {
+    if constexpr (S == Side::kRows) return Tile::Operand::blocked(A + ((int64_t)m_tile * p.a_step + s0) * kSlabElems, rows);
+    else if constexpr (S == Side::kWeight)
+      return Tile::Operand::across_weight(A + (int64_t)k0 * p.a_step + m_tile * 256, p.a_step, m_tile * 256, rows, p.k_valid - k0);
+    else return Tile::Operand::across_units(A + s0 * p.a_step * (E * E) + m_tile * kSlabElems, p.a_step, rows);
+  };
+  auto operand_b = [&](int n_tile, int rows) {
+    if constexpr (kMC) return Tile::Operand::units(B + (n_tile * (int64_t)(256 / E) * p.b_step + s0) * (E * E), p.b_step, rows);
+    else return Tile::Operand::blocked(B + ((int64_t)n_tile * p.b_step + s0) * kSlabElems, rows);
+  };
+  auto rows_of = [](int total, int tile) { const int left = total - tile * 256; return left < 256 ? left : 256; };
   typename Tile::Acc acc;
   Tile core;
   for (int k = 0; k < count; ++k) {
     const int m0 = mt * 256, n0 = nt * 256;
-    const int a_rows = (p.M - m0) < 256 ? (p.M - m0) : 256;
-    const int b_rows = (p.N - n0) < 256 ? (p.N - n0) : 256;
-    const auto op_a = Tile::Operand::blocked(static_cast<const T*>(p.A) + ((int64_t)mt * p.a_kslabs + s0) * kSlabElems, a_rows);
-    const auto op_b = Tile::Operand::blocked(static_cast<const T*>(p.B) + ((int64_t)nt * p.b_kslabs + s0) * kSlabElems, b_rows);
-    gemm_init_tile<T, OutT, kMContig>(p, acc, m0, n0, a_rows, b_rows);
+    const int a_rows = rows_of(p.M, mt), b_rows = rows_of(p.N, nt);
+    const auto op_a = operand_a(mt, a_rows);
+    const auto op_b = operand_b(nt, b_rows);
+    gemm_init_tile<T, OutT, S>(p, acc, m0, n0, a_rows, b_rows);
     if (k == 0 || !stream) core.start(op_a, op_b, nslab, lds);
-    core.next_a = Tile::hold(op_a, nslab);
-    core.next_b = Tile::hold(op_b, nslab);
-    if (stream && k + 1 < count) {
-      const int left = (kMContig ? p.N - n0 : p.M - m0) - 256;
-      const int next_rows = left < 256 ? left : 256;
-      core.next_a = kMContig ? Tile::cursor(op_a, nslab)
-                             : Tile::cursor(Tile::Operand::blocked(op_a.base + p.a_kslabs * kSlabElems, next_rows), nslab);
-      core.next_b = kMContig ? Tile::cursor(Tile::Operand::blocked(op_b.base + p.b_kslabs * kSlabElems, next_rows), nslab)
-                             : Tile::cursor(op_b, nslab);
-    }
+    if (stream && k + 1 < count)
+      core.follow(op_a, op_b, nslab, Tile::cursor_a(kMC ? op_a : operand_a(mt + 1, rows_of(p.M, mt + 1)), nslab),
+                  Tile::cursor_b(kMC ? operand_b(nt + 1, rows_of(p.N, nt + 1)) : op_b, nslab));
+    else
+      core.follow(op_a, op_b, nslab, Tile::hold_a(op_a, nslab), Tile::hold_b(op_b, nslab));
     core.run(acc, nslab);
     if (!stream || k + 1 == count) Tile::finish();
-    gemm_store_tile<T, OutT, kMContig>(p, acc, m0, n0, a_rows, b_rows, ks);
-    if (kMContig) ++nt; else ++mt;
+    gemm_store_tile<T, OutT, S>(p, acc, m0, n0, a_rows, b_rows, ks);
+    if (kMC) ++nt; else ++mt;
   }
 }
 
@@ -618,7 +624,7 @@ static size_t dhidden_partial_bytes(int64_t rows, int64_t H, int64_t ldv, int sl
 }
 
 // How the dW GEMM (C[m][n], M = vocabulary rows, N = H, K = the chunk's tokens) is launched.  With many more tiles
-// than CUs its workgroups keep one tile of hidden^T and walk runs of vocabulary tiles (see gemm_nt_kernel); the walks
+// than CUs its workgroups keep one tile of hidden^T and walk runs of vocabulary tiles (see gemm_kernel); the walks
 // are as long as the longest run, so when the vocabulary tiles do not divide by the number of walks the last
 // `n_mt % n_walk` of them keep a sixteenth of the chip busy for a whole tile period (594 tiles on 16 walks: runs of
 // 37 and 38).  The repair is the one of the dhidden GEMM: a bulk launch whose walks are all equally long, and a second
@@ -672,139 +678,11 @@ static size_t dweight_partial_bytes(int64_t rows, int64_t H, int64_t V, int slab
   return rows > 0 ? plan_dweight(V, H, round_up64(rows, 64), slab, 256, (size_t)1 << 30).partial_bytes : 0;
 }
 
-// dhidden of few rows straight from W [V, H], without W^T.  Building W^T reads and writes the weight once each (V = 151936,
-// H = 4096: 465 us), more than a contraction over a few hundred rows takes.  A wave owns 128 columns of H, 128 rows and
-// a K range.  Lane 16 g + c reads 8 vocabulary rows (k = 8 g ..) x 8 columns (8 c ..) of W, 16 bytes per row, and
-// transposes the square between registers: the result is its A fragment of 8 blocks of 16 columns each, block i
-// holding columns 8 c + i.  B fragments are 16-byte pieces of the K-blocked dz.  No LDS and no barriers: the
-// four waves of a workgroup (512 columns) meet in the L1 on the dz pieces.  Bound by reading W as long as one or
-// two blocks of 128 rows share it; with more rows the matrix work takes over, at a lower rate than the tile of
-// gemm_core.hpp (the limit and both sides' times: kFewRows).
-struct FewRowsParams {
-  const __bf16* dz;       // K-blocked, whole blocks of 256 rows
-  const __bf16* weight;
-  float* partial;         // [k_split][rows][H]
-  int64_t n_kslab;
-  int rows, H, V;
-  int n_h, n_t, k_split, slabs_per_split;
-};
-
-__global__ __launch_bounds__(256, 1) void dhidden_few_rows_kernel(FewRowsParams p) {
-  const int item = xcd_remap(blockIdx.x, gridDim.x);
-  if (item >= p.n_h * p.n_t * p.k_split) return;
-  const int tt = item % p.n_t, ks = item / p.n_t / p.n_h;
-  const int h0 = ((item / p.n_t % p.n_h) * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * 128;
-  if (h0 >= p.H) return;
-  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-  const int s0 = ks * p.slabs_per_split;
-  const int n_slab = p.n_kslab - s0 < p.slabs_per_split ? (int)(p.n_kslab - s0) : p.slabs_per_split;
-  const int last = 2 * n_slab - 1;                                // steps of 32 vocabulary rows
-  const int col = h0 + 8 * c < p.H ? h0 + 8 * c : p.H - 8;        // columns past H: any, they are not stored
-  const __bf16* z = p.dz + (((int64_t)(tt >> 1) * p.n_kslab + s0) * kBlockRows + (tt & 1) * 128 + c) * 64 + 8 * g;
-
-  // Range-checked loads from a descriptor over the step's valid rows: rows past V read as zero, and no branch stands
-  // between a request and the matrix instructions it is to overlap.  What is checked is the per-lane offset, so the row
-  // is part of it (a scalar offset is outside the check by the builtin's contract).
-  const int row_bytes = p.H * 2, voff = 8 * g * row_bytes + col * 2;
-  auto load_a = [&](u32x4 (&raw)[8], int n) __attribute__((always_inline)) {
-    const int v0 = s0 * 64 + (n < last ? n : last) * 32;
-    const int rows = p.V - v0 < 32 ? (p.V > v0 ? p.V - v0 : 0) : 32;
-    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(p.weight) + (int64_t)v0 * p.H, 0, rows * row_bytes, 0x00020000);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) raw[e] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff + e * row_bytes, 0, 0);
-  };
-  auto load_b = [&](u32x4 (&b)[8], int n) __attribute__((always_inline)) {
-    const int m = n < last ? n : last;
-    const __bf16* at = z + (int64_t)(m >> 1) * (kBlockRows * 64) + (m & 1) * 32;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) b[j] = *reinterpret_cast<const u32x4*>(at + j * 16 * 64);
-  };
-  f32x4 acc[8][8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc_set(acc[i][j], 0.f, 0.f, 0.f, 0.f);
-  u32x4 raw0[8], raw1[8], b0[8], b1[8];
-  // one step: the fragments of `raw`, the requests for the step after next into it, the products with `b`
-  auto step = [&](u32x4 (&raw)[8], const u32x4 (&b)[8], int n) __attribute__((always_inline)) {
-    u32x4 a[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        a[i][q] = __builtin_amdgcn_perm(raw[2 * q + 1][i / 2], raw[2 * q][i / 2], i % 2 ? 0x07060302u : 0x05040100u);
-    __builtin_amdgcn_sched_barrier(0);
-    load_a(raw, n + 2);
-    GemmTile<__bf16, 8>::settle();     // vector results on their way into matrix instructions
-    each<64>([&](auto m) __attribute__((always_inline)) { Mma<__bf16>::slot(acc, a, b, decltype(m)::value); });
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  load_a(raw0, 0);
-  load_b(b0, 0);
-  load_a(raw1, 1);
-  for (int s = 0; s < n_slab; ++s) {
-    load_b(b1, 2 * s + 1);
-    step(raw0, b0, 2 * s);
-    load_b(b0, 2 * s + 2);
-    step(raw1, b1, 2 * s + 1);
-  }
-  GemmTile<__bf16, 8>::settle();
-  // register r of block (i, j): column 8 (4 g + r) + i, row 16 j + c
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int t = tt * 128 + 16 * j + c;
-    if (t >= p.rows) continue;
-    float* row = p.partial + ((int64_t)ks * p.rows + t) * p.H;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int h = h0 + 8 * (4 * g + r);
-      if (h >= p.H) continue;
-      f32x4 lo, hi;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) { lo[i] = acc_get(acc[i][j], r); hi[i] = acc_get(acc[4 + i][j], r); }
-      *reinterpret_cast<f32x4*>(row + h) = lo;
-      *reinterpret_cast<f32x4*>(row + h + 4) = hi;
-    }
-  }
-}
-
-// K ranges: one workgroup per CU, none empty, at least 8 slabs each; fewer the more rows their partial sums have (384
-// rows at H = 1024, V = 32000: whole step 284 us with 32 ranges, 295 with 42).
-// Up to three blocks of 128 rows: whole training steps with W^T / without it, us, V = 151936 (H = 7168: 129280):
-//   H = 2048: 100 rows 1030 / 809, 200 1165 / 983, 384 1298 / 1183, 512 1368 / 1317, 700 1634 / 1682
-//   H = 4096: 100 rows 1669 / 1235, 200 1875 / 1556, 384 2235 / 2021, 512 2385 / 2317, 700 2997 / 3036
-//   H = 7168: 100 rows 2351 / 1704, 200 2629 / 2213, 384 3289 / 2867, 480 3505 / 3590
-constexpr int64_t kFewRows = 384;
-struct FewRowsPlan {
-  int n_h, n_t, k_split, slabs_per_split;
-  size_t partial_bytes;
-};
-static FewRowsPlan plan_few_rows(int64_t rows, int64_t H, int64_t ldv, int cus, size_t partial_cap) {
-  FewRowsPlan pl;
-  pl.n_h = (int)((H + 511) / 512);
-  pl.n_t = (int)((rows + 127) / 128);
-  const int64_t n_slab = ldv / 64;
-  int64_t s = cus / (pl.n_h * pl.n_t);
-  const int64_t most = (int64_t)(partial_cap / ((size_t)rows * H * sizeof(float)));
-  if (s > 64) s = 64;
-  if (s > 96 / pl.n_t) s = 96 / pl.n_t;
-  if (s > n_slab / 8) s = n_slab / 8;
-  if (s > most) s = most;
-  if (s < 1) s = 1;
-  pl.slabs_per_split = (int)((n_slab + s - 1) / s);
-  pl.k_split = (int)((n_slab + pl.slabs_per_split - 1) / pl.slabs_per_split);
-  pl.partial_bytes = (size_t)pl.k_split * rows * H * sizeof(float);
-  return pl;
-}
-static bool few_rows(int64_t rows, int64_t T, size_t es, bool saved, bool own_wt) {
-  return es == 2 && saved && own_wt && rows == T && rows <= kFewRows;
-}
-
 struct BwdPlan {
-  int64_t ldv;        // K extent of dz / WT (V rounded up to 64)
+  int64_t ldv;        // vocabulary extent of dz (V rounded up to 64)
   int64_t chunk;      // tokens per chunk (multiple of 256 unless >= T)
-  int64_t ldt;        // K extent of dzT / hidT for a full chunk (tokens rounded up to 64)
-  size_t off_wt, off_hidt, off_dz, off_dzt, off_part, part_bytes, total;
+  int64_t ldt;        // token extent of hidT for a full chunk (tokens rounded up to 64)
+  size_t off_hidt, off_dz, off_part, part_bytes, total;
 };
 
 static BwdPlan bwd_plan(int64_t T, int64_t H, int64_t V, size_t es, int64_t chunk_tokens, bool saved = false,
@@ -816,13 +694,9 @@ static BwdPlan bwd_plan(int64_t T, int64_t H, int64_t V, size_t es, int64_t chun
   pl.chunk = chunk;
   pl.ldt = round_up64(chunk, 64);
   size_t off = 0;
-  // K-blocked operands: whole blocks of 256 rows
-  const size_t Hb = (size_t)round_up64(H, 256), Cb = (size_t)round_up64(chunk, 256), Vb = (size_t)round_up64(V, 256);
-  const bool few = few_rows(chunk, T, es, saved, own_wt);       // reads W itself
-  pl.off_wt = off;   off += own_wt && !few ? align_up(Hb * pl.ldv * es, 256) : 0;
+  const size_t Hb = (size_t)round_up64(H, 256);                 // K-blocked: whole blocks of 256 rows
   pl.off_hidt = off; off += own_dw ? align_up(Hb * pl.ldt * es, 256) : 0;
-  pl.off_dz = off;   off += saved ? 0 : align_up(Cb * pl.ldv * es, 256);
-  pl.off_dzt = off;  off += own_dw ? align_up(Vb * pl.ldt * es, 256) : 0;
+  pl.off_dz = off;   off += saved ? 0 : align_up((size_t)pl.ldt * pl.ldv * es, 256);
   // split-K partials of the dhidden GEMM and of the dW GEMM's tail (used one after the other): what a full chunk and
   // the shorter last chunk want
   const int slab = (int)(kRowBytes / es);
@@ -830,12 +704,12 @@ static BwdPlan bwd_plan(int64_t T, int64_t H, int64_t V, size_t es, int64_t chun
   for (size_t b : {dhidden_partial_bytes(chunk, H, pl.ldv, slab), dhidden_partial_bytes(T % chunk, H, pl.ldv, slab),
                    own_dw ? dweight_partial_bytes(chunk, H, V, slab) : 0, own_dw ? dweight_partial_bytes(T % chunk, H, V, slab) : 0})
     if (b > part) part = b;
-  if (few) {
-    const size_t b = plan_few_rows(chunk, H, pl.ldv, 256, (size_t)1 << 30).partial_bytes;
-    if (b > part) part = b;
-  }
   pl.part_bytes = align_up(part, 256);
   pl.off_part = off; off += pl.part_bytes;
+  // A caller without a W^T of its own has always been asked for the room of one (up to 384 16-bit rows from kept logits
+  // excepted).  W is read as it is now; the sizes that callers plan with stay.
+  const bool few = es == 2 && saved && chunk == T && T <= 384;
+  off += own_wt && !few ? align_up(Hb * pl.ldv * es, 256) : 0;
   pl.total = off;
   return pl;
 }
@@ -860,15 +734,22 @@ static int launch_splitk_reduce(const float* partial, int k_split, int rows, int
   return check_launch("splitk_reduce_kernel");
 }
 
-template <typename T, typename OutT, bool kMContig>
-static int launch_gemm_one(const void* A, int64_t a_kslabs, int M, const void* B, int64_t b_kslabs, int N, int K, void* C,
-                           int64_t ldc, int accumulate, hipStream_t stream, float* partial, size_t partial_bytes,
-                           int k_split_wanted, const RowOrder& rows = RowOrder{nullptr, 0}) {
-  using Tile = OutTile<T, kMContig>;
-  int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_nt_kernel<T, OutT, kMContig>), Tile::kLdsBytes, "gemm_nt_kernel");
+// Operands of a contraction as GemmParams names them.
+struct GemmIn {
+  const void *A, *B;
+  int64_t a_step, b_step;
+  int k_valid;
+};
+
+template <typename T, typename OutT, Side S>
+static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64_t ldc, int accumulate, hipStream_t stream,
+                           float* partial, size_t partial_bytes, int k_split_wanted, const RowOrder& rows = RowOrder{nullptr, 0}) {
+  using Tile = OutTile<T, S>;
+  constexpr bool kMC = kMContig<S>;
+  int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_kernel<T, OutT, S>), Tile::kLdsBytes, "gemm_kernel");
   if (rc) return rc;
   GemmParams g;
-  g.A = A; g.B = B; g.C = C; g.a_kslabs = a_kslabs; g.b_kslabs = b_kslabs; g.ldc = ldc;
+  g.A = in.A; g.B = in.B; g.C = C; g.a_step = in.a_step; g.b_step = in.b_step; g.ldc = ldc; g.k_valid = in.k_valid;
   g.M = M; g.N = N; g.K = K;
   g.n_mt = (M + 255) / 256; g.n_nt = (N + 255) / 256;
   g.accumulate = accumulate;
@@ -886,7 +767,7 @@ static int launch_gemm_one(const void* A, int64_t a_kslabs, int M, const void* B
   g.partial = partial;
   // Many more tiles than CUs and no K split: let one workgroup per CU walk runs of tiles instead of
   // launching one workgroup per tile.
-  const int n_fixed = kMContig ? g.n_mt : g.n_nt, n_moving = kMContig ? g.n_nt : g.n_mt;
+  const int n_fixed = kMC ? g.n_mt : g.n_nt, n_moving = kMC ? g.n_nt : g.n_mt;
   g.n_walk = 0;
   if (g.k_split == 1 && n_fixed <= cus && g.n_mt * g.n_nt >= 4 * cus && K >= 2 * slab) {
     g.n_walk = cus / n_fixed;
@@ -899,48 +780,47 @@ static int launch_gemm_one(const void* A, int64_t a_kslabs, int M, const void* B
     if (walk_periods * 100 > plain_rounds * 104) g.n_walk = 0;
   }
   int grid = ((g.n_walk > 0 ? g.n_walk * n_fixed : g.n_mt * g.n_nt * g.k_split) + 7) / 8 * 8;
-  hipLaunchKernelGGL((gemm_nt_kernel<T, OutT, kMContig>), dim3(grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
-  rc = check_launch("gemm_nt_kernel");
+  hipLaunchKernelGGL((gemm_kernel<T, OutT, S>), dim3(grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
+  rc = check_launch("gemm_kernel");
   if (rc || g.k_split == 1) return rc;
-  return launch_splitk_reduce<OutT>(partial, g.k_split, kMContig ? N : M, kMContig ? M : N, static_cast<OutT*>(C), ldc, accumulate,
+  return launch_splitk_reduce<OutT>(partial, g.k_split, kMC ? N : M, kMC ? M : N, static_cast<OutT*>(C), ldc, accumulate,
                                     rows.order, stream);
 }
 
-// C (+)= A B^T under the launch plan of its orientation: plan_dhidden (C[n][m], with `partial`) or plan_dweight (C[m][n]).
-template <typename T, typename OutT, bool kMContig>
-static int launch_gemm(const void* A, int64_t a_kslabs, int M, const void* B, int64_t b_kslabs, int N, int K, void* C,
-                       int64_t ldc, int accumulate, hipStream_t stream, float* partial = nullptr,
-                       size_t partial_bytes = 0, const RowOrder& rows = RowOrder{nullptr, 0}) {
-  using Tile = OutTile<T, kMContig>;
-  constexpr int64_t kSlabElems = (int64_t)kBlockRows * Tile::kSlabK;
-  if (!kMContig) {
-    // dW: equally long walks over most vocabulary tiles, the rest cut into K ranges (plan_dweight)
-    const DwPlan dw = plan_dweight(M, N, K, Tile::kSlabK, device_cu_count(), partial ? partial_bytes : 0);
-    if (dw.bulk_mt == 0)
-      return launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, M, B, b_kslabs, N, K, C, ldc, accumulate, stream, nullptr, 0, 1);
-    const int bulk_rows = dw.bulk_mt * 256;
-    int rc = launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, bulk_rows, B, b_kslabs, N, K, C, ldc, accumulate, stream, nullptr, 0, 1);
-    if (rc) return rc;
-    const T* a_tail = static_cast<const T*>(A) + (int64_t)dw.bulk_mt * a_kslabs * kSlabElems;
-    OutT* c_tail = static_cast<OutT*>(C) + (int64_t)bulk_rows * ldc;
-    return launch_gemm_one<T, OutT, kMContig>(a_tail, a_kslabs, M - bulk_rows, B, b_kslabs, N, K, c_tail, ldc, accumulate, stream,
-                                              dw.k_split > 1 ? partial : nullptr, dw.k_split > 1 ? partial_bytes : 0, dw.k_split);
-  }
-  if (!(partial && partial_bytes))
-    return launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, M, B, b_kslabs, N, K, C, ldc, accumulate, stream, nullptr, 0, 1, rows);
-  const DhPlan pl = plan_dhidden(N, M, K, Tile::kSlabK, device_cu_count(), partial_bytes);
-  if (pl.bulk_nt == 0)
-    return launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, M, B, b_kslabs, N, K, C, ldc, accumulate, stream, partial,
-                                              partial_bytes, pl.k_split, rows);
+// dhidden[n][m] = sum over K of A(m, k) dz(n, k) under plan_dhidden (with `partial`).
+template <typename T, Side S>
+static int launch_dhidden(const GemmIn& in, int M, int N, int K, void* C, int64_t ldc, hipStream_t stream, float* partial,
+                          size_t partial_bytes, const RowOrder& rows) {
+  constexpr int E = Elem<T>::kSlabK;
+  if (!(partial && partial_bytes)) return launch_gemm_one<T, T, S>(in, M, N, K, C, ldc, 0, stream, nullptr, 0, 1, rows);
+  const DhPlan pl = plan_dhidden(N, M, K, E, device_cu_count(), partial_bytes);
+  if (pl.bulk_nt == 0) return launch_gemm_one<T, T, S>(in, M, N, K, C, ldc, 0, stream, partial, partial_bytes, pl.k_split, rows);
   const int bulk_rows = pl.bulk_nt * 256;
-  int rc = launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, M, B, b_kslabs, bulk_rows, K, C, ldc, accumulate, stream,
-                                              nullptr, 0, 1, rows);
+  int rc = launch_gemm_one<T, T, S>(in, M, bulk_rows, K, C, ldc, 0, stream, nullptr, 0, 1, rows);
   if (rc) return rc;
-  const T* b_tail = static_cast<const T*>(B) + (int64_t)pl.bulk_nt * b_kslabs * kSlabElems;
-  OutT* c_tail = static_cast<OutT*>(C) + (rows.order ? 0 : (int64_t)bulk_rows * ldc);
-  const RowOrder tail{rows.order ? rows.order + bulk_rows : nullptr, rows.total};
-  return launch_gemm_one<T, OutT, kMContig>(A, a_kslabs, M, b_tail, b_kslabs, N - bulk_rows, K, c_tail, ldc, accumulate,
-                                            stream, partial, partial_bytes, pl.k_split, tail);
+  GemmIn tail = in;
+  tail.B = static_cast<const T*>(in.B) + (int64_t)bulk_rows / E * in.b_step * (E * E);
+  T* c_tail = static_cast<T*>(C) + (rows.order ? 0 : (int64_t)bulk_rows * ldc);
+  const RowOrder tail_rows{rows.order ? rows.order + bulk_rows : nullptr, rows.total};
+  return launch_gemm_one<T, T, S>(tail, M, N - bulk_rows, K, c_tail, ldc, 0, stream, partial, partial_bytes, pl.k_split, tail_rows);
+}
+
+// dW[m][n] (+)= sum over K of dz(k, m) hidT(n, k): equally long walks over most vocabulary tiles, the rest cut into K
+// ranges (plan_dweight).
+template <typename T, typename OutT>
+static int launch_dweight(const GemmIn& in, int M, int N, int K, void* C, int64_t ldc, int accumulate, hipStream_t stream,
+                          float* partial, size_t partial_bytes) {
+  constexpr int E = Elem<T>::kSlabK;
+  const DwPlan dw = plan_dweight(M, N, K, E, device_cu_count(), partial ? partial_bytes : 0);
+  if (dw.bulk_mt == 0) return launch_gemm_one<T, OutT, Side::kLogits>(in, M, N, K, C, ldc, accumulate, stream, nullptr, 0, 1);
+  const int bulk_rows = dw.bulk_mt * 256;
+  int rc = launch_gemm_one<T, OutT, Side::kLogits>(in, bulk_rows, N, K, C, ldc, accumulate, stream, nullptr, 0, 1);
+  if (rc) return rc;
+  GemmIn tail = in;
+  tail.A = static_cast<const T*>(in.A) + (int64_t)bulk_rows * E;
+  OutT* c_tail = static_cast<OutT*>(C) + (int64_t)bulk_rows * ldc;
+  return launch_gemm_one<T, OutT, Side::kLogits>(tail, M - bulk_rows, N, K, c_tail, ldc, accumulate, stream,
+                                                 dw.k_split > 1 ? partial : nullptr, dw.k_split > 1 ? partial_bytes : 0, dw.k_split);
 }
 
 template <typename T>
@@ -951,18 +831,16 @@ static int launch_transpose(const T* src, int64_t ld_src, T* dst, int64_t r_dst,
   return check_launch("transpose_block_kernel");
 }
 
+// dW[v][h] (+)= sum_t dz(t, v) hidT(h, t) over k tokens of dz (n_kslab units per row of units) and hidT (ld tokens).
 template <typename T>
-static int run_dweight(const T* dzt, const T* hidt, int64_t ld, int64_t k, int64_t V, int64_t H, void* dweight, bool to_bf16,
-                       bool accumulate, void* partial, size_t partial_bytes, hipStream_t stream) {
-  // dW[v][h] (+)= sum_t dzT(v, t) hidT(h, t)   (M = V, N = H, K = the first k of ld tokens, C[m][n])
-  constexpr int slab = GemmTile<T, 4>::kSlabK;
+static int run_dweight(const T* dz, int64_t n_kslab, const T* hidt, int64_t ld, int64_t k, int64_t V, int64_t H, void* dweight,
+                       bool to_bf16, bool accumulate, void* partial, size_t partial_bytes, hipStream_t stream) {
+  const GemmIn in{dz, hidt, n_kslab, ld / Elem<T>::kSlabK, 0};
+  float* part = static_cast<float*>(partial);
   if constexpr (sizeof(T) == 2) {
-    if (to_bf16)
-      return launch_gemm<T, __bf16, false>(dzt, ld / slab, (int)V, hidt, ld / slab, (int)H, (int)k, dweight, H, 0, stream,
-                                           static_cast<float*>(partial), partial_bytes);
+    if (to_bf16) return launch_dweight<T, __bf16>(in, (int)V, (int)H, (int)k, dweight, H, 0, stream, part, partial_bytes);
   }
-  return launch_gemm<T, float, false>(dzt, ld / slab, (int)V, hidt, ld / slab, (int)H, (int)k, dweight, H, accumulate ? 1 : 0, stream,
-                                      static_cast<float*>(partial), partial_bytes);
+  return launch_dweight<T, float>(in, (int)V, (int)H, (int)k, dweight, H, accumulate ? 1 : 0, stream, part, partial_bytes);
 }
 
 template <typename T>
@@ -982,35 +860,37 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
   const BwdPlan pl = bwd_plan(T_, H, V, sizeof(T), chunk, saved, own_wt, own_dw);
   const int64_t ldz = saved ? a->ld_saved : pl.ldv;
   char* ws = static_cast<char*>(a->workspace);
-  T* wt = a->weight_t ? static_cast<T*>(a->weight_t) : reinterpret_cast<T*>(ws + pl.off_wt);
+  T* wt = static_cast<T*>(a->weight_t);
   T* dz_ws = reinterpret_cast<T*>(ws + pl.off_dz);
   const T* hidden = static_cast<const T*>(a->hidden);
   const T* weight = static_cast<const T*>(a->weight);
 
   int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&lmhead_dz_kernel<T>), Tile::kLdsBytes, "lmhead_dz_kernel");
   if (rc) return rc;
-  const bool few = few_rows(chunk, T_, sizeof(T), saved, own_wt);
-  if (a->dhidden && !few && !(a->weight_t && a->weight_t_ready)) {
-    // WT(h, v) = W[v][h], zero for V <= v < ldv, K-blocked
+  if (a->dhidden && wt && !a->weight_t_ready) {
+    // the caller keeps W^T: WT(h, v) = W[v][h], zero for V <= v < ldv, K-blocked
     rc = launch_transpose<T>(weight, H, wt, pl.ldv, (int)V, (int)H, stream);
     if (rc) return rc;
   }
   for (int64_t c0 = 0; c0 < T_; c0 += chunk) {
     const int64_t tc = (T_ - c0) < chunk ? (T_ - c0) : chunk;
     const int64_t ldt = round_up64(tc, 64);
-    // the operands of dW: this chunk's own, or its place among the ones that the caller contracts later
-    constexpr int64_t kSlabElems = (int64_t)kBlockRows * Tile::kSlabK;
+    // d(logits): in place of the kept logits, in the workspace, or in its place among the operands of dW that the caller
+    // contracts later
+    constexpr int E = Tile::kSlabK;
+    constexpr int64_t kSlabElems = (int64_t)kBlockRows * E;
     const int64_t k0 = kept ? kept->k + c0 : 0, ld_dw = kept ? kept->ld : ldt;
-    T* dzt = (kept ? static_cast<T*>(kept->dzt) : reinterpret_cast<T*>(ws + pl.off_dzt)) + k0 / Tile::kSlabK * kSlabElems;
-    T* hidt = (kept ? static_cast<T*>(kept->hidt) : reinterpret_cast<T*>(ws + pl.off_hidt)) + k0 / Tile::kSlabK * kSlabElems;
-    T* dz = saved ? static_cast<T*>(a->saved_logits) + c0 * ldz : dz_ws;
+    T* hidt = (kept ? static_cast<T*>(kept->hidt) : reinterpret_cast<T*>(ws + pl.off_hidt)) + k0 / E * kSlabElems;
+    T* z = saved ? static_cast<T*>(a->saved_logits) + c0 * ldz : nullptr;
+    T* dz = kept ? static_cast<T*>(kept->dzt) + k0 * pl.ldv : (saved ? z : dz_ws);
+    const int64_t dz_kslab = (kept ? pl.ldv : ldz) / E;
     // with an order the chunk's tokens are looked up from the start of the arrays, without they follow one another
     const int64_t t0 = rows.order ? 0 : c0;
     const int32_t* order = rows.order ? rows.order + c0 : nullptr;
     if (saved) {
       DzFromZParams q;
-      q.z = dz;
-      q.dzT = dzt;
+      q.z = z;
+      q.dz = dz;
       q.labels = a->labels + t0;
       q.label_offset = label_offset;
       q.lse = a->lse + t0;
@@ -1018,19 +898,20 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
       q.g_lp = a->g_logprob + t0;
       q.g_ent = a->g_entropy ? a->g_entropy + t0 : nullptr;
       q.order = order;
+      q.z_kslab = ldz / E;
+      q.dz_kslab = dz_kslab;
       q.Tc = (int)tc;
-      q.ldt = (int)ldt;
-      q.t_slabs = ld_dw / Tile::kSlabK;
       q.V = (int)V;
-      q.ldv = (int)ldz;
+      q.n_units = (int)(pl.ldv / E);
       q.c = a->inv_temperature * kLog2e;
       q.inv_temperature = a->inv_temperature;
-      // a workgroup walks units of one token block, so that its coefficients are fetched once; 16 workgroups per CU
-      const int64_t n_tb = (tc + kBlockRows - 1) / kBlockRows, n_units = ldz / Elem<T>::kSlabK;
-      int64_t per_tb = (16 * (int64_t)device_cu_count() + n_tb - 1) / n_tb;
-      if (per_tb > n_units) per_tb = n_units;
-      dim3 grid((unsigned)n_tb, (unsigned)per_tb);
-      hipLaunchKernelGGL(dz_from_z_kernel<T>, grid, dim3(256), 0, stream, q);
+      // a workgroup walks units of one row of units, so that its coefficients are fetched once; 16 workgroups per CU
+      const int64_t n_rows = ldt / E;
+      int64_t per_row = (16 * (int64_t)device_cu_count() + n_rows - 1) / n_rows;
+      if (per_row > q.n_units) per_row = q.n_units;
+      dim3 grid((unsigned)n_rows, (unsigned)per_row);
+      if (q.g_ent) hipLaunchKernelGGL((dz_from_z_kernel<T, true>), grid, dim3(256), 0, stream, q);
+      else hipLaunchKernelGGL((dz_from_z_kernel<T, false>), grid, dim3(256), 0, stream, q);
       rc = check_launch("dz_from_z_kernel");
       if (rc) return rc;
     } else {
@@ -1053,31 +934,20 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
       d.c = a->inv_temperature * kLog2e;
       d.inv_temperature = a->inv_temperature;
       d.dz = dz;
-      d.dzT = dzt;
       int grid = (d.n_tb * d.n_vt + 7) / 8 * 8;
       hipLaunchKernelGGL(lmhead_dz_kernel<T>, dim3(grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, d);
       rc = check_launch("lmhead_dz_kernel");
       if (rc) return rc;
     }
-    if (a->dhidden && few) {
-      const FewRowsPlan fp = plan_few_rows(tc, H, pl.ldv, device_cu_count(), pl.part_bytes);
-      FewRowsParams q;
-      q.dz = reinterpret_cast<const __bf16*>(dz);
-      q.weight = reinterpret_cast<const __bf16*>(weight);
-      q.partial = reinterpret_cast<float*>(ws + pl.off_part);
-      q.n_kslab = ldz / 64;
-      q.rows = (int)tc; q.H = (int)H; q.V = (int)V;
-      q.n_h = fp.n_h; q.n_t = fp.n_t; q.k_split = fp.k_split; q.slabs_per_split = fp.slabs_per_split;
-      hipLaunchKernelGGL(dhidden_few_rows_kernel, dim3((fp.n_h * fp.n_t * fp.k_split + 7) / 8 * 8), dim3(256), 0, stream, q);
-      rc = check_launch("dhidden_few_rows_kernel");
-      if (rc) return rc;
-      rc = launch_splitk_reduce<T>(q.partial, fp.k_split, (int)tc, (int)H, static_cast<T*>(a->dhidden) + t0 * H, H, 0, order, stream);
-      if (rc) return rc;
-    } else if (a->dhidden) {
-      // dhidden[chunk][h] = sum_v WT[h][v] dz[t][v]   (M = H, N = tokens, C[n][m])
-      rc = launch_gemm<T, T, true>(wt, pl.ldv / Tile::kSlabK, (int)H, dz, ldz / Tile::kSlabK, (int)tc, (int)pl.ldv,
-                             static_cast<T*>(a->dhidden) + t0 * H, H, 0, stream,
-                             reinterpret_cast<float*>(ws + pl.off_part), pl.part_bytes, RowOrder{order, rows.total});
+    if (a->dhidden) {
+      // dhidden[chunk][h] = sum_v W[v][h] dz[t][v]   (M = H, N = tokens, C[n][m])
+      void* out = static_cast<T*>(a->dhidden) + t0 * H;
+      float* part = reinterpret_cast<float*>(ws + pl.off_part);
+      const RowOrder out_rows{order, rows.total};
+      rc = wt ? launch_dhidden<T, Side::kRows>(GemmIn{wt, dz, pl.ldv / E, dz_kslab, 0}, (int)H, (int)tc, (int)pl.ldv, out, H,
+                                               stream, part, pl.part_bytes, out_rows)
+              : launch_dhidden<T, Side::kWeight>(GemmIn{weight, dz, H, dz_kslab, (int)V}, (int)H, (int)tc, (int)pl.ldv, out, H,
+                                                 stream, part, pl.part_bytes, out_rows);
       if (rc) return rc;
     }
     if (a->dweight || kept) {
@@ -1086,7 +956,7 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
       if (rc) return rc;
     }
     if (a->dweight && !kept) {
-      rc = run_dweight<T>(dzt, hidt, ldt, ldt, V, H, a->dweight, a->dweight_bf16 != 0, a->accumulate_dweight || c0 > 0,
+      rc = run_dweight<T>(dz, dz_kslab, hidt, ldt, ldt, V, H, a->dweight, a->dweight_bf16 != 0, a->accumulate_dweight || c0 > 0,
                           ws + pl.off_part, pl.part_bytes, stream);
       if (rc) return rc;
     }
@@ -1147,10 +1017,10 @@ extern "C" int clgrpo_dweight(const clgrpo_dweight_args* a, void* stream) {
     return fail(CLGRPO_EWORKSPACE, "%s: workspace %zu < %zu bytes", who, a->workspace_bytes, need);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (a->dtype == CLGRPO_BF16)
-    return run_dweight<__bf16>(static_cast<const __bf16*>(a->dzt), static_cast<const __bf16*>(a->hidt), a->ld, a->k, a->V, a->H,
-                               a->dweight, a->dweight_bf16 != 0, a->accumulate != 0, a->workspace, a->workspace_bytes, s);
-  return run_dweight<float>(static_cast<const float*>(a->dzt), static_cast<const float*>(a->hidt), a->ld, a->k, a->V, a->H,
-                            a->dweight, false, a->accumulate != 0, a->workspace, a->workspace_bytes, s);
+    return run_dweight<__bf16>(static_cast<const __bf16*>(a->dzt), round_up64(a->V, 64) / Elem<__bf16>::kSlabK,
+                               static_cast<const __bf16*>(a->hidt), a->ld, a->k, a->V, a->H, a->dweight, a->dweight_bf16 != 0, a->accumulate != 0, a->workspace, a->workspace_bytes, s);
+  return run_dweight<float>(static_cast<const float*>(a->dzt), round_up64(a->V, 64) / Elem<float>::kSlabK,
+                            static_cast<const float*>(a->hidt), a->ld, a->k, a->V, a->H, a->dweight, false, a->accumulate != 0, a->workspace, a->workspace_bytes, s);
 }
 
 int clgrpo::head_backward(const char* who, const clgrpo_lmhead_bwd_args* a, int64_t vocab_begin, const RowOrder& rows,

@@ -33,7 +33,7 @@ struct FwdParams {
   int T, H, V;
   int n_tb, n_split, tiles_per_split, n_vt;
   float c;  // inv_temperature * log2(e)
-  void* z_out;   // optional raw logits, K-blocked: rows x ldz entries of KeptLogit<T>
+  void* z_out;   // optional raw logits in units (see unit_index): rows x ldz entries of KeptLogit<T>
   int64_t ldz;
   const int32_t* z_row_map;  // optional [T]: destination row per token, < 0: not stored
   int z_rows;                // rows of z_out; mapped rows outside [0, z_rows) are not stored
@@ -131,11 +131,10 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
     if (stream && vt + 1 < vt_end) {
       const int v1 = v0 + kFwdBM;
       const int next_rows = (p.V - v1) < kFwdBM ? (p.V - v1) : kFwdBM;
-      core.next_a = Tile::cursor(Tile::Operand::row_major(weight + (int64_t)v1 * p.H, p.H, next_rows), nslab);
-      core.next_b = Tile::cursor(op_b, nslab);
+      core.follow(op_a, op_b, nslab, Tile::cursor_a(Tile::Operand::row_major(weight + (int64_t)v1 * p.H, p.H, next_rows), nslab),
+                  Tile::cursor_b(op_b, nslab));
     } else {
-      core.next_a = Tile::hold(op_a, nslab);
-      core.next_b = Tile::hold(op_b, nslab);
+      core.follow(op_a, op_b, nslab, Tile::hold_a(op_a, nslab), Tile::hold_b(op_b, nslab));
     }
     core.run(acc, nslab);
     if (!stream) Tile::finish();
@@ -152,7 +151,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
 
       if (STORE_Z) {
         // Raw logits for the backward: VEC consecutive vocabulary entries of a token are one 16-byte piece of
-        // the K-blocked layout.  Vocabulary rows past V hold zeros already (the operand loads are
+        // its unit.  Vocabulary rows past V hold zeros already (the operand loads are
         // range-checked), and the backward ignores whatever the padding columns hold.
         typedef typename KeptLogit<T>::type ZT;
         constexpr int AG = VEC / 4;                     // blocks whose registers make up one piece
@@ -165,7 +164,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
         if (row >= 0) {
           const int64_t n_kslab = p.ldz / Tile::kSlabK;
           char* z_row = static_cast<char*>(p.z_out) +
-                        ((int64_t)(row / kBlockRows) * n_kslab * kBlockRows + row % kBlockRows) * kRowBytes;
+                        ((int64_t)(row / Tile::kSlabK) * n_kslab * Tile::kSlabK + row % Tile::kSlabK) * kRowBytes;
 #pragma unroll
           for (int i = 0; i < MI; i += AG) {
             const int v = v0 + la + Tile::a_block(i);
@@ -173,7 +172,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
             float piece[VEC];
 #pragma unroll
             for (int e = 0; e < VEC; ++e) piece[e] = x[i * 4 + e];
-            *reinterpret_cast<u32x4*>(z_row + (int64_t)(v / Tile::kSlabK) * (kBlockRows * kRowBytes) +
+            *reinterpret_cast<u32x4*>(z_row + (int64_t)(v / Tile::kSlabK) * Tile::kUnitBytes +
                                       (v % Tile::kSlabK) * (int)sizeof(ZT)) = pack_kept(piece, (ZT*)nullptr);
           }
         }

@@ -22,8 +22,7 @@ from . import _lib, ops
 from ._lib import LOSS_GRPO, LOSS_GSPO
 
 
-# Memory one chunk's kept logits may take (they are turned into d(logits) in place; the backward's transposed
-# copy takes as much again).  The bound is on bytes, whatever the hidden size: 35328 rows of a 152k
+# Memory one chunk's kept logits may take (they are turned into d(logits) in place).  The bound is on bytes, whatever the hidden size: 35328 rows of a 152k
 # vocabulary, 41472 rows of a 129k one, in 16-bit elements - a 32768-token micro-batch in one chunk.  Only
 # what a micro-batch needs is allocated.
 DEFAULT_KEEP_LOGITS_BYTES = 10 << 30
@@ -383,7 +382,8 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
 
     ``weight_t_cache``: a dict the caller keeps while ``weight`` does not change (the micro-batches
     of one optimizer step).  The first backward leaves the transposed weight in it and later calls
-    reuse it instead of transposing again; the caller clears it after updating the weight.
+    contract with that one; the caller clears it after updating the weight.  Without it the weight is
+    read as it is, which is as fast and needs no copy.
 
     ``workspace_cache``: a dict the caller keeps between calls.  The kept-logits buffer and the forward /
     backward scratch memory (a few GB, sized by the chunk, not by T) then live in it and are reused by every
@@ -471,7 +471,7 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     if need_dhidden and weight_t_cache is not None:
         wt = weight_t_cache.get("weight_t")
         wt_ready = wt is not None
-    if need_dhidden and wt is None and (n_chunks > 1 or weight_t_cache is not None):
+    if need_dhidden and wt is None and weight_t_cache is not None:
         wt = ops.weight_t_buffer(weight)
     if wt is not None:
         ops.check_weight_t(wt, weight)
@@ -539,7 +539,7 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
             "g_logprob": glp_all, "rows_projected_bwd": rows_projected_bwd,
             "rows_projected_fwd": rows_projected_fwd, "sums": result[:8], "token_chunks": chunks,
             # device memory this call held beyond its inputs and outputs: kept logits (they become d(logits) in
-            # place), the workspace (d(logits)^T, hidden^T, W^T unless the caller's cache holds it, split-K partials;
+            # place), the workspace (hidden^T, split-K partials, the room a W^T would take unless the caller's cache holds one;
             # the forward's per-split records before that), the caller's W^T and the operands of dW that wait in a sum
             "scratch_bytes": sum(t.numel() * t.element_size() for t in (zbuf, ws, wt) if t is not None)
                              + (_dweight_sum.bytes if _dweight_sum is not None else 0)}

@@ -13,8 +13,8 @@ from . import _lib
 from ._lib import BF16, F32, F64, U8, LOSS_GRPO, LOSS_GSPO
 
 # Scratch memory a backward call may take when the caller names neither a chunk nor a workspace: the
-# token chunk is halved until the plan fits (8192 tokens of a 152k vocabulary need 6.5 GB: d(logits) in
-# both orientations, hidden^T, W^T, split-K partials).
+# token chunk is halved until the plan fits (d(logits) where no logits were kept, hidden^T, the room of a
+# W^T, split-K partials).
 DEFAULT_BWD_WORKSPACE_BYTES = 8 << 30
 
 
@@ -71,7 +71,7 @@ def saved_logits_buffer(T: int, V: int, dtype, device) -> torch.Tensor:
     """An (uninitialised) buffer the forward can keep raw logits in for the backward: T rows rounded
     up to whole blocks of 256 by the padded vocabulary extent, elements of the size of ``dtype``.  Its
     contents are opaque (``saved_logits_rowmajor`` decodes them): the forward stores the logits in the
-    layout of the backward's GEMM operands, 16-bit inputs as IEEE half; the backward overwrites them with
+    layout of the backward's GEMM operand, 16-bit inputs as IEEE half; the backward overwrites them with
     d(logits)."""
     return torch.empty(_round_up(max(T, 1), 256), _lib.lib().clgrpo_saved_logits_ld(V), dtype=dtype, device=device)
 
@@ -85,9 +85,12 @@ def _unblock(buf: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
 
 
 def saved_logits_rowmajor(buf: torch.Tensor, rows: int, V: int) -> torch.Tensor:
-    """The first ``rows`` kept rows as an ordinary fp32 [rows, V] tensor (a copy; for inspection and tests):
-    the K-blocked layout of the GEMM operands, 16-bit inputs holding IEEE half."""
-    return _unblock(buf.view(torch.float16) if buf.element_size() == 2 else buf, rows, V).float()
+    """The first ``rows`` kept rows as an ordinary fp32 [rows, V] tensor (a copy; for inspection and tests): square
+    units of 128-byte rows, a row of units after the other, 16-bit inputs holding IEEE half."""
+    buf = buf.view(torch.float16) if buf.element_size() == 2 else buf
+    e = 128 // buf.element_size()
+    n, ld = buf.shape[0] // e, buf.shape[1]
+    return buf.reshape(n, ld // e, e, e).permute(0, 2, 1, 3).reshape(n * e, ld)[:rows, :V].float()
 
 
 def weight_t_buffer(weight: torch.Tensor) -> torch.Tensor:
@@ -249,8 +252,8 @@ def lmhead_backward(hidden, weight, labels, lse, entropy, g_logprob, g_entropy=N
     """(dhidden [T,H] in hidden's dtype, dweight [V,H] fp32).  ``dweight`` may be a caller
     buffer (e.g. the fp32 main-grad) that is overwritten or, with ``accumulate_dweight``, added to.
     ``saved_logits``: the buffer the forward of these rows filled; it is overwritten with d(logits).
-    ``weight_t`` (from ``weight_t_buffer``) keeps W^T between calls that share the weight; pass
-    ``weight_t_ready=True`` once a call has filled it.  ``vocab_begin`` > 0 (or a weight that is a
+    ``weight_t`` (from ``weight_t_buffer``): contract dhidden with a W^T that is kept between calls; pass
+    ``weight_t_ready=True`` once a call has filled it.  Without it W is read as it is, which is as fast.  ``vocab_begin`` > 0 (or a weight that is a
     vocabulary shard starting at 0): ``weight`` holds rows ``[vocab_begin, vocab_begin + V)`` of the full
     matrix, ``labels`` are global ids, ``lse`` / ``entropy`` the merged ones of all shards; ``dweight`` is
     then this shard's rows and ``dhidden`` its partial sum.  ``dweight_dtype`` is that of a new dW (a

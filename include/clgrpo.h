@@ -55,8 +55,10 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *                 dweight_bf16 since 2.04.
  *   3.00 -> 3.01: clgrpo_lmhead_fwd_workspace_bytes never shrinks as T grows (up to 16 MB more for fewer than 64 blocks of
  *                 256 tokens): between 2.03 and 3.00 scratch memory sized for a longer call could be too small for a shorter one.
- *                 clgrpo_head_step refuses what a later stage would refuse (or overrun) before it enqueues anything. */
-#define CLGRPO_VERSION 301
+ *                 clgrpo_head_step refuses what a later stage would refuse (or overrun) before it enqueues anything.
+ *   3.01 -> 3.02: the opaque buffers saved_logits and kept_dzt hold square units (same sizes);
+ *                 clgrpo_lmhead_bwd_workspace_bytes no longer holds a transposed d(logits) (smaller). */
+#define CLGRPO_VERSION 302
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
 
@@ -88,9 +90,9 @@ typedef struct {
                               of sizeof(dtype) bytes.  The forward fills it with logits (16-bit inputs keep them as
                               IEEE half, a raw logit beyond +-65504 as +-65504: the backward's gradients stay
                               finite, but that token's probabilities are then formed from the saturated value), the
-                              backward overwrites it with d(logits), both in the K-blocked layout of the GEMM
-                              operands: element (row, k) at
-                              (((row / 256) * (ld_saved / E) + k / E) * 256 + row % 256) * E + k % E,
+                              backward overwrites it with d(logits), both in square units of 128-byte rows, a row of
+                              units after the other: element (row, k) at
+                              (((row / E) * (ld_saved / E) + k / E) * E + row % E) * E + k % E,
                               E = 128 / sizeof(dtype). */
   int64_t ld_saved;        /* K extent in elements, a multiple of 64, >= clgrpo_saved_logits_ld(V) */
   const int32_t* saved_row_map; /* optional [T]: row of saved_logits that receives token t's logits, or a
@@ -142,9 +144,10 @@ typedef struct {
                                buffer, ceil(T / 256) * 256 rows of ld_saved elements).  Overwritten in place
                                with d(logits); the recomputation is skipped. */
   int64_t ld_saved;
-  void* weight_t;           /* optional, `dtype`: caller-kept W^T in the same blocked layout (ceil(H / 256) * 256
-                               rows of clgrpo_saved_logits_ld(V) elements), so that several calls with the same
-                               weight (token chunks of one step) build it once */
+  void* weight_t;           /* optional, `dtype`: a caller-kept W^T that dhidden is contracted with, ceil(H / 256) * 256
+                               rows of ld = clgrpo_saved_logits_ld(V) elements, element (row, k) at
+                               (((row / 256) * (ld / E) + k / E) * 256 + row % 256) * E + k % E.  NULL: W is read as it is,
+                               which is as fast; nothing is transposed */
   int32_t weight_t_ready;   /* zero: this call fills weight_t; nonzero: it already holds W^T */
   int64_t saved_rows;       /* rows the saved_logits buffer holds; must be >= ceil(T / 256) * 256 (the backward
                                rewrites whole 256-row units) */
@@ -355,9 +358,10 @@ typedef struct {
   void* saved_logits;            /* see clgrpo_lmhead_fwd_args; NULL: the backward recomputes them */
   int64_t ld_saved, saved_rows;  /* saved_rows: at least n_live rounded up to 256 */
   void* weight_t;                /* see clgrpo_lmhead_bwd_args */
-  void* kept_dzt;                /* optional: leave both operands of dW here and compute none; needs saved_logits.  K-blocked
-                                    (see saved_logits of clgrpo_lmhead_fwd_args), rows = V and H rounded up to 256, K =
-                                    kept_ld tokens.  This chunk's rows take the place [kept_k, kept_k + ceil64(n_live)) */
+  void* kept_dzt;                /* optional: leave both operands of dW here and compute none; needs saved_logits.  Opaque: V and
+                                    H, each rounded up to 256, times kept_ld elements of `dtype` (d(logits) in the units of
+                                    saved_logits, hidden^T in the layout of weight_t).  This chunk's rows take the place
+                                    [kept_k, kept_k + ceil64(n_live)) of kept_ld tokens */
   void* kept_hidt;
   int64_t kept_ld, kept_k;       /* multiples of 64 */
 } clgrpo_head_step_args;
@@ -368,12 +372,12 @@ size_t clgrpo_head_step_workspace_bytes(int64_t T, int64_t n_live, int64_t H, in
 int64_t clgrpo_head_step_max_ordered_bytes(void);
 int clgrpo_head_step(const clgrpo_head_step_args* a, void* stream);
 
-/* dW (+)= dzT hidT^T over the operands that clgrpo_head_step calls have kept: one contraction over the tokens of several
+/* dW (+)= d(logits)^T hidden over the operands that clgrpo_head_step calls have kept: one contraction over the tokens of several
  * micro-batches in the place of one per micro-batch, each of which would read and write dW. */
 typedef struct {
   const void* dzt;               /* see kept_dzt, kept_hidt, kept_ld */
   const void* hidt;
-  int64_t ld, k;                 /* tokens per row and how many of them count, multiples of 64 */
+  int64_t ld, k;                 /* tokens they hold and how many of them count, multiples of 64 */
   int64_t H, V;
   int32_t dtype, accumulate;
   void* dweight;                 /* [V, H] out, fp32 or bf16 */
