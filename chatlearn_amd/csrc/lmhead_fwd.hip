@@ -85,6 +85,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
 
   const int lane = threadIdx.x & 63;
   const int wm = Tile::wave_m(), wn = Tile::wave_n();
+  const int wm_u = __builtin_amdgcn_readfirstlane(wm);
   const int la = wm + Tile::lane_a0();               // this lane's first vocabulary row / token of the tile
   const int lb = wn + Tile::lane_b0();
   const int t0 = tb * kFwdBN;
@@ -140,6 +141,9 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
     if (!stream) Tile::finish();
 
     const bool full = a_rows == kFwdBM;
+    // this wave's first unit of the tile, and this lane's piece in it
+    char* z_tile = static_cast<char*>(p.z_out) + (int64_t)((v0 + wm_u) / Tile::kSlabK) * Tile::kUnitBytes;
+    const int z_lane = Tile::lane_a0() * (int)sizeof(typename KeptLogit<T>::type);
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       // this token's logits of the lane's vocabulary rows
@@ -157,23 +161,22 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
         constexpr int AG = VEC / 4;                     // blocks whose registers make up one piece
         // The row is the same for every vocabulary tile, so the compiler would keep the 64-bit addresses it
         // forms from it alive across the K loops, where registers are scarcest, spill them, and reload them
-        // between the stores (a reload waits for the stores issued before it).  Re-deriving them from the
-        // 32-bit row costs a handful of instructions per tile.
+        // between the stores (a reload waits for the stores issued before it).  Re-deriving one from the 32-bit row
+        // costs a handful of instructions per tile; the pieces lie at constants from it (with an address of its own
+        // per piece, some 20 instructions each, 16384 tokens at H = 2048 took 7.55 ms for 7.44).
         int row = zrow[j];
         asm volatile("" : "+v"(row));
         if (row >= 0) {
-          const int64_t n_kslab = p.ldz / Tile::kSlabK;
-          char* z_row = static_cast<char*>(p.z_out) +
-                        ((int64_t)(row / Tile::kSlabK) * n_kslab * Tile::kSlabK + row % Tile::kSlabK) * kRowBytes;
+          const uint64_t unit_row = (uint64_t)(p.ldz / Tile::kSlabK) * Tile::kUnitBytes;
+          char* z_row = z_tile + (uint64_t)(uint32_t)(row / Tile::kSlabK) * unit_row + (row % Tile::kSlabK * kRowBytes + z_lane);
 #pragma unroll
           for (int i = 0; i < MI; i += AG) {
-            const int v = v0 + la + Tile::a_block(i);
-            if (!full && v >= p.ldz) continue;
+            if (!full && v0 + wm_u + Tile::a_block(i) / 32 * 32 >= p.ldz) continue;     // the same for all lanes
             float piece[VEC];
 #pragma unroll
             for (int e = 0; e < VEC; ++e) piece[e] = x[i * 4 + e];
-            *reinterpret_cast<u32x4*>(z_row + (int64_t)(v / Tile::kSlabK) * Tile::kUnitBytes +
-                                      (v % Tile::kSlabK) * (int)sizeof(ZT)) = pack_kept(piece, (ZT*)nullptr);
+            *reinterpret_cast<u32x4*>(z_row + Tile::a_block(i) / Tile::kSlabK * Tile::kUnitBytes +
+                                      Tile::a_block(i) % Tile::kSlabK * (int)sizeof(ZT)) = pack_kept(piece, (ZT*)nullptr);
           }
         }
       }
