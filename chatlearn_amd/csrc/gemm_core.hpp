@@ -2,7 +2,7 @@
 // way round, fp32 accumulation on the matrix cores.
 //
 // One workgroup of 2 x 2 wavefronts (64 lanes each, one per SIMD of a CU) owns a 256 x 256 tile; a wave
-// owns 128 x 128 of it as 8 x 8 blocks of 16 x 16.  K is walked in slabs of 128 bytes per row (64 bf16 or 32
+// owns 128 x 128 of it as 8 x 8 blocks of 16 x 16 (narrower along B: 8 x kNI).  K is walked in slabs of 128 bytes per row (64 bf16 or 32
 // fp32 elements), each slab in two halves of 64 bytes.
 //
 // What bounds it: on random operands the chip runs at its power limit (the shader clock settles at 1.5 -
@@ -86,7 +86,7 @@ template <typename T> struct KeptLogit;
 template <> struct KeptLogit<__bf16> { typedef _Float16 type; };
 template <> struct KeptLogit<float> { typedef float type; };
 
-// Matrix instructions of slot m (0 .. 63) of a slab half: 64 bytes of K of block (i, j) = (m / 8, m % 8), odd
+// Matrix instructions of slot m of a slab half: 64 bytes of K of block (i, j) = (m / NI, m % NI), odd
 // rows walked backwards so that neighbours share an operand.  Written as assembly because that is what ties the
 // accumulators to the accumulation registers: left to itself the compiler moves all 256 of them between the
 // register files around every loop, and spills what is in their way.  The compiler does not see the
@@ -94,9 +94,9 @@ template <> struct KeptLogit<float> { typedef float type; };
 // acc_get / acc_set for the same reason.
 template <typename T> struct Mma;
 template <> struct Mma<__bf16> {
-  template <bool kAcross = false>
-  __device__ static __forceinline__ void slot(f32x4 (&acc)[8][8], const u32x4 (&a)[8], const u32x4 (&b)[8], int m) {
-    const int i = m / 8, j = (i & 1) ? 7 - m % 8 : m % 8;
+  template <bool kAcross, int NI>
+  __device__ static __forceinline__ void slot(f32x4 (&acc)[8][NI], const u32x4 (&a)[8], const u32x4 (&b)[NI], int m) {
+    const int i = m / NI, j = (i & 1) ? NI - 1 - m % NI : m % NI;
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(a[i]), "v"(b[j]));
   }
 };
@@ -105,8 +105,9 @@ template <> struct Mma<float> {
   // step m % 8 / 2 of four blocks of row i, so that an accumulator comes up again eight instructions later.
   // kAcross: a[4 q + e] holds k = 4g + e of the four blocks 4 q .. 4 q + 3 (an A with K along its rows): the
   // transposition of a 4 x 4 square of single registers is a choice of registers.
-  template <bool kAcross = false>
-  __device__ static __forceinline__ void slot(f32x4 (&acc)[8][8], const u32x4 (&a)[8], const u32x4 (&b)[8], int m) {
+  template <bool kAcross, int NI>
+  __device__ static __forceinline__ void slot(f32x4 (&acc)[8][NI], const u32x4 (&a)[8], const u32x4 (&b)[NI], int m) {
+    static_assert(NI == 8, "four blocks of a row per slot");
     const int i = m / 8, e = m % 8 / 2;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -154,11 +155,13 @@ __device__ __forceinline__ void each(Fn fn) { each(fn, std::make_integer_sequenc
 // d(logits) pass, 256 rows at H = 4096: 471 -> 312 us, 32 rows 271 -> 242).
 enum class Side { kRows, kWeight, kLogits };
 
-// BV: consecutive B rows a lane holds (see above), 8 or 4.  kUnitsB: B is d(logits) in units (see unit_index).
-template <typename T, int BV, Side kSideA = Side::kRows, bool kUnitsB = false>
+// BV: consecutive B rows a lane holds (see above).  kUnitsB: B is d(logits) in units (see unit_index).  kNI: 16 x 16 blocks per
+// wave along B, so a tile is 32 kNI rows of B wide: 256, or less where whole tiles of 256 would be mostly padding.
+template <typename T, int BV, Side kSideA = Side::kRows, bool kUnitsB = false, int kNI = 8>
 struct GemmTile {
-  static constexpr int BM = 256, BN = 256, WM = 128, WN = 128;
-  static constexpr int MI = 8, NI = 8;                 // 16 x 16 blocks per wave along A / B
+  static constexpr int MI = 8, NI = kNI;               // 16 x 16 blocks per wave along A / B
+  static constexpr int BM = 256, BN = 32 * NI, WM = 128, WN = 16 * NI;
+  static constexpr int kSlots = MI * NI;               // matrix instructions of half a slab
   static constexpr int kThreads = 256;
   static constexpr int kSlotBytes = 256 * kRowBytes;   // one operand's slab
   static constexpr int kASlots = 3, kBSlots = 2;
@@ -171,7 +174,8 @@ struct GemmTile {
   static constexpr int kUnitBytes = kSlabK * kRowBytes;     // a unit of d(logits); a piece of a slab read across
   static constexpr int kSub = 256 / kSlabK;                 // of them per 256-wide slab
   static constexpr uint32_t kHalf = kAcross ? (uint32_t)kUnitBytes / 2 : 64u;   // from a slab's first half to its second in LDS
-  static_assert(BV == 8 || BV == 4, "B rows per lane");
+  static_assert(NI % BV == 0 && NI >= 4 && NI <= 8, "B rows per lane");
+  static_assert(!kUnitsB || BN % 64 == 0, "a tile of d(logits) is whole units");
 
   typedef f32x4 Acc[MI][NI];
   typedef __attribute__((address_space(3))) char lds_char;
@@ -200,13 +204,14 @@ struct GemmTile {
   // one bank).  In lanes (c, g): eight c's of lane group g and the other eight of g + 1.  These sixteen must fall on
   // eight chunks of either parity of rows.
   //   A rows: the swizzle of a row's chunks is enough, its rows differ in parity.
-  //   B rows (row BV c + j): all of one parity, so rows are exchanged in pairs where c is odd (b_row), and the chunks
+  //   B rows (row BV c + j): all of one parity (BV even), so rows are exchanged in pairs where c is odd (b_row), and the chunks
   //     are swizzled by the rest of c.  Without the exchange every B read took 4 cycles more (half of SQ_LDS_BANK_CONFLICT per read).
   //   A across: chunks of one row over two pieces of a slab; the odd pieces have their rows exchanged in pairs.
   // A lane reads an exchanged row at the other address of its pair: odd rows go by addresses of their own (odd_a, odd_b).
   __device__ static __forceinline__ int a_swz(int row) { return VEC == 8 ? (row & 3) | ((row >> 3) & 1) << 2 : row & 7; }
   __device__ static __forceinline__ int b_swz(int row) { return row / (2 * BV) & 7; }
-  __device__ static __forceinline__ int b_row(int row) { return row ^ (row / BV & 1); }     // its own inverse
+  static constexpr int kPairs = BV % 2 == 0;           // an odd BV gives its rows both parities by itself
+  __device__ static __forceinline__ int b_row(int row) { return row ^ (row / BV & kPairs); }     // its own inverse
 
   // Where an operand's tile lives in memory: `rows` valid rows starting at `base`, consecutive
   // rows `row_bytes` apart, consecutive 128-byte K slabs of a row `slab_bytes` apart.
@@ -268,7 +273,7 @@ struct GemmTile {
   Cursor a, b, next_a, next_b;
   __amdgpu_buffer_rsrc_t rsrc_a, rsrc_b;
   const char* unit_b;                         // this slab's unit of the next load
-  int voff_a[8], voff_b[8];
+  int voff_a[8], voff_b[NI];
   u32x4 raw[8];                               // kPerm: a half of A as it is read
   u32x4 af[2][MI], bf[2][NI];
   uint32_t a0, b0;                            // this lane's fragment addresses in slot 0 of either ring, first half of a slab
@@ -286,7 +291,7 @@ struct GemmTile {
     if constexpr (kUnitsB) { next_unit(0, 0); next_unit(1, 0); }
     else rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(b.p), 0, b.bytes, 0x00020000);
   }
-  // Load p (0 .. 7) of the slab at the cursor: 8 rows per wave, 32 per workgroup (across: 8 rows of one piece).
+  // Load p (0 .. 7, of B 0 .. NI - 1) of the slab at the cursor: 8 rows per wave, 32 per workgroup (across: 8 rows of one piece).
   __device__ __forceinline__ void load_a(int p) {
     if constexpr (kAcross)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_char*)(uintptr_t)(w0 + da + p * 4096), 16, voff_a[p], 0, 0, 0);
@@ -301,9 +306,9 @@ struct GemmTile {
   __device__ __forceinline__ void load_b(int p, uint32_t slot) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_char*)(uintptr_t)(w0 + kBB + slot + p * 4096), 16, voff_b[p], 0, 0, 0);
   }
-  __device__ __forceinline__ void load_b(uint32_t slot) {
+  __device__ __forceinline__ void load_slab_b(uint32_t slot) {
 #pragma unroll
-    for (int p = 0; p < 8; ++p) {
+    for (int p = 0; p < NI; ++p) {
       if (kUnitsB && p > 0 && p % kUnitLoads == 0) { next_unit(0, p / kUnitLoads); next_unit(1, p / kUnitLoads); }
       load_b(p, slot);
     }
@@ -345,7 +350,7 @@ struct GemmTile {
   __device__ __forceinline__ void read_b(int set, uint32_t pb, int j) {
     bf[set][j] = *(lds_vec*)(uintptr_t)((j % 2 ? pb + odd_b : pb) + b_block(j) * kRowBytes);
   }
-  // Fragment read n (0 .. 15) of a half: the first A fragment, all of B, the rest of A; across: all of A, all of B.
+  // Fragment read n (0 .. MI + NI - 1) of a half: the first A fragment, all of B, the rest of A; across: all of A, all of B.
   __device__ __forceinline__ void read(int set, uint32_t pa, uint32_t pb, int n) {
     if constexpr (kAcross) {
       if (n >= MI) read_b(set, pb, n - MI);
@@ -434,7 +439,7 @@ struct GemmTile {
       voff_a[0] = row * A.row_bytes + (chunk ^ a_swz(row)) * 16;
     }
 #pragma unroll
-    for (int p = 0; p < 8; ++p) {
+    for (int p = 0; p < NI; ++p) {
       const int r = b_row(row + 32 * p);
       const int off = kUnitsB ? r % kSlabK * kRowBytes
                               : (b_order == nullptr ? r * B.row_bytes : (r < b_rows ? b_order[r] * B.row_bytes : 0x7fffff00));
@@ -449,15 +454,15 @@ struct GemmTile {
     } else {
       a0 = lds + (wave_m() + fa) * kRowBytes + (g ^ a_swz(fa)) * 16;
     }
-    b0 = lds + kBB + (wave_n() + fb + (c & 1)) * kRowBytes + (g ^ b_swz(fb)) * 16;
-    odd_b = -2 * (c & 1) * kRowBytes;
+    b0 = lds + kBB + (wave_n() + fb + (c & kPairs)) * kRowBytes + (g ^ b_swz(fb)) * 16;
+    odd_b = -2 * (c & kPairs) * kRowBytes;
     a = cursor_a(A, nslab); b = cursor_b(B, nslab);
     follow(A, B, nslab, hold_a(A, nslab), hold_b(B, nslab));
     make_a(); make_b();
     da = sa = sb = 0;
 #pragma unroll
     for (int p = 0; p < 8; ++p) load_a(p);
-    load_b(0u);
+    load_slab_b(0);
     step_a(); step_b(); make_a(); make_b(); da = kSlotBytes;
 #pragma unroll
     for (int p = 0; p < 8; ++p) load_a(p);
@@ -465,12 +470,12 @@ struct GemmTile {
     __builtin_amdgcn_s_waitcnt(0x0F78);    // all but the youngest eight loads
     __syncthreads();
 #pragma unroll
-    for (int n = 0; n < 16; ++n) read(0, a0, b0, n);
+    for (int n = 0; n < MI + NI; ++n) read(0, a0, b0, n);
     if constexpr (kPerm) {
 #pragma unroll
       for (int n = 0; n < 4 * MI; ++n) perm(0, n);
     }
-    load_b((uint32_t)kSlotBytes);
+    load_slab_b(kSlotBytes);
   }
 
   // The schedule of a half of a slab: 64 slots of one matrix instruction (fp32: four) each.  It takes 16 cycles and its issue 4, so
@@ -478,40 +483,49 @@ struct GemmTile {
   // instructions with up to nine scalar ones in a slot were 5 % slower in the contraction that has the most of them.  Fragment
   // reads take even slots of the first 32, a load every eighth (three instructions by itself, its LDS address goes through
   // m0), scalar steps the odd slots left over, the second 32 slots the transposition.  Loads every 4 or 6 slots: no faster.
-  static constexpr int load_at(int m) { return m % 8 == 1 ? m / 8 : -1; }
+  // (Narrower tiles keep the same order in fewer slots; A's loads then come every NI.)
+  static constexpr int load_a_at(int m) { return m % NI == 1 ? m / NI : -1; }
+  static constexpr int load_b_at(int m) { return m % 8 == 1 ? m / 8 : -1; }
   static constexpr int unit_at(int m) {                // unit that begins with slot m's load of B
-    return kUnitsB && load_at(m) > 0 && load_at(m) % kUnitLoads == 0 ? load_at(m) / kUnitLoads : -1;
+    return kUnitsB && load_b_at(m) > 0 && load_b_at(m) < NI && load_b_at(m) % kUnitLoads == 0 ? load_b_at(m) / kUnitLoads : -1;
   }
-  static constexpr int step_at(int m, bool units) {    // scalar step of slot m; a unit's descriptor is made in the two slots before its load
-    if (m % 2 == 0 || load_at(m) >= 0 || (units && unit_at(m + 2) > 0)) return -1;
+  static constexpr bool spare(int h, int m) {          // odd, without a load; a unit's descriptor is made in the two slots before its load
+    return m % 2 == 1 && (h == 0 ? load_a_at(m) < 0 : load_b_at(m) < 0 && unit_at(m + 2) <= 0);
+  }
+  static constexpr int step_at(int h, int m) {         // scalar step of slot m
+    if (!spare(h, m)) return -1;
     int n = 0;
-    for (int k = 1; k < m; k += 2) n += load_at(k) < 0 && !(units && unit_at(k + 2) > 0);
+    for (int k = 1; k < m; k += 2) n += spare(h, k);
     return n;
   }
-  static constexpr int perm_from(int m) {              // registers transposed in front of slot m: none behind a load, two in the first slots
+  static constexpr int perm_from(int h, int m) {       // registers transposed in front of slot m: none behind a load, two in the first slots
+    constexpr int first = NI == 8 ? 32 : NI == 6 ? 24 : 18;
+    if (m <= first) return 0;
+    if (NI < 8) return 4 * MI * (m - first) / (kSlots - first);
     int n = 0, twice = 4;
-    for (int k = 32; k < m; ++k)
-      if (load_at(k) < 0) n += twice > 0 ? (--twice, 2) : 1;
+    for (int k = first; k < m; ++k)
+      if ((h == 0 ? load_a_at(k) : load_b_at(k)) < 0) n += twice > 0 ? (--twice, 2) : 1;
     return n;
   }
 
   // One tile's K loop of `nslab` slabs; acc must be initialised by the caller.  Between tiles of a
   // streaming workgroup LDS stays in use; after the last one call finish() before touching it.
   __device__ __forceinline__ void run(Acc& acc, int nslab) {
+#ifdef __HIP_DEVICE_COMPILE__      // the host's pass drops kernels whose body holds this many lambdas, without a word
     settle();
     for (int s = 0; s < nslab; ++s) {
-      each<MI * NI>([&](auto c) __attribute__((always_inline)) {            // first half of the slab
-        constexpr int m = decltype(c)::value, n = step_at(m, false);
-        Mma<T>::template slot<kAcross>(acc, af[0], bf[0], m);
+      each<kSlots>([&](auto c) __attribute__((always_inline)) {            // first half of the slab
+        constexpr int m = decltype(c)::value, n = step_at(0, m);
+        Mma<T>::template slot<kAcross, NI>(acc, af[0], bf[0], m);
         fence();
-        if constexpr (m % 2 == 0 && m < 32) { read(1, half_a() + sa, (b0 ^ 64) + sb, m / 2); fence(); }
-        if constexpr (load_at(m) >= 0) { load_a(load_at(m)); fence(); }
+        if constexpr (m % 2 == 0 && m < 2 * (MI + NI)) { read(1, half_a() + sa, (b0 ^ 64) + sb, m / 2); fence(); }
+        if constexpr (load_a_at(m) >= 0) { load_a(load_a_at(m)); fence(); }
         if constexpr (n >= 0 && n < kSteps) { step_b(n); fence(); }
         if constexpr (n == kSteps) { make_b(); fence(); }
         if constexpr (n == kSteps + 1) { sa1 = next_slot(sa); fence(); }
         if constexpr (kPerm) {
 #pragma unroll
-          for (int k = perm_from(m); k < perm_from(m + 1); ++k) { perm(1, k); fence(); }
+          for (int k = perm_from(0, m); k < perm_from(0, m + 1); ++k) { perm(1, k); fence(); }
         }
       });
       fence();
@@ -519,12 +533,12 @@ struct GemmTile {
       __builtin_amdgcn_s_waitcnt(0x0078);
       __builtin_amdgcn_s_barrier();
       fence();
-      each<MI * NI>([&](auto c) __attribute__((always_inline)) {            // second half, while the next slab's first fragments come in
-        constexpr int m = decltype(c)::value, n = step_at(m, kUnitsB);
-        Mma<T>::template slot<kAcross>(acc, af[1], bf[1], m);
+      each<kSlots>([&](auto c) __attribute__((always_inline)) {            // second half, while the next slab's first fragments come in
+        constexpr int m = decltype(c)::value, n = step_at(1, m);
+        Mma<T>::template slot<kAcross, NI>(acc, af[1], bf[1], m);
         fence();
-        if constexpr (m % 2 == 0 && m < 32) { read(0, a0 + sa1, b0 + (sb ^ kSlotBytes), m / 2); fence(); }
-        if constexpr (load_at(m) >= 0) { load_b(load_at(m), sb); fence(); }
+        if constexpr (m % 2 == 0 && m < 2 * (MI + NI)) { read(0, a0 + sa1, b0 + (sb ^ kSlotBytes), m / 2); fence(); }
+        if constexpr (load_b_at(m) >= 0) { load_b(load_b_at(m), sb); fence(); }
         if constexpr (unit_at(m + 2) > 0) { next_unit(0, unit_at(m + 2)); fence(); }
         if constexpr (unit_at(m + 1) > 0) { next_unit(1, unit_at(m + 1)); fence(); }
         if constexpr (n >= 0 && n < kSteps) { step_a(n); fence(); }
@@ -532,12 +546,13 @@ struct GemmTile {
         if constexpr (n == kSteps + 1) { da = next_slot(da); fence(); }
         if constexpr (kPerm) {
 #pragma unroll
-          for (int k = perm_from(m); k < perm_from(m + 1); ++k) { perm(0, k); fence(); }
+          for (int k = perm_from(1, m); k < perm_from(1, m + 1); ++k) { perm(0, k); fence(); }
         }
       });
       sa = sa1; sb ^= kSlotBytes;
     }
     settle();
+#endif
   }
 
   __device__ __forceinline__ uint32_t half_a() const { return kAcross ? a0 + kUnitBytes / 2 : a0 ^ 64; }
@@ -569,8 +584,8 @@ struct GemmTile {
 };
 
 constexpr int kHeadThreads = 256;
-// The tile of the kernels that hold logits (A = vocabulary, B = tokens): a lane's 16-byte pieces run along either.
-template <typename T> using LogitTile = GemmTile<T, 16 / (int)sizeof(T)>;
+// The tile of the kernels that hold logits (A = vocabulary, B = tokens).
+template <typename T, int NI = 8> using LogitTile = GemmTile<T, NI, Side::kRows, false, NI>;
 
 // Workgroup id -> logical work item so that the workgroups resident on one XCD
 // (hardware deals consecutive ids round-robin over the 8 XCDs) own a contiguous

@@ -243,7 +243,7 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams p) {
 //   dhidden (kMContig): C[n][m], ld = ldc, A = W^T (kWeight: W itself; kRows: the caller's K-blocked W^T), B = dz (in
 //     units).  A lane holds VEC consecutive m of a row, the 4 lane groups 64 contiguous bytes of each of 16 rows for 16-bit results.
 template <Side S> constexpr bool kMContig = S != Side::kLogits;
-template <typename T, Side S> using OutTile = GemmTile<T, kMContig<S> ? 16 / (int)sizeof(T) : 4, S, kMContig<S>>;
+template <typename T, Side S, int NI = 8> using OutTile = GemmTile<T, kMContig<S> ? NI : 4, S, kMContig<S>, NI>;
 
 struct GemmParams {
   const void* A;
@@ -270,9 +270,9 @@ struct GemmParams {
 // of them give 0 and stores are dropped.  Along the register dimension (m) nothing relies on the range check:
 // kMContig skips whole 32-row groups (its M extents are multiples of 32), and the other orientation tests
 // every row against the tile's valid rows unless the tile is a full one.
-template <typename T, typename OutT, Side S>
+template <typename T, typename OutT, Side S, int NI>
 struct TileAddr {
-  using Tile = OutTile<T, S>;
+  using Tile = OutTile<T, S, NI>;
   static constexpr bool kMContig = clgrpo::kMContig<S>;
   static constexpr int ES = (int)sizeof(OutT);
   static constexpr int kPieces = Tile::MI * 4 / Tile::VEC;  // kMContig: runs of VEC consecutive m per lane and block j
@@ -343,10 +343,10 @@ __device__ __forceinline__ void row_store(const float (&x)[4], const __amdgpu_bu
 
 // fn(values of one run of a row, per-lane offset, scalar offset), for every run of the tile that lies inside it;
 // kLoad (dW only): the values go into the accumulators afterwards.
-template <typename T, typename OutT, Side S, bool kLoad, typename AccT, typename Fn>
-__device__ __forceinline__ void for_rows(const TileAddr<T, OutT, S>& at, AccT& acc, Fn fn) {
-  using Tile = OutTile<T, S>;
-  using Addr = TileAddr<T, OutT, S>;
+template <typename T, typename OutT, Side S, int NI, bool kLoad, typename AccT, typename Fn>
+__device__ __forceinline__ void for_rows(const TileAddr<T, OutT, S, NI>& at, AccT& acc, Fn fn) {
+  using Tile = OutTile<T, S, NI>;
+  using Addr = TileAddr<T, OutT, S, NI>;
   if constexpr (kMContig<S>) {
     static_assert(!kLoad, "dhidden is never added to");
 #pragma unroll
@@ -386,39 +386,39 @@ __device__ __forceinline__ void for_rows(const TileAddr<T, OutT, S>& at, AccT& a
 // workgroup owns the whole K range of the tile - the tile's current contents.  Reading C here instead of
 // in the epilogue puts the loads' latency in front of the K loop, where the first operand slabs are in
 // flight anyway, and leaves the epilogue a pure store.
-template <typename T, typename OutT, Side S>
-__device__ __forceinline__ void gemm_init_tile(const GemmParams& p, typename OutTile<T, S>::Acc& acc, int m0, int n0,
+template <typename T, typename OutT, Side S, int NI>
+__device__ __forceinline__ void gemm_init_tile(const GemmParams& p, typename OutTile<T, S, NI>::Acc& acc, int m0, int n0,
                                                int a_rows, int b_rows) {
   constexpr bool kAdds = !kMContig<S> && sizeof(OutT) == 4;    // only an fp32 C is ever added to
-  if (!kAdds || !p.accumulate || p.k_split > 1) OutTile<T, S>::zero(acc);
+  if (!kAdds || !p.accumulate || p.k_split > 1) OutTile<T, S, NI>::zero(acc);
   if constexpr (kAdds) {
     if (!p.accumulate || p.k_split > 1) return;
-    const TileAddr<T, OutT, S> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows);
-    for_rows<T, OutT, S, true>(at, acc, [&](auto& x, int voff, int soff) { row_load(x, at.rsrc, voff, soff, (OutT*)nullptr); });
+    const TileAddr<T, OutT, S, NI> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows);
+    for_rows<T, OutT, S, NI, true>(at, acc, [&](auto& x, int voff, int soff) { row_load(x, at.rsrc, voff, soff, (OutT*)nullptr); });
   }
 }
 
 // Output tile from the accumulators: C = acc (the accumulators already hold C's previous contents
 // when the GEMM adds to it, see gemm_init_tile), or the fp32 partial of K range `ks`.
-template <typename T, typename OutT, Side S>
-__device__ __forceinline__ void gemm_store_tile(const GemmParams& p, typename OutTile<T, S>::Acc& acc, int m0, int n0,
+template <typename T, typename OutT, Side S, int NI>
+__device__ __forceinline__ void gemm_store_tile(const GemmParams& p, typename OutTile<T, S, NI>::Acc& acc, int m0, int n0,
                                                 int a_rows, int b_rows, int ks) {
   if (p.k_split > 1) {
-    const TileAddr<T, float, S> at(p.partial + (int64_t)ks * p.M * p.N, kMContig<S> ? p.M : p.N, m0, n0, a_rows, b_rows);
-    for_rows<T, float, S, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (float*)nullptr); });
+    const TileAddr<T, float, S, NI> at(p.partial + (int64_t)ks * p.M * p.N, kMContig<S> ? p.M : p.N, m0, n0, a_rows, b_rows);
+    for_rows<T, float, S, NI, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (float*)nullptr); });
     return;
   }
-  const TileAddr<T, OutT, S> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows, p.order, p.total);
-  for_rows<T, OutT, S, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (OutT*)nullptr); });
+  const TileAddr<T, OutT, S, NI> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows, p.order, p.total);
+  for_rows<T, OutT, S, NI, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (OutT*)nullptr); });
 }
 
 // Work item = (walk, fixed tile) when n_walk > 0: the workgroup keeps one operand's tile (A's m tile
 // when C is [n][m], B's n tile when C is [m][n]) and walks a contiguous run of tiles of the other, so the
 // K loops stream into each other (the next tile's first slabs are requested while the current tile
 // finishes and is stored).  Otherwise work item = (K range, m tile, n tile), one K loop per workgroup.
-template <typename T, typename OutT, Side S>
+template <typename T, typename OutT, Side S, int NI>
 __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
-  using Tile = OutTile<T, S>;
+  using Tile = OutTile<T, S, NI>;
   constexpr bool kMC = kMContig<S>;
   constexpr int E = Tile::kSlabK;
   constexpr int64_t kSlabElems = (int64_t)kBlockRows * E;   // elements of a K-blocked block's slab, and of a 256-wide row of units
@@ -457,27 +457,27 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
     else return Tile::Operand::across_units(A + s0 * p.a_step * (E * E) + m_tile * kSlabElems, p.a_step, rows);
   };
   auto operand_b = [&](int n_tile, int rows) {
-    if constexpr (kMC) return Tile::Operand::units(B + (n_tile * (int64_t)(256 / E) * p.b_step + s0) * (E * E), p.b_step, rows);
+    if constexpr (kMC) return Tile::Operand::units(B + (n_tile * (int64_t)(Tile::BN / E) * p.b_step + s0) * (E * E), p.b_step, rows);
     else return Tile::Operand::blocked(B + ((int64_t)n_tile * p.b_step + s0) * kSlabElems, rows);
   };
-  auto rows_of = [](int total, int tile) { const int left = total - tile * 256; return left < 256 ? left : 256; };
+  auto rows_of = [](int total, int tile, int width) { const int left = total - tile * width; return left < width ? left : width; };
   typename Tile::Acc acc;
   Tile core;
   for (int k = 0; k < count; ++k) {
-    const int m0 = mt * 256, n0 = nt * 256;
-    const int a_rows = rows_of(p.M, mt), b_rows = rows_of(p.N, nt);
+    const int m0 = mt * 256, n0 = nt * Tile::BN;
+    const int a_rows = rows_of(p.M, mt, 256), b_rows = rows_of(p.N, nt, Tile::BN);
     const auto op_a = operand_a(mt, a_rows);
     const auto op_b = operand_b(nt, b_rows);
-    gemm_init_tile<T, OutT, S>(p, acc, m0, n0, a_rows, b_rows);
+    gemm_init_tile<T, OutT, S, NI>(p, acc, m0, n0, a_rows, b_rows);
     if (k == 0 || !stream) core.start(op_a, op_b, nslab, lds);
     if (stream && k + 1 < count)
-      core.follow(op_a, op_b, nslab, Tile::cursor_a(kMC ? op_a : operand_a(mt + 1, rows_of(p.M, mt + 1)), nslab),
-                  Tile::cursor_b(kMC ? operand_b(nt + 1, rows_of(p.N, nt + 1)) : op_b, nslab));
+      core.follow(op_a, op_b, nslab, Tile::cursor_a(kMC ? op_a : operand_a(mt + 1, rows_of(p.M, mt + 1, 256)), nslab),
+                  Tile::cursor_b(kMC ? operand_b(nt + 1, rows_of(p.N, nt + 1, Tile::BN)) : op_b, nslab));
     else
       core.follow(op_a, op_b, nslab, Tile::hold_a(op_a, nslab), Tile::hold_b(op_b, nslab));
     core.run(acc, nslab);
     if (!stream || k + 1 == count) Tile::finish();
-    gemm_store_tile<T, OutT, S>(p, acc, m0, n0, a_rows, b_rows, ks);
+    gemm_store_tile<T, OutT, S, NI>(p, acc, m0, n0, a_rows, b_rows, ks);
     if (kMC) ++nt; else ++mt;
   }
 }
@@ -583,10 +583,15 @@ struct DhPlan {
   int bulk_nt;       // n tiles (256 token rows each) of the bulk launch; 0: one launch over all rows
   int k_split;       // K ranges of the single launch, or of the tail launch when bulk_nt > 0
   size_t partial_bytes;
+  int ni;            // the single launch's tiles are 32 * ni rows wide
 };
 
+// Narrower row tiles (16-bit operands, a single launch): where 256-row ones would be padding or too few, as in the
+// forward's fwd_plan; whole units of 64 rows, so 192 or 128.
+// dhidden and the d(logits) pass, us: H = 4096, V = 151936: 128 rows 267 -> 260, 320 469 -> 409, 384 478 -> 422; H = 2048: 320
+// 260 -> 235; H = 1024, V = 32000: 32 rows 36 -> 28, 200 45 -> 37, 320 53 -> 49.
 static DhPlan plan_dhidden(int64_t rows, int64_t H, int64_t K, int slab, int cus, size_t partial_cap) {
-  DhPlan pl{0, 1, 0};
+  DhPlan pl{0, 1, 0, 8};
   if (rows <= 0) return pl;
   const int n_mt = (int)((H + 255) / 256), n_nt = (int)((rows + 255) / 256);
   const int tiles = n_mt * n_nt;
@@ -613,7 +618,13 @@ static DhPlan plan_dhidden(int64_t rows, int64_t H, int64_t K, int slab, int cus
       return pl;
     }
   }
-  pl.partial_bytes = s_one > 1 ? (size_t)s_one * rows * H * sizeof(float) : 0;
+  for (int ni = 6; slab == 64 && ni >= 4; ni -= 2) {
+    const int t = n_mt * (int)((rows + 32 * ni - 1) / (32 * ni));
+    const int s = pick_k_split(t, (int)H, (int)rows, (int)K, slab, partial_cap, cus);
+    const double c = ni / 8.0 * (1.0 + 0.02 * (8 - ni)) * cost(t, s);
+    if (c < (pl.ni == 8 ? 0.96 : 1.0) * best) { best = c; pl.ni = ni; pl.k_split = s; }
+  }
+  pl.partial_bytes = pl.k_split > 1 ? (size_t)pl.k_split * rows * H * sizeof(float) : 0;
   return pl;
 }
 
@@ -741,17 +752,17 @@ struct GemmIn {
   int k_valid;
 };
 
-template <typename T, typename OutT, Side S>
+template <typename T, typename OutT, Side S, int NI = 8>
 static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64_t ldc, int accumulate, hipStream_t stream,
                            float* partial, size_t partial_bytes, int k_split_wanted, const RowOrder& rows = RowOrder{nullptr, 0}) {
-  using Tile = OutTile<T, S>;
+  using Tile = OutTile<T, S, NI>;
   constexpr bool kMC = kMContig<S>;
-  int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_kernel<T, OutT, S>), Tile::kLdsBytes, "gemm_kernel");
+  int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_kernel<T, OutT, S, NI>), Tile::kLdsBytes, "gemm_kernel");
   if (rc) return rc;
   GemmParams g;
   g.A = in.A; g.B = in.B; g.C = C; g.a_step = in.a_step; g.b_step = in.b_step; g.ldc = ldc; g.k_valid = in.k_valid;
   g.M = M; g.N = N; g.K = K;
-  g.n_mt = (M + 255) / 256; g.n_nt = (N + 255) / 256;
+  g.n_mt = (M + 255) / 256; g.n_nt = (N + Tile::BN - 1) / Tile::BN;
   g.accumulate = accumulate;
   g.order = rows.order; g.total = rows.total;
   const int slab = Tile::kSlabK;
@@ -780,7 +791,7 @@ static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64
     if (walk_periods * 100 > plain_rounds * 104) g.n_walk = 0;
   }
   int grid = ((g.n_walk > 0 ? g.n_walk * n_fixed : g.n_mt * g.n_nt * g.k_split) + 7) / 8 * 8;
-  hipLaunchKernelGGL((gemm_kernel<T, OutT, S>), dim3(grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
+  hipLaunchKernelGGL((gemm_kernel<T, OutT, S, NI>), dim3(grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
   rc = check_launch("gemm_kernel");
   if (rc || g.k_split == 1) return rc;
   return launch_splitk_reduce<OutT>(partial, g.k_split, kMC ? N : M, kMC ? M : N, static_cast<OutT*>(C), ldc, accumulate,
@@ -794,6 +805,10 @@ static int launch_dhidden(const GemmIn& in, int M, int N, int K, void* C, int64_
   constexpr int E = Elem<T>::kSlabK;
   if (!(partial && partial_bytes)) return launch_gemm_one<T, T, S>(in, M, N, K, C, ldc, 0, stream, nullptr, 0, 1, rows);
   const DhPlan pl = plan_dhidden(N, M, K, E, device_cu_count(), partial_bytes);
+  if constexpr (sizeof(T) == 2) {
+    if (pl.ni == 6) return launch_gemm_one<T, T, S, 6>(in, M, N, K, C, ldc, 0, stream, partial, partial_bytes, pl.k_split, rows);
+    if (pl.ni == 4) return launch_gemm_one<T, T, S, 4>(in, M, N, K, C, ldc, 0, stream, partial, partial_bytes, pl.k_split, rows);
+  }
   if (pl.bulk_nt == 0) return launch_gemm_one<T, T, S>(in, M, N, K, C, ldc, 0, stream, partial, partial_bytes, pl.k_split, rows);
   const int bulk_rows = pl.bulk_nt * 256;
   int rc = launch_gemm_one<T, T, S>(in, M, bulk_rows, K, C, ldc, 0, stream, nullptr, 0, 1, rows);

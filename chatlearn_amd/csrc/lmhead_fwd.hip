@@ -1,10 +1,10 @@
 // Fused lm_head projection + online log-softmax statistics (forward).
 //
-// z^T tile [256 vocab x 256 tokens] = W tile * hidden tile^T on the matrix cores;
+// z^T tile [256 vocab x block of tokens] = W tile * hidden tile^T on the matrix cores;
 // the vocabulary runs along the accumulator registers, the tokens along the
 // lanes, so each lane keeps a running (max, sum e^{z-max}, sum e^{z-max} z,
 // target logit) for its own tokens across all vocabulary tiles of its split.
-// A workgroup owns one block of 256 tokens and one contiguous range of
+// A workgroup owns one block of 256 tokens (or fewer, see fwd_plan) and one contiguous range of
 // vocabulary tiles ("split"); a second small kernel merges the splits with an
 // exact rescale and writes logprob / entropy / rowmax / lse.  Logits go to
 // memory only when the caller asks for a chunk's raw logits to be kept for the
@@ -17,7 +17,7 @@
 
 namespace clgrpo {
 
-constexpr int kFwdBM = 256, kFwdBN = 256;
+constexpr int kFwdBM = 256, kFwdBN = 256;   // kFwdBN: the widest token block, see fwd_plan
 constexpr float kLog2e = 1.4426950408889634f;
 // Most vocabulary splits a forward launch of n_tb token blocks uses: 4096 workgroups in all, 64 splits at least
 // (the partial records of up to 16384 tokens then stay below 17 MB).  A few token blocks need many splits to reach all
@@ -66,9 +66,9 @@ __device__ __forceinline__ void merge_state(float& m, float& s, float& u, float 
   m = nm;
 }
 
-template <typename T, bool STORE_Z>
+template <typename T, bool STORE_Z, int kNI>
 __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p) {
-  using Tile = LogitTile<T>;
+  using Tile = LogitTile<T, kNI>;
   constexpr int MI = Tile::MI, NI = Tile::NI, VEC = Tile::VEC;
   extern __shared__ __align__(16) char lds[];
 
@@ -88,8 +88,8 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
   const int wm_u = __builtin_amdgcn_readfirstlane(wm);
   const int la = wm + Tile::lane_a0();               // this lane's first vocabulary row / token of the tile
   const int lb = wn + Tile::lane_b0();
-  const int t0 = tb * kFwdBN;
-  const int b_rows = (p.T - t0) < kFwdBN ? (p.T - t0) : kFwdBN;
+  const int t0 = tb * Tile::BN;
+  const int b_rows = (p.T - t0) < Tile::BN ? (p.T - t0) : Tile::BN;
   const T* weight = static_cast<const T*>(p.weight);
   const float c = p.c;
 
@@ -347,7 +347,7 @@ static int launch_finalize(const FinalizeParams& f, hipStream_t stream) {
 //    with its partial record: 0.3 tile periods (32768 tokens at H = 7168: 22 splits x 23 tiles 45.2 ms, 4
 //    x 127 or 8 x 64 tiles 44.3 - 44.6 ms).
 // Returns the launch's cost in sixteenths of a tile period.  `cus` <= 0 plans for a 256-CU device.
-static long fwd_single_cost(int n_tb, int n_vt, int cus, int& n_split, int& tiles_per_split) {
+static double fwd_single_cost(int n_tb, int n_vt, int cus, int& n_split, int& tiles_per_split) {
   if (cus <= 0) cus = 256;
   const double xcd_wgs = cus / 8.0, full_block = 4.0 + xcd_wgs / 4.0;
   int best = 1;
@@ -364,13 +364,47 @@ static long fwd_single_cost(int n_tb, int n_vt, int cus, int& n_split, int& tile
   }
   tiles_per_split = (n_vt + best - 1) / best;
   n_split = (n_vt + tiles_per_split - 1) / tiles_per_split;
-  return (long)(best_cost + 0.5);
+  return best_cost;
+}
+
+// Width of the token blocks: 32 * ni tokens.  The last block of 256 is padding for the most part where T is a little over a
+// multiple of 256, and a launch of fewer items than CUs leaves the rest idle; a narrower tile takes ni / 8 of the time,
+// and about 2 % more of that per step down (more operand traffic and fragment reads per product).  Taken where the plan
+// then costs 4 % less; 16-bit inputs only.  Up to two wide blocks that fill the CUs are bound by reading W, so they are
+// not made into more blocks (256 tokens at H = 4096, V = 151936 as two blocks of 128: 320 us for 295).
+//   H = 4096, V = 151936, us: 128 tokens 269 -> 228, 260 428 -> 333, 400 463 -> 426, 588 638 -> 579, 900 882 -> 848, 1100 1062 -> 968
+//   H = 2048:                 128 tokens 161 -> 148, 260 229 -> 188, 588 340 -> 311, 1100 555 -> 510
+//   H = 1024, V = 32000:      200 tokens  38 ->  28, 300  40 ->  31, 588  60 ->  45, 1100  84 ->  69
+struct FwdPlan {
+  int ni, n_tb, n_split, tiles_per_split;
+};
+static FwdPlan fwd_plan(int64_t T, int n_vt, int cus, bool narrow) {
+  if (cus <= 0) cus = 256;
+  const int wide_tb = (int)((T + kFwdBN - 1) / kFwdBN);
+  FwdPlan best{8, wide_tb, 0, 0};
+  double best_cost = 0.96 * fwd_single_cost(best.n_tb, n_vt, cus, best.n_split, best.tiles_per_split);
+  for (int ni = 7; narrow && ni >= 4; --ni) {
+    FwdPlan pl{ni, (int)((T + 32 * ni - 1) / (32 * ni)), 0, 0};
+    if (pl.n_tb > wide_tb && wide_tb <= 2 && wide_tb * n_vt > cus) continue;
+    const double c = ni / 8.0 * (1.0 + 0.02 * (8 - ni)) * fwd_single_cost(pl.n_tb, n_vt, cus, pl.n_split, pl.tiles_per_split);
+    if (c < best_cost) { best_cost = c; best = pl; }
+  }
+  return best;
+}
+
+template <typename T, bool STORE_Z, int NI>
+static int launch_fwd_kernel(const FwdParams& p, const ItemGrid& ig, hipStream_t stream) {
+  using Tile = LogitTile<T, NI>;
+  const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&lmhead_fwd_kernel<T, STORE_Z, NI>), Tile::kLdsBytes, "lmhead_fwd_kernel");
+  if (rc) return rc;
+  hipLaunchKernelGGL((lmhead_fwd_kernel<T, STORE_Z, NI>), dim3(ig.grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, p);
+  return check_launch("lmhead_fwd_kernel");
 }
 
 template <typename T, bool STORE_Z>
 static int launch_fwd(const clgrpo_lmhead_fwd_args* a, hipStream_t stream, int64_t label_offset, float4* record,
                       const RowOrder& rows) {
-  using Tile = LogitTile<T>;
+  constexpr bool kNarrow = sizeof(T) == 2;
   FwdParams p;
   p.hidden = a->hidden;
   p.weight = a->weight;
@@ -379,9 +413,9 @@ static int launch_fwd(const clgrpo_lmhead_fwd_args* a, hipStream_t stream, int64
   p.T = (int)a->T;
   p.H = (int)a->H;
   p.V = (int)a->V;
-  p.n_tb = (int)((a->T + kFwdBN - 1) / kFwdBN);
   p.n_vt = (int)((a->V + kFwdBM - 1) / kFwdBM);
-  fwd_single_cost(p.n_tb, p.n_vt, device_cu_count(), p.n_split, p.tiles_per_split);
+  const FwdPlan pl = fwd_plan(a->T, p.n_vt, device_cu_count(), kNarrow);
+  p.n_tb = pl.n_tb; p.n_split = pl.n_split; p.tiles_per_split = pl.tiles_per_split;
   p.c = a->inv_temperature * kLog2e;
   p.part = static_cast<float4*>(a->workspace);
   p.z_out = a->saved_logits;
@@ -390,13 +424,16 @@ static int launch_fwd(const clgrpo_lmhead_fwd_args* a, hipStream_t stream, int64
   p.z_rows = (int)a->saved_rows;
   p.order = rows.order;
   p.total = (int)rows.total;
-  constexpr int lds_bytes = Tile::kLdsBytes;
-  int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&lmhead_fwd_kernel<T, STORE_Z>), lds_bytes, "lmhead_fwd_kernel");
-  if (rc) return rc;
   const ItemGrid ig = item_grid(p.n_tb * p.n_split, device_cu_count());
   p.xcd_wgs = ig.xcd_wgs;
-  hipLaunchKernelGGL((lmhead_fwd_kernel<T, STORE_Z>), dim3(ig.grid), dim3(Tile::kThreads), lds_bytes, stream, p);
-  rc = check_launch("lmhead_fwd_kernel");
+  int rc;
+  if constexpr (kNarrow) {
+    rc = pl.ni == 4 ? launch_fwd_kernel<T, STORE_Z, 4>(p, ig, stream) : pl.ni == 5 ? launch_fwd_kernel<T, STORE_Z, 5>(p, ig, stream)
+       : pl.ni == 6 ? launch_fwd_kernel<T, STORE_Z, 6>(p, ig, stream) : pl.ni == 7 ? launch_fwd_kernel<T, STORE_Z, 7>(p, ig, stream)
+                    : launch_fwd_kernel<T, STORE_Z, 8>(p, ig, stream);
+  } else {
+    rc = launch_fwd_kernel<T, STORE_Z, 8>(p, ig, stream);
+  }
   if (rc) return rc;
   FinalizeParams f;
   f.part = p.part;
@@ -434,12 +471,10 @@ extern "C" int64_t clgrpo_saved_logits_ld(int64_t V) { return V <= 0 ? 0 : round
 
 extern "C" int clgrpo_lmhead_fwd_launch_plan(int64_t T, int64_t V, int32_t cus, int32_t* out) {
   if (T <= 0 || V <= 0 || out == nullptr) return CLGRPO_EINVAL;
-  const int n_tb = (int)((T + kFwdBN - 1) / kFwdBN), n_vt = (int)((V + kFwdBM - 1) / kFwdBM);
-  int n_split, tps;
-  fwd_single_cost(n_tb, n_vt, cus, n_split, tps);
-  out[0] = n_tb;
-  out[1] = n_split;
-  out[2] = tps;
+  const FwdPlan pl = fwd_plan(T, (int)((V + kFwdBM - 1) / kFwdBM), cus, true);
+  out[0] = pl.n_tb;
+  out[1] = pl.n_split;
+  out[2] = pl.tiles_per_split;
   return CLGRPO_OK;
 }
 

@@ -167,8 +167,8 @@ def lmhead_forward(hidden: torch.Tensor, weight: torch.Tensor, labels: Optional[
 
 
 def lmhead_forward_launch_plan(T: int, V: int, cus: int = 0) -> Tuple[int, int, int]:
-    """(blocks of 256 tokens, vocabulary splits, vocabulary tiles per workgroup) of the forward launch for T
-    tokens on a device with ``cus`` compute units (0: 256)."""
+    """(blocks of 256 tokens or fewer, vocabulary splits, vocabulary tiles per workgroup) of the forward launch for T
+    tokens of 16-bit inputs on a device with ``cus`` compute units (0: 256)."""
     out = (C.c_int32 * 3)()
     _lib.check(_lib.lib().clgrpo_lmhead_fwd_launch_plan(int(T), int(V), int(cus), C.cast(out, C.c_void_p)))
     return int(out[0]), int(out[1]), int(out[2])
