@@ -24,6 +24,7 @@ class _PolicyLoss(torch.autograd.Function):
         # reference: assert not torch.isnan(loss).any(), "pg loss is nan"
         assert not int(res.flags.item()) & 1, "pg loss is nan"
         ctx.save_for_backward(res.dloss)
+        ctx.set_materialize_grads(False)
         ctx.in_dtype = log_probs.dtype
         out_dtype = torch.promote_types(torch.promote_types(log_probs.dtype, old_log_probs.dtype), adv.dtype)
         loss = res.loss.to(out_dtype)
@@ -35,7 +36,7 @@ class _PolicyLoss(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g, *_):
         (dloss,) = ctx.saved_tensors
-        return (g.to(dloss.dtype) * dloss).to(ctx.in_dtype), None, None, None, None, None, None, None, None
+        return None if g is None else (g.to(dloss.dtype) * dloss).to(ctx.in_dtype), None, None, None, None, None, None, None, None
 
 
 def _adv_tensor(advantages, like):

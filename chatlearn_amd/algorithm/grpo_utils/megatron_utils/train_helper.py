@@ -152,6 +152,7 @@ class _TokenLosses(torch.autograd.Function):
         assert not bits & 2, "kl loss ratio has inf values"
         assert not bits & 4, "kl loss ratio has nan values"
         ctx.save_for_backward(res.dloss)
+        ctx.set_materialize_grads(False)
         ctx.in_dtype = logprob.dtype
         # dtype of -A * ratio under torch's promotion: a list of numpy float64 advantages makes it float64
         surrogate = res.loss.to(torch.promote_types(torch.promote_types(logprob.dtype, old.dtype), adv.dtype))
@@ -265,25 +266,26 @@ def logprobs_from_hidden(module_args, hidden: torch.Tensor, output_weight: torch
 
 
 class _MaskedSums(torch.autograd.Function):
-    """One launch reduces every tensor of the loss dict under the mask; the tensors listed in
-    ``grad_slots`` get the gradient mask * g back."""
+    """One launch reduces every tensor of the loss dict under the mask: (all sums, count, one scalar of its own for each
+    tensor listed in ``grad_slots``).  Those get the gradient mask * g back.  Scalars of their own, because an entry picked
+    out of the sums costs its gradient a zero fill and a copy, and because a caller may divide the loss in place."""
 
     @staticmethod
     def forward(ctx, mask, grad_slots, averaged, *tensors):
         sums, count = ops.masked_sums(tensors, mask, averaged)
         ctx.mask, ctx.grad_slots = mask, grad_slots
         ctx.like = [(t.dtype, t.shape) for t in tensors]
-        ctx.mark_non_differentiable(count)
-        return sums, count
+        ctx.set_materialize_grads(False)
+        ctx.mark_non_differentiable(sums, count)
+        return (sums, count) + tuple(sums[j].clone() for j in grad_slots)
 
     @staticmethod
-    def backward(ctx, g_sums, _):
+    def backward(ctx, _, __, *g_slots):
         grads = [None] * len(ctx.like)
-        if g_sums is not None:
-            g_sums = g_sums.float().contiguous()
-            for j in ctx.grad_slots:
+        for j, g in zip(ctx.grad_slots, g_slots):
+            if g is not None:
                 dtype, shape = ctx.like[j]
-                grads[j] = ops.masked_sums_backward(g_sums[j:j + 1], ctx.mask, dtype, shape)
+                grads[j] = ops.masked_sums_backward(g.float().reshape(1), ctx.mask, dtype, shape)
         return (None, None, None) + tuple(grads)
 
 
@@ -299,13 +301,15 @@ def loss_func(inputs: Dict, losses: Dict[str, torch.Tensor]):
     names = list(losses)
     grad_slots = tuple(j for j, name in enumerate(names) if name in BACKPROP_KEYS and losses[name].requires_grad)
     averaged = tuple(name.endswith('_sample_average') for name in names)
-    sums, count = _MaskedSums.apply(inputs["all_token_loss_mask"], grad_slots, averaged,
-                                    *(losses[name] for name in names))
-    report = {name: sums[j].detach().clone() for j, name in enumerate(names)}
+    sums, count, *slots = _MaskedSums.apply(inputs["all_token_loss_mask"], grad_slots, averaged,
+                                            *(losses[name] for name in names))
+    report = dict(zip(names, sums.unbind(0)))          # the sums carry no gradient and belong to the report
     total = 0
     for j, name in enumerate(names):
-        if name in BACKPROP_KEYS:
+        if name in BACKPROP_KEYS and j not in grad_slots:
             total = total + sums[j]
+    for slot in slots:
+        total = slot if isinstance(total, int) else total + slot
     num_tokens = inputs.get('num_tokens_on_this_cp_rank', count[0]).to(torch.int)
     report["num_tokens"] = num_tokens
     report["num_samples"] = torch.ones_like(num_tokens)
