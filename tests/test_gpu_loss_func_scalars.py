@@ -13,7 +13,7 @@ def test_loss_divided_in_place_keeps_its_gradient_and_leaves_the_report(dev, nee
     ent = torch.randn(3, 40, generator=g).to(dev)
     mask = (torch.rand(3, 40, generator=g) < 0.6).int().to(dev)
     total, n, report = th.loss_func({"all_token_loss_mask": mask}, {"pg_loss": pg, "entropy_loss": ent})
-    want = (pg.detach() * mask).sum().float()            # 72 fp64 products, rounded to fp32 once
+    want = (pg.detach().float().double() * mask).sum().float()       # entries as fp32, summed in fp64, rounded to fp32 once
     assert torch.allclose(total.detach(), want, rtol=2.0 ** -22, atol=0)
     total /= n
     total /= 4
