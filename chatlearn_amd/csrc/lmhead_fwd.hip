@@ -144,6 +144,34 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
     // this wave's first unit of the tile, and this lane's piece in it
     char* z_tile = static_cast<char*>(p.z_out) + (int64_t)((v0 + wm_u) / Tile::kSlabK) * Tile::kUnitBytes;
     const int z_lane = Tile::lane_a0() * (int)sizeof(typename KeptLogit<T>::type);
+    const uint32_t n_units = (uint32_t)(p.ldz / Tile::kSlabK);
+    // Raw logits for the backward: VEC consecutive vocabulary entries of a token are one 16-byte piece of
+    // its unit.  Vocabulary rows past V hold zeros already (the operand loads are range-checked), and the backward
+    // ignores whatever the padding columns hold.
+    auto keep = [&](int j, const float (&x)[MI * 4], auto whole) __attribute__((always_inline)) {
+      typedef typename KeptLogit<T>::type ZT;
+      constexpr int AG = VEC / 4;                     // blocks whose registers make up one piece
+      // The row is the same for every vocabulary tile, so the compiler would keep the 64-bit addresses it
+      // forms from it alive across the K loops, where registers are scarcest, spill them, and reload them
+      // between the stores (a reload waits for the stores issued before it).  Re-deriving one from the 32-bit row
+      // costs a handful of instructions per tile; the pieces lie at constants from it (with an address of its own
+      // per piece, some 20 instructions each, 16384 tokens at H = 2048 took 7.55 ms for 7.44).
+      int row = zrow[j];
+      asm volatile("" : "+v"(row));
+      if (row >= 0) {
+        char* z_row = z_tile + ((uint64_t)(uint32_t)(row / Tile::kSlabK) * n_units) * Tile::kUnitBytes +
+                      (uint32_t)(row % Tile::kSlabK * kRowBytes + z_lane);
+#pragma unroll
+        for (int i = 0; i < MI; i += AG) {
+          if (!decltype(whole)::value && v0 + wm_u + Tile::a_block(i) / 32 * 32 >= p.ldz) continue;     // the same for all lanes
+          float piece[VEC];
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) piece[e] = x[i * 4 + e];
+          *reinterpret_cast<u32x4*>(z_row + Tile::a_block(i) / Tile::kSlabK * Tile::kUnitBytes +
+                                    Tile::a_block(i) % Tile::kSlabK * (int)sizeof(ZT)) = pack_kept(piece, (ZT*)nullptr);
+        }
+      }
+    };
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       // this token's logits of the lane's vocabulary rows
@@ -153,37 +181,11 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
 #pragma unroll
         for (int r = 0; r < 4; ++r) x[i * 4 + r] = acc_get(acc[i][j], r);
 
-      if (STORE_Z) {
-        // Raw logits for the backward: VEC consecutive vocabulary entries of a token are one 16-byte piece of
-        // its unit.  Vocabulary rows past V hold zeros already (the operand loads are
-        // range-checked), and the backward ignores whatever the padding columns hold.
-        typedef typename KeptLogit<T>::type ZT;
-        constexpr int AG = VEC / 4;                     // blocks whose registers make up one piece
-        // The row is the same for every vocabulary tile, so the compiler would keep the 64-bit addresses it
-        // forms from it alive across the K loops, where registers are scarcest, spill them, and reload them
-        // between the stores (a reload waits for the stores issued before it).  Re-deriving one from the 32-bit row
-        // costs a handful of instructions per tile; the pieces lie at constants from it (with an address of its own
-        // per piece, some 20 instructions each, 16384 tokens at H = 2048 took 7.55 ms for 7.44).
-        int row = zrow[j];
-        asm volatile("" : "+v"(row));
-        if (row >= 0) {
-          const uint64_t unit_row = (uint64_t)(p.ldz / Tile::kSlabK) * Tile::kUnitBytes;
-          char* z_row = z_tile + (uint64_t)(uint32_t)(row / Tile::kSlabK) * unit_row + (row % Tile::kSlabK * kRowBytes + z_lane);
-#pragma unroll
-          for (int i = 0; i < MI; i += AG) {
-            if (!full && v0 + wm_u + Tile::a_block(i) / 32 * 32 >= p.ldz) continue;     // the same for all lanes
-            float piece[VEC];
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) piece[e] = x[i * 4 + e];
-            *reinterpret_cast<u32x4*>(z_row + Tile::a_block(i) / Tile::kSlabK * Tile::kUnitBytes +
-                                      Tile::a_block(i) % Tile::kSlabK * (int)sizeof(ZT)) = pack_kept(piece, (ZT*)nullptr);
-          }
-        }
-      }
+      if (STORE_Z && full) keep(j, x, Const<1>{});
 
       // Target logit: only a lane whose rows of this tile hold the label looks for it.
       const int rel = lab[j] - v0;
-      if (__any((unsigned)rel < (unsigned)Tile::WM)) {
+      if (__builtin_expect(__any((unsigned)rel < (unsigned)Tile::WM), 0)) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -191,7 +193,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
             if (rel == Tile::a_block(i) + r) zt[j] = x[i * 4 + r];
       }
 
-      if (!full) {
+      if (__builtin_expect(!full, 0)) {
         // last, partial vocabulary tile: the zeros of rows past V must not count
 #pragma unroll
         for (int i = 0; i < MI; ++i)
@@ -216,6 +218,17 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
       s[j] = fmaf(s[j], scale, ls);
       u[j] = fmaf(u[j], scale, lu);
       m[j] = nm;
+    }
+    // A tile that ends inside the vocabulary keeps its logits apart: the test per piece, mixed into the loop above, put every
+    // store of every tile out of line, two jumps away (7.34 ms against 7.26 at 16384 tokens of 2048).
+    if (STORE_Z && !full) {
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        float x[MI * 4];
+#pragma unroll
+        for (int k = 0; k < MI * 4; ++k) x[k] = acc_get(acc[k / 4][j], k % 4);
+        keep(j, x, Const<0>{});
+      }
     }
   }
   if (stream) Tile::finish();
