@@ -268,8 +268,8 @@ struct GemmParams {
 // the tile's valid rows and one per-lane byte offset per group of BV (kMContig: per block) of the lane dimension.
 // Along the lane dimension (n) elements outside the tile get a per-lane offset far outside the descriptor: loads
 // of them give 0 and stores are dropped.  Along the register dimension (m) nothing relies on the range check:
-// kMContig skips whole 32-row groups (its M extents are multiples of 32), and the other orientation tests
-// every row against the tile's valid rows unless the tile is a full one.
+// kMContig skips whole 32-row groups (its M extents are multiples of 32), and in the other orientation a row past the
+// tile's valid ones gets such an offset too.
 template <typename T, typename OutT, Side S, int NI>
 struct TileAddr {
   using Tile = OutTile<T, S, NI>;
@@ -288,6 +288,7 @@ struct TileAddr {
                                       const int32_t* order = nullptr, int64_t total = 0) {
     row_bytes = (int)(ld * (int64_t)ES);
     a_rows = a_rows_;
+    if constexpr (!kMContig) asm volatile("" : "+s"(row_bytes));   // its multiples are not kept in registers across the K loops
     const int m = Tile::wave_m() + Tile::lane_a0();
     row_lim = a_rows_ - m;
     const int rows = kMContig ? b_rows : a_rows_, cols = kMContig ? a_rows_ : b_rows;
@@ -305,23 +306,11 @@ struct TileAddr {
   }
   // kMContig: piece n lies inside the tile (uniform over the wave)
   __device__ __forceinline__ bool piece_ok(int n) const { return Tile::wave_m() + (piece_off(n) & ~31) < a_rows; }
-  __device__ __forceinline__ bool full_rows() const { return a_rows == Tile::BM; }
+  // otherwise: offset of group g of the row dm rows below the lane's first
+  __device__ __forceinline__ int row_voff(int dm, int g) const { return dm < row_lim ? voff[g] : 0x7f000000; }
 };
 
-// N consecutive elements of a row: 4 or 8 floats, or 8 (T = bf16) 16-bit values.
-template <int N>
-__device__ __forceinline__ void row_load(float (&x)[N], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, float*) {
-#pragma unroll
-  for (int k = 0; k < N; k += 4) {
-    const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff + k * 4, soff, 0));
-    x[k] = v[0]; x[k + 1] = v[1]; x[k + 2] = v[2]; x[k + 3] = v[3];
-  }
-}
-__device__ __forceinline__ void row_load(float (&x)[8], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, __bf16*) {
-  const bf16x8 v = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, soff, 0));
-#pragma unroll
-  for (int k = 0; k < 8; ++k) x[k] = (float)v[k];
-}
+// N consecutive elements of a row: 4 or 8 floats, or 4 or 8 (T = bf16) 16-bit values.
 template <int N>
 __device__ __forceinline__ void row_store(const float (&x)[N], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, float*) {
 #pragma unroll
@@ -341,14 +330,13 @@ __device__ __forceinline__ void row_store(const float (&x)[4], const __amdgpu_bu
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc, voff, soff, 0);
 }
 
-// fn(values of one run of a row, per-lane offset, scalar offset), for every run of the tile that lies inside it;
-// kLoad (dW only): the values go into the accumulators afterwards.
-template <typename T, typename OutT, Side S, int NI, bool kLoad, typename AccT, typename Fn>
+// fn(values of one run of a row, per-lane offset, scalar offset), for every run of the tile that lies inside it; a
+// dW row past the tile gets an offset outside the descriptor, as elements past a row do.
+template <typename T, typename OutT, Side S, int NI, typename AccT, typename Fn>
 __device__ __forceinline__ void for_rows(const TileAddr<T, OutT, S, NI>& at, AccT& acc, Fn fn) {
   using Tile = OutTile<T, S, NI>;
   using Addr = TileAddr<T, OutT, S, NI>;
   if constexpr (kMContig<S>) {
-    static_assert(!kLoad, "dhidden is never added to");
 #pragma unroll
     for (int n = 0; n < Addr::kPieces; ++n) {
       if (!at.piece_ok(n)) continue;
@@ -361,42 +349,61 @@ __device__ __forceinline__ void for_rows(const TileAddr<T, OutT, S, NI>& at, Acc
       }
     }
   } else {
-    const bool full = at.full_rows();   // uniform over the workgroup
 #pragma unroll
     for (int i = 0; i < Tile::MI; ++i)
 #pragma unroll
-      for (int j = 0; j < Tile::NI; j += 4) {
-        float x[4][4];                    // [register of the four blocks][block]
+      for (int j = 0; j < Tile::NI; j += 4)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
+          float x[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) x[k] = acc_get(acc[i][j + k], r);
           const int dm = Tile::a_off(i, r);
-#pragma unroll
-          for (int k = 0; k < 4; ++k) x[r][k] = kLoad ? 0.f : acc_get(acc[i][j + k], r);
-          if (full || dm < at.row_lim) fn(x[r], at.voff[j / 4], dm * at.row_bytes);
+          fn(x, at.row_voff(dm, j / 4), dm * at.row_bytes);
         }
-        if (kLoad) {
-#pragma unroll
-          for (int k = 0; k < 4; ++k) acc_set(acc[i][j + k], x[0][k], x[1][k], x[2][k], x[3][k]);
-        }
-      }
   }
 }
 
-// Accumulators of output tile (m0, n0) before its K loop: zeros, or - when the GEMM adds to C and one
-// workgroup owns the whole K range of the tile - the tile's current contents.  Reading C here instead of
-// in the epilogue puts the loads' latency in front of the K loop, where the first operand slabs are in
-// flight anyway, and leaves the epilogue a pure store.
-template <typename T, typename OutT, Side S, int NI>
-__device__ __forceinline__ void gemm_init_tile(const GemmParams& p, typename OutTile<T, S, NI>::Acc& acc, int m0, int n0,
-                                               int a_rows, int b_rows) {
-  constexpr bool kAdds = !kMContig<S> && sizeof(OutT) == 4;    // only an fp32 C is ever added to
-  if (!kAdds || !p.accumulate || p.k_split > 1) OutTile<T, S, NI>::zero(acc);
-  if constexpr (kAdds) {
-    if (!p.accumulate || p.k_split > 1) return;
-    const TileAddr<T, OutT, S, NI> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows);
-    for_rows<T, OutT, S, NI, true>(at, acc, [&](auto& x, int voff, int soff) { row_load(x, at.rsrc, voff, soff, (OutT*)nullptr); });
+// The tile's contents into the accumulators (dW only).  The loads of kAhead block rows are in flight before the first is
+// used, and they are requested before the stores of the tile before: with one wave per SIMD nothing else hides their
+// latency (H = 4096 over 151936 entries, loads of half a block row at a time -> these: 256 tokens 1.24 -> 0.96 ms = 5.2 TB/s
+// over reads and writes, 1024 tokens 1.76 -> 1.48, 3520 tokens 3.55 -> 3.33).  A fourth block row ahead does not fit
+// the registers.
+template <typename T, Side S, int NI>
+struct RowLoads {
+  using Tile = OutTile<T, S, NI>;
+  static constexpr int kAhead = 3, kSlots = kAhead + 1;
+  f32x4 x[kSlots][NI / 4][4];      // [block row][group of four blocks][register of the blocks]
+  typedef TileAddr<T, float, S, NI> At;
+  __device__ __forceinline__ void fetch(const At& at, int i) {
+#pragma unroll
+    for (int g = 0; g < NI / 4; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int dm = Tile::a_off(i, r);
+        x[i % kSlots][g][r] =
+            __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(at.rsrc, at.row_voff(dm, g), dm * at.row_bytes, 0));
+      }
+    Tile::fence();
   }
-}
+  __device__ __forceinline__ void begin(const At& at) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) fetch(at, i);
+  }
+  template <typename AccT>
+  __device__ __forceinline__ void finish(const At& at, AccT& acc) {
+#pragma unroll
+    for (int i = 0; i < Tile::MI; ++i) {
+      if (i + kAhead < Tile::MI) fetch(at, i + kAhead);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        const auto& b = x[i % kSlots][j / 4];
+        acc_set(acc[i][j], b[0][j % 4], b[1][j % 4], b[2][j % 4], b[3][j % 4]);
+      }
+      Tile::fence();
+    }
+  }
+};
 
 // Output tile from the accumulators: C = acc (the accumulators already hold C's previous contents
 // when the GEMM adds to it, see gemm_init_tile), or the fp32 partial of K range `ks`.
@@ -405,11 +412,11 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, typename Ou
                                                 int a_rows, int b_rows, int ks) {
   if (p.k_split > 1) {
     const TileAddr<T, float, S, NI> at(p.partial + (int64_t)ks * p.M * p.N, kMContig<S> ? p.M : p.N, m0, n0, a_rows, b_rows);
-    for_rows<T, float, S, NI, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (float*)nullptr); });
+    for_rows<T, float, S, NI>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (float*)nullptr); });
     return;
   }
   const TileAddr<T, OutT, S, NI> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows, p.order, p.total);
-  for_rows<T, OutT, S, NI, false>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (OutT*)nullptr); });
+  for_rows<T, OutT, S, NI>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (OutT*)nullptr); });
 }
 
 // Work item = (walk, fixed tile) when n_walk > 0: the workgroup keeps one operand's tile (A's m tile
@@ -461,14 +468,30 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
     else return Tile::Operand::blocked(B + ((int64_t)n_tile * p.b_step + s0) * kSlabElems, rows);
   };
   auto rows_of = [](int total, int tile, int width) { const int left = total - tile * width; return left < width ? left : width; };
+  // Accumulators before a tile's K loop: zeros, or - when the GEMM adds to C and one workgroup owns the whole K range of
+  // the tile - the tile's current contents, which leaves the epilogue a pure store.
+  constexpr bool kCanAdd = !kMC && sizeof(OutT) == 4;     // only an fp32 C is ever added to
+  const bool adds = kCanAdd && p.accumulate && p.k_split == 1;
+  typedef RowLoads<T, S, NI> Loads;
+  auto c_tile = [&](int m_tile) {
+    return typename Loads::At(static_cast<float*>(p.C), p.ldc, m_tile * 256, nt * Tile::BN, rows_of(p.M, m_tile, 256),
+                              rows_of(p.N, nt, Tile::BN));
+  };
   typename Tile::Acc acc;
+  Loads loads;
+  if constexpr (kCanAdd) {
+    if (adds) loads.begin(c_tile(mt));
+  }
   Tile core;
   for (int k = 0; k < count; ++k) {
     const int m0 = mt * 256, n0 = nt * Tile::BN;
     const int a_rows = rows_of(p.M, mt, 256), b_rows = rows_of(p.N, nt, Tile::BN);
     const auto op_a = operand_a(mt, a_rows);
     const auto op_b = operand_b(nt, b_rows);
-    gemm_init_tile<T, OutT, S, NI>(p, acc, m0, n0, a_rows, b_rows);
+    if (!adds) Tile::zero(acc);
+    if constexpr (kCanAdd) {
+      if (adds) loads.finish(c_tile(mt), acc);
+    }
     if (k == 0 || !stream) core.start(op_a, op_b, nslab, lds);
     if (stream && k + 1 < count)
       core.follow(op_a, op_b, nslab, Tile::cursor_a(kMC ? op_a : operand_a(mt + 1, rows_of(p.M, mt + 1, 256)), nslab),
@@ -477,6 +500,9 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
       core.follow(op_a, op_b, nslab, Tile::hold_a(op_a, nslab), Tile::hold_b(op_b, nslab));
     core.run(acc, nslab);
     if (!stream || k + 1 == count) Tile::finish();
+    if constexpr (kCanAdd) {
+      if (adds && k + 1 < count) loads.begin(c_tile(mt + 1));
+    }
     gemm_store_tile<T, OutT, S, NI>(p, acc, m0, n0, a_rows, b_rows, ks);
     if (kMC) ++nt; else ++mt;
   }
