@@ -26,8 +26,18 @@ struct DwOperands {
 // `rows` are left alone), kept logits by n.  An order and kept dW operands need kept logits.
 int head_backward(const char* who, const clgrpo_lmhead_bwd_args* a, int64_t vocab_begin, const RowOrder& rows,
                   hipStream_t stream, const DwOperands* kept = nullptr);
+// What a step of several chunks reports once its last chunk's loss is known, from the sums and flag words of all of them
+// (`sums` and `flags` begin with the first chunk's, `chunk` others come before this one's); `result` NULL: nothing.
+// result: [0..7] the chunks' sums added up, [8] pg, [9] kl, [10] entropy mean, [11] total loss, [12] flags, [13] masked tokens
+struct StepResult {
+  const double* sums;
+  const int32_t* flags;
+  int chunk;
+  double scale, kl_coef, entropy_coef;
+  double* result;
+};
 // clgrpo_policy_loss with the scratch memory named apart.
 int head_policy_loss(const char* who, const clgrpo_policy_loss_args* a, void* workspace, size_t workspace_bytes,
-                     hipStream_t stream);
+                     hipStream_t stream, const StepResult& step = StepResult{});
 
 }  // namespace clgrpo

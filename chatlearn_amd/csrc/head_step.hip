@@ -32,29 +32,6 @@ __global__ __launch_bounds__(256) void zero_floats_kernel(float* p, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = 0.f;
 }
 
-// result: [0..7] the chunks' sums added up, [8] pg, [9] kl, [10] entropy mean, [11] total loss, [12] flags, [13] masked tokens
-__global__ void step_result_kernel(const double* sums, const int32_t* flags, int n_chunks, double scale, double kl_coef,
-                                   double entropy_coef, double* result) {
-  __shared__ double total[8];
-  if (threadIdx.x < 8) {
-    double s = 0.0;
-    for (int k = 0; k < n_chunks; ++k) s += sums[8 * k + threadIdx.x];
-    total[threadIdx.x] = s;
-    result[threadIdx.x] = s;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const double pg = total[0] * scale, kl = total[1] * scale, en = total[2] * scale;
-    double loss = pg;
-    if (entropy_coef > 0) loss -= entropy_coef * en;
-    if (kl_coef > 0) loss += kl_coef * kl;
-    int f = 0;
-    for (int k = 0; k < n_chunks; ++k) f |= flags[k];
-    result[8] = pg; result[9] = kl; result[10] = en; result[11] = loss;
-    result[12] = (double)f; result[13] = total[3];
-  }
-}
-
 // Scratch memory: the forward's records and the backward's operands one after the other in the same place, the
 // loss's own and the upstream gradient of the entropy beside them.
 struct StepPlan {
@@ -171,14 +148,9 @@ extern "C" int clgrpo_head_step(const clgrpo_head_step_args* a, void* stream) {
     p.grad_scale = a->grad_scale;
     p.loss = a->loss; p.kl = a->ref_logprob ? a->kl : nullptr; p.g_logprob = a->g_logprob; p.g_entropy = g_entropy;
     p.sums = a->sums + 8 * a->chunk; p.flags = a->flags + a->chunk; p.token_offset = a->token_offset;
-    int rc = head_policy_loss(who, &p, ws + pl.off_loss, pl.off_gent - pl.off_loss, s);
+    const StepResult step{a->sums, a->flags, (int)a->chunk, a->grad_scale, a->kl_coef, a->entropy_coef, a->result};
+    const int rc = head_policy_loss(who, &p, ws + pl.off_loss, pl.off_gent - pl.off_loss, s, step);
     if (rc) return rc;
-    if (a->result) {
-      hipLaunchKernelGGL(step_result_kernel, dim3(1), dim3(64), 0, s, a->sums, a->flags, a->chunk + 1, a->grad_scale, a->kl_coef,
-                         a->entropy_coef, a->result);
-      rc = check_launch("step_result_kernel");
-      if (rc) return rc;
-    }
   }
   if (a->stages & 4) {
     if (a->n_live > 0) {

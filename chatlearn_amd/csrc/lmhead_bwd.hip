@@ -137,11 +137,55 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_dz_kernel(DzParams p) 
   }
 }
 
+// dst(c, r) = src[r][c] (src[order[r]][c] with an order) for r < R, c < C and 0 for R <= r < r_dst, where dst is the K-blocked
+// operand with C rows and ld_dst K elements (see blocked_index), of which the first r_dst are written.  64x64 tiles of 256
+// threads, 16-byte accesses on both sides (C and ld_src are multiples of 32 elements here, so a 16-byte piece never
+// straddles an edge).
+template <typename T>
+struct TransposeParams {
+  const T* src;
+  T* dst;
+  int64_t ld_src, ld_dst, r_dst;
+  int R, C;
+  const int32_t* order;
+};
+template <typename T>
+__device__ __forceinline__ void transpose_tile(const TransposeParams<T>& p, int r0, int c0) {
+  constexpr int VEC = 16 / (int)sizeof(T);       // elements per 16-byte access
+  constexpr int CPR = 64 / VEC;                  // accesses per 64-wide tile row
+  constexpr int RPP = 256 / CPR;                 // tile rows covered per pass
+  constexpr int kE = kRowBytes / (int)sizeof(T);
+  __shared__ T tile[64][64 + VEC];               // [c][r], padded rows
+  const int q = threadIdx.x % CPR, row = threadIdx.x / CPR;
+  for (int rr = row; rr < 64; rr += RPP) {
+    const int r = r0 + rr, c = c0 + q * VEC;
+    alignas(16) T vals[VEC];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) vals[j] = (T)0.f;
+    if (r < p.R && c < p.C)
+      *reinterpret_cast<u32x4*>(vals) = *reinterpret_cast<const u32x4*>(p.src + (int64_t)(p.order ? p.order[r] : r) * p.ld_src + c);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) tile[q * VEC + j][rr] = vals[j];
+  }
+  __syncthreads();
+  for (int cc = row; cc < 64; cc += RPP) {
+    const int c = c0 + cc, r = r0 + q * VEC;
+    if (c < p.C && r < p.r_dst)
+      *reinterpret_cast<u32x4*>(p.dst + blocked_index<T>(c, r, p.ld_dst / kE)) = *reinterpret_cast<const u32x4*>(&tile[cc][q * VEC]);
+  }
+}
+template <typename T>
+__global__ __launch_bounds__(256) void transpose_block_kernel(TransposeParams<T> p) {
+  transpose_tile<T>(p, blockIdx.y * 64, blockIdx.x * 64);
+}
+
 // d(logits) from kept logits: in place, or into the operands of dW that the caller keeps.  HBM-bound: reads and writes the
 // chunk once.  A thread owns one 16-byte piece of one or two tokens in every unit that its workgroup walks: their
 // coefficients stay in registers, the loads of kAhead units are in flight together, and a wave's access is one kilobyte.
+// The last workgroups of the launch write hidden^T, dW's other operand, which took a launch of 5 to 12 us of its own.
 // 12126 rows of the 152k vocabulary: 2.25 -> 1.49 ms, 32768 rows 5.92 -> 3.57 ms (5.6 TB/s), against a pass that also wrote the
 // transpose.
+template <typename T>
 struct DzFromZParams {
   const void* z;      // kept logits (KeptLogit<T>): z_kslab units per row of units
   void* dz;           // d(logits) (T): dz_kslab units per row of units
@@ -154,17 +198,23 @@ struct DzFromZParams {
   const int32_t* order;   // optional [Tc]: row n is token order[n] of the per-token arrays
   int64_t z_kslab, dz_kslab;
   int Tc, V, n_units;     // n_units: units of dz per row of units
+  int n_step;             // workgroups per row of units; more of them along y turn 64 columns of hidden each
   float c, inv_temperature;
+  TransposeParams<T> turn;
 };
 
 template <typename T, bool kEntropy>
-__global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams p) {
+__global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams<T> p) {
   typedef typename KeptLogit<T>::type ZT;
   static_assert(sizeof(ZT) == sizeof(T), "d(logits) overwrites the kept logits in place");
   constexpr int E = Elem<T>::kSlabK;                // tokens and vocabulary entries of a unit (64 or 32)
   constexpr int VEC = 16 / (int)sizeof(T);          // elements per 16-byte piece
   constexpr int kRows = E / 32;                     // tokens per thread
   constexpr int kAhead = 4;                         // units in flight
+  if ((int)blockIdx.y >= p.n_step) {                // the same for the whole workgroup
+    if (blockIdx.x * E % 64 == 0) transpose_tile<T>(p.turn, blockIdx.x * E, ((int)blockIdx.y - p.n_step) * 64);
+    return;
+  }
   const int q = threadIdx.x & 7, row = threadIdx.x >> 3;
   const float it = p.inv_temperature;
   float lse[kRows], lse2[kRows], glp[kRows], gen[kRows], ent[kRows];
@@ -190,7 +240,7 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams p) {
   const int at = row * kRowBytes + q * 16;          // byte of this thread's first piece within a unit
   const char* z = static_cast<const char*>(p.z) + (int64_t)blockIdx.x * p.z_kslab * (E * kRowBytes) + at;
   char* dz = static_cast<char*>(p.dz) + (int64_t)blockIdx.x * p.dz_kslab * (E * kRowBytes) + at;
-  const int step = gridDim.y;
+  const int step = p.n_step;
   for (int k0 = blockIdx.y; k0 < p.n_units; k0 += kAhead * step) {
     u32x4 raw[kAhead][kRows];
 #pragma unroll
@@ -546,37 +596,6 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   else for (int k = 0; k < 4; ++k) dst[k] = out.x[k];
 }
 
-// dst(c, r) = src[r][c] (src[order[r]][c] with an order) for r < R, c < C and 0 for R <= r < r_dst, where dst is the K-blocked
-// operand with C rows and ld_dst K elements (see blocked_index), of which the first r_dst are written.  64x64 tiles, 16-byte accesses on
-// both sides (C and ld_src are multiples of 32 elements here, so a 16-byte piece never straddles an edge).
-template <typename T>
-__global__ __launch_bounds__(256) void transpose_block_kernel(const T* __restrict__ src, int64_t ld_src,
-                                                              T* __restrict__ dst, int64_t ld_dst, int64_t r_dst, int R, int C,
-                                                              const int32_t* __restrict__ order) {
-  constexpr int VEC = 16 / (int)sizeof(T);       // elements per 16-byte access
-  constexpr int CPR = 64 / VEC;                  // accesses per 64-wide tile row
-  constexpr int RPP = 256 / CPR;                 // tile rows covered per pass
-  constexpr int kE = kRowBytes / (int)sizeof(T);
-  __shared__ T tile[64][64 + VEC];               // [c][r], padded rows
-  const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
-  const int q = threadIdx.x % CPR, row = threadIdx.x / CPR;
-  for (int rr = row; rr < 64; rr += RPP) {
-    const int r = r0 + rr, c = c0 + q * VEC;
-    alignas(16) T vals[VEC];
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) vals[j] = (T)0.f;
-    if (r < R && c < C) *reinterpret_cast<u32x4*>(vals) = *reinterpret_cast<const u32x4*>(src + (int64_t)(order ? order[r] : r) * ld_src + c);
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) tile[q * VEC + j][rr] = vals[j];
-  }
-  __syncthreads();
-  for (int cc = row; cc < 64; cc += RPP) {
-    const int c = c0 + cc, r = r0 + q * VEC;
-    if (c < C && r < r_dst)
-      *reinterpret_cast<u32x4*>(dst + blocked_index<T>(c, r, ld_dst / kE)) = *reinterpret_cast<const u32x4*>(&tile[cc][q * VEC]);
-  }
-}
-
 // K ranges per tile that fill `cus` CUs best (1 = no split): work items = tiles x ranges, and a launch
 // takes ceil(items / cus) rounds.  At most kMaxKSplit ranges, each at least 8 slabs long and none empty,
 // and at most what `partial_bytes` can hold of fp32 partial tiles.  Fewer tiles than cus / kMaxKSplit may use twice as
@@ -865,10 +884,9 @@ static int launch_dweight(const GemmIn& in, int M, int N, int K, void* C, int64_
 }
 
 template <typename T>
-static int launch_transpose(const T* src, int64_t ld_src, T* dst, int64_t r_dst, int R, int C, hipStream_t stream,
-                            const int32_t* order = nullptr, int64_t ld_dst = 0) {
-  dim3 grid((C + 63) / 64, (int)((r_dst + 63) / 64));
-  hipLaunchKernelGGL(transpose_block_kernel<T>, grid, dim3(256), 0, stream, src, ld_src, dst, ld_dst ? ld_dst : r_dst, r_dst, R, C, order);
+static int launch_transpose(const TransposeParams<T>& p, hipStream_t stream) {
+  dim3 grid((p.C + 63) / 64, (int)((p.r_dst + 63) / 64));
+  hipLaunchKernelGGL(transpose_block_kernel<T>, grid, dim3(256), 0, stream, p);
   return check_launch("transpose_block_kernel");
 }
 
@@ -910,7 +928,7 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
   if (rc) return rc;
   if (a->dhidden && wt && !a->weight_t_ready) {
     // the caller keeps W^T: WT(h, v) = W[v][h], zero for V <= v < ldv, K-blocked
-    rc = launch_transpose<T>(weight, H, wt, pl.ldv, (int)V, (int)H, stream);
+    rc = launch_transpose(TransposeParams<T>{weight, wt, H, pl.ldv, pl.ldv, (int)V, (int)H, nullptr}, stream);
     if (rc) return rc;
   }
   for (int64_t c0 = 0; c0 < T_; c0 += chunk) {
@@ -928,8 +946,11 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
     // with an order the chunk's tokens are looked up from the start of the arrays, without they follow one another
     const int64_t t0 = rows.order ? 0 : c0;
     const int32_t* order = rows.order ? rows.order + c0 : nullptr;
+    // hidT(h, t) = hidden[c0 + t][h], zero for tc <= t < ldt, K-blocked
+    const bool want_dw = a->dweight || kept;
+    const TransposeParams<T> turn{hidden + t0 * H, hidt, H, ld_dw, ldt, (int)tc, (int)H, order};
     if (saved) {
-      DzFromZParams q;
+      DzFromZParams<T> q;
       q.z = z;
       q.dz = dz;
       q.labels = a->labels + t0;
@@ -950,7 +971,9 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
       const int64_t n_rows = ldt / E;
       int64_t per_row = (16 * (int64_t)device_cu_count() + n_rows - 1) / n_rows;
       if (per_row > q.n_units) per_row = q.n_units;
-      dim3 grid((unsigned)n_rows, (unsigned)per_row);
+      q.n_step = (int)per_row;
+      q.turn = turn;
+      dim3 grid((unsigned)n_rows, (unsigned)(per_row + (want_dw ? (H + 63) / 64 : 0)));
       if (q.g_ent) hipLaunchKernelGGL((dz_from_z_kernel<T, true>), grid, dim3(256), 0, stream, q);
       else hipLaunchKernelGGL((dz_from_z_kernel<T, false>), grid, dim3(256), 0, stream, q);
       rc = check_launch("dz_from_z_kernel");
@@ -978,6 +1001,7 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
       int grid = (d.n_tb * d.n_vt + 7) / 8 * 8;
       hipLaunchKernelGGL(lmhead_dz_kernel<T>, dim3(grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, d);
       rc = check_launch("lmhead_dz_kernel");
+      if (rc == 0 && want_dw) rc = launch_transpose(turn, stream);
       if (rc) return rc;
     }
     if (a->dhidden) {
@@ -989,11 +1013,6 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
                                                stream, part, pl.part_bytes, out_rows)
               : launch_dhidden<T, Side::kWeight>(GemmIn{weight, dz, H, dz_kslab, (int)V}, (int)H, (int)tc, (int)pl.ldv, out, H,
                                                  stream, part, pl.part_bytes, out_rows);
-      if (rc) return rc;
-    }
-    if (a->dweight || kept) {
-      // hidT(h, t) = hidden[c0 + t][h], zero for tc <= t < ldt, K-blocked
-      rc = launch_transpose<T>(hidden + t0 * H, H, hidt, ldt, (int)tc, (int)H, stream, order, ld_dw);
       if (rc) return rc;
     }
     if (a->dweight && !kept) {

@@ -52,6 +52,7 @@ struct LossParams {
   double* sums;        // [kNumSums] out (written directly by the one-workgroup kernel)
   float* seq_mean;     // workspace [B] (GSPO)
   double* partials;    // workspace [blocks][kNumSums]
+  StepResult step;
 };
 
 __device__ __forceinline__ int seq_of_token(const LossParams& p, int64_t i) {
@@ -239,6 +240,35 @@ __global__ __launch_bounds__(kLossThreads) void policy_loss_kernel(LossParams p)
 }
 
 
+// The last workgroup of a loss call: its sums and flag word (threads 0 to kNumSums pass one each), then, where a step wants
+// one, the result over all its chunks.  A launch of its own for the result took 4 to 5 us of a step
+// (200 tokens of H = 1024 over 32000 entries: 149 -> 137 us together with the launch that hidden^T had).
+__device__ __forceinline__ void write_sums(double (&total)[kNumSums], const int& flag, double* sums, int32_t* flags, const StepResult& step) {
+  const int k = threadIdx.x;
+  if (k < kNumSums) sums[k] = total[k];
+  if (k == kNumSums) flags[0] = flag;
+  if (step.result == nullptr) return;      // the same for all threads
+  if (k < kNumSums) {
+    double s = 0.0;
+    for (int c = 0; c < step.chunk; ++c) s += step.sums[kNumSums * c + k];
+    s += total[k];
+    total[k] = s;
+    step.result[k] = s;
+  }
+  __syncthreads();
+  if (k == 0) {
+    const double pg = total[0] * step.scale, kl = total[1] * step.scale, en = total[2] * step.scale;
+    double loss = pg;
+    if (step.entropy_coef > 0) loss -= step.entropy_coef * en;
+    if (step.kl_coef > 0) loss += step.kl_coef * kl;
+    int f = 0;
+    for (int c = 0; c < step.chunk; ++c) f |= step.flags[c];
+    f |= flag;
+    step.result[8] = pg; step.result[9] = kl; step.result[10] = en; step.result[11] = loss;
+    step.result[12] = (double)f; step.result[13] = total[3];
+  }
+}
+
 // The whole call in one workgroup: sequence means (one wavefront per sequence), a barrier, the
 // per-token pass, the reductions, sums and flag word.  Nothing has to be zeroed beforehand and the
 // summation order is fixed.
@@ -276,35 +306,42 @@ __global__ __launch_bounds__(kOneWgThreads) void policy_loss_onewg_kernel(LossPa
     sh_flag[wave] = flag;
   }
   __syncthreads();
+  __shared__ double total[kNumSums];
+  __shared__ int all_flags;
   if (threadIdx.x < kNumSums) {
     double t = 0;
     for (int w = 0; w < kOneWgThreads / 64; ++w) t += sh[w][threadIdx.x];
-    p.sums[threadIdx.x] = t;
+    total[threadIdx.x] = t;
   }
   if (threadIdx.x == kNumSums) {
     int f = 0;
     for (int w = 0; w < kOneWgThreads / 64; ++w) f |= sh_flag[w];
-    p.flags[0] = f;
+    all_flags = f;
   }
+  __syncthreads();
+  write_sums(total, all_flags, p.sums, p.flags, p.step);
 }
 
 // Fixed-order pass over the per-block partials: one wavefront per sum (lane l adds blocks l, l + 64, ...,
 // then a shuffle tree), and the flag word OR-ed from the blocks' flag slots.  Launched with kNumSums * 64 threads.
-__global__ void policy_loss_finalize_kernel(const double* partials, int n_blocks, double* sums, int32_t* flags) {
+__global__ void policy_loss_finalize_kernel(const double* partials, int n_blocks, double* sums, int32_t* flags, StepResult step) {
   const int k = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (k >= kNumSums) return;
+  __shared__ double total[kNumSums];
+  __shared__ int all_flags;
   if (k == kNumSums - 1) {
     int f = 0;
     for (int b = lane; b < n_blocks; b += 64) f |= (int)partials[(int64_t)b * kNumSums + k];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) f |= __shfl_xor(f, off);
-    if (lane == 0) { flags[0] = f; sums[k] = 0.0; }
-    return;
+    if (lane == 0) { all_flags = f; total[k] = 0.0; }
+  } else {
+    double t = 0;
+    for (int b = lane; b < n_blocks; b += 64) t += partials[(int64_t)b * kNumSums + k];
+    t = wave_sum(t);
+    if (lane == 0) total[k] = t;
   }
-  double t = 0;
-  for (int b = lane; b < n_blocks; b += 64) t += partials[(int64_t)b * kNumSums + k];
-  t = wave_sum(t);
-  if (lane == 0) sums[k] = t;
+  __syncthreads();
+  write_sums(total, all_flags, sums, flags, step);
 }
 
 // Masked sums of up to kMaxMaskedSums per-token tensors in one launch of one workgroup (fixed
@@ -381,7 +418,8 @@ extern "C" size_t clgrpo_policy_loss_workspace_bytes(int64_t n, int64_t B) {
 }
 
 // Validation and launches shared by the entry points; `ws` is the scratch memory they differ in.
-int clgrpo::head_policy_loss(const char* who, const clgrpo_policy_loss_args* a, void* ws_ptr, size_t ws_bytes, hipStream_t s) {
+int clgrpo::head_policy_loss(const char* who, const clgrpo_policy_loss_args* a, void* ws_ptr, size_t ws_bytes, hipStream_t s,
+                             const StepResult& step) {
   CLGRPO_REQUIRE_PTR(a, "args");
   if (a->mode != CLGRPO_LOSS_GRPO && a->mode != CLGRPO_LOSS_GSPO)
     return fail(CLGRPO_EINVAL, "%s: mode %d", who, a->mode);
@@ -422,6 +460,7 @@ int clgrpo::head_policy_loss(const char* who, const clgrpo_policy_loss_args* a, 
   p.is_pos = a->is_positive_clipped; p.is_neg = a->is_negative_clipped; p.is_clip = a->is_clipped;
   p.g_logprob = a->g_logprob; p.g_entropy = a->g_entropy; p.flags = a->flags;
   p.sums = a->sums;
+  p.step = step;
   char* ws = static_cast<char*>(ws_ptr);
   p.seq_mean = reinterpret_cast<float*>(ws);
   p.partials = reinterpret_cast<double*>(ws + align_up((size_t)a->B * sizeof(float), 256));
@@ -446,7 +485,7 @@ int clgrpo::head_policy_loss(const char* who, const clgrpo_policy_loss_args* a, 
     hipLaunchKernelGGL(policy_loss_kernel<double>, dim3(blocks), dim3(kLossThreads), 0, s, p);
   int rc = check_launch("policy_loss_kernel");
   if (rc) return rc;
-  hipLaunchKernelGGL(policy_loss_finalize_kernel, dim3(1), dim3(kNumSums * 64), 0, s, p.partials, blocks, a->sums, a->flags);
+  hipLaunchKernelGGL(policy_loss_finalize_kernel, dim3(1), dim3(kNumSums * 64), 0, s, p.partials, blocks, a->sums, a->flags, step);
   return check_launch("policy_loss_finalize_kernel");
 }
 
