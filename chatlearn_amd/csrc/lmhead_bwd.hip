@@ -308,6 +308,7 @@ struct GemmParams {
   int accumulate;
   int k_split;        // > 1: work item = (tile, K range); fp32 partial tiles go to `partial`
   int k_per_split;    // K extent of one range, a multiple of the slab
+  int xcd_wgs;        // see work_item
   int n_walk;         // > 0: workgroups walk runs of tiles (see gemm_kernel); needs k_split == 1
   float* partial;     // [k_split] copies of C's shape in fp32, densely packed (row stride N or M)
   const int32_t* order;   // kMContig, optional [N]: row n of the result is row order[n] of the `total` rows of C
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
   extern __shared__ __align__(16) char lds[];
 
   // this workgroup's tiles: (mt, nt) first, then `count - 1` steps along the walked operand; one K range
-  int item = xcd_remap(blockIdx.x, gridDim.x), mt, nt, count = 1, ks = 0, k0 = 0, k_len = p.K;
+  int item = work_item(p.xcd_wgs), mt, nt, count = 1, ks = 0, k0 = 0, k_len = p.K;
   if (p.n_walk > 0) {
     const int n_fixed = kMC ? p.n_mt : p.n_nt;       // tiles of the operand that stays
     const int n_moving = kMC ? p.n_nt : p.n_mt;      // tiles of the operand that is walked
@@ -835,8 +836,13 @@ static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64
     const long plain_rounds = ((long)g.n_mt * g.n_nt + cus - 1) / cus;
     if (walk_periods * 100 > plain_rounds * 104) g.n_walk = 0;
   }
-  int grid = ((g.n_walk > 0 ? g.n_walk * n_fixed : g.n_mt * g.n_nt * g.k_split) + 7) / 8 * 8;
-  hipLaunchKernelGGL((gemm_kernel<T, OutT, S, NI>), dim3(grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
+  // One workgroup per tile in several rounds: each round's tiles go to all XCDs, so that they stream the same stretches of
+  // the operands (dhidden of 32768 rows at H = 7168, 14 rounds: 42.4 -> 41.5 ms, of 16384 20.9 -> 20.4; dW of 8192 rows at H =
+  // 5120 9.11 -> 8.75; two and three rounds at H = 4096: no change).
+  ItemGrid grid{(g.n_walk * n_fixed + 7) / 8 * 8, 0};
+  if (g.n_walk == 0) grid = g.k_split == 1 ? item_grid(g.n_mt * g.n_nt, cus) : ItemGrid{(g.n_mt * g.n_nt * g.k_split + 7) / 8 * 8, 0};
+  g.xcd_wgs = grid.xcd_wgs;
+  hipLaunchKernelGGL((gemm_kernel<T, OutT, S, NI>), dim3(grid.grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
   rc = check_launch("gemm_kernel");
   if (rc || g.k_split == 1) return rc;
   return launch_splitk_reduce<OutT>(partial, g.k_split, kMC ? N : M, kMC ? M : N, static_cast<OutT*>(C), ldc, accumulate,

@@ -1,0 +1,31 @@
+"""Products of the backward with more tiles than compute units, one workgroup per tile: every tile is made once, whichever
+XCD its round hands it to."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# dhidden of 33 x 16 tiles, dW of 36 x 16, of 37 x 28 with ragged edges, and one tile more than a round
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,H,V", [(8200, 4096, 300), (130, 4096, 9000), (70, 7104, 9217), (64, 256, 65793)])
+def test_products_against_64_bits(dev, dtype, T, H, V):
+    """bf16: d(logits) rounded to 2^-8, the result once more; fp32: sums of at most 66000 products, 2^-16 of their norm."""
+    from chatlearn_amd import ops
+    g = torch.Generator(device=dev).manual_seed(T + V)
+    hidden = torch.randn(T, H, generator=g, device=dev).to(dtype)
+    weight = (torch.randn(V, H, generator=g, device=dev) * 0.02).to(dtype)
+    labels = torch.randint(0, V, (T,), generator=g, device=dev)
+    g_lp = torch.randn(T, generator=g, device=dev)
+    z = ops.saved_logits_buffer(T, V, dtype, dev)
+    _, _, _, lse = ops.lmhead_forward(hidden, weight, labels, saved_logits=z)
+    dh, dw = ops.lmhead_backward(hidden, weight, labels, lse, None, g_lp, saved_logits=z)
+    h64, w64 = hidden.double(), weight.double()
+    dz = -torch.softmax(h64 @ w64.t(), -1)
+    dz.scatter_add_(1, labels[:, None], torch.ones(T, 1, dtype=torch.float64, device=dev))
+    dz *= g_lp.double()[:, None]
+    tol = 3 * 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -16
+    for got, want in ((dh.double(), dz @ w64), (dw.double(), dz.t() @ h64)):
+        assert (got - want).norm() <= tol * want.norm()
+        blocks = [(got - want)[r:r + 256].norm() <= 2 * tol * want[r:r + 256].norm() + 1e-12 for r in range(0, len(want), 256)]
+        assert all(bool(b) for b in blocks)
