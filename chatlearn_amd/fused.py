@@ -352,6 +352,28 @@ class _ReadBack:
         return self.host.tolist()
 
 
+def _follow_last_use(tensors, stream):
+    """Order ``stream`` behind the calls that used these cached tensors last: on another stream they may still have their
+    backward enqueued.  The tensors' memory then also outlives what ``stream`` does with them.  A capture depends on nothing
+    outside of it: replays are ordered by whoever replays them."""
+    for t in tensors:
+        last = getattr(t, "last_use", None)
+        if last is not None and last[0] != stream and not torch.cuda.is_current_stream_capturing():
+            stream.wait_event(last[1])
+            t.record_stream(stream)
+
+
+def _leave_last_use(tensors, stream):
+    """What ``_follow_last_use`` of a later call waits for: everything this call has enqueued."""
+    if not tensors or torch.cuda.is_current_stream_capturing():
+        return
+    last = getattr(tensors[0], "last_use", None)
+    event = last[1] if last is not None and last[0] == stream else torch.cuda.Event()
+    event.record(stream)
+    for t in tensors:
+        t.last_use = (stream, event)
+
+
 def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages, cu_seqlens, loss_mask, *,
                    n_tokens_total: float, fsdp_size: int = 1, use_group_sequence_policy=False,
                    pos_clip_ratio=0.2, neg_clip_ratio=0.2, diff_clip_ratio=10, final_clip_ratio=3,
@@ -368,6 +390,11 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     per-token ``logprob``/``entropy``, the loss scalars ``pg_loss_mean``,
     ``kl_loss_mean``, ``entropy_loss_mean``, ``total_loss`` (device fp64 scalars),
     ``dhidden`` and ``dweight``.  ``advantages`` is a device tensor [B].
+
+    The call returns while its backward is still running: it waits for the loss flags only (for nothing without
+    ``check_flags``).  As with any operation on the device, inputs, results and a ``dweight`` that is added to belong to
+    the stream that is current in the call; work on another stream has to be ordered behind it (``wait_stream``).  The two
+    caches below look after themselves.
 
     ``keep_logits_chunk``: the micro-batch is walked in token chunks that keep the raw logits of at most
     this many rows (one [chunk, V] buffer of 16-bit or fp32 elements, reused chunk after chunk) so that
@@ -399,13 +426,15 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     ``weight_t_cache``: a dict the caller keeps while ``weight`` does not change (the micro-batches
     of one optimizer step).  The first backward leaves the transposed weight in it and later calls
     contract with that one; the caller clears it after updating the weight.  Without it the weight is
-    read as it is, which is as fast and needs no copy.
+    read as it is, which is as fast and needs no copy.  Calls on different streams may share it, as ``workspace_cache``.
 
     ``workspace_cache``: a dict the caller keeps between calls.  The kept-logits buffer and the forward /
     backward scratch memory (a few GB, sized by the chunk, not by T) then live in it and are reused by every
     later call they are large enough for, instead of being allocated and released per call: micro-batches of
     varying length otherwise ask the framework's allocator for differently sized multi-GB blocks each time,
-    which now and then costs a device-wide stall for a fresh allocation.
+    which now and then costs a device-wide stall for a fresh allocation.  The tensors carry the stream of the last call
+    and an event behind its work (``last_use``): a call on another stream waits for it (on the device), so successive calls may
+    share the dict whatever stream they run on; threads that run at the same time may not.
 
     ``stage_hook(name)`` is called on the host at "forward", "loss", "backward", "end" boundaries
     of every chunk (a benchmark records stream events there).
@@ -507,6 +536,10 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
         ws = cache.get("head_step")
         if ws is None or ws.numel() < need or ws.device != dev:
             ws = cache["head_step"] = torch.empty(need, dtype=torch.uint8, device=dev)
+        cached = [t for t in ((zbuf, ws) if workspace_cache is not None else ()) + ((wt,) if weight_t_cache is not None else ())
+                  if t is not None]
+        stream = torch.cuda.current_stream(dev) if cached else None
+        _follow_last_use(cached, stream)
     rows_projected_bwd = rows_projected_fwd = 0
     if T > 0:
         step = ops.HeadStep(hidden, weight, labels, old_logprob, ref_logprob, advantages, cu_seqlens, loss_mask, order,
@@ -517,30 +550,33 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
                             kl=kl_all, sums=sums_buf, flags=flags_buf, result=result, dhidden=dh_all, dweight=dw,
                             workspace=ws, saved_logits=zbuf, weight_t=wt, dweight_sum=_dweight_sum)
         stages = 7 if need_dhidden or dw is not None or _dweight_sum is not None else 3       # without a result no backward
-        for k, (lo, n, n_live, pick) in enumerate(parts):
-            live_only = bool(skip_masked_forward and pick and n_live > 0)
-            chunk = dict(lo=lo, n=n, n_live=n_live, ordered=pick, chunk=k, forward_live_only=live_only, accumulate=acc_dw,
-                         weight_t_ready=wt_ready)
-            # the flags are complete behind the last chunk's loss: they travel while the backward runs
-            read_flags = check_flags and k == n_chunks - 1
-            if stage_hook is not None:
-                for name, bit in (("forward", 1), ("loss", 2), ("backward", 4)):
-                    stage_hook(name)
-                    step.enqueue(bit & stages, **chunk)
-                    if read_flags and bit == 2:
-                        flags_read = _ReadBack(result[12:])
-                stage_hook("end")
-            elif read_flags:
-                step.enqueue(3, **chunk)
-                flags_read = _ReadBack(result[12:])
-                if stages & 4:
-                    step.enqueue(4, **chunk)
-            else:
-                step.enqueue(stages, **chunk)
-            rows_projected_fwd += n_live if live_only else n
-            rows_projected_bwd += n_live
-            wt_ready = wt_ready or n_live > 0
-            acc_dw = True
+        try:
+            for k, (lo, n, n_live, pick) in enumerate(parts):
+                live_only = bool(skip_masked_forward and pick and n_live > 0)
+                chunk = dict(lo=lo, n=n, n_live=n_live, ordered=pick, chunk=k, forward_live_only=live_only, accumulate=acc_dw,
+                             weight_t_ready=wt_ready)
+                # the flags are complete behind the last chunk's loss: they travel while the backward runs
+                read_flags = check_flags and k == n_chunks - 1
+                if stage_hook is not None:
+                    for name, bit in (("forward", 1), ("loss", 2), ("backward", 4)):
+                        stage_hook(name)
+                        step.enqueue(bit & stages, **chunk)
+                        if read_flags and bit == 2:
+                            flags_read = _ReadBack(result[12:])
+                    stage_hook("end")
+                elif read_flags:
+                    step.enqueue(3, **chunk)
+                    flags_read = _ReadBack(result[12:])
+                    if stages & 4:
+                        step.enqueue(4, **chunk)
+                else:
+                    step.enqueue(stages, **chunk)
+                rows_projected_fwd += n_live if live_only else n
+                rows_projected_bwd += n_live
+                wt_ready = wt_ready or n_live > 0
+                acc_dw = True
+        finally:
+            _leave_last_use(cached, stream)
         if weight_t_cache is not None and wt_ready:
             weight_t_cache["weight_t"] = wt
     else:
