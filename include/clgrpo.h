@@ -57,8 +57,10 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *                 256 tokens): between 2.03 and 3.00 scratch memory sized for a longer call could be too small for a shorter one.
  *                 clgrpo_head_step refuses what a later stage would refuse (or overrun) before it enqueues anything.
  *   3.01 -> 3.02: the opaque buffers saved_logits and kept_dzt hold square units (same sizes);
- *                 clgrpo_lmhead_bwd_workspace_bytes no longer holds a transposed d(logits) (smaller). */
-#define CLGRPO_VERSION 302
+ *                 clgrpo_lmhead_bwd_workspace_bytes no longer holds a transposed d(logits) (smaller).
+ *   3.02 -> 4.00: the number that 3.02 should have had: a caller built against 3.01 that reads kept logits by that header's
+ *                 formula gets entries in another order. */
+#define CLGRPO_VERSION 400
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
 
