@@ -743,7 +743,7 @@ struct BwdPlan {
 };
 
 static BwdPlan bwd_plan(int64_t T, int64_t H, int64_t V, size_t es, int64_t chunk_tokens, bool saved = false,
-                        bool own_wt = true, bool own_dw = true) {
+                        bool own_dw = true) {
   BwdPlan pl;
   pl.ldv = round_up64(V, 64);
   int64_t chunk = (chunk_tokens <= 0 || chunk_tokens >= T) ? T : round_up64(chunk_tokens, 256);
@@ -763,21 +763,17 @@ static BwdPlan bwd_plan(int64_t T, int64_t H, int64_t V, size_t es, int64_t chun
     if (b > part) part = b;
   pl.part_bytes = align_up(part, 256);
   pl.off_part = off; off += pl.part_bytes;
-  // A caller without a W^T of its own has always been asked for the room of one (up to 384 16-bit rows from kept logits
-  // excepted).  W is read as it is now; the sizes that callers plan with stay.
-  const bool few = es == 2 && saved && chunk == T && T <= 384;
-  off += own_wt && !few ? align_up(Hb * pl.ldv * es, 256) : 0;
   pl.total = off;
   return pl;
 }
 
 // Largest chunk (multiple of 256, or T itself) whose plan fits into `bytes`; 0 if none does.
-static int64_t chunk_for_workspace(int64_t T, int64_t H, int64_t V, size_t es, size_t bytes, bool saved, bool own_wt, bool own_dw) {
-  if (bwd_plan(T, H, V, es, T, saved, own_wt, own_dw).total <= bytes) return T;
+static int64_t chunk_for_workspace(int64_t T, int64_t H, int64_t V, size_t es, size_t bytes, bool saved, bool own_dw) {
+  if (bwd_plan(T, H, V, es, T, saved, own_dw).total <= bytes) return T;
   int64_t lo = 0, hi = T / 256;   // in units of 256 tokens
   while (lo < hi) {
     const int64_t mid = (lo + hi + 1) / 2;
-    if (bwd_plan(T, H, V, es, mid * 256, saved, own_wt, own_dw).total <= bytes) lo = mid; else hi = mid - 1;
+    if (bwd_plan(T, H, V, es, mid * 256, saved, own_dw).total <= bytes) lo = mid; else hi = mid - 1;
   }
   return lo * 256;
 }
@@ -914,15 +910,14 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
   using Tile = LogitTile<T>;
   const int64_t T_ = a->T, H = a->H, V = a->V;
   const bool saved = a->saved_logits != nullptr;
-  const bool own_wt = a->weight_t == nullptr;
   const bool own_dw = kept == nullptr;
-  const int64_t chunk = chunk_for_workspace(T_, H, V, sizeof(T), a->workspace_bytes, saved, own_wt, own_dw);
+  const int64_t chunk = chunk_for_workspace(T_, H, V, sizeof(T), a->workspace_bytes, saved, own_dw);
   if (chunk <= 0)
     return fail(CLGRPO_EWORKSPACE, "clgrpo_lmhead_bwd: workspace %zu bytes cannot hold a 256-token chunk (%zu needed)",
-                a->workspace_bytes, bwd_plan(T_, H, V, sizeof(T), 256, saved, own_wt, own_dw).total);
+                a->workspace_bytes, bwd_plan(T_, H, V, sizeof(T), 256, saved, own_dw).total);
   if (a->dweight_bf16 && chunk < T_)
     return fail(CLGRPO_EWORKSPACE, "clgrpo_lmhead_bwd: a 16-bit dweight needs a workspace for all %lld tokens at once", (long long)T_);
-  const BwdPlan pl = bwd_plan(T_, H, V, sizeof(T), chunk, saved, own_wt, own_dw);
+  const BwdPlan pl = bwd_plan(T_, H, V, sizeof(T), chunk, saved, own_dw);
   const int64_t ldz = saved ? a->ld_saved : pl.ldv;
   char* ws = static_cast<char*>(a->workspace);
   T* wt = static_cast<T*>(a->weight_t);
@@ -1037,8 +1032,7 @@ using namespace clgrpo;
 extern "C" size_t clgrpo_lmhead_bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int32_t dtype,
                                                     int64_t chunk_tokens, int32_t with_saved_logits) {
   if (T <= 0 || H <= 0 || V <= 0 || (dtype != CLGRPO_BF16 && dtype != CLGRPO_F32)) return 0;
-  return bwd_plan(T, H, V, dtype_bytes(dtype), chunk_tokens, (with_saved_logits & 1) != 0, (with_saved_logits & 2) == 0,
-                  (with_saved_logits & 4) == 0).total;
+  return bwd_plan(T, H, V, dtype_bytes(dtype), chunk_tokens, (with_saved_logits & 1) != 0, (with_saved_logits & 4) == 0).total;
 }
 
 extern "C" int clgrpo_lmhead_bwd_dhidden_plan(int64_t rows, int64_t H, int64_t V, int32_t dtype, int32_t cus, int32_t* out) {

@@ -600,7 +600,6 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
             "g_logprob": glp_all, "rows_projected_bwd": rows_projected_bwd,
             "rows_projected_fwd": rows_projected_fwd, "sums": result[:8], "token_chunks": chunks,
             # device memory this call held beyond its inputs and outputs: kept logits (they become d(logits) in
-            # place), the workspace (hidden^T, split-K partials, the room a W^T would take unless the caller's cache holds one;
-            # the forward's per-split records before that), the caller's W^T and the operands of dW that wait in a sum
+            # place), the workspace (hidden^T, split-K partials; the forward's per-split records before that), the caller's W^T and the operands of dW that wait in a sum
             "scratch_bytes": sum(t.numel() * t.element_size() for t in (zbuf, ws, wt) if t is not None)
                              + (_dweight_sum.bytes if _dweight_sum is not None else 0)}

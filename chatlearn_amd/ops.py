@@ -13,8 +13,7 @@ from . import _lib
 from ._lib import BF16, F32, F64, U8, LOSS_GRPO, LOSS_GSPO
 
 # Scratch memory a backward call may take when the caller names neither a chunk nor a workspace: the
-# token chunk is halved until the plan fits (d(logits) where no logits were kept, hidden^T, the room of a
-# W^T, split-K partials).
+# token chunk is halved until the plan fits (d(logits) where no logits were kept, hidden^T, split-K partials).
 DEFAULT_BWD_WORKSPACE_BYTES = 8 << 30
 
 

@@ -59,7 +59,8 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *   3.01 -> 3.02: the opaque buffers saved_logits and kept_dzt hold square units (same sizes);
  *                 clgrpo_lmhead_bwd_workspace_bytes no longer holds a transposed d(logits) (smaller).
  *   3.02 -> 4.00: the number that 3.02 should have had: a caller built against 3.01 that reads kept logits by that header's
- *                 formula gets entries in another order. */
+ *                 formula gets entries in another order.  clgrpo_lmhead_bwd_workspace_bytes (and clgrpo_head_step_workspace_bytes)
+ *                 hold no room for a W^T any more: W is read as it is. */
 #define CLGRPO_VERSION 400
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
@@ -157,7 +158,8 @@ typedef struct {
 
 /* Bytes needed to process `chunk_tokens` tokens at a time (chunk_tokens <= 0: all T at once).
  * with_saved_logits is a bit set: bit 0: the d(logits) buffer is the caller's saved_logits, not part of the
- * workspace; bit 1: the caller keeps W^T (weight_t), so the workspace holds no copy of it. */
+ * workspace; bit 1: the caller keeps W^T (weight_t), which no longer makes a difference; bit 2: both operands of dW are left
+ * in the caller's buffers (see kept_dzt of clgrpo_head_step_args). */
 size_t clgrpo_lmhead_bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int32_t dtype,
                                          int64_t chunk_tokens, int32_t with_saved_logits);
 int clgrpo_lmhead_bwd(const clgrpo_lmhead_bwd_args* a, void* stream);
@@ -368,7 +370,7 @@ typedef struct {
   int64_t kept_ld, kept_k;       /* multiples of 64 */
 } clgrpo_head_step_args;
 
-/* flags: 1 = with saved_logits, 2 = the caller keeps weight_t, 4 = with kept_dzt */
+/* flags: 1 = with saved_logits, 2 = the caller keeps weight_t (makes no difference), 4 = with kept_dzt */
 size_t clgrpo_head_step_workspace_bytes(int64_t T, int64_t n_live, int64_t H, int64_t V, int64_t B, int32_t dtype, int32_t flags,
                                         size_t recompute_cap);
 int64_t clgrpo_head_step_max_ordered_bytes(void);
