@@ -182,6 +182,14 @@ def dhidden_launch_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple
     return int(out[0]), int(out[1])
 
 
+def dhidden_tile_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple[int, int, int]:
+    """``dhidden_launch_plan`` and the token rows per tile of its (remaining) launch: 256, or 192 or 128 for 16-bit inputs."""
+    out = (C.c_int32 * 3)()
+    _lib.check(_lib.lib().clgrpo_lmhead_bwd_dhidden_tile_plan(int(rows), int(H), int(V), BF16 if dtype == torch.bfloat16 else F32,
+                                                              int(cus), -1, C.cast(out, C.c_void_p)))
+    return int(out[0]), int(out[1]), int(out[2])
+
+
 def dweight_launch_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple[int, int, int]:
     """(walks or 0, vocabulary tiles of a first launch of equally long walks or 0, K ranges of the launch over the
     remaining vocabulary tiles) for the dW contraction over a chunk of ``rows`` tokens."""

@@ -60,7 +60,7 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *                 clgrpo_lmhead_bwd_workspace_bytes no longer holds a transposed d(logits) (smaller).
  *   3.02 -> 4.00: the number that 3.02 should have had: a caller built against 3.01 that reads kept logits by that header's
  *                 formula gets entries in another order.  clgrpo_lmhead_bwd_workspace_bytes (and clgrpo_head_step_workspace_bytes)
- *                 hold no room for a W^T any more: W is read as it is. */
+ *                 hold no room for a W^T any more: W is read as it is.  clgrpo_lmhead_bwd_dhidden_tile_plan added. */
 #define CLGRPO_VERSION 400
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
@@ -168,6 +168,10 @@ int clgrpo_lmhead_bwd(const clgrpo_lmhead_bwd_args* a, void* stream);
  * all rows), out[1] = K ranges of the (remaining) launch, whose fp32 partial tiles a second pass sums.
  * Host-side arithmetic only; no counterpart in the reference. */
 int clgrpo_lmhead_bwd_dhidden_plan(int64_t rows, int64_t H, int64_t V, int32_t dtype, int32_t cus, int32_t* out);
+/* The same with out[2] = token rows per tile of the (remaining) launch (256, or 192 or 128 where that wastes less), for a
+ * workspace with room for partial_bytes of partial tiles (< 0: as much as clgrpo_lmhead_bwd_workspace_bytes asks for). */
+int clgrpo_lmhead_bwd_dhidden_tile_plan(int64_t rows, int64_t H, int64_t V, int32_t dtype, int32_t cus, int64_t partial_bytes,
+                                        int32_t* out);
 /* How the dW contraction over a chunk of `rows` tokens is launched: out[0] = walks (workgroups that keep one
  * 256-column tile of hidden^T and walk runs of vocabulary tiles; 0: one workgroup per tile), out[1] = vocabulary
  * tiles of a first launch whose walks are all equally long (0: one launch over all of them), out[2] = K ranges of
