@@ -491,6 +491,16 @@ extern "C" int clgrpo_lmhead_fwd_launch_plan(int64_t T, int64_t V, int32_t cus, 
   return CLGRPO_OK;
 }
 
+extern "C" int clgrpo_lmhead_fwd_tile_plan(int64_t T, int64_t V, int32_t dtype, int32_t cus, int32_t* out) {
+  if (T <= 0 || V <= 0 || out == nullptr || (dtype != CLGRPO_BF16 && dtype != CLGRPO_F32)) return CLGRPO_EINVAL;
+  const FwdPlan pl = fwd_plan(T, (int)((V + kFwdBM - 1) / kFwdBM), cus, dtype == CLGRPO_BF16);
+  out[0] = pl.n_tb;
+  out[1] = pl.n_split;
+  out[2] = pl.tiles_per_split;
+  out[3] = 32 * pl.ni;
+  return CLGRPO_OK;
+}
+
 extern "C" size_t clgrpo_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int32_t dtype) {
   (void)H;
   (void)dtype;

@@ -272,30 +272,34 @@ def _token_chunks(T, chunk_rows, seq_bounds, live_cum=None, n_ranges=None):
 
 def _launch_cost(chunks, live_cum, H, V, dtype=torch.bfloat16, cus=256):
     """Relative time of the three GEMM-shaped passes of every chunk, in units of one 256 x 256 tile over one
-    K element on one CU: a launch of n work items takes ceil(n / cus) rounds.  Asks the library for its
-    launch plans (vocabulary splits of the forward, bulk / K-split launches of the dhidden and dW GEMMs);
-    the passes that do not depend on the cuts (d(logits), transposes) are left out, the read of dW's previous contents by every chunk after the first is counted."""
+    K element on one CU: a launch of n work items takes ceil(n / cus) rounds, a tile of fewer tokens its share of that
+    and what its plan adds to it.  Asks the library for its launch plans (token blocks and vocabulary splits of the
+    forward, row tiles and bulk / K-split launches of the dhidden and dW GEMMs); the passes that do not
+    depend on the cuts (d(logits), transposes) are left out, the read of dW's previous contents by every chunk after the
+    first is counted."""
     n_vt = -(-V // 256)
     n_ht = -(-H // 256)
+    tile = lambda width: width / 256 * (1.0 + 0.02 * (256 - width) / 32)
     cost = 0.0
     for k, (lo, hi) in enumerate(chunks):
         rows = (hi - lo) if live_cum is None else int(live_cum[hi] - live_cum[lo])
-        n_tb, _, tps = ops.lmhead_forward_launch_plan(hi - lo, V, cus)
-        cost += -(-(n_tb * -(-n_vt // tps)) // cus) * tps * H
+        n_tb, _, tps, width = ops.lmhead_forward_tile_plan(hi - lo, V, dtype, cus)
+        cost += -(-(n_tb * -(-n_vt // tps)) // cus) * tps * H * tile(width)
         if rows == 0:
             continue
-        bulk_nt, ks = ops.dhidden_launch_plan(rows, H, V, dtype, cus)
-        n_rt = -(-rows // 256)
+        bulk_nt, ks, width = ops.dhidden_tile_plan(rows, H, V, dtype, cus)
         if bulk_nt:
             cost += -(-(bulk_nt * n_ht) // cus) * V
-        cost += -(-((n_rt - bulk_nt) * n_ht * ks) // cus) * (V / ks)
+        cost += -(-(-(-(rows - 256 * bulk_nt) // width) * n_ht * ks) // cus) * (V / ks) * tile(width)
         n_walk, bulk_vt, ks_w = ops.dweight_launch_plan(rows, H, V, dtype, cus)   # dW: walks over vocabulary tiles, K-split tail
         if bulk_vt:
             cost += (bulk_vt // n_walk) * rows + -(-((n_vt - bulk_vt) * n_ht * ks_w) // cus) * (rows / ks_w)
         else:
             cost += (-(-n_vt // n_walk) if n_walk else -(-(n_vt * n_ht) // cus)) * rows
         if k > 0:
-            cost += 0.15 * n_vt * n_ht / cus * 2048            # re-reading dW [V,H] fp32: HBM time in the same unit
+            # re-reading dW [V,H] fp32: HBM time in the same unit, which is ten times as long in fp32 (4888 rows of H = 4096, V =
+            # 32000 under a bound of 2048: 5 ranges 27.8 ms, 3 ranges 28.5)
+            cost += (0.015 if dtype == torch.float32 else 0.15) * n_vt * n_ht / cus * 2048
     return cost
 
 

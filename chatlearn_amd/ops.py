@@ -173,6 +173,14 @@ def lmhead_forward_launch_plan(T: int, V: int, cus: int = 0) -> Tuple[int, int, 
     return int(out[0]), int(out[1]), int(out[2])
 
 
+def lmhead_forward_tile_plan(T: int, V: int, dtype, cus: int = 0) -> Tuple[int, int, int, int]:
+    """``lmhead_forward_launch_plan`` for inputs of ``dtype``, and the tokens per block: 128 to 256 (fp32: 256)."""
+    out = (C.c_int32 * 4)()
+    _lib.check(_lib.lib().clgrpo_lmhead_fwd_tile_plan(int(T), int(V), BF16 if dtype == torch.bfloat16 else F32, int(cus),
+                                                      C.cast(out, C.c_void_p)))
+    return int(out[0]), int(out[1]), int(out[2]), int(out[3])
+
+
 def dhidden_launch_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple[int, int]:
     """(256-token tiles of a first launch without a K split or 0, K ranges of the remaining launch) for the
     dhidden contraction of ``rows`` tokens."""

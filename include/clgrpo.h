@@ -60,7 +60,8 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *                 clgrpo_lmhead_bwd_workspace_bytes no longer holds a transposed d(logits) (smaller).
  *   3.02 -> 4.00: the number that 3.02 should have had: a caller built against 3.01 that reads kept logits by that header's
  *                 formula gets entries in another order.  clgrpo_lmhead_bwd_workspace_bytes (and clgrpo_head_step_workspace_bytes)
- *                 hold no room for a W^T any more: W is read as it is.  clgrpo_lmhead_bwd_dhidden_tile_plan added. */
+ *                 hold no room for a W^T any more: W is read as it is.  clgrpo_lmhead_bwd_dhidden_tile_plan and
+ *                 clgrpo_lmhead_fwd_tile_plan added. */
 #define CLGRPO_VERSION 400
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
@@ -116,6 +117,8 @@ int clgrpo_lmhead_fwd(const clgrpo_lmhead_fwd_args* a, void* stream);
  * rounds of one workgroup per compute unit.  Host-side arithmetic only; no counterpart in the reference
  * (its lm_head is one library GEMM). */
 int clgrpo_lmhead_fwd_launch_plan(int64_t T, int64_t V, int32_t cus, int32_t* out);
+/* The same for inputs of `dtype`, with out[3] = tokens per block. */
+int clgrpo_lmhead_fwd_tile_plan(int64_t T, int64_t V, int32_t dtype, int32_t cus, int32_t* out);
 
 /* ------------------------------------------------------------------ *
  * Backward of the fused head: recomputes logit tiles from hidden, W and the
