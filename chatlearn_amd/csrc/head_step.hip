@@ -129,11 +129,13 @@ extern "C" int clgrpo_head_step(const clgrpo_head_step_args* a, void* stream) {
     const int rc = head_forward(who, &f, 0, nullptr, rows, s);
     if (rc) return rc;
   }
-  if (a->n_live < a->T && (((a->stages & 1) && n_fwd < a->T) || ((a->stages & 4) && a->dhidden))) {
+  const bool clear_outputs = (a->stages & 1) && n_fwd < a->T;
+  const bool clear_dhidden = a->dhidden && (a->stages & (a->stages & 8 ? 1 : 4));
+  if (a->n_live < a->T && (clear_outputs || clear_dhidden)) {
     MaskedRows m = {};
     m.rows = a->row_order + a->n_live;
-    if (a->stages & 4) { m.dhidden = static_cast<char*>(a->dhidden); m.row_bytes = a->H * (int64_t)dtype_bytes(a->dtype); }
-    if ((a->stages & 1) && n_fwd < a->T) { m.logprob = a->logprob; m.entropy = a->entropy; m.lse = a->lse; }
+    if (clear_dhidden) { m.dhidden = static_cast<char*>(a->dhidden); m.row_bytes = a->H * (int64_t)dtype_bytes(a->dtype); }
+    if (clear_outputs) { m.logprob = a->logprob; m.entropy = a->entropy; m.lse = a->lse; }
     hipLaunchKernelGGL(masked_rows_kernel, dim3((unsigned)(a->T - a->n_live)), dim3(256), 0, s, m);
     const int rc = check_launch("masked_rows_kernel");
     if (rc) return rc;

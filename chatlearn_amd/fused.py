@@ -569,10 +569,11 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
                             flags_read = _ReadBack(result[12:])
                     stage_hook("end")
                 elif read_flags:
-                    step.enqueue(3, **chunk)
+                    # 8: one launch clears all of the masked rows (four padded samples launch it 4 times instead of 8)
+                    step.enqueue(3 | 8 if stages & 4 else 3, **chunk)
                     flags_read = _ReadBack(result[12:])
                     if stages & 4:
-                        step.enqueue(4, **chunk)
+                        step.enqueue(4 | 8, **chunk)
                 else:
                     step.enqueue(stages, **chunk)
                 rows_projected_fwd += n_live if live_only else n

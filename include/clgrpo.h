@@ -61,7 +61,7 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *   3.02 -> 4.00: the number that 3.02 should have had: a caller built against 3.01 that reads kept logits by that header's
  *                 formula gets entries in another order.  clgrpo_lmhead_bwd_workspace_bytes (and clgrpo_head_step_workspace_bytes)
  *                 hold no room for a W^T any more: W is read as it is.  clgrpo_lmhead_bwd_dhidden_tile_plan and
- *                 clgrpo_lmhead_fwd_tile_plan added. */
+ *                 clgrpo_lmhead_fwd_tile_plan added, and 8 among the stages of clgrpo_head_step. */
 #define CLGRPO_VERSION 400
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
@@ -347,7 +347,10 @@ typedef struct {
   int32_t forward_live_only;     /* leave the other rows out of the forward too: their logprob / entropy / lse are 0 */
   int32_t accumulate_dweight;
   int32_t weight_t_ready;
-  int32_t stages;                /* 1 forward | 2 loss | 4 backward: which of them this call enqueues (7: all) */
+  int32_t stages;                /* 1 forward | 2 loss | 4 backward: which of them this call enqueues (7: all).  8: the dhidden
+                                    rows without a gradient are cleared by the call with the forward, in the launch that
+                                    clears their other outputs, and not by the one with the backward (a chunk whose stages
+                                    come in several calls sets it in all of them or in none) */
   float inv_temperature;
   double diff_clip_ratio, pos_clip_ratio, neg_clip_ratio, final_clip_ratio, kl_coef, entropy_coef, grad_scale;
   float* logprob;                /* [T] out */

@@ -1,4 +1,4 @@
-"""A head step returns while its backward is still enqueued, so a call on another stream that shares its caches has to be ordered
+"""What a head step enqueues, and on what: it returns while its backward is still enqueued, so a call on another stream that shares its caches has to be ordered
 behind it.  The launches are replaced by a log here; the streams and events are names."""
 import pytest
 import torch
@@ -111,3 +111,8 @@ def test_capture_neither_waits_nor_leaves_an_event(on):
     assert not any(e[0] in ("wait", "record") for e in on.log[before:])
     on("c", workspace_cache=cache)
     assert ("wait", "c", _launches(on.log, "a")) in on.log
+
+
+def test_the_two_calls_of_a_checked_step_clear_masked_rows_together(on):
+    on("a")
+    assert [e[2] for e in on.log if e[0] == "enqueue"] == [1 | 2 | 8, 4 | 8]
