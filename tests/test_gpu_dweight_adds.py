@@ -6,13 +6,16 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# walks over many vocabulary tiles with a ragged last row and column tile, their K-split tail, one workgroup per tile, fp32
+# one workgroup per tile; walks over many vocabulary tiles with a ragged last row and column tile; walks and a K-split tail behind them
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("T,H,V", [(1, 64, 3), (130, 192, 257), (200, 960, 66049), (70, 1024, 65537), (640, 1088, 70001)])
+@pytest.mark.parametrize("T,H,V", [(1, 64, 3), (130, 192, 257), (200, 960, 66049), (70, 1024, 65537), (640, 1088, 70001),
+                                   (1300, 960, 66049)])
 def test_added_equals_overwritten_plus_old(dev, dtype, T, H, V):
     """The same products are summed in the same order, from the old value instead of from 0: each of at most T additions rounds
     to 2^-24 of a partial sum, which |old| + sum over t of |g_t| max|h_t| bounds."""
     from chatlearn_amd import ops
+    n_walk, bulk, k_ranges = ops.dweight_launch_plan(T, H, V, dtype)
+    assert (n_walk > 0) == (V > 60000) and (bulk > 0 and k_ranges > 1) == (T == 1300)
     g = torch.Generator(device=dev).manual_seed(T + V)
     hidden = torch.randn(T, H, generator=g, device=dev).to(dtype)
     weight = (torch.randn(V, H, generator=g, device=dev) * 0.05).to(dtype)

@@ -6,7 +6,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# (tokens, vocabulary): the width each takes is asserted through the launch plan's number of blocks
+# (tokens, vocabulary, the block width that the plan takes)
 CASES = [(1, 300, 128), (128, 9000, 128), (129, 70000, 160), (160, 70000, 160), (161, 70000, 192), (193, 70000, 224), (224, 70000, 224),
          (225, 70000, 256), (257, 70000, 160), (321, 70000, 192), (385, 70000, 224), (449, 70000, 256), (600, 70000, 128)]
 
@@ -18,8 +18,8 @@ def test_forward_and_backward_of_every_width(dev, T, V, width, ordered):
     bf16 and the softmax rebuilt from half logits (2^-8 each at most), the result rounded once more; the bound is on rows."""
     from chatlearn_amd import ops
     H = 128
-    n_tb = ops.lmhead_forward_launch_plan(T, V)[0]
-    assert n_tb == -(-T // width)
+    n_tb, _, _, planned = ops.lmhead_forward_tile_plan(T, V, torch.bfloat16)
+    assert planned == width and n_tb == -(-T // width)
     g = torch.Generator(device=dev).manual_seed(T + V)
     hidden = torch.randn(T, H, generator=g, device=dev).bfloat16()
     weight = (torch.randn(V, H, generator=g, device=dev) * 0.1).bfloat16()
@@ -48,12 +48,16 @@ def test_forward_and_backward_of_every_width(dev, T, V, width, ordered):
     assert (dw.double() - dw64).norm() < 3 * 2.0 ** -8 * dw64.norm()
 
 
-@pytest.mark.parametrize("rows", [1, 127, 128, 129, 190, 192, 193, 257, 320, 384, 385])
-def test_dhidden_of_few_rows_matches_itself_row_by_row(dev, rows):
+@pytest.mark.parametrize("rows,H,width", [(rows, 256, 128) for rows in (1, 127, 128, 129, 190, 192, 193, 257, 320, 384, 385)] +
+                         [(1, 2048, 128), (128, 2048, 128), (129, 2048, 192), (192, 2048, 192), (193, 2048, 256), (256, 2048, 256),
+                          (257, 2048, 192), (320, 2048, 192), (384, 2048, 192), (385, 2048, 256)])
+def test_dhidden_of_few_rows_matches_itself_row_by_row(dev, rows, H, width):
     """dhidden's row tiles and K ranges depend on the number of rows; a row's gradient does not, but for the order of an fp32
     sum over 33000 entries and the rounding to bf16: 2^-8 of the row's norm."""
     from chatlearn_amd import ops
-    H, V = 256, 33000
+    V = 33000
+    bulk, k_ranges, planned = ops.dhidden_tile_plan(rows, H, V, torch.bfloat16)
+    assert bulk == 0 and k_ranges > 1 and planned == width
     g = torch.Generator(device=dev).manual_seed(5)
     hidden = torch.randn(400, H, generator=g, device=dev).bfloat16()
     weight = (torch.randn(V, H, generator=g, device=dev) * 0.1).bfloat16()

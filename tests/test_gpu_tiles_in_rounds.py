@@ -6,12 +6,18 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# dhidden of 33 x 16 tiles, dW of 36 x 16, of 37 x 28 with ragged edges, and one tile more than a round
+# dhidden of 43 x 16 tiles of 192 rows (fp32: 33 x 16 of 256); dW of 36 x 16, of 64 x 28 with ragged edges, and one tile more than a
+# round; beside them dW of 37 x 28, which workgroups walk
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("T,H,V", [(8200, 4096, 300), (130, 4096, 9000), (70, 7104, 9217), (64, 256, 65793)])
-def test_products_against_64_bits(dev, dtype, T, H, V):
+@pytest.mark.parametrize("T,H,V,plain", [(8200, 4096, 300, "dhidden"), (130, 4096, 9000, "dW"), (70, 7104, 16383, "dW"),
+                                         (64, 256, 65793, "dW"), (70, 7104, 9217, None)])
+def test_products_against_64_bits(dev, dtype, T, H, V, plain):
     """bf16: d(logits) rounded to 2^-8, the result once more; fp32: sums of at most 66000 products, 2^-16 of their norm."""
     from chatlearn_amd import ops
+    bulk, k_ranges, rows = ops.dhidden_tile_plan(T, H, V, dtype)
+    n_ht = -(-H // 256)
+    assert (plain == "dhidden") == (bulk == 0 and k_ranges == 1 and 256 < -(-T // rows) * n_ht < 1024)
+    assert (plain == "dW") == (ops.dweight_launch_plan(T, H, V, dtype) == (0, 0, 1) and -(-V // 256) * n_ht > 256)
     g = torch.Generator(device=dev).manual_seed(T + V)
     hidden = torch.randn(T, H, generator=g, device=dev).to(dtype)
     weight = (torch.randn(V, H, generator=g, device=dev) * 0.02).to(dtype)
