@@ -128,7 +128,7 @@ SIGNATURES = {
     "clgrpo_lmhead_fwd_workspace_bytes": (sz, [i64, i64, i64, i32]),
     "clgrpo_lmhead_fwd": (C.c_int, [C.POINTER(LmheadFwdArgs), vp]),
     "clgrpo_lmhead_fwd_launch_plan": (C.c_int, [i64, i64, i32, vp]),
-    "clgrpo_lmhead_fwd_tile_plan": (C.c_int, [i64, i64, i32, i32, vp]),
+    "clgrpo_lmhead_fwd_tile_plan": (C.c_int, [i64, i64, i64, i32, i32, vp]),
     "clgrpo_lmhead_bwd_dhidden_plan": (C.c_int, [i64, i64, i64, i32, i32, vp]),
     "clgrpo_lmhead_bwd_dhidden_tile_plan": (C.c_int, [i64, i64, i64, i32, i32, i64, vp]),
     "clgrpo_lmhead_bwd_dweight_plan": (C.c_int, [i64, i64, i64, i32, i32, vp]),

@@ -380,18 +380,31 @@ static double fwd_single_cost(int n_tb, int n_vt, int cus, int& n_split, int& ti
   return best_cost;
 }
 
+// A tile of 32 * ni tokens against one of 256: its time.  A step of its K loop loads as many bytes of W and reads as many of its
+// fragments, whatever the width, so the narrower tile takes more than ni / 8 of the time: 0.59 - 0.65 at ni = 4 from H = 2048 on
+// (V = 151936, launches of full rounds).  What a tile takes besides its K loop is nearer to ni / 8 and weighs more the shorter
+// the loop is: 0.56 - 0.58 at H = 512 and 1024.
+static double fwd_tile_time(int ni, int64_t H) {
+  static constexpr double kLong[9] = {0, 0, 0, 0, 0.63, 0.70, 0.81, 0.88, 1.0};
+  const double w = H <= 1024 ? 0.0 : H >= 2048 ? 1.0 : (H - 1024) / 1024.0;
+  return (1.0 - w) * ni / 8.0 * (1.0 + 0.02 * (8 - ni)) + w * kLong[ni];
+}
+
 // Width of the token blocks: 32 * ni tokens.  The last block of 256 is padding for the most part where T is a little over a
-// multiple of 256, and a launch of fewer items than CUs leaves the rest idle; a narrower tile takes ni / 8 of the time,
-// and about 2 % more of that per step down (more operand traffic and fragment reads per product).  Taken where the plan
-// then costs 4 % less; 16-bit inputs only.  Up to two wide blocks that fill the CUs are bound by reading W, so they are
-// not made into more blocks (256 tokens at H = 4096, V = 151936 as two blocks of 128: 320 us for 295).
+// multiple of 256, and a launch of fewer items than CUs leaves the rest idle.  A narrower tile is taken where the plan then
+// costs 4 % less; 16-bit inputs only.  Up to two wide blocks that fill the CUs are bound by reading W, so they are
+// not made into more blocks (256 tokens, V = 151936, as two blocks of 128 for one of 256: H = 7168 577 us for 522, 4096 315 for 285,
+// 2048 179 for 171, 1024 95 for 92; at H = 512 the two would take 52 for 58).
 //   H = 4096, V = 151936, us: 128 tokens 269 -> 228, 260 428 -> 333, 400 463 -> 426, 588 638 -> 579, 900 882 -> 848, 1100 1062 -> 968
 //   H = 2048:                 128 tokens 161 -> 148, 260 229 -> 188, 588 340 -> 311, 1100 555 -> 510
 //   H = 1024, V = 32000:      200 tokens  38 ->  28, 300  40 ->  31, 588  60 ->  45, 1100  84 ->  69
+// Over 2408 sizes (H 512 - 7168, V 9000 - 151936, 32 - 4096 tokens), each timed at all five widths: 9 % less time than 256-wide blocks
+// on average, 0.4 % more than the best width; 5 sizes more than 2 % slower than 256-wide blocks, none by more than 3.6 %.  (With the
+// time of a tile as 0.54 at ni = 4 for every H: 97 sizes, up to 33 %: 512 tokens at H = 7168, V = 32000 169 -> 211 us.)
 struct FwdPlan {
   int ni, n_tb, n_split, tiles_per_split;
 };
-static FwdPlan fwd_plan(int64_t T, int n_vt, int cus, bool narrow) {
+static FwdPlan fwd_plan(int64_t T, int64_t H, int n_vt, int cus, bool narrow) {
   if (cus <= 0) cus = 256;
   const int wide_tb = (int)((T + kFwdBN - 1) / kFwdBN);
   FwdPlan best{8, wide_tb, 0, 0};
@@ -399,7 +412,7 @@ static FwdPlan fwd_plan(int64_t T, int n_vt, int cus, bool narrow) {
   for (int ni = 7; narrow && ni >= 4; --ni) {
     FwdPlan pl{ni, (int)((T + 32 * ni - 1) / (32 * ni)), 0, 0};
     if (pl.n_tb > wide_tb && wide_tb <= 2 && wide_tb * n_vt > cus) continue;
-    const double c = ni / 8.0 * (1.0 + 0.02 * (8 - ni)) * fwd_single_cost(pl.n_tb, n_vt, cus, pl.n_split, pl.tiles_per_split);
+    const double c = fwd_tile_time(ni, H) * fwd_single_cost(pl.n_tb, n_vt, cus, pl.n_split, pl.tiles_per_split);
     if (c < best_cost) { best_cost = c; best = pl; }
   }
   return best;
@@ -427,7 +440,7 @@ static int launch_fwd(const clgrpo_lmhead_fwd_args* a, hipStream_t stream, int64
   p.H = (int)a->H;
   p.V = (int)a->V;
   p.n_vt = (int)((a->V + kFwdBM - 1) / kFwdBM);
-  const FwdPlan pl = fwd_plan(a->T, p.n_vt, device_cu_count(), kNarrow);
+  const FwdPlan pl = fwd_plan(a->T, a->H, p.n_vt, device_cu_count(), kNarrow);
   p.n_tb = pl.n_tb; p.n_split = pl.n_split; p.tiles_per_split = pl.tiles_per_split;
   p.c = a->inv_temperature * kLog2e;
   p.part = static_cast<float4*>(a->workspace);
@@ -484,20 +497,21 @@ extern "C" int64_t clgrpo_saved_logits_ld(int64_t V) { return V <= 0 ? 0 : round
 
 extern "C" int clgrpo_lmhead_fwd_launch_plan(int64_t T, int64_t V, int32_t cus, int32_t* out) {
   if (T <= 0 || V <= 0 || out == nullptr) return CLGRPO_EINVAL;
-  const FwdPlan pl = fwd_plan(T, (int)((V + kFwdBM - 1) / kFwdBM), cus, true);
+  const FwdPlan pl = fwd_plan(T, 4096, (int)((V + kFwdBM - 1) / kFwdBM), cus, true);
   out[0] = pl.n_tb;
   out[1] = pl.n_split;
   out[2] = pl.tiles_per_split;
   return CLGRPO_OK;
 }
 
-extern "C" int clgrpo_lmhead_fwd_tile_plan(int64_t T, int64_t V, int32_t dtype, int32_t cus, int32_t* out) {
-  if (T <= 0 || V <= 0 || out == nullptr || (dtype != CLGRPO_BF16 && dtype != CLGRPO_F32)) return CLGRPO_EINVAL;
-  const FwdPlan pl = fwd_plan(T, (int)((V + kFwdBM - 1) / kFwdBM), cus, dtype == CLGRPO_BF16);
+extern "C" int clgrpo_lmhead_fwd_tile_plan(int64_t T, int64_t H, int64_t V, int32_t dtype, int32_t cus, int32_t* out) {
+  if (T <= 0 || H <= 0 || V <= 0 || out == nullptr || (dtype != CLGRPO_BF16 && dtype != CLGRPO_F32)) return CLGRPO_EINVAL;
+  const FwdPlan pl = fwd_plan(T, H, (int)((V + kFwdBM - 1) / kFwdBM), cus, dtype == CLGRPO_BF16);
   out[0] = pl.n_tb;
   out[1] = pl.n_split;
   out[2] = pl.tiles_per_split;
   out[3] = 32 * pl.ni;
+  out[4] = (int32_t)(1000.0 * fwd_tile_time(pl.ni, H) + 0.5);
   return CLGRPO_OK;
 }
 

@@ -283,8 +283,8 @@ def _launch_cost(chunks, live_cum, H, V, dtype=torch.bfloat16, cus=256):
     cost = 0.0
     for k, (lo, hi) in enumerate(chunks):
         rows = (hi - lo) if live_cum is None else int(live_cum[hi] - live_cum[lo])
-        n_tb, _, tps, width = ops.lmhead_forward_tile_plan(hi - lo, V, dtype, cus)
-        cost += -(-(n_tb * -(-n_vt // tps)) // cus) * tps * H * tile(width)
+        n_tb, _, tps, _, time = ops.lmhead_forward_tile_plan(hi - lo, H, V, dtype, cus)
+        cost += -(-(n_tb * -(-n_vt // tps)) // cus) * tps * H * time
         if rows == 0:
             continue
         bulk_nt, ks, width = ops.dhidden_tile_plan(rows, H, V, dtype, cus)

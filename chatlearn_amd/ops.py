@@ -167,18 +167,19 @@ def lmhead_forward(hidden: torch.Tensor, weight: torch.Tensor, labels: Optional[
 
 def lmhead_forward_launch_plan(T: int, V: int, cus: int = 0) -> Tuple[int, int, int]:
     """(blocks of 256 tokens or fewer, vocabulary splits, vocabulary tiles per workgroup) of the forward launch for T
-    tokens of 16-bit inputs on a device with ``cus`` compute units (0: 256)."""
+    tokens of 16-bit inputs (H = 4096) on a device with ``cus`` compute units (0: 256)."""
     out = (C.c_int32 * 3)()
     _lib.check(_lib.lib().clgrpo_lmhead_fwd_launch_plan(int(T), int(V), int(cus), C.cast(out, C.c_void_p)))
     return int(out[0]), int(out[1]), int(out[2])
 
 
-def lmhead_forward_tile_plan(T: int, V: int, dtype, cus: int = 0) -> Tuple[int, int, int, int]:
-    """``lmhead_forward_launch_plan`` for inputs of ``dtype``, and the tokens per block: 128 to 256 (fp32: 256)."""
-    out = (C.c_int32 * 4)()
-    _lib.check(_lib.lib().clgrpo_lmhead_fwd_tile_plan(int(T), int(V), BF16 if dtype == torch.bfloat16 else F32, int(cus),
+def lmhead_forward_tile_plan(T: int, H: int, V: int, dtype, cus: int = 0) -> Tuple[int, int, int, int, float]:
+    """``lmhead_forward_launch_plan`` for inputs of ``dtype`` and H, the tokens per block (128 to 256; fp32: 256) and the time
+    of a tile of so many tokens against one of 256, as the plan takes it."""
+    out = (C.c_int32 * 5)()
+    _lib.check(_lib.lib().clgrpo_lmhead_fwd_tile_plan(int(T), int(H), int(V), BF16 if dtype == torch.bfloat16 else F32, int(cus),
                                                       C.cast(out, C.c_void_p)))
-    return int(out[0]), int(out[1]), int(out[2]), int(out[3])
+    return int(out[0]), int(out[1]), int(out[2]), int(out[3]), out[4] / 1000.0
 
 
 def dhidden_launch_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple[int, int]:

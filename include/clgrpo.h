@@ -111,14 +111,15 @@ int64_t clgrpo_saved_logits_ld(int64_t V);
 
 size_t clgrpo_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int32_t dtype);
 int clgrpo_lmhead_fwd(const clgrpo_lmhead_fwd_args* a, void* stream);
-/* The grid of the forward launch for T tokens of 16-bit inputs on a device with `cus` compute units (<= 0: 256):
+/* The grid of the forward launch for T tokens of 16-bit inputs, H = 4096, on a device with `cus` compute units (<= 0: 256):
  * out[0] = blocks of 256 tokens, or of fewer where that wastes less (224, 192, 160 or 128), out[1] = vocabulary splits (a workgroup owns one token block and one split),
  * out[2] = vocabulary tiles of 256 entries a workgroup walks.  The launch takes ceil(out[0] * out[1] / cus)
  * rounds of one workgroup per compute unit.  Host-side arithmetic only; no counterpart in the reference
  * (its lm_head is one library GEMM). */
 int clgrpo_lmhead_fwd_launch_plan(int64_t T, int64_t V, int32_t cus, int32_t* out);
-/* The same for inputs of `dtype`, with out[3] = tokens per block. */
-int clgrpo_lmhead_fwd_tile_plan(int64_t T, int64_t V, int32_t dtype, int32_t cus, int32_t* out);
+/* The same for inputs of `dtype` and H (the former answers for H = 4096), with out[3] = tokens per block and out[4] = the time that
+ * the plan gives a tile of so many tokens, in thousandths of a 256-wide one's. */
+int clgrpo_lmhead_fwd_tile_plan(int64_t T, int64_t H, int64_t V, int32_t dtype, int32_t cus, int32_t* out);
 
 /* ------------------------------------------------------------------ *
  * Backward of the fused head: recomputes logit tiles from hidden, W and the

@@ -18,7 +18,7 @@ def test_forward_and_backward_of_every_width(dev, T, V, width, ordered):
     bf16 and the softmax rebuilt from half logits (2^-8 each at most), the result rounded once more; the bound is on rows."""
     from chatlearn_amd import ops
     H = 128
-    n_tb, _, _, planned = ops.lmhead_forward_tile_plan(T, V, torch.bfloat16)
+    n_tb, _, _, planned, _ = ops.lmhead_forward_tile_plan(T, H, V, torch.bfloat16)
     assert planned == width and n_tb == -(-T // width)
     g = torch.Generator(device=dev).manual_seed(T + V)
     hidden = torch.randn(T, H, generator=g, device=dev).bfloat16()

@@ -22,9 +22,10 @@ def _factor(width):
 @pytest.mark.parametrize("dtype", [BF16, FP32])
 @pytest.mark.parametrize("T", [100, 256, 260, 588, 900, 1100, 3000, 16384])
 def test_forward_counts_its_blocks_at_their_width(T, dtype):
-    n_tb, n_split, tps, width = ops.lmhead_forward_tile_plan(T, V, dtype)
+    n_tb, n_split, tps, width, time = ops.lmhead_forward_tile_plan(T, 4096, V, dtype)
     assert n_tb == -(-T // width) and 128 <= width <= 256 and n_split * tps >= 594
-    assert _forward_only(T, 4096, dtype) == pytest.approx(-(-(n_tb * n_split) // 256) * tps * 4096 * _factor(width))
+    assert width / 256 <= time <= 1 and (time == 1) == (width == 256)
+    assert _forward_only(T, 4096, dtype) == pytest.approx(-(-(n_tb * n_split) // 256) * tps * 4096 * time)
     if dtype == BF16:
         assert ops.lmhead_forward_launch_plan(T, V) == (n_tb, n_split, tps)
     else:
@@ -32,7 +33,22 @@ def test_forward_counts_its_blocks_at_their_width(T, dtype):
 
 
 def test_widths_of_the_forward():
-    assert [ops.lmhead_forward_tile_plan(T, V, BF16)[3] for T in (100, 128, 260, 588, 1100, 16384)] == [128, 128, 160, 224, 224, 256]
+    assert [ops.lmhead_forward_tile_plan(T, 4096, V, BF16)[3] for T in (100, 128, 260, 588, 1100, 16384)] == [128, 128, 160, 224, 224, 256]
+
+
+# (tokens, H, V) measured at every width, us per forward for blocks of (256, 224, 192, 160, 128): a narrower block costs more than its
+# share of the products, so wide blocks that nearly fill the CUs, or their rounds, stay
+TIMES = [((512, 4096, 32000), (102.0, 135.9, 125.2, 119.3, 109.5)), ((512, 7168, 32000), (173.8, 264.2, 233.4, 211.9, 210.8)),
+         ((256, 7168, 50257), (175.6, 259.2, 241.9, 225.7, 223.0)), ((768, 4096, 50257), (250.6, 290.6, 272.2, 253.4, 287.4)),
+         ((1400, 4096, 102400), (875.4, 918.5, 912.6, 912.2, 989.5)), ((600, 4096, 151936), (642.9, 585.3, 693.8, 623.0, 674.7)),
+         ((300, 4096, 151936), (451.1, 402.1, 374.5, 341.0, 411.4)), ((384, 2048, 129280), (200.1, 183.3, 171.6, 207.4, 196.1)),
+         ((512, 1024, 32000), (40.1, 51.6, 46.7, 42.5, 38.2)), ((160, 512, 151936), (55.4, 49.6, 46.0, 42.4, 49.0))]
+
+
+@pytest.mark.parametrize("size,us", TIMES)
+def test_the_width_that_was_fastest_is_taken(size, us):
+    width = ops.lmhead_forward_tile_plan(*size, BF16)[3]
+    assert us[(256 - width) // 32] <= 1.04 * min(us)
 
 
 def test_narrow_blocks_are_cheaper_than_wide_ones():
