@@ -632,10 +632,19 @@ struct DhPlan {
   int ni;            // the single launch's tiles are 32 * ni rows wide
 };
 
+// Time of a tile of 32 * ni rows against one of 256.  A step loads as many bytes of W and transposes as many of its fragments,
+// whatever the width (launches of full rounds, H = 512 - 7168: 0.62 - 0.68 at 128 rows, 0.80 - 0.85 at 192).
+static double dh_tile_time(int ni) { return ni == 4 ? 0.63 : ni == 6 ? 0.80 : 1.0; }
+
 // Narrower row tiles (16-bit operands, a single launch): where 256-row ones would be padding or too few, as in the
-// forward's fwd_plan; whole units of 64 rows, so 192 or 128.
+// forward's fwd_plan; whole units of 64 rows, so 192 or 128.  Taken where the plan then costs 3.5 % less, the partials' traffic
+// counted: 6.6 MB per slab period of a tile (see plan_dweight).
 // dhidden and the d(logits) pass, us: H = 4096, V = 151936: 128 rows 267 -> 260, 320 469 -> 409, 384 478 -> 422; H = 2048: 320
 // 260 -> 235; H = 1024, V = 32000: 32 rows 36 -> 28, 200 45 -> 37, 320 53 -> 49.
+// Over 2398 sizes (H 512 - 7168, V 9000 - 151936, 32 - 4096 rows), each timed at all three widths: 6 % less time than 256-row tiles on
+// average, 0.3 % more than the best width; 21 sizes more than 2 % slower than 256-row tiles, by at most 8.6 %.  (With the time of a
+// tile as 0.54 and 0.78 and a flat 2 % for partials: 135 sizes, up to 80 %: 640 rows at H = 7168, V = 129280 in five tiles of 128
+// rows 1312 us, in three of 256 1007.)
 static DhPlan plan_dhidden(int64_t rows, int64_t H, int64_t K, int slab, int cus, size_t partial_cap) {
   DhPlan pl{0, 1, 0, 8};
   if (rows <= 0) return pl;
@@ -664,11 +673,16 @@ static DhPlan plan_dhidden(int64_t rows, int64_t H, int64_t K, int slab, int cus
       return pl;
     }
   }
+  auto full_cost = [&](long items, int s, int ni) {
+    const long rounds = (items * s + cus - 1) / cus;
+    return dh_tile_time(ni) * (double)rounds * (double)((k_slabs + s - 1) / s) + (s > 1 ? 2.0 * (double)s * rows * H * sizeof(float) / 6.6e6 : 0.0);
+  };
+  best = 0.965 * full_cost(tiles, s_one, 8);
   for (int ni = 6; slab == 64 && ni >= 4; ni -= 2) {
     const int t = n_mt * (int)((rows + 32 * ni - 1) / (32 * ni));
     const int s = pick_k_split(t, (int)H, (int)rows, (int)K, slab, partial_cap, cus);
-    const double c = ni / 8.0 * (1.0 + 0.02 * (8 - ni)) * cost(t, s);
-    if (c < (pl.ni == 8 ? 0.96 : 1.0) * best) { best = c; pl.ni = ni; pl.k_split = s; }
+    const double c = full_cost(t, s, ni);
+    if (c < best) { best = c; pl.ni = ni; pl.k_split = s; }
   }
   pl.partial_bytes = pl.k_split > 1 ? (size_t)pl.k_split * rows * H * sizeof(float) : 0;
   return pl;
@@ -1053,6 +1067,7 @@ extern "C" int clgrpo_lmhead_bwd_dhidden_tile_plan(int64_t rows, int64_t H, int6
   out[0] = pl.bulk_nt;
   out[1] = pl.k_split;
   out[2] = 32 * pl.ni;
+  out[3] = (int32_t)(1000.0 * dh_tile_time(pl.ni) + 0.5);
   return CLGRPO_OK;
 }
 

@@ -279,7 +279,6 @@ def _launch_cost(chunks, live_cum, H, V, dtype=torch.bfloat16, cus=256):
     first is counted."""
     n_vt = -(-V // 256)
     n_ht = -(-H // 256)
-    tile = lambda width: width / 256 * (1.0 + 0.02 * (256 - width) / 32)
     cost = 0.0
     for k, (lo, hi) in enumerate(chunks):
         rows = (hi - lo) if live_cum is None else int(live_cum[hi] - live_cum[lo])
@@ -287,10 +286,10 @@ def _launch_cost(chunks, live_cum, H, V, dtype=torch.bfloat16, cus=256):
         cost += -(-(n_tb * -(-n_vt // tps)) // cus) * tps * H * time
         if rows == 0:
             continue
-        bulk_nt, ks, width = ops.dhidden_tile_plan(rows, H, V, dtype, cus)
+        bulk_nt, ks, width, time = ops.dhidden_tile_plan(rows, H, V, dtype, cus)
         if bulk_nt:
             cost += -(-(bulk_nt * n_ht) // cus) * V
-        cost += -(-(-(-(rows - 256 * bulk_nt) // width) * n_ht * ks) // cus) * (V / ks) * tile(width)
+        cost += -(-(-(-(rows - 256 * bulk_nt) // width) * n_ht * ks) // cus) * (V / ks) * time
         n_walk, bulk_vt, ks_w = ops.dweight_launch_plan(rows, H, V, dtype, cus)   # dW: walks over vocabulary tiles, K-split tail
         if bulk_vt:
             cost += (bulk_vt // n_walk) * rows + -(-((n_vt - bulk_vt) * n_ht * ks_w) // cus) * (rows / ks_w)

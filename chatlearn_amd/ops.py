@@ -191,12 +191,13 @@ def dhidden_launch_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple
     return int(out[0]), int(out[1])
 
 
-def dhidden_tile_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple[int, int, int]:
-    """``dhidden_launch_plan`` and the token rows per tile of its (remaining) launch: 256, or 192 or 128 for 16-bit inputs."""
-    out = (C.c_int32 * 3)()
+def dhidden_tile_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple[int, int, int, float]:
+    """``dhidden_launch_plan``, the token rows per tile of its (remaining) launch (256, or 192 or 128 for 16-bit inputs) and
+    the time of a tile of so many rows against one of 256, as the plan takes it."""
+    out = (C.c_int32 * 4)()
     _lib.check(_lib.lib().clgrpo_lmhead_bwd_dhidden_tile_plan(int(rows), int(H), int(V), BF16 if dtype == torch.bfloat16 else F32,
                                                               int(cus), -1, C.cast(out, C.c_void_p)))
-    return int(out[0]), int(out[1]), int(out[2])
+    return int(out[0]), int(out[1]), int(out[2]), out[3] / 1000.0
 
 
 def dweight_launch_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple[int, int, int]:

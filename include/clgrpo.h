@@ -172,8 +172,9 @@ int clgrpo_lmhead_bwd(const clgrpo_lmhead_bwd_args* a, void* stream);
  * all rows), out[1] = K ranges of the (remaining) launch, whose fp32 partial tiles a second pass sums.
  * Host-side arithmetic only; no counterpart in the reference. */
 int clgrpo_lmhead_bwd_dhidden_plan(int64_t rows, int64_t H, int64_t V, int32_t dtype, int32_t cus, int32_t* out);
-/* The same with out[2] = token rows per tile of the (remaining) launch (256, or 192 or 128 where that wastes less), for a
- * workspace with room for partial_bytes of partial tiles (< 0: as much as clgrpo_lmhead_bwd_workspace_bytes asks for). */
+/* The same with out[2] = token rows per tile of the (remaining) launch (256, or 192 or 128 where that wastes less) and out[3] = the
+ * time that the plan gives such a tile, in thousandths of a 256-row one's, for a workspace with room for partial_bytes of partial
+ * tiles (< 0: as much as clgrpo_lmhead_bwd_workspace_bytes asks for). */
 int clgrpo_lmhead_bwd_dhidden_tile_plan(int64_t rows, int64_t H, int64_t V, int32_t dtype, int32_t cus, int64_t partial_bytes,
                                         int32_t* out);
 /* How the dW contraction over a chunk of `rows` tokens is launched: out[0] = walks (workgroups that keep one

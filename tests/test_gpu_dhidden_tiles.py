@@ -11,7 +11,7 @@ PLANS = [((1537, 7168, 129280), (0, 1, 192)), ((1728, 7168, 300), (0, 1, 192)), 
 @pytest.mark.parametrize("size,plan", PLANS)
 def test_reported_tiles(lib, size, plan):
     from chatlearn_amd import ops
-    assert ops.dhidden_tile_plan(*size, torch.bfloat16) == plan
+    assert ops.dhidden_tile_plan(*size, torch.bfloat16)[:3] == plan
     assert ops.dhidden_launch_plan(*size, torch.bfloat16) == plan[:2]
     assert ops.dhidden_tile_plan(*size, torch.float32)[2] == 256           # fp32 has no narrower tiles
 
@@ -19,13 +19,13 @@ def test_reported_tiles(lib, size, plan):
 def test_a_plan_without_partial_sums_is_launched_as_planned(lib):
     """Whatever the scratch memory holds for partial sums: nothing where neither contraction wants any."""
     from chatlearn_amd import _lib, ops
-    out = (_lib.i32 * 3)()
+    out = (_lib.i32 * 4)()
     for rows, H in ((1537, 7168), (1728, 7168), (3329, 3584)):
         assert lib.clgrpo_lmhead_bwd_dhidden_tile_plan(rows, H, 129280, _lib.BF16, 256, 0, out) == 0
-        assert tuple(out) == (0, 1, 192)
+        assert tuple(out)[:3] == (0, 1, 192)
         # with memory for none, a plan that would like some still takes the best tile without a K split
         assert lib.clgrpo_lmhead_bwd_dhidden_tile_plan(128, H, 129280, _lib.BF16, 256, 0, out) == 0
-        assert tuple(out) == (0, 1, 128)
+        assert tuple(out)[:3] == (0, 1, 128)
 
 
 @pytest.mark.gpu
@@ -45,7 +45,7 @@ def test_tiles_of_192_rows_without_a_k_split(dev, rows, ordered):
     labels = torch.randint(0, V, (T,), generator=g, device=dev)
     mask = torch.zeros(T, dtype=torch.int32, device=dev)
     mask[torch.randperm(T, generator=g, device=dev)[:rows]] = 1
-    assert ops.dhidden_tile_plan(rows, H, V, torch.bfloat16) == (0, 1, 192)
+    assert ops.dhidden_tile_plan(rows, H, V, torch.bfloat16)[:3] == (0, 1, 192)
     out = grpo_head_step(hidden, weight, labels, torch.full((T,), -6.0, device=dev), None, torch.ones(1, device=dev),
                          torch.tensor([0, T], dtype=torch.int32, device=dev), mask, n_tokens_total=1.0, loss_mask_host=mask.cpu())
     h64, w64, g64 = hidden.double(), weight.double(), out["g_logprob"].double()[:, None]
@@ -62,7 +62,7 @@ def test_tiles_of_192_rows_without_a_k_split(dev, rows, ordered):
     assert (err <= bound)[live].all(), float((err / bound)[live].max())
     # and the products of the same rows in tiles of another width, bit for bit: no K split either way
     some = torch.nonzero(live).flatten()[:700]
-    assert ops.dhidden_tile_plan(700, H, V, torch.bfloat16)[1:] != (1, 192)
+    assert ops.dhidden_tile_plan(700, H, V, torch.bfloat16)[1:3] in ((1, 128), (1, 256))
     z = ops.saved_logits_buffer(700, V, torch.bfloat16, dev)
     y, g_lp = labels[some], out["g_logprob"][some]
     lse = ops.lmhead_forward(hidden[some], weight, y, saved_logits=z)[3]

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 def test_products_against_64_bits(dev, dtype, T, H, V, plain):
     """bf16: d(logits) rounded to 2^-8, the result once more; fp32: sums of at most 66000 products, 2^-16 of their norm."""
     from chatlearn_amd import ops
-    bulk, k_ranges, rows = ops.dhidden_tile_plan(T, H, V, dtype)
+    bulk, k_ranges, rows, _ = ops.dhidden_tile_plan(T, H, V, dtype)
     n_ht = -(-H // 256)
     assert (plain == "dhidden") == (bulk == 0 and k_ranges == 1 and 256 < -(-T // rows) * n_ht < 1024)
     assert (plain == "dW") == (ops.dweight_launch_plan(T, H, V, dtype) == (0, 0, 1) and -(-V // 256) * n_ht > 256)
