@@ -344,11 +344,11 @@ class _ReadBack:
     the flags of a micro-batch read behind its backward, the GPU stood still until the next one was prepared and launched:
     four padded samples 12.9 -> 12.3 ms, a 200-token step 212 -> 149 us."""
 
-    def __init__(self, values):
+    def __init__(self, values, stream):
         self.host = torch.empty(values.shape, dtype=values.dtype, pin_memory=True)
         self.host.copy_(values, non_blocking=True)
         self.done = torch.cuda.Event()
-        self.done.record(torch.cuda.current_stream(values.device))
+        self.done.record(stream)
 
     def tolist(self):
         self.done.synchronize()
@@ -356,23 +356,27 @@ class _ReadBack:
 
 
 def _follow_last_use(tensors, stream):
-    """Order ``stream`` behind the calls that used these cached tensors last: on another stream they may still have their
-    backward enqueued.  The tensors' memory then also outlives what ``stream`` does with them.  A capture depends on nothing
+    """Order ``stream`` behind the calls that used these cached tensors (of its device) last: on another stream they may still
+    have their backward enqueued.  The tensors' memory then also outlives what ``stream`` does with them.  A capture depends on nothing
     outside of it: replays are ordered by whoever replays them."""
     for t in tensors:
         last = getattr(t, "last_use", None)
-        if last is not None and last[0] != stream and not torch.cuda.is_current_stream_capturing():
-            stream.wait_event(last[1])
+        if last is not None and last[0].cuda_stream != stream.cuda_stream and not torch.cuda.is_current_stream_capturing():
+            stream.wait_event(last[1] if last[1] is not None else last[0].record_event())
             t.record_stream(stream)
 
 
 def _leave_last_use(tensors, stream):
-    """What ``_follow_last_use`` of a later call waits for: everything this call has enqueued."""
+    """What ``_follow_last_use`` of a later call waits for: everything this call has enqueued.  An event behind it costs the
+    stream a few us (a 200-token step by itself 215 -> 224 us), and the default stream is there for good: an event is recorded on
+    it when another stream asks.  Any other stream may be gone by then."""
     if not tensors or torch.cuda.is_current_stream_capturing():
         return
-    last = getattr(tensors[0], "last_use", None)
-    event = last[1] if last is not None and last[0] == stream else torch.cuda.Event()
-    event.record(stream)
+    event = None
+    if stream.cuda_stream != 0:
+        last = getattr(tensors[0], "last_use", None)
+        event = last[1] if last is not None and last[0].cuda_stream == stream.cuda_stream else torch.cuda.Event()
+        event.record(stream)
     for t in tensors:
         t.last_use = (stream, event)
 
@@ -436,7 +440,7 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
     later call they are large enough for, instead of being allocated and released per call: micro-batches of
     varying length otherwise ask the framework's allocator for differently sized multi-GB blocks each time,
     which now and then costs a device-wide stall for a fresh allocation.  The tensors carry the stream of the last call
-    and an event behind its work (``last_use``): a call on another stream waits for it (on the device), so successive calls may
+    and where it is not the default one an event behind its work (``last_use``): a call on another stream waits for it (on the device), so successive calls may
     share the dict whatever stream they run on; threads that run at the same time may not.
 
     ``stage_hook(name)`` is called on the host at "forward", "loss", "backward", "end" boundaries
@@ -541,7 +545,7 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
             ws = cache["head_step"] = torch.empty(need, dtype=torch.uint8, device=dev)
         cached = [t for t in ((zbuf, ws) if workspace_cache is not None else ()) + ((wt,) if weight_t_cache is not None else ())
                   if t is not None]
-        stream = torch.cuda.current_stream(dev) if cached else None
+        stream = torch.cuda.current_stream(dev)
         _follow_last_use(cached, stream)
     rows_projected_bwd = rows_projected_fwd = 0
     if T > 0:
@@ -557,7 +561,7 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
             for k, (lo, n, n_live, pick) in enumerate(parts):
                 live_only = bool(skip_masked_forward and pick and n_live > 0)
                 chunk = dict(lo=lo, n=n, n_live=n_live, ordered=pick, chunk=k, forward_live_only=live_only, accumulate=acc_dw,
-                             weight_t_ready=wt_ready)
+                             weight_t_ready=wt_ready, stream=stream)
                 # the flags are complete behind the last chunk's loss: they travel while the backward runs
                 read_flags = check_flags and k == n_chunks - 1
                 if stage_hook is not None:
@@ -565,14 +569,16 @@ def grpo_head_step(hidden, weight, labels, old_logprob, ref_logprob, advantages,
                         stage_hook(name)
                         step.enqueue(bit & stages, **chunk)
                         if read_flags and bit == 2:
-                            flags_read = _ReadBack(result[12:])
+                            flags_read = _ReadBack(result[12:], stream)
                     stage_hook("end")
                 elif read_flags:
-                    # 8: one launch clears all of the masked rows (four padded samples launch it 4 times instead of 8)
-                    step.enqueue(3 | 8 if stages & 4 else 3, **chunk)
-                    flags_read = _ReadBack(result[12:])
+                    # 8: one launch clears all of the masked rows, where the forward's call has one for its outputs anyway
+                    # (four padded samples launch it 4 times instead of 8); elsewhere it would only make the flags later
+                    together = 8 if live_only and stages & 4 else 0
+                    step.enqueue(3 | together, **chunk)
+                    flags_read = _ReadBack(result[12:], stream)
                     if stages & 4:
-                        step.enqueue(4 | 8, **chunk)
+                        step.enqueue(4 | together, **chunk)
                 else:
                     step.enqueue(stages, **chunk)
                 rows_projected_fwd += n_live if live_only else n

@@ -421,7 +421,8 @@ class DweightSum:
 
 class HeadStep:
     """The token chunks of one micro-batch through clgrpo_head_step: the tensors of the whole micro-batch, checked
-    once; ``enqueue`` launches one chunk (or one stage of it) on the current stream."""
+    once; ``enqueue`` launches one chunk (or one stage of it) on the current stream (``stream``: which the caller has looked
+    up already, 2 us a time)."""
 
     def __init__(self, hidden, weight, labels, old_logprob, ref_logprob, advantages, cu_seqlens, loss_mask, order, *, mode,
                  temperature, diff_clip_ratio, pos_clip_ratio, neg_clip_ratio, final_clip_ratio, kl_coef, entropy_coef,
@@ -471,14 +472,16 @@ class HeadStep:
         if saved_logits is not None:
             a.saved_logits, a.ld_saved, a.saved_rows = _ptr(saved_logits), saved_logits.shape[1], saved_logits.shape[0]
         a.weight_t = _ptr(weight_t)
-        self.device = hidden.device
+        self.device, self.at = hidden.device, None
 
-    def enqueue(self, stages, *, lo, n, n_live, ordered, chunk, forward_live_only, accumulate, weight_t_ready):
+    def enqueue(self, stages, *, lo, n, n_live, ordered, chunk, forward_live_only, accumulate, weight_t_ready, stream=None):
         a = self.args
-        for name, base in self.base.items():
-            setattr(a, name, None if base is None else base + lo * self.row_bytes[name])
-        if not ordered:
-            a.row_order = None
+        if self.at != (lo, ordered):           # several calls for one chunk: its addresses are set once
+            for name, base in self.base.items():
+                setattr(a, name, None if base is None else base + lo * self.row_bytes[name])
+            if not ordered:
+                a.row_order = None
+            self.at = (lo, ordered)
         a.T, a.n_live, a.token_offset, a.chunk = n, n_live, lo, chunk
         a.forward_live_only, a.accumulate_dweight, a.weight_t_ready = int(forward_live_only), int(accumulate), int(weight_t_ready)
         a.stages = stages
@@ -488,7 +491,7 @@ class HeadStep:
             a.kept_dzt, a.kept_hidt, a.kept_ld, a.kept_k = _ptr(keep.dzt), _ptr(keep.hidt), keep.capacity, keep.used
             if stages & 4:
                 keep.used += _round_up(n_live, 64)
-        _lib.call("clgrpo_head_step", a, torch.cuda.current_stream(self.device).cuda_stream)
+        _lib.call("clgrpo_head_step", a, (stream or torch.cuda.current_stream(self.device)).cuda_stream)
 
 
 # --------------------------------------------------------------------------- stats from logits
