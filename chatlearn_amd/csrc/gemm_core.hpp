@@ -12,10 +12,10 @@
 //    TFLOP/s), 6 % in this loop.
 //  - every instruction's place is fixed in the source (see the schedule): with one wave per SIMD nothing else would
 //    fill a gap.
-// At 12288 tokens, H = 4096, V = 151936 (bf16, counters): matrix cores busy 0.865 of the cycles at 1.64 GHz, 1.50 - 1.54
-// PFLOP/s for either contraction of the backward.  With the barriers and load waits left out (wrong results) they are busy
-// 0.88 and the clock falls: 0.5 % less time.  The eight-wave 32x32x16 form of this tile with two 64 KB stages ran
-// 13 % slower.
+// 12126 rows, H = 4096, V = 151936 (bf16): 1.46 - 1.54 PFLOP/s for either contraction of the backward, by the machine; under the
+// counters matrix cores busy 0.85 of the cycles at 1.61 GHz (profiles/head_gemm_kernels_c2_sq_counters.txt).  With the barriers
+// and load waits left out (wrong results) they were busy 1.5 % of the cycles more and the clock fell: 0.5 % less time.  The
+// eight-wave 32x32x16 form of this tile with two 64 KB stages ran 13 % slower.
 //
 // Operand slabs travel HBM/L2 -> LDS directly (buffer loads with an LDS destination; no registers, no LDS
 // store instructions) into two rings of 32 KB slots, three for A and two for B: all 160 KB.  While the matrix

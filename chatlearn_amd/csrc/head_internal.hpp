@@ -16,8 +16,8 @@ constexpr int64_t kMaxOrderedBytes = 0x7f000000;
 // Forward of the a->T rows of `rows`; per-token outputs and labels are indexed by order[n], kept logits by n.
 int head_forward(const char* who, const clgrpo_lmhead_fwd_args* a, int64_t vocab_begin, void* record, const RowOrder& rows,
                  hipStream_t stream);
-// Both operands of the dW contraction, kept beyond the call: K-blocked with `ld` tokens, of which the first `k` (a
-// multiple of 64) are in use.  A backward that is given one leaves its rows behind those and computes no dW.
+// Both operands of the dW contraction, kept beyond the call: d(logits) in units and hidden^T K-blocked, `ld` tokens each, of
+// which the first `k` (a multiple of 64) are in use.  A backward that is given one leaves its rows behind those and computes no dW.
 struct DwOperands {
   void *dzt, *hidt;
   int64_t ld, k;

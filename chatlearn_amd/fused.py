@@ -342,7 +342,7 @@ def head_step_chunks(T, keep_logits_chunk, sequence_level, cu_seqlens, loss_mask
 class _ReadBack:
     """A few device values on their way to the host: waiting for them does not wait for what is enqueued behind them.  With
     the flags of a micro-batch read behind its backward, the GPU stood still until the next one was prepared and launched:
-    four padded samples 12.9 -> 12.3 ms, a 200-token step 212 -> 149 us."""
+    four padded samples 12.9 -> 12.3 ms, 200-token steps one behind the other 212 -> 149 us each."""
 
     def __init__(self, values, stream):
         self.host = torch.empty(values.shape, dtype=values.dtype, pin_memory=True)

@@ -156,8 +156,7 @@ typedef struct {
                                (((row / 256) * (ld / E) + k / E) * 256 + row % 256) * E + k % E.  NULL: W is read as it is,
                                which is as fast; nothing is transposed */
   int32_t weight_t_ready;   /* zero: this call fills weight_t; nonzero: it already holds W^T */
-  int64_t saved_rows;       /* rows the saved_logits buffer holds; must be >= ceil(T / 256) * 256 (the backward
-                               rewrites whole 256-row units) */
+  int64_t saved_rows;       /* rows the saved_logits buffer holds; must be >= ceil(T / 256) * 256 */
 } clgrpo_lmhead_bwd_args;
 
 /* Bytes needed to process `chunk_tokens` tokens at a time (chunk_tokens <= 0: all T at once).
