@@ -604,8 +604,8 @@ __device__ __forceinline__ int xcd_remap(int bid, int grid) {
 // the last-level cache then serves to all of them from one HBM read - instead of eight stretches a
 // eighth of the launch apart.  Bit-identical results; measured on the forward, with a core of eight waves: 32768 tokens at H = 7168
 // (22 vocabulary splits, 11 rounds) 48.1 -> 45.2 ms, 16640 tokens at H = 4096 (35 splits, 9 rounds) 16.1 ->
-// 15.4 ms, no change for launches of one or two rounds.  Used by the forward and by the plain launches of
-// the backward's products; the kernel that recomputes d(logits) tile by tile got 6 % slower with it.
+// 15.4 ms, no change for launches of one or two rounds.  Used by the forward and by plain launches of
+// the backward's products (see launch_gemm_one); the kernel that recomputes d(logits) tile by tile got 6 % slower with it.
 __device__ __forceinline__ int xcd_round_remap(int bid, int xcd_wgs) {
   const int x = bid & 7, slot = bid >> 3;
   return ((slot / xcd_wgs) * 8 + x) * xcd_wgs + slot % xcd_wgs;

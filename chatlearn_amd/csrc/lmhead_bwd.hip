@@ -848,9 +848,14 @@ static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64
   }
   // One workgroup per tile in several rounds: each round's tiles go to all XCDs, so that they stream the same stretches of
   // the operands (dhidden of 32768 rows at H = 7168, 14 rounds: 42.4 -> 41.5 ms, of 16384 20.9 -> 20.4; dW of 8192 rows at H =
-  // 5120 9.11 -> 8.75; two and three rounds at H = 4096: no change).
+  // 5120 9.11 -> 8.56; two and three rounds at H = 4096: no change).  dW of some hundred rows writes more than it reads, and eight
+  // XCDs writing one stretch of dW at a time are slower than each its own (V = 151936, plain -> rounds, us: H = 5120 412 rows
+  // 925 -> 1010, 1024 1432 -> 1534, 2048 2382 -> 2380, 4096 4569 -> 4397; H = 1536 768 rows 458 -> 472, 4096 1676 -> 1634); up to 128
+  // rows it is the reads of hidden^T and dz that count again (H = 4096, 64 rows 479 -> 457).  fp32 tiles take ten times as long
+  // for the same bytes: no gain from it, up to 4 % lost (dW of 64 rows at H = 1536 356 -> 371).
+  const bool rounds = g.k_split == 1 && sizeof(T) == 2 && (kMC || K >= 2048 || K <= 128);
   ItemGrid grid{(g.n_walk * n_fixed + 7) / 8 * 8, 0};
-  if (g.n_walk == 0) grid = g.k_split == 1 ? item_grid(g.n_mt * g.n_nt, cus) : ItemGrid{(g.n_mt * g.n_nt * g.k_split + 7) / 8 * 8, 0};
+  if (g.n_walk == 0) grid = rounds ? item_grid(g.n_mt * g.n_nt, cus) : ItemGrid{(g.n_mt * g.n_nt * g.k_split + 7) / 8 * 8, 0};
   g.xcd_wgs = grid.xcd_wgs;
   hipLaunchKernelGGL((gemm_kernel<T, OutT, S, NI>), dim3(grid.grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
   rc = check_launch("gemm_kernel");

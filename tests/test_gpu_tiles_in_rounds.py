@@ -1,16 +1,17 @@
 """Products of the backward with more tiles than compute units, one workgroup per tile: every tile is made once, whichever
-XCD its round hands it to."""
+XCD it is handed to, round by round (dhidden, dW of up to 128 or from 2048 rows on) or an eighth of the launch each."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 
-# dhidden of 43 x 16 tiles of 192 rows (fp32: 33 x 16 of 256); dW of 36 x 16, of 64 x 28 with ragged edges, and one tile more than a
-# round; beside them dW of 37 x 28, which workgroups walk
+# dhidden of 43 x 16 tiles of 192 rows (fp32: 33 x 16 of 256); dW of 36 x 16, of 64 x 28 with ragged edges, of 43 x 6, and one tile
+# more than a round; beside them dW of 37 x 28, which workgroups walk
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("T,H,V,plain", [(8200, 4096, 300, "dhidden"), (130, 4096, 9000, "dW"), (70, 7104, 16383, "dW"),
-                                         (64, 256, 65793, "dW"), (70, 7104, 9217, None)])
+@pytest.mark.parametrize("T,H,V,plain", [(8200, 4096, 300, "dhidden"), (130, 4096, 9000, "dW"), (2050, 1536, 11000, "dW"), (70, 7104, 16383, "dW"),
+                                         (64, 256, 65793, "dW"),
+                                         (70, 7104, 9217, None)])
 def test_products_against_64_bits(dev, dtype, T, H, V, plain):
     """bf16: d(logits) rounded to 2^-8, the result once more; fp32: sums of at most 66000 products, 2^-16 of their norm."""
     from chatlearn_amd import ops
