@@ -643,7 +643,7 @@ static double dh_tile_time(int ni) { return ni == 4 ? 0.63 : ni == 6 ? 0.80 : 1.
 // 260 -> 235; H = 1024, V = 32000: 32 rows 36 -> 28, 200 45 -> 37, 320 53 -> 49.
 // Over 2398 sizes (H 512 - 7168, V 9000 - 151936, 32 - 4096 rows), each timed at all three widths: 6 % less time than 256-row tiles on
 // average, 0.3 % more than the best width; 21 sizes more than 2 % slower than 256-row tiles, by at most 8.6 %.  (With the time of a
-// tile as 0.54 and 0.78 and a flat 2 % for partials: 135 sizes, up to 80 %: 640 rows at H = 7168, V = 129280 in five tiles of 128
+// tile as 0.54 and 0.78 and a flat 2 % for partials: 135 sizes, up to 80 %; 640 rows at H = 7168, V = 129280 in five tiles of 128
 // rows 1312 us, in three of 256 1007.)
 static DhPlan plan_dhidden(int64_t rows, int64_t H, int64_t K, int slab, int cus, size_t partial_cap) {
   DhPlan pl{0, 1, 0, 8};

@@ -400,7 +400,7 @@ static double fwd_tile_time(int ni, int64_t H) {
 //   H = 1024, V = 32000:      200 tokens  38 ->  28, 300  40 ->  31, 588  60 ->  45, 1100  84 ->  69
 // Over 2408 sizes (H 512 - 7168, V 9000 - 151936, 32 - 4096 tokens), each timed at all five widths: 9 % less time than 256-wide blocks
 // on average, 0.4 % more than the best width; 5 sizes more than 2 % slower than 256-wide blocks, none by more than 3.6 %.  (With the
-// time of a tile as 0.54 at ni = 4 for every H: 97 sizes, up to 33 %: 512 tokens at H = 7168, V = 32000 169 -> 211 us.)
+// time of a tile as 0.54 at ni = 4 for every H: 97 sizes, up to 33 %; 512 tokens at H = 7168, V = 32000 169 -> 211 us.)
 struct FwdPlan {
   int ni, n_tb, n_split, tiles_per_split;
 };
