@@ -170,6 +170,7 @@ struct GemmTile {
   static constexpr int VEC = 16 / (int)sizeof(T);      // elements per 16-byte piece
   static constexpr int kBB = kASlots * kSlotBytes;     // LDS offset of the B ring
   static constexpr bool kAcross = kSideA != Side::kRows;
+  static constexpr bool kSplit = false;                     // see SplitTile
   static constexpr bool kPerm = kAcross && VEC == 8;   // fragments are made from what is read
   static constexpr int kUnitBytes = kSlabK * kRowBytes;     // a unit of d(logits); a piece of a slab read across
   static constexpr int kSub = 256 / kSlabK;                 // of them per 256-wide slab
@@ -412,9 +413,8 @@ struct GemmTile {
     jump_b = nb.p - (reinterpret_cast<const char*>(B.base) + (int64_t)(nslab - 1) * B.slab_bytes);
   }
 
-  // First tile of a workgroup (or of a run that does not stream): nothing is in flight, LDS is free.
   // b_order: row r of the B tile is row b_order[r] of B.base (B.rows: rows of the whole array; b_rows of them used).
-  __device__ __forceinline__ void start(const Operand& A, const Operand& B, int nslab, char* shared,
+  __device__ __forceinline__ void place(const Operand& A, const Operand& B, int nslab, char* shared,
                                         const int32_t* b_order = nullptr, int b_rows = 0) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t lds = (uint32_t)(uintptr_t)(lds_char*)shared;
@@ -460,12 +460,20 @@ struct GemmTile {
     follow(A, B, nslab, hold_a(A, nslab), hold_b(B, nslab));
     make_a(); make_b();
     da = sa = sb = 0;
+  }
+  __device__ __forceinline__ void load_slab_a() {
 #pragma unroll
     for (int p = 0; p < 8; ++p) load_a(p);
+  }
+
+  // First tile of a workgroup (or of a run that does not stream): nothing is in flight, LDS is free.
+  __device__ __forceinline__ void start(const Operand& A, const Operand& B, int nslab, char* shared,
+                                        const int32_t* b_order = nullptr, int b_rows = 0) {
+    place(A, B, nslab, shared, b_order, b_rows);
+    load_slab_a();
     load_slab_b(0);
     step_a(); step_b(); make_a(); make_b(); da = kSlotBytes;
-#pragma unroll
-    for (int p = 0; p < 8; ++p) load_a(p);
+    load_slab_a();
     step_a(); make_a(); da = 2 * kSlotBytes;
     __builtin_amdgcn_s_waitcnt(0x0F78);    // all but the youngest eight loads
     __syncthreads();
@@ -583,9 +591,234 @@ struct GemmTile {
   }
 };
 
+// The tile of fp32 operands, on the 16-bit matrix cores.
+//
+// An operand element is the sum of three 16-bit floats: x0 = x rounded to 8 bits of mantissa, x1 the rest rounded, x2 what is
+// left (24 bits in all: of 4 M random values none had a remainder; below 2^-108 the last parts lose bits to the smallest exponent).  A
+// product takes the six of the nine partial products that are above 2^-26 of it, into the same fp32 accumulators: six v_mfma 16x16x32
+// of 16 cycles in the place of eight v_mfma 16x16x4_f32 of 32, and six additions to an accumulator in the place of 32.
+//   1536 tokens, H = 1024, V = 151936, us: forward 3270 -> 2020, dhidden 3360 -> 1915, dW 3220 -> 1870
+//   error against 64 bits there (2-norm): logprob 6.5e-8 -> 6.1e-8, dhidden 2.2e-6 -> 1.2e-6, dW 6.8e-7 -> 3.3e-7; the same or better
+//   over eight sizes of 96 - 4096 tokens, H 512 - 2048, V 32000 - 151936
+// What bounds it: issue beside the matrix cores and their power (busy 0.68 - 0.75 of the cycles at 1.9 GHz, where the fp32
+// instructions were busy 0.86 - 0.93 at 2.4).
+//
+// The operands stay fp32 in memory and in LDS.  A wave splits the fragments it has read, 44 instructions for the eight elements
+// that a lane has of a block, 704 beside the 384 matrix instructions of a slab, each of which covers two (a third costs 5
+// cycles).  v_dot2_f32_bf16 with (-1, 0), which leaves the rest of an element in one instruction, holds up the matrix cores: 34 cycles
+// per matrix instruction with one of them beside each.
+// Registers decide the order: the parts of all eight B blocks are kept (96), those of A are made a pair of blocks ahead (2 x 24).
+// A slab is four pairs q of A blocks, a pair eight steps j of B blocks, a step twelve matrix instructions.  Beside them
+//   steps 1 - 7 of a pair            split the next pair of A blocks;
+//   steps 1 - 7 of the last pair     split B blocks 0 - 3 of the next slab, into the registers of this one's, which are used up;
+//   steps 0 - 6 of the first pair    split B blocks 4 - 7, each before its first use;
+//   the last / the first pair        request A of the slab after next / B of the next slab.
+// One barrier per slab, behind the third pair: the next slab has landed, and what is left of this one is in registers.  Two slots
+// per operand are enough, as a slab takes three times as long as one of 16-bit elements.
+//
+// What is not finite has no such parts (inf - inf): a tile with a NaN among its sums is computed again by the fp32
+// instructions (see redo), whose result stands.
+template <int BV, Side kSideA = Side::kRows, bool kUnitsB = false>
+struct SplitTile : GemmTile<float, BV, kSideA, kUnitsB> {
+  using Whole = GemmTile<float, BV, kSideA, kUnitsB>;
+  using typename Whole::Acc;
+  using typename Whole::Operand;
+  using typename Whole::lds_vec;
+  static constexpr bool kSplit = true, kAcross = Whole::kAcross;
+  static constexpr int kSlotBytes = Whole::kSlotBytes, kUnitBytes = Whole::kUnitBytes, kVec = Whole::VEC;
+
+  u32x4 xa[kAcross ? 8 : 4];      // A as it is read: two halves of two blocks, or (across, where a read covers four) eight k of four
+  u32x4 xb[2][2];                 // B as it is read: a block's two halves
+  u32x4 pa[2][2][3], pb[8][3];    // parts: [set][block of the pair][part], [block][part]
+  uint32_t ra[8], rb[8], wa, wb;  // what is left of the elements being split, a part of one
+
+  // Instruction n (0 .. 43) of splitting eight elements x(0) .. x(7): round two of them, widen one, subtract it.
+  static constexpr int kSplitOps = 44;
+  template <int n, typename X>
+  __device__ static __forceinline__ void split(u32x4 (&part)[3], uint32_t (&rest)[8], uint32_t& wide, X x) {
+    constexpr int t = n / 20, k = n % 20, e = (k - 4) / 2;
+    auto left = [&](int i) { return t == 0 ? x(i) : rest[i]; };
+    if constexpr (k < 4) {
+      uint32_t r;
+      asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(left(2 * k)), "v"(left(2 * k + 1)));
+      part[t][k] = r;
+    } else if constexpr (k % 2 == 0) {
+      wide = e % 2 ? part[t][e / 2] & 0xffff0000u : part[t][e / 2] << 16;
+    } else {
+      rest[e] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, left(e)) - __builtin_bit_cast(float, wide));
+    }
+    Whole::fence();
+  }
+  // of block b of the pair q of A, of block j of B
+  template <int n, int b, int q>
+  __device__ __forceinline__ void split_a() {
+    split<n>(pa[q % 2][b], ra, wa, [&](int e) { return kAcross ? xa[e][(2 * q + b) % 4] : xa[2 * b + e / 4][e % 4]; });
+  }
+  template <int n, int j>
+  __device__ __forceinline__ void split_b() {
+    split<n>(pb[j], rb, wb, [&](int e) { return xb[j % 2][e / 4][e % 4]; });
+  }
+  // Reads of the pair q of A (across: of the four blocks it begins) and of block j of B in the slot at `slot`.
+  static constexpr int kReadsA = kAcross ? 8 : 4;
+  template <int n, int q>
+  __device__ __forceinline__ void read_a(uint32_t slot) {
+    if constexpr (kAcross) {
+      const uint32_t at = this->a0 + slot + n / 4 * (kUnitBytes / 2);
+      xa[n] = *(lds_vec*)(uintptr_t)((n % 2 ? at + this->odd_a : at) + q / 2 * 2 * kUnitBytes + n % 4 * kRowBytes);
+    } else {
+      xa[n] = *(lds_vec*)(uintptr_t)((n % 2 ? this->a0 ^ 64 : this->a0) + slot + Whole::a_block(2 * q + n / 2) * kRowBytes);
+    }
+    Whole::fence();
+  }
+  template <int n, int j>
+  __device__ __forceinline__ void read_b(uint32_t slot) {
+    const uint32_t at = (n ? this->b0 ^ 64 : this->b0) + slot;
+    xb[j % 2][n] = *(lds_vec*)(uintptr_t)((j % 2 ? at + this->odd_b : at) + Whole::b_block(j) * kRowBytes);
+    Whole::fence();
+  }
+
+  __device__ __forceinline__ void start(const Operand& A, const Operand& B, int nslab, char* shared,
+                                        const int32_t* b_order = nullptr, int b_rows = 0) {
+    this->place(A, B, nslab, shared, b_order, b_rows);
+    this->load_slab_a();
+    this->load_slab_b(0);
+    this->step_a(); this->step_b(); this->make_a(); this->make_b();
+    this->da = kSlotBytes;
+    this->load_slab_a();
+    __builtin_amdgcn_s_waitcnt(0x0F78);    // all but the youngest eight loads
+    __syncthreads();
+  }
+
+  // The parts a slab's first pair begins with, for a tile's first slab.
+  __device__ __forceinline__ void prime() {
+    each<kReadsA>([&](auto n) __attribute__((always_inline)) { read_a<decltype(n)::value, 0>(this->sa); });
+    each<2>([&](auto b) __attribute__((always_inline)) {
+      each<kSplitOps>([&](auto n) __attribute__((always_inline)) { split_a<decltype(n)::value, decltype(b)::value, 0>(); });
+    });
+    each<5>([&](auto c) __attribute__((always_inline)) {
+      constexpr int j = decltype(c)::value;
+      read_b<0, j>(this->sa);
+      read_b<1, j>(this->sa);
+      if constexpr (j > 0) each<kSplitOps>([&](auto n) __attribute__((always_inline)) { split_b<decltype(n)::value, j - 1>(); });
+    });
+  }
+
+  // The B blocks are split one after another from the second step of a slab's last pair on.  The block that a step reads: each
+  // before its first instruction, in the registers of the one before the last, which is through.
+  static constexpr int b_step(int q, int j) { return q == 3 ? j : q == 0 ? 8 + j : -1; }
+  static constexpr int b_read(int step) {
+    return step == 0 ? 0 : step == 2 ? 1 : step == 3 ? 2 : step == 5 ? 3 : step == 7 ? 4 : step == 8 ? 5 : step == 10 ? 6 : step == 12 ? 7 : -1;
+  }
+  static constexpr int kStepSlots = 12;
+  // Instructions of splitting `blocks` blocks over `steps` steps that stand in front of slot m of them.
+  static constexpr int at(int m, int steps, int blocks) { return blocks * kSplitOps * m / (steps * kStepSlots); }
+
+  // What stands behind matrix instruction m of step j of pair q.
+  template <int q, int j, int m>
+  __device__ __forceinline__ void beside() {
+    constexpr int step = b_step(q, j), next = (q + 1) % 4;
+    const uint32_t other = this->sa ^ kSlotBytes;
+    if constexpr (b_read(step) >= 0 && m < 2) read_b<m, b_read(step)>(q == 3 ? other : this->sa);
+    if constexpr (j == 0 && m >= 2 && m < 2 + kReadsA && (!kAcross || next % 2 == 0)) read_a<m - 2, next>(q == 3 ? other : this->sa);
+    if constexpr (step >= 1 && step <= 14) {
+      constexpr int from = at((step - 1) * kStepSlots + m, 14, 8), to = at((step - 1) * kStepSlots + m + 1, 14, 8);
+      each<to - from>([&](auto c) __attribute__((always_inline)) {
+        constexpr int n = from + decltype(c)::value;
+        split_b<n % kSplitOps, n / kSplitOps>();
+      });
+    }
+    if constexpr (j >= 1) {
+      constexpr int from = at((j - 1) * kStepSlots + m, 7, 2), to = at((j - 1) * kStepSlots + m + 1, 7, 2);
+      each<to - from>([&](auto c) __attribute__((always_inline)) {
+        constexpr int n = from + decltype(c)::value;
+        split_a<n % kSplitOps, n / kSplitOps, next>();
+      });
+    }
+    if constexpr (q == 3 && m == 6) { this->load_a(j); Whole::fence(); }
+    if constexpr (q == 0 && kUnitsB && j > 0 && (m == 3 || m == 4)) { this->next_unit(m - 3, j); Whole::fence(); }
+    if constexpr (q == 0 && m == 6) { this->load_b(j, other); Whole::fence(); }
+    if constexpr (q == 1 && m == 10) {
+      if constexpr (j < Whole::kSteps) this->step_a(j);
+      if constexpr (j == Whole::kSteps) this->make_a();
+      if constexpr (j == Whole::kSteps + 1) this->da = this->sa;
+      Whole::fence();
+    }
+    if constexpr (q == 2 && m == 10) {
+      if constexpr (j < Whole::kSteps) this->step_b(j);
+      if constexpr (j == Whole::kSteps) this->make_b();
+      Whole::fence();
+    }
+  }
+
+  __device__ __forceinline__ void run(Acc& acc, int nslab) {
+#ifdef __HIP_DEVICE_COMPILE__
+    Whole::settle();
+    prime();
+    for (int s = 0; s < nslab; ++s) {
+      each<4>([&](auto cq) __attribute__((always_inline)) {
+        each<8>([&](auto cj) __attribute__((always_inline)) {
+          each<kStepSlots>([&](auto cm) __attribute__((always_inline)) {
+            constexpr int q = decltype(cq)::value, j = decltype(cj)::value, m = decltype(cm)::value;
+            constexpr int of_a[6] = {0, 0, 1, 1, 0, 2}, of_b[6] = {2, 1, 1, 0, 0, 0};
+            asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                         : "+a"(acc[2 * q + m % 2][j]) : "v"(pa[q % 2][m % 2][of_a[m / 2]]), "v"(pb[j][of_b[m / 2]]));
+            Whole::fence();
+            beside<q, j, m>();
+          });
+        });
+        if constexpr (decltype(cq)::value == 2) {
+          __builtin_amdgcn_s_waitcnt(0x0070);      // the next slab has landed, this one's reads are through
+          __builtin_amdgcn_s_barrier();
+          Whole::fence();
+        }
+      });
+      this->sa ^= kSlotBytes;
+    }
+    Whole::settle();
+#endif
+  }
+
+  // Behind run(): whether the tile had to be computed again.  An operand element that is not finite makes every sum of its row NaN
+  // (its parts are, and 0 * NaN is), so a sum of every row and one of every column tell.  `init` sets the accumulators as they were
+  // before run().  LDS is free then, and the next tile begins with start().
+  template <typename Init>
+  __device__ __forceinline__ bool redo(Acc& acc, const Operand& A, const Operand& B, int nslab, char* shared, Init init,
+                                       const int32_t* b_order = nullptr, int b_rows = 0) {
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < Whole::MI; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum += acc_get(acc[i][0], r);
+#pragma unroll
+    for (int j = 1; j < Whole::NI; ++j) sum += acc_get(acc[0][j], 0);
+    // the flags are in the third slot of A, which this tile does not use
+    typedef __attribute__((address_space(3))) volatile uint32_t lds_flag;
+    lds_flag* flag = (lds_flag*)(uintptr_t)((uint32_t)(uintptr_t)(typename Whole::lds_char*)shared + 2 * kSlotBytes);
+    const bool bad = __any(sum != sum);
+    if ((threadIdx.x & 63) == 0) flag[threadIdx.x >> 6] = bad;
+    __builtin_amdgcn_s_waitcnt(0xC07F);      // this wave's flag is written (loads stay outstanding)
+    __builtin_amdgcn_s_barrier();
+    const uint32_t any = flag[0] | flag[1] | flag[2] | flag[3];
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(any) == 0, 1)) return false;
+    Whole::finish();
+    init();
+    Whole whole;
+    whole.start(A, B, nslab, shared, b_order, b_rows);
+    whole.run(acc, nslab);
+    Whole::finish();
+    return true;
+  }
+};
+
+// The tile for operands of type T.
+template <typename T, int BV, Side S = Side::kRows, bool kUnitsB = false, int NI = 8>
+struct TileOf { typedef GemmTile<T, BV, S, kUnitsB, NI> type; };
+template <int BV, Side S, bool kUnitsB>
+struct TileOf<float, BV, S, kUnitsB, 8> { typedef SplitTile<BV, S, kUnitsB> type; };
+
 constexpr int kHeadThreads = 256;
 // The tile of the kernels that hold logits (A = vocabulary, B = tokens).
-template <typename T, int NI = 8> using LogitTile = GemmTile<T, NI, Side::kRows, false, NI>;
+template <typename T, int NI = 8> using LogitTile = typename TileOf<T, NI, Side::kRows, false, NI>::type;
 
 // Workgroup id -> logical work item so that the workgroups resident on one XCD
 // (hardware deals consecutive ids round-robin over the 8 XCDs) own a contiguous

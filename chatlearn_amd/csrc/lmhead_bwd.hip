@@ -87,8 +87,10 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_dz_kernel(DzParams p) 
   if (block_live) {
     Tile core;
     const int nslab = p.H / Tile::kSlabK;
-    core.start(Tile::Operand::row_major(weight, p.H, a_rows), Tile::Operand::row_major(hidden, p.H, b_rows), nslab, lds);
+    const auto op_a = Tile::Operand::row_major(weight, p.H, a_rows), op_b = Tile::Operand::row_major(hidden, p.H, b_rows);
+    core.start(op_a, op_b, nslab, lds);
     core.run(acc, nslab);
+    if constexpr (Tile::kSplit) core.redo(acc, op_a, op_b, nslab, lds, [&] { Tile::zero(acc); });
     Tile::finish();
   }
 
@@ -293,7 +295,7 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams<T> p) {
 //   dhidden (kMContig): C[n][m], ld = ldc, A = W^T (kWeight: W itself; kRows: the caller's K-blocked W^T), B = dz (in
 //     units).  A lane holds VEC consecutive m of a row, the 4 lane groups 64 contiguous bytes of each of 16 rows for 16-bit results.
 template <Side S> constexpr bool kMContig = S != Side::kLogits;
-template <typename T, Side S, int NI = 8> using OutTile = GemmTile<T, kMContig<S> ? NI : 4, S, kMContig<S>, NI>;
+template <typename T, Side S, int NI = 8> using OutTile = typename TileOf<T, kMContig<S> ? NI : 4, S, kMContig<S>, NI>::type;
 
 struct GemmParams {
   const void* A;
@@ -305,7 +307,6 @@ struct GemmParams {
   int M, N, K;
   int k_valid;              // kWeight: rows of W; the rest of K reads as zero
   int n_mt, n_nt;
-  int accumulate;
   int k_split;        // > 1: work item = (tile, K range); fp32 partial tiles go to `partial`
   int k_per_split;    // K extent of one range, a multiple of the slab
   int xcd_wgs;        // see work_item
@@ -420,10 +421,10 @@ __device__ __forceinline__ void for_rows(const TileAddr<T, OutT, S, NI>& at, Acc
 // latency (H = 4096 over 151936 entries, loads of half a block row at a time -> these: 256 tokens 1.24 -> 0.96 ms = 5.2 TB/s
 // over reads and writes, 1024 tokens 1.76 -> 1.48, 3520 tokens 3.55 -> 3.33).  A fourth block row ahead does not fit
 // the registers.
-template <typename T, Side S, int NI>
+template <typename T, Side S, int NI, int kAhead = 3>
 struct RowLoads {
   using Tile = OutTile<T, S, NI>;
-  static constexpr int kAhead = 3, kSlots = kAhead + 1;
+  static constexpr int kSlots = kAhead + 1;
   f32x4 x[kSlots][NI / 4][4];      // [block row][group of four blocks][register of the blocks]
   typedef TileAddr<T, float, S, NI> At;
   __device__ __forceinline__ void fetch(const At& at, int i) {
@@ -474,7 +475,9 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, typename Ou
 // when C is [n][m], B's n tile when C is [m][n]) and walks a contiguous run of tiles of the other, so the
 // K loops stream into each other (the next tile's first slabs are requested while the current tile
 // finishes and is stored).  Otherwise work item = (K range, m tile, n tile), one K loop per workgroup.
-template <typename T, typename OutT, Side S, int NI>
+// kAdds: C is added to, and one workgroup owns the whole K range of a tile (an argument in its place had fp32 tiles spill
+// 400 registers).
+template <typename T, typename OutT, Side S, int NI, bool kAdds>
 __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
   using Tile = OutTile<T, S, NI>;
   constexpr bool kMC = kMContig<S>;
@@ -521,38 +524,44 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
   auto rows_of = [](int total, int tile, int width) { const int left = total - tile * width; return left < width ? left : width; };
   // Accumulators before a tile's K loop: zeros, or - when the GEMM adds to C and one workgroup owns the whole K range of
   // the tile - the tile's current contents, which leaves the epilogue a pure store.
-  constexpr bool kCanAdd = !kMC && sizeof(OutT) == 4;     // only an fp32 C is ever added to
-  const bool adds = kCanAdd && p.accumulate && p.k_split == 1;
-  typedef RowLoads<T, S, NI> Loads;
+  static_assert(!kAdds || (!kMC && sizeof(OutT) == 4), "only an fp32 dW is ever added to");
+  typedef RowLoads<T, S, NI, Tile::kSplit ? 1 : 3> Loads;
   auto c_tile = [&](int m_tile) {
     return typename Loads::At(static_cast<float*>(p.C), p.ldc, m_tile * 256, nt * Tile::BN, rows_of(p.M, m_tile, 256),
                               rows_of(p.N, nt, Tile::BN));
   };
   typename Tile::Acc acc;
   Loads loads;
-  if constexpr (kCanAdd) {
-    if (adds) loads.begin(c_tile(mt));
-  }
+  if constexpr (kAdds) loads.begin(c_tile(mt));
   Tile core;
+  bool again = false;      // the tile before was computed twice: nothing of this one has been requested
   for (int k = 0; k < count; ++k) {
     const int m0 = mt * 256, n0 = nt * Tile::BN;
     const int a_rows = rows_of(p.M, mt, 256), b_rows = rows_of(p.N, nt, Tile::BN);
     const auto op_a = operand_a(mt, a_rows);
     const auto op_b = operand_b(nt, b_rows);
-    if (!adds) Tile::zero(acc);
-    if constexpr (kCanAdd) {
-      if (adds) loads.finish(c_tile(mt), acc);
-    }
-    if (k == 0 || !stream) core.start(op_a, op_b, nslab, lds);
+    if constexpr (kAdds) loads.finish(c_tile(mt), acc);
+    else Tile::zero(acc);
+    if (k == 0 || !stream || again) core.start(op_a, op_b, nslab, lds);
     if (stream && k + 1 < count)
       core.follow(op_a, op_b, nslab, Tile::cursor_a(kMC ? op_a : operand_a(mt + 1, rows_of(p.M, mt + 1, 256)), nslab),
                   Tile::cursor_b(kMC ? operand_b(nt + 1, rows_of(p.N, nt + 1, Tile::BN)) : op_b, nslab));
     else
       core.follow(op_a, op_b, nslab, Tile::hold_a(op_a, nslab), Tile::hold_b(op_b, nslab));
     core.run(acc, nslab);
+    if constexpr (Tile::kSplit) {
+      again = core.redo(acc, op_a, op_b, nslab, lds, [&] {
+        if constexpr (kAdds) {
+          RowLoads<T, S, NI, 0> old;
+          old.finish(c_tile(mt), acc);
+        } else {
+          Tile::zero(acc);
+        }
+      });
+    }
     if (!stream || k + 1 == count) Tile::finish();
-    if constexpr (kCanAdd) {
-      if (adds && k + 1 < count) loads.begin(c_tile(mt + 1));
+    if constexpr (kAdds) {
+      if (k + 1 < count) loads.begin(c_tile(mt + 1));
     }
     gemm_store_tile<T, OutT, S, NI>(p, acc, m0, n0, a_rows, b_rows, ks);
     if (kMC) ++nt; else ++mt;
@@ -813,13 +822,10 @@ static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64
                            float* partial, size_t partial_bytes, int k_split_wanted, const RowOrder& rows = RowOrder{nullptr, 0}) {
   using Tile = OutTile<T, S, NI>;
   constexpr bool kMC = kMContig<S>;
-  int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(&gemm_kernel<T, OutT, S, NI>), Tile::kLdsBytes, "gemm_kernel");
-  if (rc) return rc;
   GemmParams g;
   g.A = in.A; g.B = in.B; g.C = C; g.a_step = in.a_step; g.b_step = in.b_step; g.ldc = ldc; g.k_valid = in.k_valid;
   g.M = M; g.N = N; g.K = K;
   g.n_mt = (M + 255) / 256; g.n_nt = (N + Tile::BN - 1) / Tile::BN;
-  g.accumulate = accumulate;
   g.order = rows.order; g.total = rows.total;
   const int slab = Tile::kSlabK;
   const int cus = device_cu_count();
@@ -857,8 +863,17 @@ static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64
   ItemGrid grid{(g.n_walk * n_fixed + 7) / 8 * 8, 0};
   if (g.n_walk == 0) grid = rounds ? item_grid(g.n_mt * g.n_nt, cus) : ItemGrid{(g.n_mt * g.n_nt * g.k_split + 7) / 8 * 8, 0};
   g.xcd_wgs = grid.xcd_wgs;
-  hipLaunchKernelGGL((gemm_kernel<T, OutT, S, NI>), dim3(grid.grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
-  rc = check_launch("gemm_kernel");
+  auto launch = [&](auto kernel) {
+    const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), Tile::kLdsBytes, "gemm_kernel");
+    if (rc) return rc;
+    hipLaunchKernelGGL(kernel, dim3(grid.grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
+    return check_launch("gemm_kernel");
+  };
+  int rc;
+  if constexpr (!kMC && sizeof(OutT) == 4)
+    rc = accumulate && g.k_split == 1 ? launch(&gemm_kernel<T, OutT, S, NI, true>) : launch(&gemm_kernel<T, OutT, S, NI, false>);
+  else
+    rc = launch(&gemm_kernel<T, OutT, S, NI, false>);
   if (rc || g.k_split == 1) return rc;
   return launch_splitk_reduce<OutT>(partial, g.k_split, kMC ? N : M, kMC ? M : N, static_cast<OutT*>(C), ldc, accumulate,
                                     rows.order, stream);

@@ -122,13 +122,14 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
                                              order ? p.total : b_rows);
   const int vt_begin = vs * p.tiles_per_split;
   const int vt_end = (vt_begin + p.tiles_per_split) < p.n_vt ? (vt_begin + p.tiles_per_split) : p.n_vt;
+  bool again = false;      // the tile before was computed twice: nothing of this one has been requested
   for (int vt = vt_begin; vt < vt_end; ++vt) {
     const int v0 = vt * kFwdBM;
     const int a_rows = (p.V - v0) < kFwdBM ? (p.V - v0) : kFwdBM;
     const auto op_a = Tile::Operand::row_major(weight + (int64_t)v0 * p.H, p.H, a_rows);
     typename Tile::Acc acc;
     Tile::zero(acc);
-    if (vt == vt_begin || !stream) core.start(op_a, op_b, nslab, lds, order, b_rows);
+    if (vt == vt_begin || !stream || again) core.start(op_a, op_b, nslab, lds, order, b_rows);
     if (stream && vt + 1 < vt_end) {
       const int v1 = v0 + kFwdBM;
       const int next_rows = (p.V - v1) < kFwdBM ? (p.V - v1) : kFwdBM;
@@ -138,6 +139,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
       core.follow(op_a, op_b, nslab, Tile::hold_a(op_a, nslab), Tile::hold_b(op_b, nslab));
     }
     core.run(acc, nslab);
+    if constexpr (Tile::kSplit) again = core.redo(acc, op_a, op_b, nslab, lds, [&] { Tile::zero(acc); }, order, b_rows);
     if (!stream) Tile::finish();
 
     const bool full = a_rows == kFwdBM;
