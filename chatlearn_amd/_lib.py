@@ -131,6 +131,7 @@ SIGNATURES = {
     "clgrpo_lmhead_fwd_tile_plan": (C.c_int, [i64, i64, i64, i32, i32, vp]),
     "clgrpo_lmhead_bwd_dhidden_plan": (C.c_int, [i64, i64, i64, i32, i32, vp]),
     "clgrpo_lmhead_bwd_dhidden_tile_plan": (C.c_int, [i64, i64, i64, i32, i32, i64, vp]),
+    "clgrpo_lmhead_bwd_guest_plan": (C.c_int, [i64, i64, i64, i32, i64, vp]),
     "clgrpo_lmhead_bwd_dweight_plan": (C.c_int, [i64, i64, i64, i32, i32, vp]),
     "clgrpo_saved_logits_ld": (i64, [i64]),
     "clgrpo_lmhead_bwd_workspace_bytes": (sz, [i64, i64, i64, i32, i64, i32]),

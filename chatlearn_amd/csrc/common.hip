@@ -26,7 +26,7 @@ int check_launch(const char* what) {
 // The limit is a per-device property of a kernel; a process may drive several devices and call from
 // several threads.  Small fixed table: at most kMaxKernels kernels on kMaxDevices devices.
 int ensure_dynamic_lds(const void* kernel, int bytes, const char* name) {
-  constexpr int kMaxKernels = 32, kMaxDevices = 64;
+  constexpr int kMaxKernels = 64, kMaxDevices = 64;
   static std::atomic<const void*> keys[kMaxKernels];
   static std::atomic<unsigned char> done[kMaxKernels][kMaxDevices];
   int dev = 0;

@@ -516,51 +516,83 @@ struct GemmTile {
     return n;
   }
 
+  // A slab, and what a guest does beside it: guest.first<m>() and guest.second<m>() stand behind matrix instruction m of
+  // either half, and have issued Guest::kOps vector memory accesses between one half's loads and the next one's.
+  struct NoGuest {
+    static constexpr int kOps = 0;
+    template <int m> __device__ __forceinline__ void first() {}
+    template <int m> __device__ __forceinline__ void second() {}
+  };
+  template <typename Guest>
+  __device__ __forceinline__ void slab(Acc& acc, Guest& guest) {
+#ifdef __HIP_DEVICE_COMPILE__      // the host's pass drops kernels whose body holds this many lambdas, without a word
+    each<kSlots>([&](auto c) __attribute__((always_inline)) {            // first half of the slab
+      constexpr int m = decltype(c)::value, n = step_at(0, m);
+      Mma<T>::template slot<kAcross, NI>(acc, af[0], bf[0], m);
+      fence();
+      if constexpr (m % 2 == 0 && m < 2 * (MI + NI)) { read(1, half_a() + sa, (b0 ^ 64) + sb, m / 2); fence(); }
+      if constexpr (load_a_at(m) >= 0) { load_a(load_a_at(m)); fence(); }
+      if constexpr (n >= 0 && n < kSteps) { step_b(n); fence(); }
+      if constexpr (n == kSteps) { make_b(); fence(); }
+      if constexpr (n == kSteps + 1) { sa1 = next_slot(sa); fence(); }
+      if constexpr (kPerm) {
+#pragma unroll
+        for (int k = perm_from(0, m); k < perm_from(0, m + 1); ++k) { perm(1, k); fence(); }
+      }
+      guest.template first<m>();
+    });
+    fence();
+    // every wave has the last fragments of this slab, and the next one's loads have landed: all but the youngest eight, A of the slab
+    // after it, and what the guest has issued around them
+    __builtin_amdgcn_s_waitcnt(0x0070 + 8 + Guest::kOps);
+    static_assert(8 + Guest::kOps < 16, "the wait's upper bits are elsewhere");
+    __builtin_amdgcn_s_barrier();
+    fence();
+    each<kSlots>([&](auto c) __attribute__((always_inline)) {            // second half, while the next slab's first fragments come in
+      constexpr int m = decltype(c)::value, n = step_at(1, m);
+      Mma<T>::template slot<kAcross, NI>(acc, af[1], bf[1], m);
+      fence();
+      if constexpr (m % 2 == 0 && m < 2 * (MI + NI)) { read(0, a0 + sa1, b0 + (sb ^ kSlotBytes), m / 2); fence(); }
+      if constexpr (load_b_at(m) >= 0) { load_b(load_b_at(m), sb); fence(); }
+      if constexpr (unit_at(m + 2) > 0) { next_unit(0, unit_at(m + 2)); fence(); }
+      if constexpr (unit_at(m + 1) > 0) { next_unit(1, unit_at(m + 1)); fence(); }
+      if constexpr (n >= 0 && n < kSteps) { step_a(n); fence(); }
+      if constexpr (n == kSteps) { make_a(); fence(); }
+      if constexpr (n == kSteps + 1) { da = next_slot(da); fence(); }
+      if constexpr (kPerm) {
+#pragma unroll
+        for (int k = perm_from(1, m); k < perm_from(1, m + 1); ++k) { perm(0, k); fence(); }
+      }
+      guest.template second<m>();
+    });
+    sa = sa1; sb ^= kSlotBytes;
+#endif
+  }
+
   // One tile's K loop of `nslab` slabs; acc must be initialised by the caller.  Between tiles of a
   // streaming workgroup LDS stays in use; after the last one call finish() before touching it.
   __device__ __forceinline__ void run(Acc& acc, int nslab) {
-#ifdef __HIP_DEVICE_COMPILE__      // the host's pass drops kernels whose body holds this many lambdas, without a word
     settle();
-    for (int s = 0; s < nslab; ++s) {
-      each<kSlots>([&](auto c) __attribute__((always_inline)) {            // first half of the slab
-        constexpr int m = decltype(c)::value, n = step_at(0, m);
-        Mma<T>::template slot<kAcross, NI>(acc, af[0], bf[0], m);
-        fence();
-        if constexpr (m % 2 == 0 && m < 2 * (MI + NI)) { read(1, half_a() + sa, (b0 ^ 64) + sb, m / 2); fence(); }
-        if constexpr (load_a_at(m) >= 0) { load_a(load_a_at(m)); fence(); }
-        if constexpr (n >= 0 && n < kSteps) { step_b(n); fence(); }
-        if constexpr (n == kSteps) { make_b(); fence(); }
-        if constexpr (n == kSteps + 1) { sa1 = next_slot(sa); fence(); }
-        if constexpr (kPerm) {
-#pragma unroll
-          for (int k = perm_from(0, m); k < perm_from(0, m + 1); ++k) { perm(1, k); fence(); }
-        }
-      });
-      fence();
-      // every wave has the last fragments of this slab, and the next one's loads have landed
-      __builtin_amdgcn_s_waitcnt(0x0078);
-      __builtin_amdgcn_s_barrier();
-      fence();
-      each<kSlots>([&](auto c) __attribute__((always_inline)) {            // second half, while the next slab's first fragments come in
-        constexpr int m = decltype(c)::value, n = step_at(1, m);
-        Mma<T>::template slot<kAcross, NI>(acc, af[1], bf[1], m);
-        fence();
-        if constexpr (m % 2 == 0 && m < 2 * (MI + NI)) { read(0, a0 + sa1, b0 + (sb ^ kSlotBytes), m / 2); fence(); }
-        if constexpr (load_b_at(m) >= 0) { load_b(load_b_at(m), sb); fence(); }
-        if constexpr (unit_at(m + 2) > 0) { next_unit(0, unit_at(m + 2)); fence(); }
-        if constexpr (unit_at(m + 1) > 0) { next_unit(1, unit_at(m + 1)); fence(); }
-        if constexpr (n >= 0 && n < kSteps) { step_a(n); fence(); }
-        if constexpr (n == kSteps) { make_a(); fence(); }
-        if constexpr (n == kSteps + 1) { da = next_slot(da); fence(); }
-        if constexpr (kPerm) {
-#pragma unroll
-          for (int k = perm_from(1, m); k < perm_from(1, m + 1); ++k) { perm(0, k); fence(); }
-        }
-      });
-      sa = sa1; sb ^= kSlotBytes;
-    }
+    NoGuest none;
+    for (int s = 0; s < nslab; ++s) slab(acc, none);
     settle();
-#endif
+  }
+  // The same with a guest in the first 2 `pairs` slabs; at least one pair and one slab more.  (A loop that may not run at all, between
+  // the accumulators' clearing and another one, had them moved and 200 registers spilled.)
+  template <typename Guest>
+  __device__ __forceinline__ void run_with(Acc& acc, int nslab, int pairs, Guest& guest) {
+    settle();
+    int s = 0;
+    do {
+      auto even = guest.template turn<0>();
+      slab(acc, even);
+      auto odd = guest.template turn<1>();
+      slab(acc, odd);
+    } while (++s < pairs);
+    NoGuest none;
+    s = 2 * pairs;
+    do slab(acc, none); while (++s < nslab);
+    settle();
   }
 
   __device__ __forceinline__ uint32_t half_a() const { return kAcross ? a0 + kUnitBytes / 2 : a0 ^ 64; }

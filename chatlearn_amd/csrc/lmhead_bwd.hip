@@ -12,6 +12,7 @@
 // Algorithmic work: 4*T*H*V flop (dhidden + dW); the z recomputation (2*T*H*V) is overhead.
 #include "head_internal.hpp"
 #include "gemm_core.hpp"
+#include <type_traits>
 
 namespace clgrpo {
 
@@ -187,10 +188,7 @@ __global__ __launch_bounds__(256) void transpose_block_kernel(TransposeParams<T>
 // The last workgroups of the launch write hidden^T, dW's other operand, which took a launch of 5 to 12 us of its own.
 // 12126 rows of the 152k vocabulary: 2.25 -> 1.49 ms, 32768 rows 5.92 -> 3.57 ms (5.6 TB/s), against a pass that also wrote the
 // transpose.
-template <typename T>
-struct DzFromZParams {
-  const void* z;      // kept logits (KeptLogit<T>): z_kslab units per row of units
-  void* dz;           // d(logits) (T): dz_kslab units per row of units
+struct DzTokens {
   const int64_t* labels;
   int64_t label_offset;
   const float* lse;
@@ -198,10 +196,47 @@ struct DzFromZParams {
   const float* g_lp;
   const float* g_ent;
   const int32_t* order;   // optional [Tc]: row n is token order[n] of the per-token arrays
-  int64_t z_kslab, dz_kslab;
-  int Tc, V, n_units;     // n_units: units of dz per row of units
-  int n_step;             // workgroups per row of units; more of them along y turn 64 columns of hidden each
+  int Tc, V;
   float c, inv_temperature;
+};
+// d(logits) of a row from its raw logits z, tau = 1 / inv_temperature:  x = z c - lse log2(e);
+// dz = tau^-1 (g_lp (1[v = y] - 2^x) - g_H 2^x (x ln 2 + H))  =  2^x (k1 + k2 x) + [v = y] top.
+struct DzRow {
+  float shift, k1, k2, top;   // shift = -lse log2(e)
+  int label;                  // or -1
+  bool live;                  // rows past the chunk and rows without a gradient give zeros
+  template <bool kEntropy>
+  __device__ __forceinline__ static DzRow of(const DzTokens& p, int n) {
+    DzRow r;
+    const bool ok = n < p.Tc;
+    const int t = ok && p.order ? p.order[n] : n;
+    const float glp = ok ? p.g_lp[t] : 0.f, gen = kEntropy && ok ? p.g_ent[t] : 0.f, ent = kEntropy && ok ? p.entropy[t] : 0.f;
+    r.shift = ok ? -(p.lse[t] * kLog2e) : 0.f;
+    r.top = p.inv_temperature * glp;
+    r.k1 = kEntropy ? -p.inv_temperature * fmaf(gen, ent, glp) : -r.top;
+    r.k2 = kEntropy ? -p.inv_temperature * gen * 0.6931471805599453f : 0.f;
+    r.live = glp != 0.f || gen != 0.f;
+    r.label = -1;
+    if (ok) {
+      const int64_t rel = p.labels[t] - p.label_offset;
+      if (rel >= 0 && rel < p.V) r.label = (int)rel;
+    }
+    return r;
+  }
+};
+
+template <typename T>
+struct DzFromZParams {
+  const void* z;      // kept logits (KeptLogit<T>): z_kslab units per row of units
+  void* dz;           // d(logits) (T): dz_kslab units per row of units
+  DzTokens t;
+  int64_t z_kslab, dz_kslab;
+  int n_units;        // units of dz per row of units
+  int row0, row_units;   // rows of units to convert
+  int n_step;            // workgroups per row of units
+  int whole;             // units of such a row to convert
+  int n_edge;            // rows of units, from the first on, of which the units from `whole` on are converted
+  int turn_rows;         // workgroups behind those turn 64 x 64 hidden states each, this many of them along the tokens
   TransposeParams<T> turn;
 };
 
@@ -213,41 +248,33 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams<T> p) {
   constexpr int VEC = 16 / (int)sizeof(T);          // elements per 16-byte piece
   constexpr int kRows = E / 32;                     // tokens per thread
   constexpr int kAhead = 4;                         // units in flight
-  if ((int)blockIdx.y >= p.n_step) {                // the same for the whole workgroup
-    if (blockIdx.x * E % 64 == 0) transpose_tile<T>(p.turn, blockIdx.x * E, ((int)blockIdx.y - p.n_step) * 64);
+  // the same for the whole workgroup: its row of units and first unit, or its square of hidden states
+  int item = blockIdx.x, unit_row, unit, end = p.whole, step = p.n_step;
+  if (item < p.row_units * p.n_step) {
+    unit_row = p.row0 + item % p.row_units;
+    unit = item / p.row_units;
+  } else if ((item -= p.row_units * p.n_step) < p.n_edge) {
+    unit_row = item;
+    unit = p.whole;
+    end = p.n_units;
+    step = 1;
+  } else {
+    item -= p.n_edge;
+    transpose_tile<T>(p.turn, item % p.turn_rows * 64, item / p.turn_rows * 64);
     return;
   }
   const int q = threadIdx.x & 7, row = threadIdx.x >> 3;
-  const float it = p.inv_temperature;
-  float lse[kRows], lse2[kRows], glp[kRows], gen[kRows], ent[kRows];
-  int lab[kRows];
-  bool live[kRows];
+  DzRow r[kRows];
 #pragma unroll
-  for (int h = 0; h < kRows; ++h) {
-    const int n = blockIdx.x * E + h * 32 + row;
-    const bool ok = n < p.Tc;                       // rows past the chunk and rows without a gradient give zeros
-    const int t = ok && p.order ? p.order[n] : n;
-    glp[h] = ok ? p.g_lp[t] : 0.f;
-    gen[h] = kEntropy && ok ? p.g_ent[t] : 0.f;
-    lse[h] = ok ? p.lse[t] : 0.f;
-    ent[h] = kEntropy && ok ? p.entropy[t] : 0.f;
-    lse2[h] = lse[h] * kLog2e;
-    live[h] = glp[h] != 0.f || gen[h] != 0.f;
-    lab[h] = -1;
-    if (ok) {
-      const int64_t rel = p.labels[t] - p.label_offset;
-      if (rel >= 0 && rel < p.V) lab[h] = (int)rel;
-    }
-  }
+  for (int h = 0; h < kRows; ++h) r[h] = DzRow::of<kEntropy>(p.t, unit_row * E + h * 32 + row);
   const int at = row * kRowBytes + q * 16;          // byte of this thread's first piece within a unit
-  const char* z = static_cast<const char*>(p.z) + (int64_t)blockIdx.x * p.z_kslab * (E * kRowBytes) + at;
-  char* dz = static_cast<char*>(p.dz) + (int64_t)blockIdx.x * p.dz_kslab * (E * kRowBytes) + at;
-  const int step = p.n_step;
-  for (int k0 = blockIdx.y; k0 < p.n_units; k0 += kAhead * step) {
+  const char* z = static_cast<const char*>(p.z) + (int64_t)unit_row * p.z_kslab * (E * kRowBytes) + at;
+  char* dz = static_cast<char*>(p.dz) + (int64_t)unit_row * p.dz_kslab * (E * kRowBytes) + at;
+  for (int k0 = unit; k0 < end; k0 += kAhead * step) {
     u32x4 raw[kAhead][kRows];
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
-      const int ks = k0 + u * step < p.n_units ? k0 + u * step : k0;
+      const int ks = k0 + u * step < end ? k0 + u * step : k0;
 #pragma unroll
       for (int h = 0; h < kRows; ++h)
         raw[u][h] = *reinterpret_cast<const u32x4*>(z + (int64_t)ks * (E * kRowBytes) + h * 32 * kRowBytes);
@@ -255,37 +282,175 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams<T> p) {
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
       const int ks = k0 + u * step;
-      if (ks >= p.n_units) break;
+      if (ks >= end) break;
       const int v = ks * E + q * VEC;
 #pragma unroll
       for (int h = 0; h < kRows; ++h) {
         const ZT* in = reinterpret_cast<const ZT*>(&raw[u][h]);
         float d[VEC];
+        const bool here = (unsigned)(r[h].label - v) < (unsigned)VEC;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-          const float zraw = (float)in[e];
-          const float pr = __builtin_amdgcn_exp2f(fmaf(zraw, p.c, -lse2[h]));
-          float up = glp[h];
-          if (kEntropy) up = fmaf(gen[h], fmaf(zraw, it, -lse[h]) + ent[h], up);
-          d[e] = -it * pr * up;
+          const float x = fmaf((float)in[e], p.t.c, r[h].shift);
+          d[e] = __builtin_amdgcn_exp2f(x) * (kEntropy ? fmaf(x, r[h].k2, r[h].k1) : r[h].k1);
         }
-        if ((unsigned)(lab[h] - v) < (unsigned)VEC) {
+        if (here) {
 #pragma unroll
           for (int e = 0; e < VEC; ++e)
-            if (lab[h] - v == e) d[e] += it * glp[h];
+            if (r[h].label - v == e) {
+              const float x = fmaf((float)in[e], p.t.c, r[h].shift);
+              d[e] = fmaf(__builtin_amdgcn_exp2f(x), kEntropy ? fmaf(x, r[h].k2, r[h].k1) : r[h].k1, r[h].top);
+            }
         }
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) d[e] = live[h] ? d[e] : 0.f;
-        if (v + VEC > p.V) {                        // vocabulary padding columns give zeros
+        for (int e = 0; e < VEC; ++e) d[e] = r[h].live ? d[e] : 0.f;
+        if (v + VEC > p.t.V) {                      // vocabulary padding columns give zeros
 #pragma unroll
           for (int e = 0; e < VEC; ++e)
-            if (v + e >= p.V) d[e] = 0.f;
+            if (v + e >= p.t.V) d[e] = 0.f;
         }
         *reinterpret_cast<u32x4*>(dz + (int64_t)ks * (E * kRowBytes) + h * 32 * kRowBytes) = pack_vec(d, (T*)nullptr);
       }
     }
   }
 }
+
+// The same conversion, bit for bit, as a guest of dhidden's K loop (16-bit operands): while the matrix cores contract the rows of
+// one launch, its workgroups convert the rows of the next.  The pass by itself is bound by HBM and leaves the matrix cores idle;
+// the K loop leaves HBM idle, and covers two vector instructions per matrix instruction of which it uses one in two: a piece is about
+// 60 of the 190 left in a slab (two where H < 3072 asks for them: 32768 rows of 2048, V = 151936, 15.85 -> 15.63 ms; 12288 of 4096
+// 10.57 -> 10.70).  What it still costs is power (see plan_hosts).
+// A workgroup takes a run of units of one row of units, a thread kRows pieces of 16 bytes of every slab: requested two slabs before
+// they are looked at, written a slab later, all by range-checked accesses, so that what lies past the run is neither read nor
+// written.  The accesses stand behind a half's operand loads: the wait in the middle of a slab leaves the youngest of them out.
+template <bool kEntropy, int kRowsOf>
+struct DzGuest {
+  static constexpr bool kHosts = true;
+  static constexpr int kRows = kRowsOf, kOps = 2 * kRows, kUnitBytes = 64 * kRowBytes;
+  static_assert(kRows == 1 || kRows == 2, "rows 32 apart of a unit");
+  struct Params {
+    const char* z;      // of the first row of units to convert
+    char* dz;
+    DzTokens t;
+    int64_t z_kslab, dz_kslab;
+    int n0;             // its first row
+    int runs, run_rows, n_units, per_run;   // runs per row of units x rows of units; units, units of a run
+  };
+  __amdgpu_buffer_rsrc_t rsrc_z, rsrc_dz;
+  int load_at, store_at, store_next;
+  int rel[kRows];                  // label - vocabulary entry of the piece that is finished
+  float shift[kRows], k1[kRows], k2[kRows], top[kRows], c;
+  uint32_t live[kRows];
+  u32x4 raw[2][kRows], out[kRows];
+  float x[kRows][8], pr[kRows][8];
+  int pairs;                       // pairs of slabs that the run takes
+
+  __device__ __forceinline__ static int pieces(const Params& p, int item) {
+    const int row = item / p.runs, run = item % p.runs;
+    const int left = p.n_units - run * p.per_run;
+    return row < p.run_rows && left > 0 ? (left < p.per_run ? left : p.per_run) : 0;
+  }
+  __device__ __forceinline__ void place(const Params& p, int item) {
+    constexpr int kParts = 2 / kRows;            // of a row of units
+    const int n = pieces(p, item);
+    pairs = (n + 2) / 2;                         // one slab more, to write the last piece in
+    const int row = n > 0 ? item / p.runs : 0, run = n > 0 ? item % p.runs : 0;
+    const int lane_row = (int)(threadIdx.x >> 3) + row % kParts * 32, q = threadIdx.x & 7;
+    const int64_t first = (int64_t)run * p.per_run;
+    rsrc_z = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.z + (row / kParts * p.z_kslab + first) * kUnitBytes), 0, n * kUnitBytes, 0x00020000);
+    rsrc_dz = __builtin_amdgcn_make_buffer_rsrc(p.dz + (row / kParts * p.dz_kslab + first) * kUnitBytes, 0, n * kUnitBytes, 0x00020000);
+    load_at = store_next = lane_row * kRowBytes + q * 16;
+    store_at = 0x7f000000;                       // there is no piece before the first
+    c = p.t.c;
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+      const DzRow r = DzRow::of<kEntropy>(p.t, p.n0 + row / kParts * 64 + h * 32 + lane_row);
+      rel[h] = r.label < 0 ? -0x40000000 : r.label - ((int)first - 1) * 64 - q * 8;
+      shift[h] = r.shift; k1[h] = r.k1; k2[h] = r.k2; top[h] = r.top;
+      live[h] = r.live ? 0xffffffffu : 0u;
+      out[h] = u32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[h][e] = pr[h][e] = 0.f;
+    }
+  }
+  template <int par>
+  __device__ __forceinline__ void request(int h) {
+    raw[par][h] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_z, load_at + h * 32 * kRowBytes, 0, 0);
+  }
+  __device__ __forceinline__ void begin() {
+    // what the rows need has arrived: not a wait in the K loop
+#pragma unroll
+    for (int h = 0; h < kRows; ++h)
+      asm volatile("" : "+v"(shift[h]), "+v"(k1[h]), "+v"(k2[h]), "+v"(top[h]), "+v"(rel[h]), "+v"(live[h]));
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) request<0>(h);
+    load_at += kUnitBytes;
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) request<1>(h);
+    load_at += kUnitBytes;
+  }
+  template <int par>
+  struct Turn {
+    DzGuest& g;
+    static constexpr int kOps = DzGuest::kOps;
+    __device__ __forceinline__ static void fence() { __builtin_amdgcn_sched_barrier(0); }
+    // second half of a slab: exponents and exponentials of its piece; the request two slabs ahead
+    template <int m>
+    __device__ __forceinline__ void second() {
+      constexpr int kEvery = 2 / kRows, n = m / kEvery, h = n / 16, i = n % 16;
+      // not looked at before the wait in front of this half: what does is volatile, as that is
+      if constexpr (m == 0)
+        for (int r = 0; r < kRows; ++r) asm volatile("" : "+v"(g.raw[par][r]));
+      if constexpr (m % kEvery == 0 && n < 16 * kRows) {
+        if constexpr (i < 8) g.x[h][i] = fmaf((float)reinterpret_cast<const _Float16*>(&g.raw[par][h])[i], g.c, g.shift[h]);
+        else g.pr[h][i - 8] = __builtin_amdgcn_exp2f(g.x[h][i - 8]);
+        fence();
+      }
+      if constexpr (m >= 60 && m < 60 + kRows) { g.template request<par>(m - 60); fence(); }
+      if constexpr (m == 63) { g.load_at += kUnitBytes; fence(); }
+    }
+    // first half of the next one: its d(logits), and the store
+    template <int m>
+    __device__ __forceinline__ void first() {
+      constexpr int kEvery = 4 / kRows, n = m / kEvery, h = n / 8, e = n % 8;
+      if constexpr (n < 8 * kRows) {
+        if constexpr (m % kEvery == 0) {
+          if constexpr (kEntropy) g.x[h][e] = fmaf(g.x[h][e], g.k2[h], g.k1[h]);
+          else g.x[h][e] = g.rel[h] == e ? g.top[h] : 0.f;
+          fence();
+        }
+        if constexpr (m % kEvery == kEvery / 2) {
+          const float k = kEntropy ? g.x[h][e] : g.k1[h];
+          g.pr[h][e] = fmaf(g.pr[h][e], k, kEntropy ? (g.rel[h] == e ? g.top[h] : 0.f) : g.x[h][e]);
+          fence();
+        }
+      }
+      constexpr int w = m - 34;
+      if constexpr (w >= 0 && w < 8 * kRows && w % 2 == 0) {
+        constexpr int o = w / 2, hh = o / 4, k = o % 4;
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        const bf16x2 two = {(__bf16)g.pr[hh][2 * k], (__bf16)g.pr[hh][2 * k + 1]};
+        g.out[hh][k] = __builtin_bit_cast(uint32_t, two) & g.live[hh];
+        fence();
+      }
+      if constexpr (m >= 60 && m < 60 + kRows) {
+        __builtin_amdgcn_raw_buffer_store_b128(g.out[m - 60], g.rsrc_dz, g.store_at + (m - 60) * 32 * kRowBytes, 0, 0);
+        fence();
+      }
+      if constexpr (m == 63) {
+        g.store_at = g.store_next;
+        g.store_next += kUnitBytes;
+        for (int i = 0; i < kRows; ++i) g.rel[i] -= 64;
+        fence();
+      }
+    }
+  };
+  template <int par> __device__ __forceinline__ Turn<par> turn() { return Turn<par>{*this}; }
+};
+struct NoDz {
+  static constexpr bool kHosts = false;
+  struct Params {};
+};
 
 // C (+)= A B^T with A [M x K] and B [N x K], C row-major in one of two orientations; either way
 // a lane's 16-byte pieces lie along C's rows and a store instruction covers runs of at least 64 bytes:
@@ -477,8 +642,8 @@ __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, typename Ou
 // finishes and is stored).  Otherwise work item = (K range, m tile, n tile), one K loop per workgroup.
 // kAdds: C is added to, and one workgroup owns the whole K range of a tile (an argument in its place had fp32 tiles spill
 // 400 registers).
-template <typename T, typename OutT, Side S, int NI, bool kAdds>
-__global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
+template <typename T, typename OutT, Side S, int NI, bool kAdds, typename G>
+__global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p, typename G::Params guest_of) {
   using Tile = OutTile<T, S, NI>;
   constexpr bool kMC = kMContig<S>;
   constexpr int E = Tile::kSlabK;
@@ -487,6 +652,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
 
   // this workgroup's tiles: (mt, nt) first, then `count - 1` steps along the walked operand; one K range
   int item = work_item(p.xcd_wgs), mt, nt, count = 1, ks = 0, k0 = 0, k_len = p.K;
+  const int whole_item = item;
   if (p.n_walk > 0) {
     const int n_fixed = kMC ? p.n_mt : p.n_nt;       // tiles of the operand that stays
     const int n_moving = kMC ? p.n_nt : p.n_mt;      // tiles of the operand that is walked
@@ -542,13 +708,20 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p) {
     const auto op_b = operand_b(nt, b_rows);
     if constexpr (kAdds) loads.finish(c_tile(mt), acc);
     else Tile::zero(acc);
+    [[maybe_unused]] std::conditional_t<G::kHosts, G, int> guest;
+    if constexpr (G::kHosts) guest.place(guest_of, whole_item);     // one tile per workgroup
     if (k == 0 || !stream || again) core.start(op_a, op_b, nslab, lds);
     if (stream && k + 1 < count)
       core.follow(op_a, op_b, nslab, Tile::cursor_a(kMC ? op_a : operand_a(mt + 1, rows_of(p.M, mt + 1, 256)), nslab),
                   Tile::cursor_b(kMC ? operand_b(nt + 1, rows_of(p.N, nt + 1, Tile::BN)) : op_b, nslab));
     else
       core.follow(op_a, op_b, nslab, Tile::hold_a(op_a, nslab), Tile::hold_b(op_b, nslab));
-    core.run(acc, nslab);
+    if constexpr (G::kHosts) {
+      guest.begin();
+      core.run_with(acc, nslab, guest.pairs, guest);
+    } else {
+      core.run(acc, nslab);
+    }
     if constexpr (Tile::kSplit) {
       again = core.redo(acc, op_a, op_b, nslab, lds, [&] {
         if constexpr (kAdds) {
@@ -817,9 +990,10 @@ struct GemmIn {
   int k_valid;
 };
 
-template <typename T, typename OutT, Side S, int NI = 8>
+template <typename T, typename OutT, Side S, int NI = 8, typename G = NoDz>
 static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64_t ldc, int accumulate, hipStream_t stream,
-                           float* partial, size_t partial_bytes, int k_split_wanted, const RowOrder& rows = RowOrder{nullptr, 0}) {
+                           float* partial, size_t partial_bytes, int k_split_wanted, const RowOrder& rows = RowOrder{nullptr, 0},
+                           const typename G::Params& guest = typename G::Params{}) {
   using Tile = OutTile<T, S, NI>;
   constexpr bool kMC = kMContig<S>;
   GemmParams g;
@@ -842,7 +1016,7 @@ static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64
   // launching one workgroup per tile.
   const int n_fixed = kMC ? g.n_mt : g.n_nt, n_moving = kMC ? g.n_nt : g.n_mt;
   g.n_walk = 0;
-  if (g.k_split == 1 && n_fixed <= cus && g.n_mt * g.n_nt >= 4 * cus && K >= 2 * slab) {
+  if (!G::kHosts && g.k_split == 1 && n_fixed <= cus && g.n_mt * g.n_nt >= 4 * cus && K >= 2 * slab) {
     g.n_walk = cus / n_fixed;
     if (g.n_walk > n_moving) g.n_walk = n_moving;
     // A walk is as long as its longest run; one workgroup per tile takes ceil(tiles / CUs) rounds.  Streaming the K
@@ -866,14 +1040,14 @@ static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64
   auto launch = [&](auto kernel) {
     const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), Tile::kLdsBytes, "gemm_kernel");
     if (rc) return rc;
-    hipLaunchKernelGGL(kernel, dim3(grid.grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g);
+    hipLaunchKernelGGL(kernel, dim3(grid.grid), dim3(Tile::kThreads), Tile::kLdsBytes, stream, g, guest);
     return check_launch("gemm_kernel");
   };
   int rc;
   if constexpr (!kMC && sizeof(OutT) == 4)
-    rc = accumulate && g.k_split == 1 ? launch(&gemm_kernel<T, OutT, S, NI, true>) : launch(&gemm_kernel<T, OutT, S, NI, false>);
+    rc = accumulate && g.k_split == 1 ? launch(&gemm_kernel<T, OutT, S, NI, true, NoDz>) : launch(&gemm_kernel<T, OutT, S, NI, false, NoDz>);
   else
-    rc = launch(&gemm_kernel<T, OutT, S, NI, false>);
+    rc = launch(&gemm_kernel<T, OutT, S, NI, false, G>);
   if (rc || g.k_split == 1) return rc;
   return launch_splitk_reduce<OutT>(partial, g.k_split, kMC ? N : M, kMC ? M : N, static_cast<OutT*>(C), ldc, accumulate,
                                     rows.order, stream);
@@ -925,6 +1099,115 @@ static int launch_transpose(const TransposeParams<T>& p, hipStream_t stream) {
   dim3 grid((p.C + 63) / 64, (int)((p.r_dst + 63) / 64));
   hipLaunchKernelGGL(transpose_block_kernel<T>, grid, dim3(256), 0, stream, p);
   return check_launch("transpose_block_kernel");
+}
+
+// d(logits): the first `whole` units of `row_units` rows of units from row0 on, the others of the first n_edge rows; with `turn` hidden^T.
+template <typename T>
+static int launch_dz(DzFromZParams<T>& q, int row0, int row_units, int whole, int n_edge, bool turn, hipStream_t stream) {
+  q.whole = whole;
+  q.row0 = row0;
+  q.row_units = row_units;
+  q.n_edge = n_edge;
+  // a workgroup walks units of one row of units, so that its coefficients are fetched once; 16 workgroups per CU
+  int64_t per_row = row_units > 0 ? (16 * (int64_t)device_cu_count() + row_units - 1) / row_units : 0;
+  if (per_row > whole) per_row = whole;
+  q.n_step = (int)per_row;
+  q.turn_rows = (int)((q.turn.r_dst + 63) / 64);
+  const int64_t grid = (int64_t)row_units * per_row + n_edge + (turn ? (int64_t)q.turn_rows * ((q.turn.C + 63) / 64) : 0);
+  if (grid == 0) return CLGRPO_OK;
+  if (q.t.g_ent) hipLaunchKernelGGL((dz_from_z_kernel<T, true>), dim3((unsigned)grid), dim3(256), 0, stream, q);
+  else hipLaunchKernelGGL((dz_from_z_kernel<T, false>), dim3((unsigned)grid), dim3(256), 0, stream, q);
+  return check_launch("dz_from_z_kernel");
+}
+
+// Row tiles (of 256) of the launches in which dhidden's workgroups convert the next launch's d(logits): as many as fill one round
+// of the CUs, the first launch what is left over (K ranges fill it).  0: dhidden and the conversion apart.
+struct HostPlan {
+  int first_nt, first_split, per_nt;
+};
+// Taken where it is the cheaper one, in periods of a tile's slab: rounds x slabs of the launches, 6.6 MB of a partial sum's traffic or
+// 7.15 MB of the conversion's (5 TB/s) per period, of what guests convert the 0.35 that it still costs (12288 rows at H = 4096 in
+// three launches: 1.0 ms less to convert in front of them, 0.66 ms gained).  What it loses is a round that whole row tiles do not fill
+// (12836 rows at H = 2560, V = 32000: 510 tiles are two rounds of 256, not of 250), or a first launch without room for K ranges.
+//   dhidden and d(logits), apart -> hosted, ms: H = 4096, V = 151936: 12288 rows 11.23 -> 10.57, 13397 12.45 -> 11.63; H = 2048: 10139
+//   5.35 -> 4.97, 32768 16.9 -> 15.6; H = 7168, V = 129280: 32768 43.3 -> 41.1; H = 2560, V = 32000: 18657 2.74 -> 2.42
+static HostPlan plan_hosts(int64_t rows, int64_t H, int64_t V, int cus, size_t partial_cap) {
+  HostPlan hp{0, 1, 0};
+  const int n_mt = (int)((H + 255) / 256), n_nt = (int)((rows + 255) / 256), per = cus / n_mt;
+  if (per < 1 || n_nt <= per || V > (1 << 22)) return hp;     // a guest's run of units is within 32-bit offsets
+  const int64_t K = round_up64(V, 64);
+  const long slabs = (long)(K / 64);
+  auto launch = [&](long tiles, int split, int64_t launch_rows) {
+    const double partial = split > 1 ? 2.0 * split * (double)launch_rows * H * sizeof(float) / 6.6e6 : 0.0;
+    return (double)((tiles * split + cus - 1) / cus) * (double)((slabs + split - 1) / split) + partial;
+  };
+  const double convert = 4.0 * (double)K / 7.15e6;      // per row
+  const DhPlan dh = plan_dhidden(rows, H, K, 64, cus, partial_cap);
+  double apart = rows * convert;
+  if (dh.bulk_nt > 0) {
+    const int64_t tail = rows - (int64_t)dh.bulk_nt * 256;
+    apart += launch((long)dh.bulk_nt * n_mt, 1, 0) + launch((long)(n_nt - dh.bulk_nt) * n_mt, dh.k_split, tail);
+  } else {
+    apart += dh_tile_time(dh.ni) * launch((long)n_mt * ((rows + 32 * dh.ni - 1) / (32 * dh.ni)), dh.k_split, rows);
+  }
+  const int first = n_nt % per ? n_nt % per : per;
+  const int split = pick_k_split(first * n_mt, (int)H, first * 256, (int)K, 64, partial_cap, cus);
+  const double hosted = launch((long)first * n_mt, split, first * 256) + (double)((n_nt - first) / per) * slabs +
+                        convert * (first * 256 + 0.35 * (rows - first * 256));
+  if (hosted < 0.99 * apart) hp = HostPlan{first, split, per};
+  return hp;
+}
+
+// d(logits) and dhidden of a chunk by plan_hosts, with G for a guest; with `turn` hidden^T as well.
+template <typename T, typename G>
+static int launch_hosted(const HostPlan& hp, DzFromZParams<T>& q, int n_rows, bool turn, const T* weight, int64_t H, T* out,
+                         float* partial, size_t partial_bytes, const RowOrder& rows, hipStream_t stream) {
+  constexpr int E = Elem<T>::kSlabK, kTileUnits = 256 / E, kParts = 2 / G::kRows;
+  const int n_mt = (int)((H + 255) / 256), n_nt = (q.t.Tc + 255) / 256, slabs = q.n_units;
+  const int whole = q.t.V / E;                          // units of a row that guests convert: the last one may end inside the vocabulary
+  auto units_of = [&](int nt) { return nt * kTileUnits < n_rows ? nt * kTileUnits : n_rows; };    // rows of units of the first nt tiles
+  int done = units_of(hp.first_nt);                     // of them are converted
+  int rc = launch_dz(q, 0, done, whole, whole < q.n_units ? n_rows : 0, turn, stream);
+  for (int nt = 0, width = hp.first_nt; rc == CLGRPO_OK && nt < n_nt; nt += width, width = hp.per_nt) {
+    const int split = nt == 0 ? hp.first_split : 1;
+    const int upto = units_of(nt + width + hp.per_nt);
+    // Guests: as many of the next launch's rows as the workgroups have slabs for, all but one pair of theirs (see run_with).  The
+    // last K range, if it is much the shortest, goes without.
+    typename G::Params g{};
+    const int per = (slabs + split - 1) / split, last = slabs - (split - 1) * per;
+    const bool use_last = last * 10 >= per * 9;
+    const int items = width * n_mt * (use_last ? split : split - 1), most = ((use_last ? last : per) - 1) / 2 * 2 - 1;
+    int left = upto - done;
+    if (left > 0 && most > 0 && last >= 3) {
+      const int fit = items / (kParts * ((whole + most - 1) / most)), take = left < fit ? left : fit;
+      if (take > 0) {
+        const int row0 = upto - take;
+        g.runs = items / (kParts * take);
+        g.per_run = (whole + g.runs - 1) / g.runs;
+        g.run_rows = kParts * take;
+        g.n_units = whole;
+        g.t = q.t;
+        g.n0 = row0 * E;
+        g.z_kslab = q.z_kslab;
+        g.dz_kslab = q.dz_kslab;
+        g.z = static_cast<const char*>(q.z) + (int64_t)row0 * q.z_kslab * G::kUnitBytes;
+        g.dz = static_cast<char*>(q.dz) + (int64_t)row0 * q.dz_kslab * G::kUnitBytes;
+        left -= take;
+      }
+    }
+    const int r0 = nt * 256, r1 = (nt + width) * 256 < q.t.Tc ? (nt + width) * 256 : q.t.Tc;
+    const GemmIn in{weight, static_cast<const T*>(q.dz) + (int64_t)r0 / E * q.dz_kslab * (E * E), H, q.dz_kslab, q.t.V};
+    T* c = out + (rows.order ? 0 : (int64_t)r0 * H);
+    float* part = split > 1 ? partial : nullptr;
+    const size_t part_bytes = split > 1 ? partial_bytes : 0;
+    const RowOrder c_rows{rows.order ? rows.order + r0 : nullptr, rows.total};
+    rc = g.run_rows > 0
+             ? launch_gemm_one<T, T, Side::kWeight, 8, G>(in, (int)H, r1 - r0, slabs * E, c, H, 0, stream, part, part_bytes, split, c_rows, g)
+             : launch_gemm_one<T, T, Side::kWeight>(in, (int)H, r1 - r0, slabs * E, c, H, 0, stream, part, part_bytes, split, c_rows);
+    if (rc == CLGRPO_OK && left > 0) rc = launch_dz(q, done, left, whole, 0, false, stream);
+    done = upto;
+  }
+  return rc;
 }
 
 // dW[v][h] (+)= sum_t dz(t, v) hidT(h, t) over k tokens of dz (n_kslab units per row of units) and hidT (ld tokens).
@@ -985,35 +1268,47 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
     // hidT(h, t) = hidden[c0 + t][h], zero for tc <= t < ldt, K-blocked
     const bool want_dw = a->dweight || kept;
     const TransposeParams<T> turn{hidden + t0 * H, hidt, H, ld_dw, ldt, (int)tc, (int)H, order};
+    DzFromZParams<T> q;
+    bool dhidden_done = false;
     if (saved) {
-      DzFromZParams<T> q;
       q.z = z;
       q.dz = dz;
-      q.labels = a->labels + t0;
-      q.label_offset = label_offset;
-      q.lse = a->lse + t0;
-      q.entropy = a->g_entropy ? a->entropy + t0 : nullptr;
-      q.g_lp = a->g_logprob + t0;
-      q.g_ent = a->g_entropy ? a->g_entropy + t0 : nullptr;
-      q.order = order;
+      q.t.labels = a->labels + t0;
+      q.t.label_offset = label_offset;
+      q.t.lse = a->lse + t0;
+      q.t.entropy = a->g_entropy ? a->entropy + t0 : nullptr;
+      q.t.g_lp = a->g_logprob + t0;
+      q.t.g_ent = a->g_entropy ? a->g_entropy + t0 : nullptr;
+      q.t.order = order;
+      q.t.Tc = (int)tc;
+      q.t.V = (int)V;
+      q.t.c = a->inv_temperature * kLog2e;
+      q.t.inv_temperature = a->inv_temperature;
       q.z_kslab = ldz / E;
       q.dz_kslab = dz_kslab;
-      q.Tc = (int)tc;
-      q.V = (int)V;
       q.n_units = (int)(pl.ldv / E);
-      q.c = a->inv_temperature * kLog2e;
-      q.inv_temperature = a->inv_temperature;
-      // a workgroup walks units of one row of units, so that its coefficients are fetched once; 16 workgroups per CU
-      const int64_t n_rows = ldt / E;
-      int64_t per_row = (16 * (int64_t)device_cu_count() + n_rows - 1) / n_rows;
-      if (per_row > q.n_units) per_row = q.n_units;
-      q.n_step = (int)per_row;
       q.turn = turn;
-      dim3 grid((unsigned)n_rows, (unsigned)(per_row + (want_dw ? (H + 63) / 64 : 0)));
-      if (q.g_ent) hipLaunchKernelGGL((dz_from_z_kernel<T, true>), grid, dim3(256), 0, stream, q);
-      else hipLaunchKernelGGL((dz_from_z_kernel<T, false>), grid, dim3(256), 0, stream, q);
-      rc = check_launch("dz_from_z_kernel");
-      if (rc) return rc;
+      if constexpr (sizeof(T) == 2) {
+        if (a->dhidden && !wt) {
+          // a launch's d(logits) while the one before it is contracted
+          const HostPlan hp = plan_hosts(tc, H, V, device_cu_count(), pl.part_bytes);
+          if (hp.first_nt > 0) {
+            auto hosted = [&](auto guest) {
+              return launch_hosted<T, decltype(guest)>(hp, q, (int)(ldt / E), want_dw, weight, H, static_cast<T*>(a->dhidden) + t0 * H,
+                                                       reinterpret_cast<float*>(ws + pl.off_part), pl.part_bytes,
+                                                       RowOrder{order, rows.total}, stream);
+            };
+            // a guest's two pieces per slab, where one would take more slabs than there are (the rows of a launch have 2048 / H of them)
+            rc = q.t.g_ent ? hosted(DzGuest<true, 1>{}) : H < 3072 ? hosted(DzGuest<false, 2>{}) : hosted(DzGuest<false, 1>{});
+            if (rc) return rc;
+            dhidden_done = true;
+          }
+        }
+      }
+      if (!dhidden_done) {
+        rc = launch_dz(q, 0, (int)(ldt / E), q.n_units, 0, want_dw, stream);
+        if (rc) return rc;
+      }
     } else {
       DzParams d;
       d.hidden = hidden + c0 * H;
@@ -1040,7 +1335,7 @@ static int run_bwd(const clgrpo_lmhead_bwd_args* a, hipStream_t stream, int64_t 
       if (rc == 0 && want_dw) rc = launch_transpose(turn, stream);
       if (rc) return rc;
     }
-    if (a->dhidden) {
+    if (a->dhidden && !dhidden_done) {
       // dhidden[chunk][h] = sum_v W[v][h] dz[t][v]   (M = H, N = tokens, C[n][m])
       void* out = static_cast<T*>(a->dhidden) + t0 * H;
       float* part = reinterpret_cast<float*>(ws + pl.off_part);
@@ -1088,6 +1383,15 @@ extern "C" int clgrpo_lmhead_bwd_dhidden_tile_plan(int64_t rows, int64_t H, int6
   out[1] = pl.k_split;
   out[2] = 32 * pl.ni;
   out[3] = (int32_t)(1000.0 * dh_tile_time(pl.ni) + 0.5);
+  return CLGRPO_OK;
+}
+
+extern "C" int clgrpo_lmhead_bwd_guest_plan(int64_t rows, int64_t H, int64_t V, int32_t cus, int64_t partial_bytes, int32_t* out) {
+  if (rows <= 0 || H <= 0 || V <= 0 || out == nullptr) return CLGRPO_EINVAL;
+  const HostPlan hp = plan_hosts(rows, H, V, cus > 0 ? cus : 256, partial_bytes < 0 ? (size_t)1 << 30 : (size_t)partial_bytes);
+  out[0] = hp.first_nt;
+  out[1] = hp.first_split;
+  out[2] = hp.per_nt;
   return CLGRPO_OK;
 }
 

@@ -200,6 +200,14 @@ def dhidden_tile_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple[i
     return int(out[0]), int(out[1]), int(out[2]), out[3] / 1000.0
 
 
+def dhidden_guest_plan(rows: int, H: int, V: int, cus: int = 0, partial_bytes: int = -1) -> Tuple[int, int, int]:
+    """(256-token tiles of the first launch or 0, its K ranges, tiles of each launch behind it) where dhidden's launches over 16-bit
+    kept logits also turn the next launch's logits into d(logits)."""
+    out = (C.c_int32 * 3)()
+    _lib.check(_lib.lib().clgrpo_lmhead_bwd_guest_plan(int(rows), int(H), int(V), int(cus), int(partial_bytes), C.cast(out, C.c_void_p)))
+    return int(out[0]), int(out[1]), int(out[2])
+
+
 def dweight_launch_plan(rows: int, H: int, V: int, dtype, cus: int = 0) -> Tuple[int, int, int]:
     """(walks or 0, vocabulary tiles of a first launch of equally long walks or 0, K ranges of the launch over the
     remaining vocabulary tiles) for the dW contraction over a chunk of ``rows`` tokens."""

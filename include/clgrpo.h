@@ -61,8 +61,9 @@ typedef enum { CLGRPO_BF16 = 0, CLGRPO_F32 = 1, CLGRPO_F64 = 2, CLGRPO_U8 = 3 /*
  *   3.02 -> 4.00: the number that 3.02 should have had: a caller built against 3.01 that reads kept logits by that header's
  *                 formula gets entries in another order.  clgrpo_lmhead_bwd_workspace_bytes (and clgrpo_head_step_workspace_bytes)
  *                 hold no room for a W^T any more: W is read as it is.  clgrpo_lmhead_bwd_dhidden_tile_plan and
- *                 clgrpo_lmhead_fwd_tile_plan added, and 8 among the stages of clgrpo_head_step. */
-#define CLGRPO_VERSION 400
+ *                 clgrpo_lmhead_fwd_tile_plan added, and 8 among the stages of clgrpo_head_step.
+ *   4.00 -> 4.01: clgrpo_lmhead_bwd_guest_plan added. */
+#define CLGRPO_VERSION 401
 int clgrpo_version(void);
 const char* clgrpo_last_error_string(void);
 
@@ -176,6 +177,11 @@ int clgrpo_lmhead_bwd_dhidden_plan(int64_t rows, int64_t H, int64_t V, int32_t d
  * tiles (< 0: as much as clgrpo_lmhead_bwd_workspace_bytes asks for). */
 int clgrpo_lmhead_bwd_dhidden_tile_plan(int64_t rows, int64_t H, int64_t V, int32_t dtype, int32_t cus, int64_t partial_bytes,
                                         int32_t* out);
+/* From kept logits of 16-bit inputs, without a weight_t, more rows than one round of the device's units takes may be contracted in
+ * several launches, in which the workgroups of one also turn the next one's kept logits into d(logits), beside the matrix instructions:
+ * out[0] = 256-token tiles of the first launch (0: not done so, and the two plans above hold), out[1] = its K ranges, out[2] =
+ * 256-token tiles of each launch behind it.  partial_bytes as above. */
+int clgrpo_lmhead_bwd_guest_plan(int64_t rows, int64_t H, int64_t V, int32_t cus, int64_t partial_bytes, int32_t* out);
 /* How the dW contraction over a chunk of `rows` tokens is launched: out[0] = walks (workgroups that keep one
  * 256-column tile of hidden^T and walk runs of vocabulary tiles; 0: one workgroup per tile), out[1] = vocabulary
  * tiles of a first launch whose walks are all equally long (0: one launch over all of them), out[2] = K ranges of
