@@ -6,8 +6,8 @@
 // V*sizeof(dtype) bytes per row read (+ the same written).  A row may start anywhere: what lies before its first
 // and behind its last 16-byte boundary goes element by element, the rest in 16-byte pieces (519 rows of 32003 fp32,
 // three quarters of them misaligned: 48 -> 16 us, gradients 73 -> 28 us; as bf16 47 -> 13 and 46 -> 17.5 us).
-// 2048 rows of the 152k vocabulary, bf16: statistics 116 us = 5.4 TB/s, gradients 239 us = 5.2 TB/s, where a copy of
-// 1 GB reaches 5.0 TB/s on this card.
+// 2048 rows of the 152k vocabulary, bf16: statistics 111 us = 5.6 TB/s, gradients 190 us = 6.5 TB/s (a part of it the last-level
+// cache's, see kKeptBytes), where a copy of 1 GB reaches 5.0 TB/s on this card.
 #include "common.hpp"
 
 namespace clgrpo {
@@ -92,7 +92,30 @@ struct RowSpan {
   }
 };
 
-template <typename T, int BLOCK>
+// What passes over logits leave in the last-level cache (256 MB), which allocates on loads and stores alike: with more logits than
+// fit, each line that a pass brings in pushes one out that was written before and has to go to memory first.  Such passes
+// go around the cache (kOnce) where nobody will find in it what they bring: the statistics for all rows but the last kKeptBytes; the
+// gradients, which take the rows from the last one on, for their loads and for the stores in front of which another
+// kKeptGradients follow.  Fewer logits are better off in the cache altogether.
+//   logits just written -> statistics -> gradients -> a pass that reads the gradients, us:  2048 rows of the 152k vocabulary, bf16
+//   566 -> 502, 800 235 -> 210, 600 175 -> 167, 4096 of 129280 913 -> 873, 1024 of 50257 fp32 184 -> 168; statistics alone 146 -> 111
+//   for 2048 rows.  With all of it around the cache 300 rows of 152k (91 MB) 100 -> 107, 519 of 32003 fp32 76 -> 86; with all
+//   gradients stored around it 514 and 179 for the 502 and 168.
+constexpr int64_t kKeptBytes = 160 << 20, kKeptGradients = 128 << 20;
+
+// Copies of a loop and not a condition inside it: the compiler makes one access of the two sides, without the hint.
+template <bool kOnce>
+__device__ __forceinline__ u32x4_t load16(const u32x4_t* p) {
+  if constexpr (kOnce) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool kOnce>
+__device__ __forceinline__ void store16(u32x4_t v, u32x4_t* p) {
+  if constexpr (kOnce) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
+template <typename T, int BLOCK, bool kOnce>
 __device__ RowStats row_stats(const T* row, int64_t V) {
   constexpr int N = Vec16<T>::N;
   RowStats st{-INFINITY, 0.f, 0.f};
@@ -112,10 +135,10 @@ __device__ RowStats row_stats(const T* row, int64_t V) {
   if (i + 3 * BLOCK < span.pieces) {
     u32x4_t cur[4], nxt[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) cur[k] = rv[i + k * BLOCK];
+    for (int k = 0; k < 4; ++k) cur[k] = load16<kOnce>(rv + i + k * BLOCK);
     for (i += 4 * BLOCK; i + 3 * BLOCK < span.pieces; i += 4 * BLOCK) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) nxt[k] = rv[i + k * BLOCK];
+      for (int k = 0; k < 4; ++k) nxt[k] = load16<kOnce>(rv + i + k * BLOCK);
       __builtin_amdgcn_sched_barrier(0);
       four(cur);
 #pragma unroll
@@ -153,7 +176,8 @@ template <typename T, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void softmax_stats_kernel(clgrpo_softmax_stats_args a) {
   const int64_t r = blockIdx.x;
   const T* row = static_cast<const T*>(a.logits) + r * a.ld;
-  const RowStats st = row_stats<T, BLOCK>(row, a.V);
+  const bool once = (a.R - r) * a.ld * (int64_t)sizeof(T) > kKeptBytes;
+  const RowStats st = once ? row_stats<T, BLOCK, true>(row, a.V) : row_stats<T, BLOCK, false>(row, a.V);
   if (threadIdx.x == 0) {
     const float lse = st.m + logf(st.s);
     if (a.lse) a.lse[r] = lse;
@@ -167,21 +191,11 @@ __global__ __launch_bounds__(BLOCK) void softmax_stats_kernel(clgrpo_softmax_sta
 
 // d(logits) of one row: with the row's lse (and entropy, when it carries a gradient) from the forward the
 // row is read once and written once; without them the statistics are rebuilt by one more pass over it.
-template <typename T, int BLOCK>
-__global__ __launch_bounds__(BLOCK) void softmax_stats_bwd_kernel(clgrpo_softmax_stats_bwd_args a) {
+template <typename T, int BLOCK, bool kOnce>
+__device__ __forceinline__ void row_gradients(const clgrpo_softmax_stats_bwd_args& a, int64_t r, float lse, float ent) {
   constexpr int N = Vec16<T>::N;
-  const int64_t r = blockIdx.x;
   const T* row = static_cast<const T*>(a.logits) + r * a.ld;
   T* out = static_cast<T*>(a.dlogits) + r * a.V;
-  float lse, ent;
-  if (a.lse != nullptr && (a.g_entropy == nullptr || a.entropy != nullptr)) {
-    lse = a.lse[r];
-    ent = a.g_entropy ? a.entropy[r] : 0.f;
-  } else {
-    const RowStats st = row_stats<T, BLOCK>(row, a.V);
-    lse = st.m + logf(st.s);
-    ent = lse - st.u / st.s;
-  }
   const float glp = a.g_logprob ? a.g_logprob[r] : 0.f;
   const float gen = a.g_entropy ? a.g_entropy[r] : 0.f;
   const int64_t y = a.g_logprob ? a.labels[r] : -1;
@@ -201,11 +215,12 @@ __global__ __launch_bounds__(BLOCK) void softmax_stats_bwd_kernel(clgrpo_softmax
       Vec16<T>::unpack(raw, z);
 #pragma unroll
       for (int k = 0; k < N; ++k) d[k] = dz(z[k], span.head + i * N + k);
-      ov[i] = Vec16<T>::pack(d);
+      store16<kOnce>(Vec16<T>::pack(d), ov + i);
     };
     int64_t i = threadIdx.x;
     for (; i + 3 * BLOCK < span.pieces; i += 4 * BLOCK) {
-      const u32x4_t r0 = rv[i], r1 = rv[i + BLOCK], r2 = rv[i + 2 * BLOCK], r3 = rv[i + 3 * BLOCK];
+      const u32x4_t r0 = load16<kOnce>(rv + i), r1 = load16<kOnce>(rv + i + BLOCK), r2 = load16<kOnce>(rv + i + 2 * BLOCK),
+                    r3 = load16<kOnce>(rv + i + 3 * BLOCK);
       one(r0, i); one(r1, i + BLOCK); one(r2, i + 2 * BLOCK); one(r3, i + 3 * BLOCK);
     }
     for (; i < span.pieces; i += BLOCK) one(rv[i], i);
@@ -215,6 +230,22 @@ __global__ __launch_bounds__(BLOCK) void softmax_stats_bwd_kernel(clgrpo_softmax
     // rows a stride apart that shifts them against the packed result
     for (int64_t v = threadIdx.x; v < a.V; v += BLOCK) out[v] = (T)dz(to_f32<T>(row[v]), v);
   }
+}
+template <typename T, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void softmax_stats_bwd_kernel(clgrpo_softmax_stats_bwd_args a) {
+  const bool once = a.R * a.ld * (int64_t)sizeof(T) > kKeptBytes;
+  const int64_t r = once ? (int64_t)gridDim.x - 1 - blockIdx.x : blockIdx.x;     // the cache has the last rows
+  float lse, ent;
+  if (a.lse != nullptr && (a.g_entropy == nullptr || a.entropy != nullptr)) {
+    lse = a.lse[r];
+    ent = a.g_entropy ? a.entropy[r] : 0.f;
+  } else {
+    const RowStats st = row_stats<T, BLOCK, false>(static_cast<const T*>(a.logits) + r * a.ld, a.V);
+    lse = st.m + logf(st.s);
+    ent = lse - st.u / st.s;
+  }
+  if (once && r * a.V * (int64_t)sizeof(T) > kKeptGradients) row_gradients<T, BLOCK, true>(a, r, lse, ent);
+  else row_gradients<T, BLOCK, false>(a, r, lse, ent);
 }
 
 // Threads per row.  Measured with 256 / 512 / 1024 (us): statistics of 48 bf16 rows of the 152k vocabulary 15.6 / 13.9 /
