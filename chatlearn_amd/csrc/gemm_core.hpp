@@ -94,10 +94,13 @@ template <> struct KeptLogit<float> { typedef float type; };
 // acc_get / acc_set for the same reason.
 template <typename T> struct Mma;
 template <> struct Mma<__bf16> {
-  template <bool kAcross, int NI>
+  template <bool kAcross, bool kFresh, int NI>
   __device__ static __forceinline__ void slot(f32x4 (&acc)[8][NI], const u32x4 (&a)[8], const u32x4 (&b)[NI], int m) {
     const int i = m / NI, j = (i & 1) ? NI - 1 - m % NI : m % NI;
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(a[i]), "v"(b[j]));
+    // kFresh: the product alone.  The accumulator stays an operand that is read, for the compiler: as a plain result it is given other
+    // registers, and hundreds are spilled.
+    if constexpr (kFresh) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "+a"(acc[i][j]) : "v"(a[i]), "v"(b[j]));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(a[i]), "v"(b[j]));
   }
 };
 template <> struct Mma<float> {
@@ -105,8 +108,9 @@ template <> struct Mma<float> {
   // step m % 8 / 2 of four blocks of row i, so that an accumulator comes up again eight instructions later.
   // kAcross: a[4 q + e] holds k = 4g + e of the four blocks 4 q .. 4 q + 3 (an A with K along its rows): the
   // transposition of a 4 x 4 square of single registers is a choice of registers.
-  template <bool kAcross, int NI>
+  template <bool kAcross, bool kFresh, int NI>
   __device__ static __forceinline__ void slot(f32x4 (&acc)[8][NI], const u32x4 (&a)[8], const u32x4 (&b)[NI], int m) {
+    static_assert(!kFresh, "sixteen bits only");
     static_assert(NI == 8, "four blocks of a row per slot");
     const int i = m / 8, e = m % 8 / 2;
 #pragma unroll
@@ -523,12 +527,12 @@ struct GemmTile {
     template <int m> __device__ __forceinline__ void first() {}
     template <int m> __device__ __forceinline__ void second() {}
   };
-  template <typename Guest>
+  template <bool kFresh = false, typename Guest>
   __device__ __forceinline__ void slab(Acc& acc, Guest& guest) {
 #ifdef __HIP_DEVICE_COMPILE__      // the host's pass drops kernels whose body holds this many lambdas, without a word
     each<kSlots>([&](auto c) __attribute__((always_inline)) {            // first half of the slab
       constexpr int m = decltype(c)::value, n = step_at(0, m);
-      Mma<T>::template slot<kAcross, NI>(acc, af[0], bf[0], m);
+      Mma<T>::template slot<kAcross, kFresh, NI>(acc, af[0], bf[0], m);
       fence();
       if constexpr (m % 2 == 0 && m < 2 * (MI + NI)) { read(1, half_a() + sa, (b0 ^ 64) + sb, m / 2); fence(); }
       if constexpr (load_a_at(m) >= 0) { load_a(load_a_at(m)); fence(); }
@@ -550,7 +554,7 @@ struct GemmTile {
     fence();
     each<kSlots>([&](auto c) __attribute__((always_inline)) {            // second half, while the next slab's first fragments come in
       constexpr int m = decltype(c)::value, n = step_at(1, m);
-      Mma<T>::template slot<kAcross, NI>(acc, af[1], bf[1], m);
+      Mma<T>::template slot<kAcross, false, NI>(acc, af[1], bf[1], m);
       fence();
       if constexpr (m % 2 == 0 && m < 2 * (MI + NI)) { read(0, a0 + sa1, b0 + (sb ^ kSlotBytes), m / 2); fence(); }
       if constexpr (load_b_at(m) >= 0) { load_b(load_b_at(m), sb); fence(); }
@@ -577,7 +581,17 @@ struct GemmTile {
     for (int s = 0; s < nslab; ++s) slab(acc, none);
     settle();
   }
-  // The same with a guest in the first 2 `pairs` slabs; at least one pair and one slab more.  (A loop that may not run at all, between
+  // The same over accumulators that hold anything.  Clearing them takes 256 instructions per tile that no matrix instruction covers
+  // (forward, V = 151936: 16384 tokens of 2048 7.32 -> 7.28 ms, of 4096 without kept logits 13.11 -> 13.03, 588 tokens 602 -> 598 us; 8192
+  // of 1024, V = 102400 1.424 -> 1.408 ms; with H = 7168, and up to a few tiles per workgroup, no difference).
+  __device__ __forceinline__ void run_fresh(Acc& acc, int nslab) {
+    settle();
+    NoGuest none;
+    slab<true>(acc, none);
+    for (int s = 1; s < nslab; ++s) slab(acc, none);
+    settle();
+  }
+  // The same as run() with a guest in the first 2 `pairs` slabs; at least one pair and one slab more.  (A loop that may not run at all, between
   // the accumulators' clearing and another one, had them moved and 200 registers spilled.)
   template <typename Guest>
   __device__ __forceinline__ void run_with(Acc& acc, int nslab, int pairs, Guest& guest) {

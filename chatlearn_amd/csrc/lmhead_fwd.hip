@@ -123,12 +123,13 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
   const int vt_begin = vs * p.tiles_per_split;
   const int vt_end = (vt_begin + p.tiles_per_split) < p.n_vt ? (vt_begin + p.tiles_per_split) : p.n_vt;
   bool again = false;      // the tile before was computed twice: nothing of this one has been requested
+  typename Tile::Acc acc;
+  Tile::zero(acc);
   for (int vt = vt_begin; vt < vt_end; ++vt) {
     const int v0 = vt * kFwdBM;
     const int a_rows = (p.V - v0) < kFwdBM ? (p.V - v0) : kFwdBM;
     const auto op_a = Tile::Operand::row_major(weight + (int64_t)v0 * p.H, p.H, a_rows);
-    typename Tile::Acc acc;
-    Tile::zero(acc);
+    if constexpr (Tile::kSplit) Tile::zero(acc);
     if (vt == vt_begin || !stream || again) core.start(op_a, op_b, nslab, lds, order, b_rows);
     if (stream && vt + 1 < vt_end) {
       const int v1 = v0 + kFwdBM;
@@ -138,7 +139,8 @@ __global__ __launch_bounds__(kHeadThreads, 1) void lmhead_fwd_kernel(FwdParams p
     } else {
       core.follow(op_a, op_b, nslab, Tile::hold_a(op_a, nslab), Tile::hold_b(op_b, nslab));
     }
-    core.run(acc, nslab);
+    if constexpr (Tile::kSplit) core.run(acc, nslab);
+    else core.run_fresh(acc, nslab);
     if constexpr (Tile::kSplit) again = core.redo(acc, op_a, op_b, nslab, lds, [&] { Tile::zero(acc); }, order, b_rows);
     if (!stream) Tile::finish();
 
