@@ -74,74 +74,92 @@ class PolicyStep:
         (policy_trainer.py:80-172).  The all-reduce of the response-token count is the identity here."""
         response_token_length_total = ops.upload(
             torch.tensor(sum(data["response_token_length"] for data in data_list)), self.device) / 1
+        return response_token_length_total, [self._process(mb, training) for mb in self._split(data_list, training)]
+
+    def _split(self, data_list, training: bool):
         if self.packing:
-            microbatch_list = split_microbatch(data_list=data_list, max_train_token=self.max_token_in_seq,
-                                               packing=self.packing)
+            return split_microbatch(data_list=data_list, max_train_token=self.max_token_in_seq, packing=self.packing)
+        size = self.train_micro_batch_size if training else self.generate_micro_batch_size
+        return split_microbatch(data_list=data_list, micro_batch_size=size, packing=self.packing)
+
+    def _process(self, micro_batch, training: bool, shifted_host: Optional[torch.Tensor] = None):
+        data_b = batching(micro_batch)
+        tokens_ = data_b["all_tokens"].long()
+        ori_batch_size, ori_seq_len = tokens_.size()
+        plen, rlen = ([int(x) for x in data_b[key]] for key in ("prompt_token_length", "response_token_length"))
+        text = 'position_ids' not in data_b and self.model_type != "vlm"
+        if text:
+            # the masks stay on the device: nothing the host needs of them cannot be had from the lengths
+            tokens_ = self._put(tokens_)
+        # vision-language samples carry their prompt's three position channels and the image tensors
+        attn_mask, loss_mask, position_ids = generate_loss_mask_position_ids(
+            tokens_, plen, rlen, data_b.get("position_ids", None))
+        if 'loss_mask' in data_b:
+            loss_mask = data_b['loss_mask']
+        indices = cu_seqlens = None
+        if self.packing and text:
+            # unpad_input of tokens and position ids plus the label roll (policy_trainer.py:143-162) in
+            # one device pass driven by the length lists; no device value is read back
+            packed = ops.thd_pack(tokens_, plen, rlen, align=1, pad_token=0, want_loss_mask=False,
+                                  want_position_ids=True, verify_on_device=False)
+            tokens = packed["tokens"].unsqueeze(0)
+            position_ids = packed["position_ids"].unsqueeze(0)
+            labels = packed["labels"].unsqueeze(0)
+            indices, cu_seqlens = packed["indices"], packed["cu_seqlens_padded"]
+            width = packed["max_seqlen_padded"]
+            if width != ori_seq_len:      # the batch is padded wider than its longest sample
+                indices = (indices // width) * ori_seq_len + indices % width
         else:
-            size = self.train_micro_batch_size if training else self.generate_micro_batch_size
-            microbatch_list = split_microbatch(data_list=data_list, micro_batch_size=size, packing=self.packing)
-        data_after_process = []
-        for data_b in (batching(mb) for mb in microbatch_list):
-            tokens_ = data_b["all_tokens"].long()
-            ori_batch_size, ori_seq_len = tokens_.size()
-            plen, rlen = ([int(x) for x in data_b[key]] for key in ("prompt_token_length", "response_token_length"))
-            text = 'position_ids' not in data_b and self.model_type != "vlm"
-            if text:
-                # the masks stay on the device: nothing the host needs of them cannot be had from the lengths
-                tokens_ = self._put(tokens_)
-            # vision-language samples carry their prompt's three position channels and the image tensors
-            attn_mask, loss_mask, position_ids = generate_loss_mask_position_ids(
-                tokens_, plen, rlen, data_b.get("position_ids", None))
-            if 'loss_mask' in data_b:
-                loss_mask = data_b['loss_mask']
-            indices = cu_seqlens = None
-            if self.packing and text:
-                # unpad_input of tokens and position ids plus the label roll (policy_trainer.py:143-162) in
-                # one device pass driven by the length lists; no device value is read back
-                packed = ops.thd_pack(tokens_, plen, rlen, align=1, pad_token=0, want_loss_mask=False,
-                                      want_position_ids=True, verify_on_device=False)
-                tokens = packed["tokens"].unsqueeze(0)
-                position_ids = packed["position_ids"].unsqueeze(0)
-                labels = packed["labels"].unsqueeze(0)
-                indices, cu_seqlens = packed["indices"], packed["cu_seqlens_padded"]
-                width = packed["max_seqlen_padded"]
-                if width != ori_seq_len:      # the batch is padded wider than its longest sample
-                    indices = (indices // width) * ori_seq_len + indices % width
-            else:
-                if self.packing:
-                    tokens_, indices, cu_seqlens, _ = unpad_input(tokens_.unsqueeze(-1).to(self.device),
-                                                                  attn_mask.to(self.device))
-                    tokens_ = tokens_.permute(1, 0)
-                    position_ids, *_ = unpad_input(position_ids.unsqueeze(-1).to(self.device),
-                                                   attn_mask.to(self.device))
-                    if self.model_type == "vlm":
-                        position_ids = position_ids.permute(0, 2, 1)        # [3, 1, T] (policy_trainer.py:121-123)
-                        if self.prepend_text_position_channel:
-                            position_ids = torch.cat([position_ids[0:1], position_ids], dim=0)
-                    else:
-                        position_ids = position_ids.permute(1, 0)
-                tokens = tokens_
-                # labels roll along the (packed or padded) token row (policy_trainer.py:135,160)
-                labels, _ = ops.shift_labels(self._put(tokens).contiguous(), None, zero_last=False)
-            # the training mask rolls along the padded rows and loses its last column (policy_trainer.py:161-162)
-            shifted = shifted_host = None
-            if training:
-                _, shifted = ops.shift_labels(None, self._put(loss_mask).to(torch.int32).contiguous(), zero_last=True)
+            if self.packing:
+                tokens_, indices, cu_seqlens, _ = unpad_input(tokens_.unsqueeze(-1).to(self.device),
+                                                              attn_mask.to(self.device))
+                tokens_ = tokens_.permute(1, 0)
+                position_ids, *_ = unpad_input(position_ids.unsqueeze(-1).to(self.device),
+                                               attn_mask.to(self.device))
+                if self.model_type == "vlm":
+                    position_ids = position_ids.permute(0, 2, 1)        # [3, 1, T] (policy_trainer.py:121-123)
+                    if self.prepend_text_position_channel:
+                        position_ids = torch.cat([position_ids[0:1], position_ids], dim=0)
+                else:
+                    position_ids = position_ids.permute(1, 0)
+            tokens = tokens_
+            # labels roll along the (packed or padded) token row (policy_trainer.py:135,160)
+            labels, _ = ops.shift_labels(self._put(tokens).contiguous(), None, zero_last=False)
+        # the training mask rolls along the padded rows and loses its last column (policy_trainer.py:161-162)
+        shifted = None
+        if training:
+            _, shifted = ops.shift_labels(None, self._put(loss_mask).to(torch.int32).contiguous(), zero_last=True)
+            if shifted_host is None:
                 shifted_host = self._shifted_mask_host(data_b.get('loss_mask', None), plen, rlen, ori_seq_len)
-            data_obj = {"all_tokens": tokens, "position_ids": position_ids, "labels": labels,
-                        "ori_seq_len": ori_seq_len, "indices": indices, "cu_seqlens": cu_seqlens,
-                        "ori_batch_size": ori_batch_size, "sample_ids": data_b["id_in_list"],
-                        "attention_mask": attn_mask, "pad_size": 0,
-                        "sample_lengths": [min(p + r, ori_seq_len) for p, r in zip(plen, rlen)]}   # as many as attn_mask marks
-            if self.model_type == "vlm":
-                data_obj.update({"pixel_values": data_b.get("pixel_values", None),
-                                 "image_grid_thw": data_b.get("image_grid_thw", None)})
-            if training:
-                data_obj.update({"loss_mask": shifted, "loss_mask_host": shifted_host,
-                                 "old_logprobs": data_b["old_logprobs"],
-                                 "ref_logprobs": data_b["ref_logprobs"], "advantages": data_b["advantages"]})
-            data_after_process.append(data_obj)
-        return response_token_length_total, data_after_process
+        data_obj = {"all_tokens": tokens, "position_ids": position_ids, "labels": labels,
+                    "ori_seq_len": ori_seq_len, "indices": indices, "cu_seqlens": cu_seqlens,
+                    "ori_batch_size": ori_batch_size, "sample_ids": data_b["id_in_list"],
+                    "attention_mask": attn_mask, "pad_size": 0,
+                    "sample_lengths": [min(p + r, ori_seq_len) for p, r in zip(plen, rlen)]}   # as many as attn_mask marks
+        if self.model_type == "vlm":
+            data_obj.update({"pixel_values": data_b.get("pixel_values", None),
+                             "image_grid_thw": data_b.get("image_grid_thw", None)})
+        if training:
+            data_obj.update({"loss_mask": shifted, "loss_mask_host": shifted_host,
+                             "old_logprobs": data_b["old_logprobs"],
+                             "ref_logprobs": data_b["ref_logprobs"], "advantages": data_b["advantages"]})
+        return data_obj
+
+    def _masks_ahead(self, micro_batches):
+        """The shifted host masks of micro-batches that may be processed one by one while the device works on the ones before:
+        what their processing would refuse has to be refused before any gradient is made, so only text samples
+        without a mask of their own whose lengths are in order.  None for others."""
+        masks = []
+        for mb in micro_batches:
+            plen, rlen = ([int(d[key]) for d in mb] for key in ("prompt_token_length", "response_token_length"))
+            width = max((d["all_tokens"].shape[0] for d in mb), default=0)
+            if self.model_type == "vlm" or not mb or any("loss_mask" in d or "position_ids" in d or d["all_tokens"].dim() != 1 for d in mb) \
+                    or any(p < 0 or r < 0 or p + r > width for p, r in zip(plen, rlen)) \
+                    or any(set(d) != set(mb[0]) or any(d[k].shape != d["all_tokens"].shape for k in ("old_logprobs", "ref_logprobs"))
+                           for d in mb):
+                return None
+            masks.append(self._shifted_mask_host(None, plen, rlen, width))
+        return masks
 
     def _shifted_mask_host(self, given, plen, rlen, width):
         """The shifted training mask on the host, flattened the way the kernels see the tokens: it tells the head
@@ -199,12 +217,24 @@ class PolicyStep:
         args = self.module_args
         # the same fp32 value that preprocess_data_list leaves on the device
         n_tok_f = float(np.float32(float(sum(data["response_token_length"] for data in data_list))))
-        _, data_list = self.preprocess_data_list(data_list=data_list, training=True)
+        # A micro-batch is processed when its turn comes, behind the one before it, whose backward still runs (48 samples packed into
+        # four rows of H = 2048: 56.7 -> 55.6 ms a step; four padded ones of 4096 11.90 -> 11.56).
+        if type(self).preprocess_data_list is PolicyStep.preprocess_data_list:
+            micro_batches = self._split(data_list, True)
+            masks = self._masks_ahead(micro_batches)
+            if masks is not None:
+                data_list = (self._process(mb, True, m) for mb, m in zip(micro_batches, masks))
+            else:
+                data_list = [self._process(mb, True) for mb in micro_batches]
+        else:
+            masks, (_, data_list) = None, self.preprocess_data_list(data_list=data_list, training=True)
+        if masks is None:
+            masks = [inputs["loss_mask_host"] for inputs in data_list]
         sums = torch.zeros(8, dtype=torch.float64, device=self.device)
         dw = self.dweight_buffer
         accumulate = dw is not None
         need_dw = dw is not None or self.weight.requires_grad
-        dw_sum = self._dweight_sum(data_list) if need_dw and data_list else None
+        dw_sum = self._dweight_sum([{"loss_mask_host": m} for m in masks]) if need_dw and masks else None
         ws_cache = {}   # kept logits and head scratch memory, shared by the micro-batches of this step
         for inputs in data_list:
             inputs = self._to_device(inputs)
