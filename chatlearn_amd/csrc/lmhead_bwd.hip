@@ -527,24 +527,36 @@ struct TileAddr {
   __device__ __forceinline__ int row_voff(int dm, int g) const { return dm < row_lim ? voff[g] : 0x7f000000; }
 };
 
+// What a contraction does with the previous contents of C.  kAddsAround: the same as kAdds, loads and stores around the last-level
+// cache (256 MB; the accesses' non-temporal bit), which otherwise gives up hidden^T and d(logits), read again by the workgroups of
+// every column of tiles, for lines of dW that nobody reads before they are gone.  From 112 MB of dW on:
+//   dW added to, us: 300 tokens at H = 4096, V = 151936 976 -> 925, 1024 1476 -> 1428, 3573 3656 -> 3586; 1200 at 1536, V = 65536 300 -> 274;
+//   2000 at 2048, V = 32000 265 -> 252; 6000 at 5120, V = 102400 4478 -> 4436; below it 600 at 512, V = 50257 (103 MB) 65.2 -> 67.8,
+//   500 at 1024, V = 32000 (131 MB) 70.5 -> 71.5 where dW was in the cache, 78 -> 69 where it was not.
+// A dW that is only written is as fast either way.
+enum Adds : int { kOverwrites, kAdds, kAddsAround };
+constexpr int64_t kAddsAroundBytes = 112 << 20;
+constexpr int kNonTemporal = 2;                  // of the buffer accesses' cache policy
+
 // N consecutive elements of a row: 4 or 8 floats, or 4 or 8 (T = bf16) 16-bit values.
-template <int N>
+template <int kPolicy, int N>
 __device__ __forceinline__ void row_store(const float (&x)[N], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, float*) {
 #pragma unroll
   for (int k = 0; k < N; k += 4) {
     const f32x4 v = {x[k], x[k + 1], x[k + 2], x[k + 3]};
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, voff + k * 4, soff, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, voff + k * 4, soff, kPolicy);
   }
 }
+template <int kPolicy>
 __device__ __forceinline__ void row_store(const float (&x)[8], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, __bf16*) {
-  __builtin_amdgcn_raw_buffer_store_b128(pack_vec(x, (__bf16*)nullptr), rsrc, voff, soff, 0);
+  __builtin_amdgcn_raw_buffer_store_b128(pack_vec(x, (__bf16*)nullptr), rsrc, voff, soff, kPolicy);
 }
-
+template <int kPolicy>
 __device__ __forceinline__ void row_store(const float (&x)[4], const __amdgpu_buffer_rsrc_t& rsrc, int voff, int soff, __bf16*) {
   typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
   const bf16x4 v = {(__bf16)x[0], (__bf16)x[1], (__bf16)x[2], (__bf16)x[3]};
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc, voff, soff, 0);
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc, voff, soff, kPolicy);
 }
 
 // fn(values of one run of a row, per-lane offset, scalar offset), for every run of the tile that lies inside it; a
@@ -586,7 +598,7 @@ __device__ __forceinline__ void for_rows(const TileAddr<T, OutT, S, NI>& at, Acc
 // latency (H = 4096 over 151936 entries, loads of half a block row at a time -> these: 256 tokens 1.24 -> 0.96 ms = 5.2 TB/s
 // over reads and writes, 1024 tokens 1.76 -> 1.48, 3520 tokens 3.55 -> 3.33).  A fourth block row ahead does not fit
 // the registers.
-template <typename T, Side S, int NI, int kAhead = 3>
+template <typename T, Side S, int NI, int kPolicy, int kAhead = 3>
 struct RowLoads {
   using Tile = OutTile<T, S, NI>;
   static constexpr int kSlots = kAhead + 1;
@@ -599,7 +611,7 @@ struct RowLoads {
       for (int r = 0; r < 4; ++r) {
         const int dm = Tile::a_off(i, r);
         x[i % kSlots][g][r] =
-            __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(at.rsrc, at.row_voff(dm, g), dm * at.row_bytes, 0));
+            __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(at.rsrc, at.row_voff(dm, g), dm * at.row_bytes, kPolicy));
       }
     Tile::fence();
   }
@@ -624,28 +636,29 @@ struct RowLoads {
 
 // Output tile from the accumulators: C = acc (the accumulators already hold C's previous contents
 // when the GEMM adds to it, see gemm_init_tile), or the fp32 partial of K range `ks`.
-template <typename T, typename OutT, Side S, int NI>
+template <typename T, typename OutT, Side S, int NI, int kPolicy>
 __device__ __forceinline__ void gemm_store_tile(const GemmParams& p, typename OutTile<T, S, NI>::Acc& acc, int m0, int n0,
                                                 int a_rows, int b_rows, int ks) {
   if (p.k_split > 1) {
     const TileAddr<T, float, S, NI> at(p.partial + (int64_t)ks * p.M * p.N, kMContig<S> ? p.M : p.N, m0, n0, a_rows, b_rows);
-    for_rows<T, float, S, NI>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (float*)nullptr); });
+    for_rows<T, float, S, NI>(at, acc, [&](auto& x, int voff, int soff) { row_store<0>(x, at.rsrc, voff, soff, (float*)nullptr); });
     return;
   }
   const TileAddr<T, OutT, S, NI> at(static_cast<OutT*>(p.C), p.ldc, m0, n0, a_rows, b_rows, p.order, p.total);
-  for_rows<T, OutT, S, NI>(at, acc, [&](auto& x, int voff, int soff) { row_store(x, at.rsrc, voff, soff, (OutT*)nullptr); });
+  for_rows<T, OutT, S, NI>(at, acc, [&](auto& x, int voff, int soff) { row_store<kPolicy>(x, at.rsrc, voff, soff, (OutT*)nullptr); });
 }
 
 // Work item = (walk, fixed tile) when n_walk > 0: the workgroup keeps one operand's tile (A's m tile
 // when C is [n][m], B's n tile when C is [m][n]) and walks a contiguous run of tiles of the other, so the
 // K loops stream into each other (the next tile's first slabs are requested while the current tile
 // finishes and is stored).  Otherwise work item = (K range, m tile, n tile), one K loop per workgroup.
-// kAdds: C is added to, and one workgroup owns the whole K range of a tile (an argument in its place had fp32 tiles spill
-// 400 registers).
-template <typename T, typename OutT, Side S, int NI, bool kAdds, typename G>
+// kC: whether C is added to (see Adds), where one workgroup owns the whole K range of a tile (an argument in its place had fp32 tiles
+// spill 400 registers).
+template <typename T, typename OutT, Side S, int NI, Adds kC, typename G>
 __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p, typename G::Params guest_of) {
   using Tile = OutTile<T, S, NI>;
-  constexpr bool kMC = kMContig<S>;
+  constexpr bool kMC = kMContig<S>, kLoadsC = kC != kOverwrites;
+  constexpr int kPolicy = kC == kAddsAround ? kNonTemporal : 0;
   constexpr int E = Tile::kSlabK;
   constexpr int64_t kSlabElems = (int64_t)kBlockRows * E;   // elements of a K-blocked block's slab, and of a 256-wide row of units
   extern __shared__ __align__(16) char lds[];
@@ -690,15 +703,15 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p, typ
   auto rows_of = [](int total, int tile, int width) { const int left = total - tile * width; return left < width ? left : width; };
   // Accumulators before a tile's K loop: zeros, or - when the GEMM adds to C and one workgroup owns the whole K range of
   // the tile - the tile's current contents, which leaves the epilogue a pure store.
-  static_assert(!kAdds || (!kMC && sizeof(OutT) == 4), "only an fp32 dW is ever added to");
-  typedef RowLoads<T, S, NI, Tile::kSplit ? 1 : 3> Loads;
+  static_assert(!kLoadsC || (!kMC && sizeof(OutT) == 4), "only an fp32 dW is ever added to");
+  typedef RowLoads<T, S, NI, kPolicy, Tile::kSplit ? 1 : 3> Loads;
   auto c_tile = [&](int m_tile) {
     return typename Loads::At(static_cast<float*>(p.C), p.ldc, m_tile * 256, nt * Tile::BN, rows_of(p.M, m_tile, 256),
                               rows_of(p.N, nt, Tile::BN));
   };
   typename Tile::Acc acc;
   Loads loads;
-  if constexpr (kAdds) loads.begin(c_tile(mt));
+  if constexpr (kLoadsC) loads.begin(c_tile(mt));
   Tile core;
   bool again = false;      // the tile before was computed twice: nothing of this one has been requested
   for (int k = 0; k < count; ++k) {
@@ -706,7 +719,7 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p, typ
     const int a_rows = rows_of(p.M, mt, 256), b_rows = rows_of(p.N, nt, Tile::BN);
     const auto op_a = operand_a(mt, a_rows);
     const auto op_b = operand_b(nt, b_rows);
-    if constexpr (kAdds) loads.finish(c_tile(mt), acc);
+    if constexpr (kLoadsC) loads.finish(c_tile(mt), acc);
     else Tile::zero(acc);
     [[maybe_unused]] std::conditional_t<G::kHosts, G, int> guest;
     if constexpr (G::kHosts) guest.place(guest_of, whole_item);     // one tile per workgroup
@@ -724,8 +737,8 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p, typ
     }
     if constexpr (Tile::kSplit) {
       again = core.redo(acc, op_a, op_b, nslab, lds, [&] {
-        if constexpr (kAdds) {
-          RowLoads<T, S, NI, 0> old;
+        if constexpr (kLoadsC) {
+          RowLoads<T, S, NI, kPolicy, 0> old;
           old.finish(c_tile(mt), acc);
         } else {
           Tile::zero(acc);
@@ -733,10 +746,10 @@ __global__ __launch_bounds__(kHeadThreads, 1) void gemm_kernel(GemmParams p, typ
       });
     }
     if (!stream || k + 1 == count) Tile::finish();
-    if constexpr (kAdds) {
+    if constexpr (kLoadsC) {
       if (k + 1 < count) loads.begin(c_tile(mt + 1));
     }
-    gemm_store_tile<T, OutT, S, NI>(p, acc, m0, n0, a_rows, b_rows, ks);
+    gemm_store_tile<T, OutT, S, NI, kPolicy>(p, acc, m0, n0, a_rows, b_rows, ks);
     if (kMC) ++nt; else ++mt;
   }
 }
@@ -1045,9 +1058,11 @@ static int launch_gemm_one(const GemmIn& in, int M, int N, int K, void* C, int64
   };
   int rc;
   if constexpr (!kMC && sizeof(OutT) == 4)
-    rc = accumulate && g.k_split == 1 ? launch(&gemm_kernel<T, OutT, S, NI, true, NoDz>) : launch(&gemm_kernel<T, OutT, S, NI, false, NoDz>);
+    rc = !accumulate || g.k_split > 1                                ? launch(&gemm_kernel<T, OutT, S, NI, kOverwrites, NoDz>)
+         : (int64_t)M * N * (int64_t)sizeof(OutT) > kAddsAroundBytes ? launch(&gemm_kernel<T, OutT, S, NI, kAddsAround, NoDz>)
+                                                                     : launch(&gemm_kernel<T, OutT, S, NI, kAdds, NoDz>);
   else
-    rc = launch(&gemm_kernel<T, OutT, S, NI, false, G>);
+    rc = launch(&gemm_kernel<T, OutT, S, NI, kOverwrites, G>);
   if (rc || g.k_split == 1) return rc;
   return launch_splitk_reduce<OutT>(partial, g.k_split, kMC ? N : M, kMC ? M : N, static_cast<OutT*>(C), ldc, accumulate,
                                     rows.order, stream);

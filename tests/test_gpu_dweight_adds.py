@@ -6,10 +6,11 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# one workgroup per tile; walks over many vocabulary tiles with a ragged last row and column tile; walks and a K-split tail behind them
+# one workgroup per tile; walks over many vocabulary tiles with a ragged last row and column tile; walks and a K-split tail behind them;
+# the last dW (H = 960) that is added to through the last-level cache and the first that goes around it
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T,H,V", [(1, 64, 3), (130, 192, 257), (200, 960, 66049), (70, 1024, 65537), (640, 1088, 70001),
-                                   (1300, 960, 66049)])
+                                   (1300, 960, 66049), (500, 320, 40000), (70, 960, 30583), (70, 960, 30584)])
 def test_added_equals_overwritten_plus_old(dev, dtype, T, H, V):
     """The same products are summed in the same order, from the old value instead of from 0: each of at most T additions rounds
     to 2^-24 of a partial sum, which |old| + sum over t of |g_t| max|h_t| bounds."""
