@@ -185,6 +185,10 @@ __global__ __launch_bounds__(256) void transpose_block_kernel(TransposeParams<T>
 // d(logits) from kept logits: in place, or into the operands of dW that the caller keeps.  HBM-bound: reads and writes the
 // chunk once.  A thread owns one 16-byte piece of one or two tokens in every unit that its workgroup walks: their
 // coefficients stay in registers, the loads of kAhead units are in flight together, and a wave's access is one kilobyte.
+// The units are walked from the vocabulary's end on, whose logits a forward of several rounds has written last, which the last-level
+// cache still has, and dhidden, which begins at the other end, finds there what was written last here.  The pass and dhidden
+// behind the forward, us: 143 rows at H = 1024, V = 32000 40.0 -> 38.4, 1064 at 2048, V = 151936 669 -> 661; loss dict of 6680 tokens
+// at H = 2048 and its backward 8.78 -> 8.74 ms, a step of 200 tokens 148 -> 147 us.  Loads or stores around the cache: nothing.
 // The last workgroups of the launch write hidden^T, dW's other operand, which took a launch of 5 to 12 us of its own.
 // 12126 rows of the 152k vocabulary: 2.25 -> 1.49 ms, 32768 rows 5.92 -> 3.57 ms (5.6 TB/s), against a pass that also wrote the
 // transpose.
@@ -248,15 +252,15 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams<T> p) {
   constexpr int VEC = 16 / (int)sizeof(T);          // elements per 16-byte piece
   constexpr int kRows = E / 32;                     // tokens per thread
   constexpr int kAhead = 4;                         // units in flight
-  // the same for the whole workgroup: its row of units and first unit, or its square of hidden states
-  int item = blockIdx.x, unit_row, unit, end = p.whole, step = p.n_step;
+  // the same for the whole workgroup: its row of units, its last unit and the least it may reach, or its square of hidden states
+  int item = blockIdx.x, unit_row, unit, least = 0, step = p.n_step;
   if (item < p.row_units * p.n_step) {
     unit_row = p.row0 + item % p.row_units;
-    unit = item / p.row_units;
+    unit = p.whole - 1 - item / p.row_units;
   } else if ((item -= p.row_units * p.n_step) < p.n_edge) {
     unit_row = item;
-    unit = p.whole;
-    end = p.n_units;
+    unit = p.n_units - 1;
+    least = p.whole;
     step = 1;
   } else {
     item -= p.n_edge;
@@ -270,19 +274,19 @@ __global__ __launch_bounds__(256) void dz_from_z_kernel(DzFromZParams<T> p) {
   const int at = row * kRowBytes + q * 16;          // byte of this thread's first piece within a unit
   const char* z = static_cast<const char*>(p.z) + (int64_t)unit_row * p.z_kslab * (E * kRowBytes) + at;
   char* dz = static_cast<char*>(p.dz) + (int64_t)unit_row * p.dz_kslab * (E * kRowBytes) + at;
-  for (int k0 = unit; k0 < end; k0 += kAhead * step) {
+  for (int k0 = unit; k0 >= least; k0 -= kAhead * step) {
     u32x4 raw[kAhead][kRows];
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
-      const int ks = k0 + u * step < end ? k0 + u * step : k0;
+      const int ks = k0 - u * step >= least ? k0 - u * step : k0;
 #pragma unroll
       for (int h = 0; h < kRows; ++h)
         raw[u][h] = *reinterpret_cast<const u32x4*>(z + (int64_t)ks * (E * kRowBytes) + h * 32 * kRowBytes);
     }
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
-      const int ks = k0 + u * step;
-      if (ks >= end) break;
+      const int ks = k0 - u * step;
+      if (ks < least) break;
       const int v = ks * E + q * VEC;
 #pragma unroll
       for (int h = 0; h < kRows; ++h) {
