@@ -32,7 +32,7 @@ from chatlearn_amd._lib import LOSS_GRPO, LOSS_GSPO  # noqa: E402
 from chatlearn_amd.fused import default_keep_rows, grpo_head_step, head_step_chunks  # noqa: E402
 
 PEAK_BF16_TFLOPS = 2500.0   # MI355X dense bf16 MFMA
-PEAK_F32_TFLOPS = 157.3
+PEAK_F32_TFLOPS = 2500.0 / 6     # fp32 operands as three 16-bit parts each: six of the bf16 matrix products per product
 PEAK_HBM_GBS = 8000.0
 
 # HBM-side bytes per forward launch are read from this summary of two rocprofv3 --pmc runs (FETCH_SIZE, WRITE_SIZE,
@@ -324,7 +324,8 @@ def gemm_kernels(w, keep, reps=3):
     """The three GEMM-shaped kernels on the largest token chunk of the step, each against the matrix-core peak
     on the rows it ran: the forward launch timed directly; dhidden and dW as the differences between the
     whole backward of the chunk and the backward without that output (what remains in either is the
-    d(logits) pass and a transpose)."""
+    d(logits) pass and a transpose; dhidden's launches take over a part of that pass, so its figure is what it adds
+    to the pass by itself)."""
     cfg = w.cfg
     chunks = head_step_chunks(w.T, keep, cfg.loss == "gspo", w.cu_host, w.mask_host, shape=(cfg.H, cfg.V), dtype=cfg.dtype)
     lo, hi = max(chunks, key=lambda c: c[1] - c[0])
