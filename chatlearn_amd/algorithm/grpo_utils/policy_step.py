@@ -149,14 +149,20 @@ class PolicyStep:
         """The shifted host masks of micro-batches that may be processed one by one while the device works on the ones before:
         what their processing would refuse has to be refused before any gradient is made, so only text samples
         without a mask of their own whose lengths are in order.  None for others."""
+        first = micro_batches[0][0] if micro_batches and micro_batches[0] else {}
+        tensors = ("all_tokens", "old_logprobs", "ref_logprobs")
+
+        def plain(d):
+            return set(d) == set(first) and {k for k, v in d.items() if isinstance(v, torch.Tensor)} == set(tensors) and \
+                all(d[k].shape == d["all_tokens"].shape and d[k].dim() == 1 and d[k].device == first[k].device for k in tensors)
+
+        if self.model_type == "vlm" or "position_ids" in first or "loss_mask" in first or not all(plain(d) for mb in micro_batches for d in mb):
+            return None
         masks = []
         for mb in micro_batches:
             plen, rlen = ([int(d[key]) for d in mb] for key in ("prompt_token_length", "response_token_length"))
             width = max((d["all_tokens"].shape[0] for d in mb), default=0)
-            if self.model_type == "vlm" or not mb or any("loss_mask" in d or "position_ids" in d or d["all_tokens"].dim() != 1 for d in mb) \
-                    or any(p < 0 or r < 0 or p + r > width for p, r in zip(plen, rlen)) \
-                    or any(set(d) != set(mb[0]) or any(d[k].shape != d["all_tokens"].shape for k in ("old_logprobs", "ref_logprobs"))
-                           for d in mb):
+            if not mb or any(p < 0 or r < 0 or p + r > width for p, r in zip(plen, rlen)):
                 return None
             masks.append(self._shifted_mask_host(None, plen, rlen, width))
         return masks

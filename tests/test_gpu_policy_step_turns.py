@@ -76,3 +76,14 @@ def test_a_length_beyond_the_sample_is_refused_first(dev):
     with pytest.raises(ValueError):
         step.train_step(data)
     assert not hiddens and weight.grad is None
+
+
+@pytest.mark.parametrize("change", [lambda d: d.pop("advantages"), lambda d: d.update(extra=torch.ones(3)),
+                                    lambda d: d.update(old_logprobs=d["old_logprobs"][:-1]),
+                                    lambda d: d.update(ref_logprobs=d["ref_logprobs"].tolist())])
+def test_samples_that_differ_are_processed_in_front(dev, change):
+    step, _, _ = _step(dev, False)
+    data = _samples(5, 3, 1031)
+    assert step._masks_ahead(step._split(data, True)) is not None
+    change(data[-1])
+    assert step._masks_ahead(step._split(data, True)) is None
